@@ -11,18 +11,19 @@ from a hipGraph) over the whole state, which stays resident in HBM.
 
 Prints one JSON line:
   value          site*dir RK4 updates/s = nx*nz*nv*K / wall(K steps)
-  roofline       for the dominant kernel (RK4 stage 2): algorithmic bytes per
-                 launch (4 state passes x 8 fields x sizeof(real) per update)
-                 / its average duration from HIP events, against 8 TB/s
-  step_roofline  the same for a whole step (12 passes: 768 B per update in
-                 FP64), plus vs_16pass_ceiling = updates/s over 8 TB/s / 1024 B
+  roofline       for the dominant kernel (RK4 stages 3+4; stage 2 where a step
+                 is not made of stage pairs): algorithmic bytes per launch (4
+                 state passes x 8 fields x sizeof(real) per update) / its
+                 average duration from HIP events, against 8 TB/s
+  step_roofline  the same for a whole step (7 passes: 448 B per update in
+                 FP64; 12 where it is not made of stage pairs), plus vs_16pass_ceiling = updates/s over 8 TB/s / 1024 B
                  (FP64; 512 B FP32), the ceiling of the 16-pass RK4 streaming
                  in which the per-update targets are stated
   fp32           (default box run) the same workload in the FP32 form: value,
                  speed-up over FP64, its stage-2 roofline
   batched        (default box run) the 64-run batched scan (FP32), 20 steps:
                  aggregate updates/s together and one after another, the
-                 speed-up, and each mode's HBM fraction at 384 B per update
+                 speed-up, and each mode's HBM fraction at 224 B per update
   served         (default box run) the run server, FP32: 20 s of Poisson
                  0.35/s arrivals of runs drawn like the batched scan's (grids
                  64..384 squared, steps U[100,1000]): p50/p99 request latency
@@ -55,6 +56,8 @@ HBM_PEAK_GBS = 8000.0
 # state passes per update of each stage (read + write of the 8 fields):
 # S1 u -> Y2; S2 Y2, u -> Y3, A; S3 Y3, u -> Y4; S4 Y4, A -> u'
 STAGE_PASSES = (2, 4, 3, 3)
+# the same in stage pairs: u -> Y3, A; Y3, u, A -> u'
+PAIR_PASSES = (3, 0, 4, 0)
 
 
 def parse():
@@ -110,13 +113,13 @@ TRAFFIC_FILE = "profiles/stage_traffic.json"
 
 
 def traffic_from_profiles(precision):
-    """HBM bytes per stage-2 launch measured with rocprofv3 --pmc (FETCH_SIZE +
-    WRITE_SIZE, scaled by a copy-kernel calibration), if recorded."""
+    """HBM bytes per stages-3+4 launch measured with rocprofv3 --pmc (FETCH_SIZE
+    + WRITE_SIZE, scaled by a copy-kernel calibration), if recorded."""
     path = os.path.join(ROOT, TRAFFIC_FILE)
     try:
         with open(path) as f:
             d = json.load(f)
-        return d.get(f"fp{precision}", {}).get("stage2_bytes")
+        return d.get(f"fp{precision}", {}).get("pair2_bytes")
     except Exception:
         return None
 
@@ -447,7 +450,6 @@ def measure_box(N, a, precision):
     esize = 8 if precision == 64 else 4
     three = a.nflavor == 3
     nvar = 18 if three else 8
-    passes = STAGE_PASSES
     pmo = 1.0 if three else 0.0
     column = a.shape == "column"
     if column:   # the 1-D open column of the precision workload
@@ -471,7 +473,7 @@ def measure_box(N, a, precision):
 
     g.step_rk4(a.warmup)
     g.synchronize()
-    # per-stage kernel durations from HIP events around each stage kernel on
+    # durations from HIP events around each stage (or stage-pair) kernel on
     # the library's stream, right before the timed steps
     stage_ms = g.profile_stages(3)
     t0 = time.perf_counter()
@@ -484,8 +486,12 @@ def measure_box(N, a, precision):
     g.close()
 
     value = upd * a.steps / wall
-    s2_bytes = STAGE_PASSES[1] * nvar * esize * upd
-    s2_gbs = s2_bytes / (stage_ms[1] * 1e-3) / 1e9
+    # the largest kernel: stages 3+4 where a step is two stage pairs, else stage 2
+    pairs = stage_ms[1] == 0
+    passes = PAIR_PASSES if pairs else STAGE_PASSES
+    main = 2 if pairs else 1
+    s2_bytes = passes[main] * nvar * esize * upd
+    s2_gbs = s2_bytes / (stage_ms[main] * 1e-3) / 1e9
     step_bytes = sum(passes) * nvar * esize * upd
     step_gbs = step_bytes / (wall / a.steps) / 1e9
     traffic = None if (three or column) else traffic_from_profiles(precision)
@@ -512,7 +518,7 @@ def measure_box(N, a, precision):
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": "k_stage3z stage 2" if three else "k_stage stage 2",
+            "kernel": "k_stage3z stage 2" if three else ("k_pair stages 3+4" if pairs else "k_stage stage 2"),
             "achieved": s2_gbs,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
@@ -521,7 +527,7 @@ def measure_box(N, a, precision):
             "traffic_source": (f"{TRAFFIC_FILE}: rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE of this workload, "
                                "scaled by a plain copy's readings; not measured in this run") if traffic else None,
             "algorithmic_bytes_per_launch": s2_bytes,
-            "launch_ms": stage_ms[1],
+            "launch_ms": stage_ms[main],
         },
         "step_roofline": {
             "achieved": step_gbs,
@@ -540,7 +546,7 @@ def batched_leg(N, a, runs=64, steps=20):
     """The batched-scan workload (64 uneven runs, FP32) for a few steps:
     aggregate updates/s stepped all together (at the autotuned z-segment
     length and launch form; the other launch form is timed too) and one
-    after another, and each mode's HBM fraction at 384 B per FP32 update
+    after another, and each mode's HBM fraction at 224 B per FP32 update
     (12 passes x 8 fields)."""
     import numpy as np
     rng = np.random.default_rng(7)
@@ -578,7 +584,7 @@ def batched_leg(N, a, runs=64, steps=20):
     b.close()
     for g in sims:
         g.close()
-    bpu = 12 * 8 * 4
+    bpu = sum(PAIR_PASSES) * 8 * 4
     v_bat, v_seq = upd * steps / t_bat, upd * steps / t_seq
     return {
         "value": v_bat, "unit": "updates/s", "sequential_value": v_seq, "speedup_vs_sequential": t_seq / t_bat,

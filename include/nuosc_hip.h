@@ -245,14 +245,17 @@ int nuosc_last_step_ms(nuosc_sim* sim, double* ms);
 
 /* Measurement helper: run nsteps RK4 steps eagerly with a pair of HIP events
  * around each of the four stage kernels (on the handle's stream) and return
- * the average duration of each stage kernel in stage_ms[4] (ms).  Advances
- * the state and phy_time like nuosc_step_rk4. */
+ * the average duration of each stage kernel in stage_ms[4] (ms).  Handles
+ * that step in stage pairs (2 flavours, periodic, the default discretisation)
+ * report the kernel of stages 1+2 in stage_ms[0], that of stages 3+4 in
+ * stage_ms[2] and zeros.  Advances the state and phy_time like
+ * nuosc_step_rk4. */
 int nuosc_profile_stages(nuosc_sim* sim, int nsteps, double* stage_ms);
 
 /* Stage-kernel decomposition (no reference counterpart).  Each wavefront
  * marches along z over a segment of zlen sites; nuosc_autotune times RK4
- * stages 1-3 (with their boundary fills and moment totals) on this handle's
- * own grid for zlen in {8, ..., 256}, the candidates in turn for trials
+ * stages 1-3 (with their boundary fills and moment totals), or the two stage
+ * pairs, on this handle's own grid for zlen in {8, ..., 256}, the candidates in turn for trials
  * rounds after a warm-up round, keeps each candidate's fastest time and
  * selects the best.  Call it at a step boundary: it overwrites only the RK4
  * scratch copies, never the state.  Results are cached per (nx, nz, nv,
@@ -287,14 +290,14 @@ const char* nuosc_batch_last_error(const nuosc_batch* batch);
 /* z-segment length of the batched stage kernels, shared by every member
  * (default 64, capped at each member's nz; 0 = each member's own plan).  A
  * common length gives every block of a batched launch the same work.
- * batch_autotune times the batched stage-1 kernel for zlen in {16, ..., 256}
+ * batch_autotune times the batched stages-1+2 kernel for zlen in {16, ..., 256}
  * and both launch forms (trials launches each, the fastest kept; only the
  * RK4 scratch copies are written) and keeps the best pair (the launch form
  * it chose: nuosc_batch_get_launch).  Results do not depend on zlen or the
  * launch form. */
 int nuosc_batch_set_zlen(nuosc_batch* batch, int zlen);
 int nuosc_batch_autotune(nuosc_batch* batch, int trials, int* best_zlen, double* best_ms);
-/* Launch form of the batched stage kernels: NUOSC_BATCH_GRID (default: one
+/* Launch form of the batched stage-pair kernels: NUOSC_BATCH_GRID (default: one
  * block per logical block of every member) or NUOSC_BATCH_PERSISTENT (one
  * grid of as many blocks as the GPU holds at once, drawing logical blocks
  * from per-XCD work queues until they are empty).  get_launch returns the

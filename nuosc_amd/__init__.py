@@ -318,7 +318,8 @@ class NuOsc:
         return ms.value
 
     def profile_stages(self, nsteps=2):
-        """Average device time (ms) of each of the four stage kernels."""
+        """Average device time (ms) of each of the four stage kernels (stage
+        pairs: of stages 1+2 and 3+4 at indices 0 and 2)."""
         ms = np.zeros(4)
         self._check(lib().nuosc_profile_stages(self._h, int(nsteps), _ptr(ms)))
         return ms
@@ -430,7 +431,7 @@ class Batch:
 
     def autotune(self, trials=2):
         """Pick the fastest shared z-segment length and launch form; returns
-        (zlen, stage-1 ms); the form chosen is `launch`."""
+        (zlen, stages-1+2 ms); the form chosen is `launch`."""
         z, ms = C.c_int(), C.c_double()
         self._check(lib().nuosc_batch_autotune(self._h, int(trials), C.byref(z), C.byref(ms)))
         return z.value, ms.value

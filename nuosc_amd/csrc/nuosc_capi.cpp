@@ -7,6 +7,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -48,6 +49,7 @@ struct nuosc_sim {
     double* mom_u = nullptr;     // totals of u, yA, yB (3 flavours: mom_u the stage input's, mom_a calRHS scratch)
     double* mom_a = nullptr;
     double* mom_b = nullptr;
+    double* pair_tot = nullptr;  // direction sums of u (handles that step in stage pairs)
     double* d_vgrid = nullptr;  // vx | vy | vz | vw
     double* d_g0 = nullptr;     // G0 | G0b
     double* d_part = nullptr;
@@ -59,11 +61,16 @@ struct nuosc_sim {
     long long device_bytes = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t graph_exec = nullptr;
-    hipGraph_t graph3 = nullptr;          // SSP-RK3 step
-    hipGraphExec_t graph3_exec = nullptr;
-    bool have_moments = false;
+    // captured steps, [RK4 or SSP-RK3][flip]
+    hipGraph_t graph[2][2] = {};
+    hipGraphExec_t graph_exec[2][2] = {};
+    bool have_moments = false;            // mom_u holds the moments of u
+    bool have_sums = false;               // pair_tot holds the direction sums of u
+    // RK4 in stage pairs: the new state goes to st_ya, which then becomes
+    // st_u; flip counts those exchanges (mod 2)
+    bool pairs = false;
+    int flip = 0;
+    int pair_zlen = 0;                    // z-segment length of the pair kernels
     int steps_in_last_call = 0;
     Geometry geo{};
     Physics ph{};
@@ -117,16 +124,28 @@ CopyLayout copy_layout(int nx, int nz, int nzs, int nvp, int nch, int esize, int
     return CopyLayout{gq.srec, gq.xrow, 4 * copy_elems(gq), true};
 }
 
+// RK4 in stage pairs: 2 flavours, periodic box, the default discretisation
+bool steps_in_pairs(const nuosc_config& c) {
+    return c.nflavor != 3 && c.bc == NUOSC_BC_PERIODIC && c.ko_order != 5 && c.adv == NUOSC_ADV_CFD4;
+}
+// doubles of the partial moment records (with the spare x row's) and of the
+// partial direction sums, which share one buffer
+long long part_doubles(long long nx, long long nz, long long nv, long long nch, int nf, bool pairs) {
+    if (nf == kNVar3) return nx * nz * ((nv + 63) / 64) * kNMom3;
+    const long long stage = (nx + 1) * nz * nch * kMomRec;
+    return pairs ? std::max(stage, nx * nz * nch * kPairRec) : stage;
+}
+
 void drop_graph(nuosc_sim* s) {
     // (teardown: errors of the destroy calls leave nothing to recover)
-    if (s->graph_exec) (void)hipGraphExecDestroy(s->graph_exec);
-    if (s->graph) (void)hipGraphDestroy(s->graph);
-    if (s->graph3_exec) (void)hipGraphExecDestroy(s->graph3_exec);
-    if (s->graph3) (void)hipGraphDestroy(s->graph3);
-    s->graph_exec = nullptr;
-    s->graph = nullptr;
-    s->graph3_exec = nullptr;
-    s->graph3 = nullptr;
+    for (int k = 0; k < 4; ++k) {
+        hipGraphExec_t& x = s->graph_exec[k / 2][k % 2];
+        hipGraph_t& g = s->graph[k / 2][k % 2];
+        if (x) (void)hipGraphExecDestroy(x);
+        if (g) (void)hipGraphDestroy(g);
+        x = nullptr;
+        g = nullptr;
+    }
 }
 
 int ensure_tmp(nuosc_sim* s, size_t bytes) {
@@ -251,6 +270,40 @@ int enqueue_step3_srk3(nuosc_sim* s) {
     return NUOSC_OK;
 }
 
+PairBuffers pair_buffers(const nuosc_sim* s) {
+    return PairBuffers{s->st_u, s->st_w,   s->st_yb,  s->st_ya,   s->mom_u,
+                       s->mom_b, s->mom_a, s->mom_part, s->pair_tot};
+}
+
+// direction sums of the state y (partial records, then totals)
+template <typename T>
+hipError_t enqueue_sums(nuosc_sim* s, const T* y) {
+    const hipError_t e = launch_pair_sums<T>(s->geo, y, s->mom_part, s->stream);
+    return e != hipSuccess ? e : launch_pair_totals(s->geo, sizeof(T) == 4, pair_buffers(s), s->stream);
+}
+
+// One RK4 step in two stage pairs (nuosc_pair.hip) from st_u into st_ya; the
+// caller exchanges the two.  Events ev[0], ev[1] bracket the first pair's
+// kernel alone, ev[4], ev[5] the second's.
+template <typename T>
+int enqueue_step_pairs(nuosc_sim* s, hipEvent_t* ev = nullptr) {
+    const PairBuffers b = pair_buffers(s);
+    const bool comp = sizeof(T) == 4;
+    for (int pair = 1; pair <= 2; ++pair) {
+        HIPCK(s, launch_pair_predict(pair, s->geo, s->ph, b, s->dt, s->stream));
+        if (ev) HIPCK(s, hipEventRecord(ev[4 * pair - 4], s->stream));
+        HIPCK(s, launch_pair<T>(pair, s->geo, s->ph, s->pair_zlen, b, s->dt, s->stream));
+        if (ev) HIPCK(s, hipEventRecord(ev[4 * pair - 3], s->stream));
+        if (pair == 2 && s->cfg.renorm) {
+            T* u = static_cast<T*>(b.unew);
+            HIPCK(s, launch_renorm<T>(s->geo, u, s->d_g0, s->d_g0 + s->nv, s->stream));
+            HIPCK(s, launch_pair_sums<T>(s->geo, u, b.part, s->stream));
+        }
+        HIPCK(s, launch_pair_totals(s->geo, comp, b, s->stream));
+    }
+    return NUOSC_OK;
+}
+
 // One RK4 step: the four stage launches (+ optional renormalisation).  With
 // ev != nullptr events ev[2k], ev[2k+1] bracket the stage-(k+1) kernel alone
 // (not its boundary fill or moment-total pass).
@@ -367,6 +420,71 @@ int refresh_moments(nuosc_sim* s) {
     return NUOSC_OK;
 }
 
+// z-segment length of the stage kernels (of the stage pairs too)
+void set_plan(nuosc_sim* s, int zlen) {
+    s->plan = plan_stage_zlen(s->geo, zlen);
+    if (s->pairs) s->pair_zlen = s->plan.zlen;
+}
+
+// what an RK4 step needs of the state u: its direction sums (stage pairs) or
+// its moments
+int refresh_rk4(nuosc_sim* s) {
+    if (!s->pairs) return refresh_moments(s);
+    if (is64(s)) HIPCK(s, enqueue_sums<double>(s, (double*)s->st_u));
+    else HIPCK(s, enqueue_sums<float>(s, (float*)s->st_u));
+    s->have_sums = true;
+    return NUOSC_OK;
+}
+bool rk4_ready(const nuosc_sim* s) { return s->pairs ? s->have_sums : s->have_moments; }
+
+// the stage pairs leave the new state in st_ya
+void state_stepped(nuosc_sim* s) {
+    std::swap(s->st_u, s->st_ya);
+    s->flip ^= 1;
+    s->have_moments = false;
+}
+
+// nsteps steps on the handle's stream, replayed from a captured graph if the
+// handle uses them
+enum StepKind { kRk4 = 0, kSrk3 = 1 };
+int run_steps(nuosc_sim* s, StepKind kind, int nsteps) {
+    const bool pairs = kind == kRk4 && s->pairs;
+    auto enqueue = [&] {
+        if (pairs) return is64(s) ? enqueue_step_pairs<double>(s) : enqueue_step_pairs<float>(s);
+        if (kind == kRk4) return is64(s) ? enqueue_step<double>(s) : enqueue_step<float>(s);
+        return is64(s) ? enqueue_step_srk3<double>(s) : enqueue_step_srk3<float>(s);
+    };
+    HIPCK(s, hipEventRecord(s->ev0, s->stream));
+    for (int n = 0; n < nsteps; ++n) {
+        if (s->cfg.use_graph) {
+            hipGraphExec_t& exec = s->graph_exec[kind][s->flip];
+            if (!exec) {
+                HIPCK(s, hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
+                const int rc = enqueue();
+                hipGraph_t gr = nullptr;
+                const hipError_t e = hipStreamEndCapture(s->stream, &gr);
+                if (rc) {
+                    if (gr) (void)hipGraphDestroy(gr);
+                    return rc;
+                }
+                if (e != hipSuccess) return fail(s, NUOSC_EHIP, std::string("graph capture: ") + hipGetErrorString(e));
+                s->graph[kind][s->flip] = gr;
+                HIPCK(s, hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0));
+            }
+            HIPCK(s, hipGraphLaunch(exec, s->stream));
+        } else {
+            const int rc = enqueue();
+            if (rc) return rc;
+        }
+        if (pairs) state_stepped(s);
+        else s->have_sums = false;
+        s->phy_time += s->dt;   // accumulated, as nuosc_class.cpp:423, 448
+    }
+    HIPCK(s, hipEventRecord(s->ev1, s->stream));
+    s->steps_in_last_call = nsteps;
+    return NUOSC_OK;
+}
+
 // Device analysis sums -> host (kNAna doubles).
 int analysis_sums(nuosc_sim* s, double* h) {
     if (is64(s))
@@ -410,8 +528,15 @@ int check_field(nuosc_sim* s, int f) {
 
 // RK4 stages 1-3 with their boundary fills and moment totals: they write only
 // the scratch copies A (w), yA, yB and the scratch moment records, never u.
+// (Stage pairs: both of them, which write st_ya, A, Y3 and the scratch records
+// only, with whatever the inner moments hold: their values do not matter here.)
 template <typename T>
 hipError_t enqueue_scratch_stages(nuosc_sim* s) {
+    if (s->pairs) {
+        const PairBuffers b = pair_buffers(s);
+        const hipError_t e1 = launch_pair<T>(1, s->geo, s->ph, s->pair_zlen, b, s->dt, s->stream);
+        return e1 != hipSuccess ? e1 : launch_pair<T>(2, s->geo, s->ph, s->pair_zlen, b, s->dt, s->stream);
+    }
     const double dt = s->dt, c2 = dt / 2;
     const Geometry& g = s->geo;
     T* u = static_cast<T*>(s->st_u);
@@ -560,8 +685,8 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
 
     const size_t state_bytes = (size_t)s->state_elems * s->esize;
     const bool three = s->nf == kNVar3;
-    const size_t part_bytes = three ? (size_t)s->nx * s->nz * ((s->nv + 63) / 64) * kNMom3 * sizeof(double)
-                                    : (size_t)(s->nx + 1) * s->nz * s->nch * kMomRec * sizeof(double);
+    s->pairs = steps_in_pairs(c);
+    const size_t part_bytes = (size_t)part_doubles(s->nx, s->nz, s->nv, s->nch, s->nf, s->pairs) * sizeof(double);
     const size_t mom_bytes = (size_t)s->nx * s->nz * (three ? kNMom3 : kMomStride) * sizeof(double);
     void** states[4] = {&s->st_u, &s->st_w, &s->st_ya, &s->st_yb};
     {
@@ -572,10 +697,11 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
             if (hipMemsetAsync(*p, 0, copy_bytes, s->stream) != hipSuccess) return bail(NUOSC_EHIP, "memset failed");
         }
     }
-    double** moms[4] = {&s->mom_part, &s->mom_u, &s->mom_a, &s->mom_b};
+    double** moms[5] = {&s->mom_part, &s->mom_u, &s->mom_a, &s->mom_b, &s->pair_tot};
     for (double** p : moms) {
         if (three && p == &s->mom_b) continue;   // 3 flavours: totals of the stage input and a calRHS scratch
-        const size_t b = (p == &s->mom_part) ? part_bytes : mom_bytes;
+        if (!s->pairs && p == &s->pair_tot) continue;
+        const size_t b = (p == &s->mom_part) ? part_bytes : (p == &s->pair_tot ? (size_t)s->nx * s->nz * kPairRec * sizeof(double) : mom_bytes);
         if (hipMalloc((void**)p, b) != hipSuccess) return bail(NUOSC_ENOMEM, "moment allocation failed");
         s->device_bytes += (long long)b;
         if (hipMemsetAsync(*p, 0, b, s->stream) != hipSuccess) return bail(NUOSC_EHIP, "memset failed");
@@ -634,6 +760,7 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, c.device) != hipSuccess) return bail(NUOSC_EHIP, "device query failed");
     s->plan = plan_stage(s->geo, prop.multiProcessorCount);
+    if (s->pairs) s->pair_zlen = plan_pair_zlen(s->geo, (int)s->esize, prop.multiProcessorCount);
     if (hipStreamSynchronize(s->stream) != hipSuccess) return bail(NUOSC_EHIP, "stream sync failed");
     s->G0h.assign(s->nv, 0.0);
     s->G0bh.assign(s->nv, 0.0);
@@ -651,7 +778,7 @@ int nuosc_destroy(nuosc_sim* s) {
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     drop_graph(s);
     void* bufs[] = {s->st_u, s->st_w, s->st_ya, s->st_yb, s->mom_part, s->mom_u, s->mom_a, s->mom_b,
-                    s->d_vgrid, s->d_g0, s->d_part, s->d_ana, s->d_tmp, s->d_time};
+                    s->pair_tot, s->d_vgrid, s->d_g0, s->d_part, s->d_ana, s->d_tmp, s->d_time};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
     if (s->ev0) (void)hipEventDestroy(s->ev0);
@@ -787,7 +914,8 @@ int nuosc_fill_init(nuosc_sim* s, int ipt, double alpha, double eps0, double sig
     drop_graph(s);
     rc = set_device_time(s);
     if (rc) return rc;
-    rc = refresh_moments(s);
+    s->have_moments = false;
+    rc = refresh_rk4(s);
     if (rc) return rc;
     HIPCK(s, hipStreamSynchronize(s->stream));
     return NUOSC_OK;
@@ -796,39 +924,11 @@ int nuosc_fill_init(nuosc_sim* s, int ipt, double alpha, double eps0, double sig
 int nuosc_step_rk4(nuosc_sim* s, int nsteps) {
     if (!s) return NUOSC_EINVAL;
     if (nsteps < 0) return fail(s, NUOSC_EINVAL, "negative step count");
-    if (!s->have_moments) {
-        int rc = refresh_moments(s);
+    if (!rk4_ready(s)) {
+        int rc = refresh_rk4(s);
         if (rc) return rc;
     }
-    HIPCK(s, hipEventRecord(s->ev0, s->stream));
-    if (s->cfg.use_graph && nsteps > 0) {
-        if (!s->graph_exec) {
-            HIPCK(s, hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-            int rc = is64(s) ? enqueue_step<double>(s) : enqueue_step<float>(s);
-            hipGraph_t gr = nullptr;
-            hipError_t e = hipStreamEndCapture(s->stream, &gr);
-            if (rc) {
-                if (gr) (void)hipGraphDestroy(gr);
-                return rc;
-            }
-            if (e != hipSuccess) return fail(s, NUOSC_EHIP, std::string("graph capture: ") + hipGetErrorString(e));
-            s->graph = gr;
-            HIPCK(s, hipGraphInstantiate(&s->graph_exec, s->graph, nullptr, nullptr, 0));
-        }
-        for (int n = 0; n < nsteps; ++n) {
-            HIPCK(s, hipGraphLaunch(s->graph_exec, s->stream));
-            s->phy_time += s->dt;
-        }
-    } else {
-        for (int n = 0; n < nsteps; ++n) {
-            int rc = is64(s) ? enqueue_step<double>(s) : enqueue_step<float>(s);
-            if (rc) return rc;
-            s->phy_time += s->dt;  // accumulated, as nuosc_class.cpp:423
-        }
-    }
-    HIPCK(s, hipEventRecord(s->ev1, s->stream));
-    s->steps_in_last_call = nsteps;
-    return NUOSC_OK;
+    return run_steps(s, kRk4, nsteps);
 }
 
 int nuosc_step_srk3(nuosc_sim* s, int nsteps) {
@@ -838,35 +938,7 @@ int nuosc_step_srk3(nuosc_sim* s, int nsteps) {
         int rc = refresh_moments(s);
         if (rc) return rc;
     }
-    HIPCK(s, hipEventRecord(s->ev0, s->stream));
-    if (s->cfg.use_graph && nsteps > 0) {
-        if (!s->graph3_exec) {
-            HIPCK(s, hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-            int rc = is64(s) ? enqueue_step_srk3<double>(s) : enqueue_step_srk3<float>(s);
-            hipGraph_t gr = nullptr;
-            hipError_t e = hipStreamEndCapture(s->stream, &gr);
-            if (rc) {
-                if (gr) (void)hipGraphDestroy(gr);
-                return rc;
-            }
-            if (e != hipSuccess) return fail(s, NUOSC_EHIP, std::string("graph capture: ") + hipGetErrorString(e));
-            s->graph3 = gr;
-            HIPCK(s, hipGraphInstantiate(&s->graph3_exec, s->graph3, nullptr, nullptr, 0));
-        }
-        for (int n = 0; n < nsteps; ++n) {
-            HIPCK(s, hipGraphLaunch(s->graph3_exec, s->stream));
-            s->phy_time += s->dt;
-        }
-    } else {
-        for (int n = 0; n < nsteps; ++n) {
-            int rc = is64(s) ? enqueue_step_srk3<double>(s) : enqueue_step_srk3<float>(s);
-            if (rc) return rc;
-            s->phy_time += s->dt;  // nuosc_class.cpp:448
-        }
-    }
-    HIPCK(s, hipEventRecord(s->ev1, s->stream));
-    s->steps_in_last_call = nsteps;
-    return NUOSC_OK;
+    return run_steps(s, kSrk3, nsteps);
 }
 
 int nuosc_synchronize(nuosc_sim* s) {
@@ -886,8 +958,8 @@ int nuosc_last_step_ms(nuosc_sim* s, double* ms) {
 
 int nuosc_profile_stages(nuosc_sim* s, int nsteps, double* stage_ms) {
     if (!s || !stage_ms || nsteps < 1) return NUOSC_EINVAL;
-    if (!s->have_moments) {
-        int rc = refresh_moments(s);
+    if (!rk4_ready(s)) {
+        int rc = refresh_rk4(s);
         if (rc) return rc;
     }
     hipEvent_t ev[8] = {};
@@ -896,14 +968,16 @@ int nuosc_profile_stages(nuosc_sim* s, int nsteps, double* stage_ms) {
     double acc[4] = {0, 0, 0, 0};
     int rc = NUOSC_OK;
     for (int n = 0; n < nsteps && rc == NUOSC_OK; ++n) {
-        rc = is64(s) ? enqueue_step<double>(s, ev) : enqueue_step<float>(s, ev);
+        if (s->pairs) rc = is64(s) ? enqueue_step_pairs<double>(s, ev) : enqueue_step_pairs<float>(s, ev);
+        else rc = is64(s) ? enqueue_step<double>(s, ev) : enqueue_step<float>(s, ev);
         if (rc) break;
+        if (s->pairs) state_stepped(s);
         s->phy_time += s->dt;
-        if (hipEventSynchronize(ev[7]) != hipSuccess) {
+        if (hipEventSynchronize(ev[s->pairs ? 5 : 7]) != hipSuccess) {
             rc = fail(s, NUOSC_EHIP, "event sync failed");
             break;
         }
-        for (int k = 0; k < 4 && rc == NUOSC_OK; ++k) {
+        for (int k = 0; k < 4 && rc == NUOSC_OK; k += s->pairs ? 2 : 1) {
             float f = 0;
             if (hipEventElapsedTime(&f, ev[2 * k], ev[2 * k + 1]) != hipSuccess)
                 rc = fail(s, NUOSC_EHIP, "event timing failed");
@@ -917,15 +991,15 @@ int nuosc_profile_stages(nuosc_sim* s, int nsteps, double* stage_ms) {
 
 int nuosc_get_plan(const nuosc_sim* s, int* zlen, int* waves) {
     if (!s) return NUOSC_EINVAL;
-    if (zlen) *zlen = s->plan.zlen;
-    if (waves) *waves = s->plan.ntask;
+    if (zlen) *zlen = s->pairs ? s->pair_zlen : s->plan.zlen;
+    if (waves) *waves = s->pairs ? pair_waves(s->geo, (int)s->esize, s->pair_zlen) : s->plan.ntask;
     return NUOSC_OK;
 }
 
 int nuosc_set_zlen(nuosc_sim* s, int zlen) {
     if (!s || zlen < 1) return NUOSC_EINVAL;
     HIPCK(s, hipStreamSynchronize(s->stream));
-    s->plan = plan_stage_zlen(s->geo, zlen);
+    set_plan(s, zlen);
     drop_graph(s);
     if (s->batch) batch_member_changed(s->batch);
     return NUOSC_OK;
@@ -951,20 +1025,25 @@ int nuosc_autotune(nuosc_sim* s, int trials, int* best_zlen, double* best_ms) {
         std::lock_guard<std::mutex> g(g_tune_mu);
         auto it = g_tune_cache.find(key);
         if (it != g_tune_cache.end()) {
-            int rc = nuosc_set_zlen(s, it->second);
+            HIPCK(s, hipStreamSynchronize(s->stream));
+            if (s->pairs) s->pair_zlen = std::min(it->second, s->nz);
+            else s->plan = plan_stage_zlen(s->geo, it->second);
+            drop_graph(s);
+            if (s->batch) batch_member_changed(s->batch);
             if (best_zlen) *best_zlen = it->second;
             if (best_ms) *best_ms = -1;
-            return rc;
+            return NUOSC_OK;
         }
     }
-    if (!s->have_moments) {
-        int rc = refresh_moments(s);
+    if (!rk4_ready(s)) {
+        int rc = refresh_rk4(s);
         if (rc) return rc;
     }
     hipEvent_t e0, e1;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
         return fail(s, NUOSC_EHIP, "event creation failed");
     const StagePlan keep = s->plan;
+    const int keep_pair = s->pair_zlen;
     std::vector<int> cand;
     for (int zl = 8; zl <= 256; zl *= 2) {
         if (zl > s->nz && zl != 8) break;
@@ -976,7 +1055,7 @@ int nuosc_autotune(nuosc_sim* s, int trials, int* best_zlen, double* best_ms) {
     int rc = NUOSC_OK;
     for (int t = 0; t < trials + 1 && rc == NUOSC_OK; ++t)
         for (size_t k = 0; k < cand.size() && rc == NUOSC_OK; ++k) {
-            s->plan = plan_stage_zlen(s->geo, cand[k]);
+            set_plan(s, cand[k]);
             (void)hipEventRecord(e0, s->stream);
             const hipError_t le =
                 is64(s) ? enqueue_scratch_stages<double>(s) : enqueue_scratch_stages<float>(s);
@@ -991,15 +1070,15 @@ int nuosc_autotune(nuosc_sim* s, int trials, int* best_zlen, double* best_ms) {
         }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    if (rc) {
-        s->plan = keep;
-        return rc;
-    }
+    s->plan = keep;
+    s->pair_zlen = keep_pair;
+    if (rc) return rc;
     size_t kb = 0;
     for (size_t k = 1; k < cand.size(); ++k)
         if (tmin[k] < tmin[kb]) kb = k;
     const int best = cand[kb];
-    s->plan = plan_stage_zlen(s->geo, best);
+    if (s->pairs) s->pair_zlen = std::min(best, s->nz);   // (RK4 only: the SSP-RK3 stages keep their plan)
+    else s->plan = plan_stage_zlen(s->geo, best);
     drop_graph(s);
     if (s->batch) batch_member_changed(s->batch);
     {
@@ -1084,7 +1163,8 @@ int nuosc_renormalize(nuosc_sim* s) {
     if (!s) return NUOSC_EINVAL;
     if (is64(s)) HIPCK(s, launch_renorm<double>(s->geo, (double*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->stream));
     else HIPCK(s, launch_renorm<float>(s->geo, (float*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->stream));
-    return refresh_moments(s);
+    s->have_moments = false;
+    return refresh_rk4(s);
 }
 
 int nuosc_download_field(nuosc_sim* s, int f, double* host) {
@@ -1133,13 +1213,14 @@ int nuosc_upload_field(nuosc_sim* s, int f, const double* host) {
     if (is64(s)) HIPCK(s, launch_unpack<double>(s->geo, s->d_tmp, (double*)s->st_u, f, s->stream));
     else HIPCK(s, launch_unpack<float>(s->geo, s->d_tmp, (float*)s->st_u, f, s->stream));
     HIPCK(s, hipStreamSynchronize(s->stream));
-    s->have_moments = false;
+    s->have_moments = s->have_sums = false;
     return NUOSC_OK;
 }
 
 int nuosc_state_updated(nuosc_sim* s) {
     if (!s) return NUOSC_EINVAL;
-    int rc = refresh_moments(s);
+    s->have_moments = false;
+    int rc = refresh_rk4(s);
     if (rc) return rc;
     HIPCK(s, hipStreamSynchronize(s->stream));
     return NUOSC_OK;
@@ -1181,8 +1262,12 @@ struct nuosc_batch {
     hipStream_t stream = nullptr;
     BatchTables tables;
     bool dirty = true;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t graph_exec = nullptr;
+    // the tables hold both exchanges of the members' state copies: at flip f
+    // member k's state is in copies[k][f]
+    int flip = 0;
+    std::vector<std::array<const void*, 2>> copies;
+    hipGraph_t graph[2] = {};
+    hipGraphExec_t graph_exec[2] = {};
     // z-segment length shared by all members (0: each member's own plan).
     // One length gives every block of the batched launch the same amount of
     // work, so the contiguous block ranges of the 8 XCDs stay balanced.
@@ -1199,10 +1284,12 @@ int bfail(nuosc_batch* b, int code, const std::string& m) {
     return code;
 }
 void batch_drop_graph(nuosc_batch* b) {
-    if (b->graph_exec) (void)hipGraphExecDestroy(b->graph_exec);
-    if (b->graph) (void)hipGraphDestroy(b->graph);
-    b->graph_exec = nullptr;
-    b->graph = nullptr;
+    for (int f = 0; f < 2; ++f) {
+        if (b->graph_exec[f]) (void)hipGraphExecDestroy(b->graph_exec[f]);
+        if (b->graph[f]) (void)hipGraphDestroy(b->graph[f]);
+        b->graph_exec[f] = nullptr;
+        b->graph[f] = nullptr;
+    }
 }
 void batch_member_changed(nuosc_batch* b) { b->dirty = true; }
 void batch_detach(nuosc_batch* b, nuosc_sim* s) {
@@ -1220,22 +1307,12 @@ namespace {
 // (re)build the device tables of the batched launches from the members
 int batch_tables(nuosc_batch* b) {
     std::vector<BatchMember> ms;
+    b->copies.clear();
+    b->flip = 0;
     for (nuosc_sim* m : b->members) {
-        BatchMember bm;
-        bm.g = m->geo;
-        bm.g.nox = 0;   // the batched stage kernel has no NOX form
-        bm.ph = m->ph;
-        bm.pl = plan_stage_zlen(bm.g, b->zlen > 0 ? std::min(b->zlen, m->nz) : m->plan.zlen);
-        bm.u = m->st_u;
-        bm.w = m->st_w;
-        bm.ya = m->st_ya;
-        bm.yb = m->st_yb;
-        bm.mpart = m->mom_part;
-        bm.mu = m->mom_u;
-        bm.ma = m->mom_a;
-        bm.mb = m->mom_b;
-        bm.dt = m->dt;
-        ms.push_back(bm);
+        const int zlen = b->zlen > 0 ? std::min(b->zlen, m->nz) : m->pair_zlen;
+        ms.push_back(BatchMember{m->geo, m->ph, zlen, pair_buffers(m), m->dt});
+        b->copies.push_back({m->st_u, m->st_ya});
     }
     hipError_t e = batch_build(b->tables, ms, is64(b->members[0]) ? 8 : 4, b->launch, b->stream);
     if (e != hipSuccess) return bfail(b, NUOSC_EHIP, std::string("batch tables: ") + hipGetErrorString(e));
@@ -1246,7 +1323,7 @@ int batch_tables(nuosc_batch* b) {
 int batch_sync_members(nuosc_batch* b) {
     for (nuosc_sim* m : b->members) {
         if (m->cfg.renorm) return bfail(b, NUOSC_EINVAL, "renormalising runs cannot be batched");
-        if (!m->have_moments && refresh_moments(m) != NUOSC_OK) return bfail(b, NUOSC_EHIP, m->err);
+        if (!rk4_ready(m) && refresh_rk4(m) != NUOSC_OK) return bfail(b, NUOSC_EHIP, m->err);
         if (hipStreamSynchronize(m->stream) != hipSuccess) return bfail(b, NUOSC_EHIP, "member stream sync failed");
     }
     return NUOSC_OK;
@@ -1320,27 +1397,37 @@ int nuosc_batch_step(nuosc_batch* b, int nsteps) {
     if (b->members.empty() || nsteps == 0) return NUOSC_OK;
     int rc0 = batch_sync_members(b);
     if (rc0) return rc0;
+    // a member stepped alone meanwhile may have exchanged its copies
+    for (size_t k = 0; k < b->members.size() && !b->dirty; ++k)
+        b->dirty = b->members[k]->st_u != b->copies[k][b->flip];
     if (b->dirty) {
         batch_drop_graph(b);
         int rc = batch_tables(b);
         if (rc) return rc;
-        if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
-            return bfail(b, NUOSC_EHIP, "capture failed");
-        hipError_t le = batch_step(b->tables, b->stream);
-        hipGraph_t gr = nullptr;
-        hipError_t ce = hipStreamEndCapture(b->stream, &gr);
-        if (le != hipSuccess || ce != hipSuccess) {
-            if (gr) (void)hipGraphDestroy(gr);
-            return bfail(b, NUOSC_EHIP, "batched step capture failed");
-        }
-        b->graph = gr;
-        if (hipGraphInstantiate(&b->graph_exec, b->graph, nullptr, nullptr, 0) != hipSuccess)
-            return bfail(b, NUOSC_EHIP, "graph instantiation failed");
         b->dirty = false;
     }
     for (int n = 0; n < nsteps; ++n) {
-        if (hipGraphLaunch(b->graph_exec, b->stream) != hipSuccess) return bfail(b, NUOSC_EHIP, "graph launch failed");
-        for (nuosc_sim* m : b->members) m->phy_time += m->dt;
+        hipGraphExec_t& exec = b->graph_exec[b->flip];
+        if (!exec) {
+            if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
+                return bfail(b, NUOSC_EHIP, "capture failed");
+            hipError_t le = batch_step(b->tables, b->flip, b->stream);
+            hipGraph_t gr = nullptr;
+            hipError_t ce = hipStreamEndCapture(b->stream, &gr);
+            if (le != hipSuccess || ce != hipSuccess) {
+                if (gr) (void)hipGraphDestroy(gr);
+                return bfail(b, NUOSC_EHIP, "batched step capture failed");
+            }
+            b->graph[b->flip] = gr;
+            if (hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0) != hipSuccess)
+                return bfail(b, NUOSC_EHIP, "graph instantiation failed");
+        }
+        if (hipGraphLaunch(exec, b->stream) != hipSuccess) return bfail(b, NUOSC_EHIP, "graph launch failed");
+        b->flip ^= 1;
+        for (nuosc_sim* m : b->members) {
+            state_stepped(m);
+            m->phy_time += m->dt;
+        }
     }
     if (hipStreamSynchronize(b->stream) != hipSuccess) return bfail(b, NUOSC_EHIP, "batch stream sync failed");
     return NUOSC_OK;
@@ -1387,8 +1474,8 @@ int nuosc_batch_autotune(nuosc_batch* b, int trials, int* best_zlen, double* bes
             rc = batch_tables(b);
             if (rc) break;
             (void)hipEventRecord(e0, b->stream);
-            // stage 1 writes only the RK4 scratch copies (w, yA), never the state
-            hipError_t le = batch_stage(b->tables, 1, b->stream);
+            // pair 1 writes only the RK4 scratch copies (A, Y3) and records, never the state
+            hipError_t le = batch_pair(b->tables, 1, 0, b->stream);
             (void)hipEventRecord(e1, b->stream);
             if (le != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
                 rc = bfail(b, NUOSC_EHIP, "autotune launch failed");
@@ -1429,8 +1516,9 @@ int nuosc_estimate_device_bytes(const nuosc_config* c, long long* bytes) {
     const CopyLayout L = copy_layout((int)nx, (int)nz, (int)nzs, (int)nvp, (int)nch, esize, nf);
     if (!L.ok) return NUOSC_EINVAL;
     long long b = L.elems * esize;                                     // u, w, yA, yB
-    if (nf == kNVar3) b += nx * nz * ((nv + 63) / 64 + 2) * kNMom3 * 8;   // moments: partials, 2 totals
-    else b += (nx + 1) * nz * nch * kMomRec * 8 + 3ll * nx * nz * kMomStride * 8;
+    const bool pairs = steps_in_pairs(*c);
+    b += part_doubles(nx, nz, nv, nch, nf, pairs) * 8;                 // moments: partials, totals
+    b += (nf == kNVar3 ? 2ll * kNMom3 : 3ll * kMomStride + (pairs ? kPairRec : 0)) * nx * nz * 8;
     b += 4 * nv * 8 + 2 * nv * 8 + 2048ll * kNAna * 16 + kNAna * 8;    // v-grid, G0, analysis
     b += 2 * nz * 8;                                                   // init tables
     *bytes = b;

@@ -45,6 +45,7 @@ constexpr int kWave = 64;
 constexpr int kMomStride = 16;   // doubles per per-site moment total record (12 used)
 constexpr int kMomRec = 12;      // doubles per (site, chunk) partial moment record
 constexpr int kNMom = 12;
+constexpr int kPairRec = 54;     // doubles per (site, chunk) record of direction sums (stage pairs)
 constexpr int kNAna = 12;        // analysis accumulators (see AnaIdx)
 constexpr int kXg = 3;           // stored periodic ghost x rows at each end (the widest stencil's radius)
 
@@ -211,42 +212,68 @@ template <typename T>
 hipError_t launch_p3_slice(const Geometry& g, const T* y, const double* G0, const int* xi, int sx,
                            const int* vi, int sv, double* dst, hipStream_t s);
 
+// Stage pairs (nuosc_pair.hip): RK4 stages 1+2 and 3+4 in one pass each, for
+// 2-flavour periodic boxes with the default discretisation.  A step is
+//   predict(1), pair(1), totals, predict(2), pair(2), totals
+// and needs the direction sums tot of u; it leaves those of unew, and the new
+// state in unew (u is not touched).
+struct PairBuffers {
+    const void* u;
+    void *a, *y3, *unew;        // A = Y2 + u + dt k2, Y3, the new state
+    double *mu, *m3, *min;      // mu times the moments of u, Y3 and the inner input (Y2, then Y4), [site][kMomStride]
+    double *part, *tot;         // direction sums: [site][chunk][kPairRec] partial, [site][kPairRec] total
+};
+bool pair_capable(const Geometry& g);
+// blocks and wavefronts of one pair kernel with z segments of zlen sites
+int pair_blocks(const Geometry& g, int esize, int zlen);
+int pair_waves(const Geometry& g, int esize, int zlen);
+// z-segment length the pair kernels start with
+int plan_pair_zlen(const Geometry& g, int esize, int num_cus);
+template <typename T>
+hipError_t launch_pair(int pair, const Geometry& g, const Physics& ph, int zlen, const PairBuffers& b, double dt,
+                       hipStream_t s);
+hipError_t launch_pair_predict(int pair, const Geometry& g, const Physics& ph, const PairBuffers& b, double dt,
+                               hipStream_t s);
+hipError_t launch_pair_totals(const Geometry& g, bool compensated, const PairBuffers& b, hipStream_t s);
+// partial direction sums of a state
+template <typename T>
+hipError_t launch_pair_sums(const Geometry& g, const T* y, double* part, hipStream_t s);
+
 // Batched runs: every member run advances one RK4 step per batch_step call
-// with one launch per stage for all members (plus one moment-total launch per
-// stage).  Members keep their own buffers, plans and physics; all share the
-// precision (esize) of the tables.
+// with one launch of each kernel of a step for all members.  Members keep
+// their own buffers, segments and physics; all share the precision (esize) of
+// the tables.
 struct BatchMember {
     Geometry g;
     Physics ph;
-    StagePlan pl;
-    void *u, *w, *ya, *yb;          // state copies
-    double *mpart, *mu, *ma, *mb;   // partial records; totals of u, yA, yB
+    int zlen;
+    PairBuffers b;   // of flip 0; with flip 1 u and unew change places
     double dt;
 };
-// Launch forms of the batched stage kernel: an ordinary grid of one block
+// Launch forms of the batched pair kernels: an ordinary grid of one block
 // per logical block, or a persistent grid of resident blocks drawing logical
 // blocks from per-XCD work queues.
 constexpr int kBatchGrid = 0, kBatchPersistent = 1;
-constexpr int kBatchCounters = 32;   // 8 XCD counters for each of the 4 stages
+constexpr int kBatchCounters = 16;   // 8 XCD counters for each of the 2 pairs
 
 struct BatchTables {
-    void* args[4] = {nullptr, nullptr, nullptr, nullptr};  // per-stage StageArgs arrays
-    void* tot[4] = {nullptr, nullptr, nullptr, nullptr};   // per-stage moment-total arrays
-    void* xg[4] = {nullptr, nullptr, nullptr, nullptr};    // per-stage x-ghost refresh arrays
-    int* bmap = nullptr;   // logical block -> (member, block of member)
-    int* tmap = nullptr;
-    int* xmap = nullptr;
-    int* ctr = nullptr;    // work-queue counters of the persistent launch
-    int nblocks = 0, tblocks = 0, xblocks = 0, esize = 8;
+    void* buf = nullptr;   // one device buffer holds all of the following
+    size_t bytes = 0;
+    void* args[2][2] = {};   // [pair][flip] PairArgs arrays
+    void* pre[2][2] = {};    // [pair][flip] PredictArgs arrays
+    void* sum = nullptr;     // totals arguments
+    int *bmap = nullptr, *tmap = nullptr, *pmap = nullptr;   // logical block -> (member, block of member)
+    int* ctr = nullptr;      // work-queue counters of the persistent launch
+    int nblocks = 0, tblocks = 0, pblocks = 0, esize = 8;
     int launch = kBatchGrid, pgrid = 0;   // launch form; resident blocks of the persistent grid
 };
 hipError_t batch_build(BatchTables& t, const std::vector<BatchMember>& members, int esize, int launch,
                        hipStream_t s);
 void batch_free(BatchTables& t);
-hipError_t batch_step(const BatchTables& t, hipStream_t s);
-// one stage kernel of every member (no ghost refresh, no moment totals):
-// autotuner timing
-hipError_t batch_stage(const BatchTables& t, int stage, hipStream_t s);
+// one step of every member; flip: which of its two state copies holds u
+hipError_t batch_step(const BatchTables& t, int flip, hipStream_t s);
+// one pair kernel of every member alone (autotuner timing)
+hipError_t batch_pair(const BatchTables& t, int pair, int flip, hipStream_t s);
 
 // Open z boundary: fill the zoff ghost rows at both z ends of state y for
 // time t = *t_dev + cdt (inflow directions: the Inflow pulse state;

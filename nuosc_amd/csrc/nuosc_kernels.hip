@@ -791,59 +791,6 @@ __global__ __launch_bounds__(64 * StageShape<T>::W) __attribute__((amdgpu_waves_
     stage_body<T, R, W, RAD, STAGE, COMP, NOX>(a, xcd_remap(blockIdx.x, gridDim.x), wib, slab);
 }
 
-// Many independent runs in one launch: logical block -> (run, block of run)
-// from bmap; each run's arguments from the runs table (read with scalar loads).
-template <typename T, int R, int STAGE, bool COMP>
-__global__ __launch_bounds__(64 * StageShape<T>::W) __attribute__((amdgpu_waves_per_eu(stage_waves<T, STAGE>()))) void k_stage_batch(
-    const StageArgs<T>* __restrict__ runs, const int* __restrict__ bmap) {
-    constexpr int W = StageShape<T>::W;
-    __shared__ Slab<T, R, W, 2> slab;
-    const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lb = xcd_remap(blockIdx.x, gridDim.x);
-    const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)bmap;
-    const int run = cm[2 * lb], blk = cm[2 * lb + 1];
-    const StageArgs<T> a = runs[run];   // uniform, read-only: scalar loads
-    stage_body<T, R, W, 2, STAGE, COMP>(a, blk, wib, slab);
-}
-
-// The same work as a persistent kernel: a grid of resident blocks takes
-// logical blocks from a work queue until it is empty.  Logical blocks keep
-// the split of xcd_remap (one contiguous range per XCD, block b of the grid
-// runs on XCD b % 8), and each XCD's blocks draw from their range through
-// their own counter ctr[x], so neighbouring logical blocks still run on one
-// XCD at about the same time.  Every block leaves the loop once its XCD's
-// counter passes the range (the exit every wave reaches); the counters are
-// zeroed by k_zero_ints before each launch.
-template <typename T, int R, int STAGE, bool COMP>
-__global__ __launch_bounds__(64 * StageShape<T>::W) __attribute__((amdgpu_waves_per_eu(stage_waves<T, STAGE>()))) void k_stage_batch_q(
-    const StageArgs<T>* __restrict__ runs, const int* __restrict__ bmap, int* __restrict__ ctr, int nitems) {
-    constexpr int W = StageShape<T>::W;
-    __shared__ Slab<T, R, W, 2> slab;
-    __shared__ int next;
-    const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int x = blockIdx.x % 8;
-    const int per = nitems / 8, rem = nitems % 8;
-    const int start = x < rem ? x * (per + 1) : rem * (per + 1) + (x - rem) * per;
-    const int count = per + (x < rem ? 1 : 0);
-    const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)bmap;
-    for (;;) {
-        if (threadIdx.x == 0) next = atomicAdd(&ctr[x], 1);
-        __syncthreads();
-        const int k = __builtin_amdgcn_readfirstlane(next);
-        __syncthreads();   // every wave has read next before thread 0 rewrites it
-        if (k >= count) break;
-        const int lb = start + k;
-        const int run = cm[2 * lb], blk = cm[2 * lb + 1];
-        const StageArgs<T> a = runs[run];   // uniform, read-only: scalar loads
-        stage_body<T, R, W, 2, STAGE, COMP>(a, blk, wib, slab);
-    }
-}
-
-__global__ void k_zero_ints(int* __restrict__ p, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
-}
-
 int rows_per_wave(int esize) { return esize == 8 ? StageShape<double>::R : StageShape<float>::R; }
 int waves_per_block(int esize) { return esize == 8 ? StageShape<double>::W : StageShape<float>::W; }
 int dirs_per_chunk(int esize) {
@@ -1023,26 +970,12 @@ __device__ __forceinline__ void xg_body(const XgArgs& a, long long blk) {
 
 __global__ __launch_bounds__(256) void k_xghosts(const XgArgs a) { xg_body(a, blockIdx.x); }
 
-__global__ __launch_bounds__(256) void k_xghosts_batch(const XgArgs* __restrict__ runs, const int* __restrict__ xmap) {
-    const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)xmap;
-    const int run = cm[2 * blockIdx.x], blk = cm[2 * blockIdx.x + 1];
-    const XgArgs a = runs[run];
-    xg_body(a, blk);
-}
-
 template <typename T>
 hipError_t launch_xghosts(const Geometry& g, T* y, hipStream_t s) {
     const XgArgs a = xg_args(g, y, sizeof(T));
     hipLaunchKernelGGL(k_xghosts, dim3((unsigned)xg_blocks(a.words)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
-
-struct TotArgs {
-    const double* part;
-    double* tot;
-    int nch;
-    long long nsites;
-};
 
 template <bool COMP>
 __device__ __forceinline__ void totals_body(const double* __restrict__ part, int nch, long long nsites,
@@ -1084,185 +1017,6 @@ hipError_t launch_moment_totals(const Geometry& g, bool compensated, const doubl
     const dim3 grid((unsigned)((n + 255) / 256)), block(256);
     if (compensated) hipLaunchKernelGGL((k_moment_totals<true>), grid, block, 0, s, part, g.nch, nsites, tot);
     else hipLaunchKernelGGL((k_moment_totals<false>), grid, block, 0, s, part, g.nch, nsites, tot);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// batched runs: one launch per RK4 stage (and one per moment-total pass) for
-// every member run; the runs keep their own buffers, plans and physics
-// ---------------------------------------------------------------------------
-template <bool COMP>
-__global__ __launch_bounds__(256) void k_moment_totals_batch(const TotArgs* __restrict__ runs,
-                                                             const int* __restrict__ bmap) {
-    const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)bmap;
-    const int run = cm[2 * blockIdx.x], blk = cm[2 * blockIdx.x + 1];
-    const TotArgs ta = runs[run];
-    totals_body<COMP>(ta.part, ta.nch, ta.nsites, ta.tot, (long long)blk * 256 + threadIdx.x);
-}
-
-template <typename T>
-static hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hipStream_t s) {
-    const int n = (int)ms.size();
-    std::vector<int> bmap, tmap, xmap;
-    for (int r = 0; r < n; ++r)
-        for (int b = 0; b < ms[r].pl.nblocks; ++b) {
-            bmap.push_back(r);
-            bmap.push_back(b);
-        }
-    for (int r = 0; r < n; ++r) {
-        const long long ent = (long long)ms[r].g.nx * ms[r].g.nz * kMomStride;
-        const int nb = (int)((ent + 255) / 256);
-        for (int b = 0; b < nb; ++b) {
-            tmap.push_back(r);
-            tmap.push_back(b);
-        }
-    }
-    for (int r = 0; r < n; ++r) {
-        const long long nb = xg_blocks(xg_args(ms[r].g, nullptr, sizeof(T)).words);
-        for (long long b = 0; b < nb; ++b) {
-            xmap.push_back(r);
-            xmap.push_back((int)b);
-        }
-    }
-    t.nblocks = (int)bmap.size() / 2;
-    t.tblocks = (int)tmap.size() / 2;
-    t.xblocks = (int)xmap.size() / 2;
-    hipError_t e;
-    // persistent launch: one counter per XCD per stage, and a grid of as many
-    // blocks as the GPU holds at once (stage 2, the largest, sets the count)
-    if ((e = hipMalloc((void**)&t.ctr, kBatchCounters * sizeof(int))) != hipSuccess) return e;
-    {
-        int dev = 0, cus = 0, bpc = 0;
-        if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
-        if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
-        constexpr int R = StageShape<T>::R;
-        if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_stage_batch_q<T, R, 2, sizeof(T) == 4>,
-                                                              64 * StageShape<T>::W, 0)) != hipSuccess)
-            return e;
-        t.pgrid = std::max(8, (cus * std::max(bpc, 1) + 7) / 8 * 8);
-    }
-    for (auto [dst, v] : {std::pair<int**, std::vector<int>*>{&t.bmap, &bmap}, {&t.tmap, &tmap}, {&t.xmap, &xmap}}) {
-        if ((e = hipMalloc((void**)dst, v->size() * sizeof(int))) != hipSuccess) return e;
-        if ((e = hipMemcpyAsync(*dst, v->data(), v->size() * sizeof(int), hipMemcpyHostToDevice, s)) != hipSuccess)
-            return e;
-    }
-    for (int st = 1; st <= 4; ++st) {
-        std::vector<StageArgs<T>> args(n);
-        std::vector<TotArgs> tots(n);
-        std::vector<XgArgs> xgs(n);
-        for (int r = 0; r < n; ++r) {
-            const BatchMember& m = ms[r];
-            const double dt = m.dt, c6 = 1.0 / 6.0 * dt, c2 = 0.5 * dt;
-            T *u = (T*)m.u, *w = (T*)m.w, *ya = (T*)m.ya, *yb = (T*)m.yb;
-            T* yin;
-            const T* uu;
-            T* yout;
-            const double* mt;
-            double* mo;
-            double cw, cy;
-            switch (st) {
-                case 1: yin = u; uu = u; yout = ya; mt = m.mu; mo = m.ma; cw = 0.0; cy = c2; break;
-                case 2: yin = ya; uu = u; yout = yb; mt = m.ma; mo = m.mb; cw = dt; cy = c2; break;
-                case 3: yin = yb; uu = u; yout = ya; mt = m.mb; mo = m.ma; cw = 0.0; cy = dt; break;
-                default: yin = ya; uu = ya; yout = u; mt = m.ma; mo = m.mu; cw = c6; cy = 0.0; break;
-            }
-            args[r] = make_stage_args<T>(m.g, m.ph, m.pl, yin, uu, w, yout, mt, m.mpart, cw, cy);
-            tots[r] = TotArgs{m.mpart, mo, m.g.nch, (long long)m.g.nx * m.g.nz};
-            xgs[r] = xg_args(m.g, yin, sizeof(T));
-        }
-        if ((e = hipMalloc(&t.args[st - 1], n * sizeof(StageArgs<T>))) != hipSuccess) return e;
-        if ((e = hipMalloc(&t.tot[st - 1], n * sizeof(TotArgs))) != hipSuccess) return e;
-        if ((e = hipMalloc(&t.xg[st - 1], n * sizeof(XgArgs))) != hipSuccess) return e;
-        if ((e = hipMemcpyAsync(t.args[st - 1], args.data(), n * sizeof(StageArgs<T>), hipMemcpyHostToDevice, s)) !=
-            hipSuccess)
-            return e;
-        if ((e = hipMemcpyAsync(t.tot[st - 1], tots.data(), n * sizeof(TotArgs), hipMemcpyHostToDevice, s)) !=
-            hipSuccess)
-            return e;
-        if ((e = hipMemcpyAsync(t.xg[st - 1], xgs.data(), n * sizeof(XgArgs), hipMemcpyHostToDevice, s)) !=
-            hipSuccess)
-            return e;
-    }
-    return hipStreamSynchronize(s);
-}
-
-hipError_t batch_build(BatchTables& t, const std::vector<BatchMember>& ms, int esize, int launch, hipStream_t s) {
-    batch_free(t);
-    t.esize = esize;
-    t.launch = launch;
-    if (ms.empty()) return hipSuccess;
-    for (const auto& m : ms) {
-        if (!buffer_addressable(m.g, esize)) return hipErrorInvalidValue;
-        if (m.g.lpr != dirs_per_chunk(esize) || m.g.wpb != waves_per_block(esize) || m.g.nox)
-            return hipErrorInvalidValue;
-    }
-    return esize == 8 ? batch_build_t<double>(t, ms, s) : batch_build_t<float>(t, ms, s);
-}
-
-void batch_free(BatchTables& t) {
-    for (int k = 0; k < 4; ++k) {
-        if (t.args[k]) (void)hipFree(t.args[k]);
-        if (t.tot[k]) (void)hipFree(t.tot[k]);
-        if (t.xg[k]) (void)hipFree(t.xg[k]);
-        t.args[k] = t.tot[k] = t.xg[k] = nullptr;
-    }
-    for (int** m : {&t.bmap, &t.tmap, &t.xmap, &t.ctr}) {
-        if (*m) (void)hipFree(*m);
-        *m = nullptr;
-    }
-    t.nblocks = t.tblocks = t.xblocks = t.pgrid = 0;
-}
-
-template <typename T>
-static hipError_t batch_stage_t(const BatchTables& t, int st, hipStream_t s) {
-    constexpr int R = StageShape<T>::R;
-    constexpr bool COMP = sizeof(T) == 4;
-    const dim3 grid(t.nblocks), block(64 * StageShape<T>::W);
-    const StageArgs<T>* a = (const StageArgs<T>*)t.args[st - 1];
-    if (t.launch == kBatchPersistent) {
-        int* c = t.ctr + 8 * (st - 1);
-        hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, c, 8);   // a kernel node, not a memset, in graphs
-        const dim3 pg(t.pgrid);
-        const int n = t.nblocks;
-        switch (st) {
-            case 1: hipLaunchKernelGGL((k_stage_batch_q<T, R, 1, COMP>), pg, block, 0, s, a, t.bmap, c, n); break;
-            case 2: hipLaunchKernelGGL((k_stage_batch_q<T, R, 2, COMP>), pg, block, 0, s, a, t.bmap, c, n); break;
-            case 3: hipLaunchKernelGGL((k_stage_batch_q<T, R, 3, COMP>), pg, block, 0, s, a, t.bmap, c, n); break;
-            default: hipLaunchKernelGGL((k_stage_batch_q<T, R, 4, COMP>), pg, block, 0, s, a, t.bmap, c, n); break;
-        }
-        return hipGetLastError();
-    }
-    switch (st) {
-        case 1: hipLaunchKernelGGL((k_stage_batch<T, R, 1, COMP>), grid, block, 0, s, a, t.bmap); break;
-        case 2: hipLaunchKernelGGL((k_stage_batch<T, R, 2, COMP>), grid, block, 0, s, a, t.bmap); break;
-        case 3: hipLaunchKernelGGL((k_stage_batch<T, R, 3, COMP>), grid, block, 0, s, a, t.bmap); break;
-        default: hipLaunchKernelGGL((k_stage_batch<T, R, 4, COMP>), grid, block, 0, s, a, t.bmap); break;
-    }
-    return hipGetLastError();
-}
-
-hipError_t batch_stage(const BatchTables& t, int stage, hipStream_t s) {
-    if (t.nblocks == 0) return hipSuccess;
-    if (stage < 1 || stage > 4) return hipErrorInvalidValue;
-    return t.esize == 8 ? batch_stage_t<double>(t, stage, s) : batch_stage_t<float>(t, stage, s);
-}
-
-// per stage: x ghost rows of every member's stage input, the stage kernel,
-// the moment totals of its output
-hipError_t batch_step(const BatchTables& t, hipStream_t s) {
-    if (t.nblocks == 0) return hipSuccess;
-    const bool comp = t.esize == 4;
-    for (int st = 1; st <= 4; ++st) {
-        hipLaunchKernelGGL(k_xghosts_batch, dim3(t.xblocks), dim3(256), 0, s, (const XgArgs*)t.xg[st - 1], t.xmap);
-        const hipError_t e = t.esize == 8 ? batch_stage_t<double>(t, st, s) : batch_stage_t<float>(t, st, s);
-        if (e != hipSuccess) return e;
-        if (comp)
-            hipLaunchKernelGGL((k_moment_totals_batch<true>), dim3(t.tblocks), dim3(256), 0, s,
-                               (const TotArgs*)t.tot[st - 1], t.tmap);
-        else
-            hipLaunchKernelGGL((k_moment_totals_batch<false>), dim3(t.tblocks), dim3(256), 0, s,
-                               (const TotArgs*)t.tot[st - 1], t.tmap);
-    }
     return hipGetLastError();
 }
 

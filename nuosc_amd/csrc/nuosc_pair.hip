@@ -1,0 +1,1019 @@
+// nuosc_pair.hip -- CDNA4 (gfx950) kernels that advance two RK4 stages in one
+// pass over the state (2 flavours, periodic box, the default discretisation).
+//
+// The stage-by-stage form (k_stage, nuosc_kernels.hip) writes and re-reads
+// every stage input: 12 passes over the state per step.  k_pair does stages
+// 1+2 and stages 3+4 as two kernels that keep the inner stage input in
+// registers and LDS:
+//   pair 1: read u       -> Y2 (on chip) -> Y3 = u + dt/2 k2, A = Y2 + u + dt k2
+//   pair 2: read Y3, u, A -> Y4 (on chip) -> u' = (A + Y4)/3 + dt/6 k4
+// 3 + 4 = 7 passes (448 B per FP64 update instead of 768).
+//
+// What made the passes separate is the interaction term of the inner input Y:
+// it needs the velocity moments of Y at each site, a sum over all directions,
+// while a block holds 64 of them.  But Y = u + c k(y), and the moments of
+// k(y) follow from sums over directions of y itself: the stencil terms are
+// linear, and the interaction term is a product of the moments of y with the
+// fields, so with the nine sums over w u_a u_b (u = (1, vx, vy, vz);
+// vy^2 = 1 - vx^2 - vz^2) of emr, emi and ee - mm, and of their antineutrino
+// partners, the moments of k(y) -- and so of Y -- are known at every site
+// before any Y is formed:
+//   k_pair_totals   adds a site's partial sums over its direction chunks;
+//   k_pair_predict  forms from them the moments of y and of Y (per site: the
+//                   same stencils on 24 numbers instead of on 8 nv);
+//   k_pair          writes the 2 x 27 partial sums of its output.
+// The sums are FP64 in both precisions.
+//
+// The neutrino and antineutrino fields couple only through the moments, so
+// the work unit of a wavefront is 4 fields (one of the two) of one x row and
+// 64 directions.
+#include <hip/hip_runtime.h>
+
+#include "nuosc_dev.h"
+#include "nuosc_lanes.h"
+
+#include <algorithm>
+#include <cstring>
+#include <type_traits>
+#include <vector>
+
+namespace nuosc {
+namespace {
+
+constexpr int kF = 4;           // fields of a unit: ee, mm, emr, emi (or the antineutrino ones)
+constexpr double kThirdRest = 0x1.5555555555555p-56;   // 1/3 minus its double
+constexpr int kMono = 9;        // 1, x, y, z, xx, xy, xz, yz, zz
+constexpr int kRec = 3 * kMono; // sums of one unit: [mono][emr, emi, ee - mm]
+static_assert(2 * kRec == kPairRec, "record of a site: neutrinos, then antineutrinos");
+
+typedef __attribute__((ext_vector_type(2))) unsigned int pu32x2;
+constexpr int kPairRsrc3 = 0x00020000;   // gfx9 raw-buffer descriptor word 3
+
+// AUX: cache policy bits (2: non-temporal)
+template <typename T, int AUX = 0>
+__device__ __forceinline__ T pld(__amdgpu_buffer_rsrc_t r, unsigned vo, unsigned so) {
+    if constexpr (sizeof(T) == 8)
+        return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, vo, so, AUX));
+    else
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, vo, so, AUX));
+}
+template <typename T>
+__device__ __forceinline__ void pst(T v, __amdgpu_buffer_rsrc_t r, unsigned vo, unsigned so) {
+    if constexpr (sizeof(T) == 8)
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(pu32x2, v), r, vo, so, 2);
+    else
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, vo, so, 2);
+}
+// descriptor of the bytes [base, base + bytes); the empty asm keeps it from
+// being held in scalar registers across the z loop
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t prs(unsigned long long base, unsigned bytes) {
+    asm volatile("" : "+s"(base));
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, kPairRsrc3);
+}
+
+// constant address space: uniform loads from it become scalar loads
+typedef const __attribute__((address_space(4))) double pcdouble;
+// the compiler divides integers in vector registers and may then keep what is
+// derived from the quotient there; this puts a wave-uniform value back
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+// ---------------------------------------------------------------------------
+// Direction sums on the matrix cores.  V_MFMA_F64_4X4X4 multiplies four pairs
+// of 4 x 4 matrices; lane l holds A[i = l % 4][q] and B[q][j = l % 4], where
+// q = l / 4 runs over the four blocks and the four columns of A (rows of B)
+// of each.  With lane l's A value of step t the weighted monomial 4 m + i of
+// direction (l & ~3) + t and its B value the field combination j of that
+// direction, four steps sum a chunk's 64 directions in four blocks, which two
+// DPP adds join.  The combinations move from "lane = direction" to the B
+// layout through a small LDS array (each lane needs combination l % 4 of the
+// four directions of its quad).  27 sums cost 12 matrix instructions and
+// about 45 others; as wavefront reductions they took 160.
+// ---------------------------------------------------------------------------
+constexpr int kStageStride = 66;   // doubles between the combinations: 16-byte aligned quads, other banks
+struct SumStage {
+    double v[3 * kStageStride];
+};
+struct SumTable {
+    double2 v[6][64];   // [pair of steps and tiles][lane]: A values 2k, 2k+1 of the 12 = 3 tiles x 4 steps
+};
+
+// w mono_n of direction d (0 past nv)
+__device__ __forceinline__ double weighted_mono(const Geometry& g, int d, int n) {
+    if (d >= g.nv || n >= kMono) return 0.0;
+    const double x = g.vx[d], y = g.vy[d], z = g.vz[d], w = g.vw[d];
+    const double p = n == 0 || n == 1 || n == 2 || n == 3 ? 1.0 : (n < 7 ? x : (n == 7 ? y : z));
+    const double q = n == 0 ? 1.0 : (n == 1 || n == 4 ? x : (n == 2 || n == 5 ? y : z));
+    return p * q * w;
+}
+// the table entries of one lane, chunk ch
+__device__ __forceinline__ void fill_table(const Geometry& g, SumTable& t, int ch, int lane) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        double e[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int m = (2 * k + h) / 4, s = (2 * k + h) % 4;
+            e[h] = weighted_mono(g, ch * 64 + (lane & ~3) + s, 4 * m + (lane & 3));
+        }
+        t.v[k][lane] = make_double2(e[0], e[1]);
+    }
+}
+
+__device__ __forceinline__ double dpp_add_ror(double x, bool eight) {
+    // x + x of lane +-8 / +-4 within the 16-lane row
+    return eight ? x + dpp_f64<kDppRowRor8, 0xF>(x, x) : x + dpp_f64<0x124, 0xF>(x, x);
+}
+
+// Direction sums of (c0, c1, c2) over the chunk, stored as one record of 27
+// doubles at so under descriptor rp (vrec: the lane's offset from sum_offset).
+__device__ __forceinline__ void direction_sums(double c0, double c1, double c2, SumStage& st, const SumTable& tab,
+                                               int lane, __amdgpu_buffer_rsrc_t rp, unsigned vrec, unsigned so) {
+    st.v[lane] = c0;
+    st.v[kStageStride + lane] = c1;
+    st.v[2 * kStageStride + lane] = c2;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    // (lanes of the unused fourth column read the third combination)
+    const double* q = &st.v[min(lane & 3, 2) * kStageStride + (lane & ~3)];
+    const double b[4] = {q[0], q[1], q[2], q[3]};
+    double d[3];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+        const double2 a01 = tab.v[2 * m][lane], a23 = tab.v[2 * m + 1][lane];
+        double acc = __builtin_amdgcn_mfma_f64_4x4x4f64(a01.x, b[0], 0.0, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_4x4x4f64(a01.y, b[1], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_4x4x4f64(a23.x, b[2], acc, 0, 0, 0);
+        d[m] = __builtin_amdgcn_mfma_f64_4x4x4f64(a23.y, b[3], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int m = 0; m < 3; ++m) d[m] = dpp_add_ror(dpp_add_ror(d[m], true), false);
+    // every block's lanes hold the joined sums: block m stores tile m
+    const int blk = (lane >> 2) & 3;
+    const double v = blk == 0 ? d[0] : (blk == 1 ? d[1] : d[2]);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(pu32x2, v), rp, vrec, so, 0);
+}
+// lane l of D holds row i = l / 16, column j = l % 4 of block (l / 4) % 4:
+// sum 4 m + i of combination j; lanes without one point past the record array
+__device__ __forceinline__ unsigned sum_offset(int lane, unsigned past) {
+    const int m = (lane >> 2) & 3, i = lane >> 4, j = lane & 3, n = 4 * m + i;
+    return (m < 3 && j < 3 && n < kMono) ? (unsigned)(n * 3 + j) * 8u : past;
+}
+
+// ---------------------------------------------------------------------------
+// the stage pair
+// ---------------------------------------------------------------------------
+template <typename T>
+struct PairArgs {
+    Geometry g;
+    unsigned long long y;      // stencil input (stored x row 0): u (pair 1), Y3 (pair 2)
+    unsigned long long u;      // pair 2: u
+    unsigned long long a;      // A: written by pair 1, read by pair 2
+    unsigned long long out;    // Y3 (pair 1), u' (pair 2); no input of the pass
+    unsigned long long m1, m2; // moments of y and of the inner input, times mu: [site][kMomStride]
+    unsigned long long part;   // partial sums of out: [site][chunk][2][kRec]
+    double c1, c2, cA;         // inner input u + c1 k; output factor c2; A's factor cA
+    double pst, p2ct;          // pmo st, 2 pmo ct
+    int zlen, xgroups, nunits;
+};
+
+// x rows a block writes: R, from R + 4 rows of the inner input and R + 8 of y
+template <typename T>
+struct PairShape {
+    static constexpr int R = sizeof(T) == 8 ? 8 : 12;
+};
+
+template <typename T, int R>
+struct PairSlab {
+    T y[2][R + 9][kF][64];   // rows -4 .. R+3 of y at the inner input's z, and a slot idle lanes write
+    T m[2][R + 4][kF][64];   // rows -2 .. R+1 of the inner input
+    SumTable tab;
+    SumStage st[R];
+};
+// one x row: no neighbours to share
+template <int W>
+struct PairRowLds {
+    SumTable tab[W];
+    SumStage st[W];
+};
+
+// Per-direction and physics factors of k(y)
+template <typename T>
+struct PairConst {
+    double vx, vy, vz;
+    T fx, fz;          // -v / (12 h)
+    T kx, kz, k6;      // -ko / (16 h) per axis; 6 (kx + kz)
+    double pst, p2ct;
+};
+
+// Interaction and vacuum terms as one precession: with the projections A, B, C
+// of the site's moments (INP, nuosc_class.cpp:187), here times mu,
+//   k_ee = 2 (q emi + b emr), k_mm = -k_ee, k_emr = -(b d + c emi),
+//   k_emi = c emr - q d,  d = ee - mm,  q = A - pmo st, b = B, c = C + 2 pmo ct
+// (the terms of nuosc_class.cpp:193-200, 280-287 collected).
+template <typename T>
+struct Precession {
+    T q2, b2, q, b, c;
+};
+template <typename T>
+__device__ __forceinline__ Precession<T> precession(const PairConst<T>& k, const double (&m)[kNMom]) {
+    const double A = m[0] - m[1] * k.vx - m[2] * k.vy - m[3] * k.vz;
+    const double B = m[4] - m[5] * k.vx - m[6] * k.vy - m[7] * k.vz;
+    const double C = m[8] - m[9] * k.vx - m[10] * k.vy - m[11] * k.vz;
+    const double q = A - k.pst, c = C + k.p2ct;
+    return Precession<T>{(T)(2 * q), (T)(2 * B), (T)q, (T)B, (T)c};
+}
+
+__device__ __forceinline__ void load_moments(unsigned long long site, double (&m)[kNMom]) {
+    pcdouble* p = (pcdouble*)site;
+#pragma unroll
+    for (int q = 0; q < kNMom; ++q) m[q] = p[q];
+}
+
+// k(y) of the 4 fields: c centre values, z neighbours, x neighbours through
+// the callable.  The stencils (nuosc_class.cpp:122-123, 182-183) are taken on
+// differences and sums of opposite neighbours, so that the advection term
+// keeps the exact differences, and added to the local terms one by one.
+template <typename T, typename XN>
+__device__ __forceinline__ void rhs_unit(const PairConst<T>& k, const Precession<T>& r, const T (&c)[kF],
+                                         const T (&zm2)[kF], const T (&zm1)[kF], const T (&zp1)[kF],
+                                         const T (&zp2)[kF], XN xn, T (&out)[kF]) {
+    const T d = c[0] - c[1], ee = r.q2 * c[3] + r.b2 * c[2];
+    const T loc[kF] = {ee, -ee, -(r.b * d + r.c * c[3]), r.c * c[2] - r.q * d};
+#pragma unroll
+    for (int f = 0; f < kF; ++f) {
+        T xm2, xm1, xp1, xp2;
+        xn(f, xm2, xm1, xp1, xp2);
+        T t = loc[f] + k.k6 * c[f];
+        t += k.kz * ((zm2[f] + zp2[f]) - (T)4 * (zm1[f] + zp1[f]));
+        t += k.kx * ((xm2 + xp2) - (T)4 * (xm1 + xp1));
+        t += k.fz * ((zm2[f] - zp2[f]) - (T)8 * (zm1[f] - zp1[f]));
+        t += k.fx * ((xm2 - xp2) - (T)8 * (xm1 - xp1));
+        out[f] = t;
+    }
+}
+
+// One wavefront of a pair: x row `row`, unit (chunk ch, neutrinos grp = 0 or
+// antineutrinos 1), z segment [j0, j1).  Step j forms the inner input at
+// z = j + 2 and, from step j0 on, the output at z = j; the four steps before
+// j0 fill the inner input's z window.
+//   OUT   the wave writes its row; otherwise the row only feeds neighbours
+//         (and the wave loads an edge row of y)
+//   NOX   one x row: x neighbours are the point itself, no slab, no barrier
+// Per step each wave puts its row of y at z = j + 2 and of the inner input at
+// z = j into the slab of the step's parity, passes the one barrier, and reads
+// its x neighbours; the other parity's slab is rewritten only after the next
+// barrier, which every wave reaches after its reads.  The rows of y and u that
+// step j loads are used from step j + 1 on, so a wave does not wait for what
+// it has just asked for: the waves of a block move in step, and one block
+// fills a CU's registers.  Edge rows are loaded at the z at which the
+// neighbouring blocks load them as their own (L2 hits).
+// The z windows are rings of six slots and a step is compiled for each of the
+// six phases, so that no register is moved to shift a window (54 of 354
+// vector instructions per step before).
+template <typename T, int PAIR, bool OUT, bool NOX, typename LDS>
+__device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch, int grp, int j0, int j1, int slot_m,
+                                          int erow, int slot_e, SumTable& tab, SumStage& sst, LDS* lds) {
+    const Geometry& g = a.g;
+    const int lane = threadIdx.x & 63, nz = g.nz;
+    const unsigned rowb = (unsigned)g.nvp * (unsigned)sizeof(T);
+    const unsigned siteb = (unsigned)(g.srec * (long long)sizeof(T));
+    const unsigned long long xrowb = (unsigned long long)g.xrow * sizeof(T);
+    const unsigned gofs = (unsigned)(grp * kF) * rowb;
+    const unsigned long long rbase = (unsigned long long)(row + kXg) * xrowb + gofs;
+    const unsigned long long ebase = (unsigned long long)(max(erow, 0) + kXg) * xrowb + gofs;
+    const unsigned rbytes = (unsigned)xrowb - gofs;
+    const int pv = min(ch * 64 + lane, g.nv - 1);   // lanes past nv work on the last direction (and store its bits)
+    const unsigned vo = (unsigned)pv * (unsigned)sizeof(T);
+    const unsigned ve = erow >= 0 ? vo : rbytes;    // no edge row: past the range, nothing is fetched
+    const unsigned zrec = (unsigned)(g.nch * kPairRec * 8);   // bytes of a site's partial records
+    const unsigned rec0 = (unsigned)(ch * kPairRec + grp * kRec) * 8;
+    const unsigned long long prow = a.part + (unsigned long long)row * nz * zrec + rec0;
+    const unsigned pbytes = (unsigned)nz * zrec - rec0;
+    const unsigned vrec = sum_offset(lane, pbytes);
+    const unsigned long long mrow = (unsigned long long)row * nz * (kMomStride * 8);
+    const unsigned mbytes = (unsigned)nz * (kMomStride * 8), vm = (unsigned)(lane & 15) * 8;
+    PairConst<T> k;
+    k.vx = g.vx[pv];
+    k.vy = g.vy[pv];
+    k.vz = g.vz[pv];
+    k.fx = (T)(-k.vx / g.twelve_dx);
+    k.fz = (T)(-k.vz / g.twelve_dz);
+    k.kx = (T)g.ko_x;
+    k.kz = (T)g.ko_z;
+    k.k6 = (T)(6 * (g.ko_x + g.ko_z));
+    k.pst = a.pst;
+    k.p2ct = a.p2ct;
+    const T c1 = (T)a.c1, c2 = (T)a.c2, cA = (T)a.cA;
+
+    T U[6][kF];    // y of the own row, z = j .. j+4, and j+5 on its way: slot (phase + z - j) % 6
+    T Y[6][kF];    // inner input, z = j-2 .. j+2: slot (phase + 2 + z - j) % 6 (not OUT: from j on)
+    T E[6][kF];    // not OUT: edge row of y, z = j+2 .. j+5, in the slots of U
+    T uc[kF];      // pair 2: u at z = j+2 (of the next step, once used)
+    auto next = [&](int z) { return z + 1 == nz ? 0 : z + 1; };
+    auto load = [&](unsigned long long base, unsigned v, int z, T (&x)[kF]) {
+        const __amdgpu_buffer_rsrc_t r = prs(base, rbytes);
+#pragma unroll
+        for (int f = 0; f < kF; ++f) x[f] = pld<T>(r, v, (unsigned)z * siteb + f * rowb);
+    };
+    int j = j0 - 4;   // the step; z5, z3, z2: wrapped j+5, j+3, j+2
+    int z5 = uniform(wrapi(j + 5, nz)), z3 = uniform(wrapi(j + 3, nz)), z2 = uniform(wrapi(j + 2, nz));
+    int z1 = uniform(wrapi(j + 1, nz));
+#pragma unroll
+    for (int q = 0; q < 5; ++q) load(a.y + rbase, vo, wrapi(j + q, nz), U[q]);
+    if constexpr (!OUT && !NOX) {
+#pragma unroll
+        for (int q = 2; q < 5; ++q) load(a.y + ebase, ve, wrapi(j + q, nz), E[q]);
+    }
+    if constexpr (PAIR == 2) load(a.u + rbase, vo, z2, uc);
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int f = 0; f < kF; ++f) Y[q][f] = (T)0;
+
+    // phase P: the step's number modulo 6; WRITE: step j0 or later
+    auto step = [&](auto phase, auto write) {
+        constexpr int P = decltype(phase)::value;
+        constexpr bool WRITE = decltype(write)::value;
+        constexpr int b = P & 1;
+        const auto& U0 = U[P % 6];
+        const auto& U1 = U[(P + 1) % 6];
+        const auto& U2 = U[(P + 2) % 6];
+        const auto& U3 = U[(P + 3) % 6];
+        const auto& U4 = U[(P + 4) % 6];
+        const auto& Y0 = Y[P % 6];
+        const auto& Y1 = Y[(P + 1) % 6];
+        const auto& Y2 = Y[(P + 2) % 6];
+        const auto& Y3 = Y[(P + 3) % 6];
+        auto& Y4 = Y[(P + 4) % 6];
+        // ---- loads for the next steps (A: for the end of this one)
+        load(a.y + rbase, vo, z5, U[(P + 5) % 6]);
+        if constexpr (!OUT && !NOX) load(a.y + ebase, ve, z5, E[(P + 5) % 6]);
+        T ac[kF];
+        if constexpr (PAIR == 2 && WRITE) {
+            const __amdgpu_buffer_rsrc_t ra = prs(a.a + rbase, rbytes);
+#pragma unroll
+            for (int f = 0; f < kF; ++f) ac[f] = pld<T, 2>(ra, vo, (unsigned)j * siteb + f * rowb);
+        }
+        // the moment records of the next step: into L2, for the scalar loads
+        const __amdgpu_buffer_rsrc_t rm1 = prs(a.m1 + mrow, mbytes), rm2 = prs(a.m2 + mrow, mbytes);
+        const unsigned w1 = __builtin_amdgcn_raw_buffer_load_b32(rm1, vm, (unsigned)z3 * (kMomStride * 8), 0);
+        unsigned w2 = 0;
+        if constexpr (OUT) w2 = __builtin_amdgcn_raw_buffer_load_b32(rm2, vm, (unsigned)z1 * (kMomStride * 8), 0);
+        // moments of y at z = j + 2 (uniform: scalar loads, which arrive with the
+        // barrier)
+        double m1[kNMom], m2[kNMom];
+        load_moments(a.m1 + mrow + (unsigned)z2 * (kMomStride * 8), m1);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!NOX) {
+#pragma unroll
+            for (int f = 0; f < kF; ++f) lds->y[b][slot_m + 2][f][lane] = U2[f];
+#pragma unroll
+            for (int f = 0; f < kF; ++f) lds->m[b][slot_m][f][lane] = Y2[f];
+            if constexpr (!OUT) {
+#pragma unroll
+                for (int f = 0; f < kF; ++f) lds->y[b][slot_e][f][lane] = E[(P + 2) % 6][f];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        }
+        {   // ---- the inner input at z = j + 2
+            const Precession<T> r1 = precession(k, m1);
+            // (and the inner input's moments at z = j, for the output)
+            if constexpr (OUT && WRITE) load_moments(a.m2 + mrow + (unsigned)j * (kMomStride * 8), m2);
+            __builtin_amdgcn_sched_barrier(0);
+            T kk[kF];
+            rhs_unit<T>(k, r1, U2, U0, U1, U3, U4,
+                        [&](int f, T& xm2, T& xm1, T& xp1, T& xp2) {
+                            if constexpr (NOX) {
+                                xm2 = xm1 = xp1 = xp2 = U2[f];
+                            } else {
+                                xm2 = lds->y[b][slot_m][f][lane];
+                                xm1 = lds->y[b][slot_m + 1][f][lane];
+                                xp1 = lds->y[b][slot_m + 3][f][lane];
+                                xp2 = lds->y[b][slot_m + 4][f][lane];
+                            }
+                        },
+                        kk);
+#pragma unroll
+            for (int f = 0; f < kF; ++f) {
+                Y4[f] = (PAIR == 1 ? U2[f] : uc[f]) + c1 * kk[f];
+                // (not OUT: computed here, not sunk to its use two steps on,
+                // which kept every operand alive and spilled)
+                if constexpr (!OUT) asm volatile("" : "+v"(Y4[f]));
+            }
+        }
+        if constexpr (PAIR == 2) {
+            load(a.u + rbase, vo, z3, uc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (OUT && WRITE) {   // ---- the output at z = j
+            const Precession<T> r2 = precession(k, m2);
+            T kk[kF], yo[kF];
+            rhs_unit<T>(k, r2, Y2, Y0, Y1, Y3, Y4,
+                        [&](int f, T& xm2, T& xm1, T& xp1, T& xp2) {
+                            if constexpr (NOX) {
+                                xm2 = xm1 = xp1 = xp2 = Y2[f];
+                            } else {
+                                xm2 = lds->m[b][slot_m - 2][f][lane];
+                                xm1 = lds->m[b][slot_m - 1][f][lane];
+                                xp1 = lds->m[b][slot_m + 1][f][lane];
+                                xp2 = lds->m[b][slot_m + 2][f][lane];
+                            }
+                        },
+                        kk);
+            const unsigned so = (unsigned)j * siteb;
+            const __amdgpu_buffer_rsrc_t ro = prs(a.out + rbase, rbytes);
+            if constexpr (PAIR == 1) {   // A = Y2 + u + dt k2, Y3 = u + dt/2 k2
+                const __amdgpu_buffer_rsrc_t ra = prs(a.a + rbase, rbytes);
+#pragma unroll
+                for (int f = 0; f < kF; ++f) {
+                    yo[f] = U0[f] + c2 * kk[f];
+                    pst<T>((Y2[f] + U0[f]) + cA * kk[f], ra, vo, so + f * rowb);
+                }
+            } else {                     // u' = (A + Y4) / 3 + dt/6 k4
+                // (1/3 in two parts: a third rounded to T alone grows u by
+                // 3e-8 (FP32) or 6e-17 of itself every step)
+                const T third = (T)(1.0 / 3.0), rest = sizeof(T) == 4 ? (T)(1.0 / 3.0 - (double)third) : (T)kThirdRest;
+#pragma unroll
+                for (int f = 0; f < kF; ++f) {
+                    const T s = ac[f] + Y2[f];
+                    yo[f] = s * third + (s * rest + c2 * kk[f]);
+                }
+            }
+#pragma unroll
+            for (int f = 0; f < kF; ++f) pst<T>(yo[f], ro, vo, so + f * rowb);
+            direction_sums((double)yo[2], (double)yo[3], (double)yo[0] - (double)yo[1], sst, tab, lane,
+                           prs(prow, pbytes), vrec, (unsigned)j * zrec);
+        }
+        asm volatile("" ::"v"(w1), "v"(w2));
+        ++j;
+        z5 = next(z5);
+        z3 = next(z3);
+        z2 = next(z2);
+        z1 = next(z1);
+    };
+    using std::integral_constant;
+    step(integral_constant<int, 0>{}, std::false_type{});
+    step(integral_constant<int, 1>{}, std::false_type{});
+    step(integral_constant<int, 2>{}, std::false_type{});
+    step(integral_constant<int, 3>{}, std::false_type{});
+    for (;;) {
+        step(integral_constant<int, 4>{}, std::true_type{});
+        if (j == j1) break;
+        step(integral_constant<int, 5>{}, std::true_type{});
+        if (j == j1) break;
+        step(integral_constant<int, 0>{}, std::true_type{});
+        if (j == j1) break;
+        step(integral_constant<int, 1>{}, std::true_type{});
+        if (j == j1) break;
+        step(integral_constant<int, 2>{}, std::true_type{});
+        if (j == j1) break;
+        step(integral_constant<int, 3>{}, std::true_type{});
+        if (j == j1) break;
+    }
+}
+
+// logical block -> (x group fastest, unit, z segment): neighbouring blocks,
+// which share edge rows, run on one XCD at about the same time
+template <typename T, int PAIR, int R>
+__device__ __forceinline__ void pair_block(const PairArgs<T>& a, int lb, int wib, PairSlab<T, R>& lds) {
+    const int xg = uniform(lb % a.xgroups), rest = uniform(lb / a.xgroups);
+    const int un = uniform(rest % a.nunits), j0 = uniform(rest / a.nunits) * a.zlen;
+    const int ch = un >> 1, grp = un & 1;
+    const int nx = a.g.nx, j1 = min(a.g.nz, j0 + a.zlen), ib = xg * R;
+    if (wib == 0) fill_table(a.g, lds.tab, ch, threadIdx.x & 63);   // (read after the first barriers)
+    // wave wib works on x row ib - 2 + wib; rows past either end wrap (the box
+    // is periodic), and rows past the last one write nothing
+    const int r = ib - 2 + wib, row = uniform(wrapi(r, nx));
+    if (wib >= 2 && wib < R + 2 && r < nx) {
+        pair_wave<T, PAIR, true, false>(a, row, ch, grp, j0, j1, wib, -1, 0, lds.tab, lds.st[wib - 2], &lds);
+    } else {
+        // the first and last two waves also load the rows beyond: -4, -3, R+2, R+3
+        const bool lo = wib < 2, hi = wib >= R + 2;
+        const int er = lo ? ib - 4 + wib : ib + wib;
+        pair_wave<T, PAIR, false, false>(a, row, ch, grp, j0, j1, wib, lo || hi ? uniform(wrapi(er, nx)) : -1,
+                                         lo ? wib : (hi ? wib + 4 : R + 8), lds.tab, lds.st[0], &lds);
+    }
+}
+
+// Waves per SIMD the register allocation aims at: 12 waves of one block per
+// CU (FP64: its slab takes 137 KB), two blocks in FP32.
+template <typename T>
+constexpr int pair_simd_waves() {
+    return sizeof(T) == 8 ? 3 : 4;
+}
+
+template <typename T, int PAIR>
+__global__ __launch_bounds__(64 * (PairShape<T>::R + 4)) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
+void k_pair(const PairArgs<T> a) {
+    constexpr int R = PairShape<T>::R;
+    __shared__ PairSlab<T, R> lds;
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    pair_block<T, PAIR, R>(a, xcd_remap(blockIdx.x, gridDim.x), wib, lds);
+}
+
+// Many independent runs in one launch: logical block -> (run, block of run)
+// from bmap; each run's arguments from the runs table (read with scalar loads).
+template <typename T, int PAIR>
+__global__ __launch_bounds__(64 * (PairShape<T>::R + 4)) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
+void k_pair_batch(const PairArgs<T>* __restrict__ runs, const int* __restrict__ bmap) {
+    constexpr int R = PairShape<T>::R;
+    __shared__ PairSlab<T, R> lds;
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lb = xcd_remap(blockIdx.x, gridDim.x);
+    const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)bmap;
+    const int run = cm[2 * lb], blk = cm[2 * lb + 1];
+    const PairArgs<T> a = runs[run];   // uniform, read-only: scalar loads
+    pair_block<T, PAIR, R>(a, blk, wib, lds);
+}
+
+// The same work as a persistent kernel: a grid of resident blocks takes
+// logical blocks from a work queue until it is empty.  Logical blocks keep
+// the split of xcd_remap (one contiguous range per XCD, block b of the grid
+// runs on XCD b % 8), and each XCD's blocks draw from their range through
+// their own counter ctr[x], so neighbouring logical blocks still run on one
+// XCD at about the same time.  Every block leaves the loop once its XCD's
+// counter passes the range (the exit every wave reaches); the counters are
+// zeroed by k_zero_ints before each launch.
+template <typename T, int PAIR>
+__global__ __launch_bounds__(64 * (PairShape<T>::R + 4)) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
+void k_pair_batch_q(const PairArgs<T>* __restrict__ runs, const int* __restrict__ bmap, int* __restrict__ ctr,
+                    int nitems) {
+    constexpr int R = PairShape<T>::R;
+    __shared__ PairSlab<T, R> lds;
+    __shared__ int next;
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int x = blockIdx.x % 8;
+    const int per = nitems / 8, rem = nitems % 8;
+    const int start = x < rem ? x * (per + 1) : rem * (per + 1) + (x - rem) * per;
+    const int count = per + (x < rem ? 1 : 0);
+    const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)bmap;
+    for (;;) {
+        if (threadIdx.x == 0) next = atomicAdd(&ctr[x], 1);
+        __syncthreads();   // (also: every wave is done with the slab of the last block)
+        const int k = __builtin_amdgcn_readfirstlane(next);
+        __syncthreads();   // every wave has read next before thread 0 rewrites it
+        if (k >= count) break;
+        const int lb = start + k;
+        const int run = cm[2 * lb], blk = cm[2 * lb + 1];
+        const PairArgs<T> a = runs[run];   // uniform, read-only: scalar loads
+        pair_block<T, PAIR, R>(a, blk, wib, lds);
+    }
+}
+
+__global__ void k_zero_ints(int* __restrict__ p, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = 0;
+}
+
+constexpr int kRowWaves = 4;   // waves per block of the one-row form, a unit each
+
+template <typename T, int PAIR>
+__global__ __launch_bounds__(64 * kRowWaves) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
+void k_pair_row(const PairArgs<T> a) {
+    __shared__ PairRowLds<kRowWaves> lds;
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lb = xcd_remap(blockIdx.x, gridDim.x);
+    const int groups = (a.nunits + kRowWaves - 1) / kRowWaves;
+    const int un = uniform(lb % groups) * kRowWaves + wib, j0 = uniform(lb / groups) * a.zlen;
+    if (un >= a.nunits) return;
+    fill_table(a.g, lds.tab[wib], un >> 1, threadIdx.x & 63);   // (the wave's own: its LDS accesses stay in order)
+    pair_wave<T, PAIR, true, true>(a, 0, un >> 1, un & 1, j0, min(a.g.nz, j0 + a.zlen), 0, -1, 0, lds.tab[wib],
+                                   lds.st[wib], (PairRowLds<kRowWaves>*)nullptr);
+}
+
+// ---------------------------------------------------------------------------
+// partial sums of a state (after init, upload or renormalisation): a wave per
+// unit and run of sites
+// ---------------------------------------------------------------------------
+constexpr int kSumSites = 16;   // sites per wave
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_pair_sums(const Geometry g, const T* __restrict__ y, double* __restrict__ part) {
+    __shared__ PairRowLds<4> lds;
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const long long nsites = (long long)g.nx * g.nz, runs = (nsites + kSumSites - 1) / kSumSites;
+    const long long id = (long long)blockIdx.x * 4 + wib;
+    const int nu = 2 * g.nch;
+    if (id >= runs * nu) return;
+    const int un = (int)(id % nu), ch = un >> 1, grp = un & 1;
+    fill_table(g, lds.tab[wib], ch, lane);
+    const int pv = min(ch * 64 + lane, g.nv - 1);
+    const long long s0 = id / nu * kSumSites, s1 = min(nsites, s0 + kSumSites);
+    const unsigned vrec = sum_offset(lane, kRec * 8);
+    for (long long s = s0; s < s1; ++s) {
+        const T* p = y + site_off(g, s) + (long long)(grp * kF) * g.nvp + pv;
+        const double ee = p[0], mm = p[g.nvp], emr = p[2 * (long long)g.nvp], emi = p[3 * (long long)g.nvp];
+        direction_sums(emr, emi, ee - mm, lds.st[wib], lds.tab[wib], lane,
+                       prs((unsigned long long)(part + (s * g.nch + ch) * kPairRec + grp * kRec), kRec * 8), vrec, 0);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// totals of a site's partial sums in chunk order, and the moments they give
+// ---------------------------------------------------------------------------
+template <bool COMP>
+__device__ __forceinline__ void pair_totals_body(const double* __restrict__ part, int nch, long long nsites,
+                                                 double* __restrict__ tot, long long n) {
+    if (n >= nsites * kPairRec) return;
+    const long long site = n / kPairRec;
+    const double* rec = part + site * nch * kPairRec + n % kPairRec;
+    double sum = rec[0], err = 0.0;
+    for (int c = 1; c < nch; ++c) {
+        const double x = rec[(long long)c * kPairRec];
+        if constexpr (COMP) {   // (FP32 form: as k_moment_totals)
+            const double s = sum + x, bb = s - sum;
+            err += (sum - (s - bb)) + (x - bb);
+            sum = s;
+        } else {
+            sum += x;
+        }
+    }
+    tot[n] = sum + err;
+}
+
+struct PredictArgs {
+    const double* tot;    // [site][2][kMono][3]
+    const double* base;   // what the prediction starts from (an m, or null: that of tot's state)
+    double* m;            // mu times the moments of tot's state
+    double* inner;        // mu times the moments of base + c k
+    double c;
+    double mu, mu2, p2st, p2ct, pmo, ct2, st;
+    double twelve_dx, twelve_dz, ko_x, ko_z;
+    int nx, nz;
+};
+
+// index of u_a u_b among the monomials; yy (a = b = 2) is 1 - xx - zz
+__device__ __forceinline__ double second(const double* t, int a, int b, int c) {
+    const int lo = min(a, b), hi = max(a, b);
+    if (lo == 0) return t[hi * 3 + c];
+    if (lo == 2 && hi == 2) return t[c] - t[4 * 3 + c] - t[8 * 3 + c];
+    return t[(lo == 1 ? 3 + hi : 5 + lo) * 3 + c];   // xx, xy, xz; yz, zz
+}
+
+// Thread (site, s): moment component a = s % 4 of vector s / 4 (A: bemr - emr,
+// B: bemi + emi, C: bee - bmm - ee + mm).  The moments of k follow
+// nuosc_class.cpp:115-287 summed over directions with w u_a.
+__device__ __forceinline__ void predict_body(const PredictArgs& p, long long n) {
+    const long long nsites = (long long)p.nx * p.nz;
+    const long long site = n / kMomStride;
+    const int s = (int)(n % kMomStride);
+    if (site >= nsites) return;
+    if (s >= kNMom) {
+        p.m[n] = p.inner[n] = 0.0;
+        return;
+    }
+    const int a = s & 3, v = s >> 2;
+    const int i = (int)(site / p.nz), j = (int)(site % p.nz);
+    const double* t = p.tot + site * kPairRec;
+    const double* tb = t + kRec;
+    // the vector's combination of the two halves: bar - nu, bar + nu, bar - nu
+    const double sg = v == 1 ? 1.0 : -1.0;
+    auto comb = [&](const double* q, int b) { return second(q + kRec, a, b, v) + sg * second(q, a, b, v); };
+    const double m0 = t[kRec + a * 3 + v] + sg * t[a * 3 + v];
+    // transport: advection multiplies by vx or vz, Kreiss-Oliger by nothing
+    double kt = 0.0;
+#pragma unroll
+    for (int ax = 0; ax < 2; ++ax) {
+        double d[4], e[4];
+        const int b = ax ? 3 : 1;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int o = q < 2 ? q - 2 : q - 1;
+            const long long ns = ax ? (long long)i * p.nz + wrapi(j + o, p.nz) : (long long)wrapi(i + o, p.nx) * p.nz + j;
+            const double* tn = p.tot + ns * kPairRec;
+            d[q] = comb(tn, b);
+            e[q] = tn[kRec + a * 3 + v] + sg * tn[a * 3 + v];
+        }
+        kt += -((d[0] - d[3]) - 8.0 * (d[1] - d[2])) / (ax ? p.twelve_dz : p.twelve_dx);
+        kt += (ax ? p.ko_z : p.ko_x) * (e[0] + e[3] - 4 * (e[1] + e[2]) + 6 * m0);
+    }
+    // interaction: sum over b of s_b (moment b) (second moment a b), s = (1, -1, -1, -1)
+    double loc = 0.0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const double Ab = tb[b * 3] - t[b * 3], Bb = tb[b * 3 + 1] + t[b * 3 + 1], Cb = tb[b * 3 + 2] - t[b * 3 + 2];
+        double x;
+        if (v == 0)        // k_emr of bar minus nu: -mu [ d3 B + (bemi - emi) C ]
+            x = -p.mu * ((second(tb, a, b, 2) - second(t, a, b, 2)) * Bb + Cb * (second(tb, a, b, 1) - second(t, a, b, 1)));
+        else if (v == 1)   // k_emi: mu [ -(bee - bmm + ee - mm) A + (bemr + emr) C ]
+            x = p.mu * (Cb * (second(tb, a, b, 0) + second(t, a, b, 0)) - (second(tb, a, b, 2) + second(t, a, b, 2)) * Ab);
+        else               // k_ee - k_mm = 2 k_ee: 2 mu2 [ (bemi - emi) A + (bemr - emr) B ]
+            x = 2 * p.mu2 * ((second(tb, a, b, 1) - second(t, a, b, 1)) * Ab + (second(tb, a, b, 0) - second(t, a, b, 0)) * Bb);
+        loc += b == 0 ? x : -x;
+    }
+    const double r1 = tb[a * 3] + t[a * 3], i1 = tb[a * 3 + 1] - t[a * 3 + 1], e1 = tb[a * 3 + 2] + t[a * 3 + 2];
+    const double vac = v == 0 ? -p.p2ct * i1 : (v == 1 ? p.pmo * (p.ct2 * r1 + p.st * e1) : -2 * p.p2st * i1);
+    const double mm = p.mu * m0;
+    p.m[n] = mm;
+    p.inner[n] = (p.base ? p.base[n] : mm) + p.mu * (p.c * (loc + kt + vac));
+}
+
+template <bool COMP>
+__global__ __launch_bounds__(256) void k_pair_totals(const double* __restrict__ part, int nch, long long nsites,
+                                                     double* __restrict__ tot) {
+    pair_totals_body<COMP>(part, nch, nsites, tot, (long long)blockIdx.x * 256 + threadIdx.x);
+}
+__global__ __launch_bounds__(256) void k_pair_predict(const PredictArgs p) {
+    predict_body(p, (long long)blockIdx.x * 256 + threadIdx.x);
+}
+
+struct SumArgs {
+    const double* part;
+    double* tot;
+    int nch;
+    long long nsites;
+};
+template <bool COMP>
+__global__ __launch_bounds__(256) void k_pair_totals_batch(const SumArgs* __restrict__ runs, const int* __restrict__ map) {
+    const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)map;
+    const SumArgs a = runs[cm[2 * blockIdx.x]];
+    pair_totals_body<COMP>(a.part, a.nch, a.nsites, a.tot, (long long)cm[2 * blockIdx.x + 1] * 256 + threadIdx.x);
+}
+__global__ __launch_bounds__(256) void k_pair_predict_batch(const PredictArgs* __restrict__ runs, const int* __restrict__ map) {
+    const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)map;
+    const PredictArgs p = runs[cm[2 * blockIdx.x]];
+    predict_body(p, (long long)cm[2 * blockIdx.x + 1] * 256 + threadIdx.x);
+}
+
+template <typename T>
+PairArgs<T> pair_args(const Geometry& g, const Physics& ph, int zlen, int pair, const PairBuffers& b, double dt) {
+    PairArgs<T> a{};
+    a.g = g;
+    a.y = (unsigned long long)(pair == 1 ? b.u : b.y3);
+    a.u = (unsigned long long)b.u;
+    a.a = (unsigned long long)b.a;
+    a.out = (unsigned long long)(pair == 1 ? b.y3 : b.unew);
+    a.m1 = (unsigned long long)(pair == 1 ? b.mu : b.m3);
+    a.m2 = (unsigned long long)b.min;
+    a.part = (unsigned long long)b.part;
+    a.c1 = pair == 1 ? 0.5 * dt : dt;
+    a.c2 = pair == 1 ? 0.5 * dt : 1.0 / 6.0 * dt;
+    a.cA = dt;
+    a.pst = ph.pmo * ph.st;
+    a.p2ct = ph.pmo * 2 * ph.ct;
+    a.zlen = zlen;
+    a.xgroups = g.nx == 1 ? 1 : (g.nx + PairShape<T>::R - 1) / PairShape<T>::R;
+    a.nunits = 2 * g.nch;
+    return a;
+}
+
+PredictArgs predict_args(const Geometry& g, const Physics& ph, int pair, const PairBuffers& b, double dt) {
+    PredictArgs p{};
+    p.tot = b.tot;
+    p.base = pair == 1 ? nullptr : b.mu;
+    p.m = pair == 1 ? b.mu : b.m3;
+    p.inner = b.min;
+    p.c = pair == 1 ? 0.5 * dt : dt;
+    p.mu = ph.mu;
+    p.mu2 = 2 * ph.mu;
+    p.p2st = ph.pmo * 2 * ph.st;
+    p.p2ct = ph.pmo * 2 * ph.ct;
+    p.pmo = ph.pmo;
+    p.ct2 = 2 * ph.ct;
+    p.st = ph.st;
+    p.twelve_dx = g.twelve_dx;
+    p.twelve_dz = g.twelve_dz;
+    p.ko_x = g.ko_x;
+    p.ko_z = g.ko_z;
+    p.nx = g.nx;
+    p.nz = g.nz;
+    return p;
+}
+
+unsigned blocks_of(long long n) { return (unsigned)((n + 255) / 256); }
+
+}  // namespace
+
+bool pair_capable(const Geometry& g) {
+    return g.nf == kNVar && g.bc == 0 && !g.ko5 && g.adv == kAdvCfd4;
+}
+
+int pair_blocks(const Geometry& g, int esize, int zlen) {
+    const long long nseg = (g.nz + zlen - 1) / zlen, nu = 2ll * g.nch;
+    const int R = esize == 8 ? PairShape<double>::R : PairShape<float>::R;
+    return (int)(nseg * (g.nx == 1 ? (nu + kRowWaves - 1) / kRowWaves : nu * ((g.nx + R - 1) / R)));
+}
+
+int pair_waves(const Geometry& g, int esize, int zlen) {
+    const int R = esize == 8 ? PairShape<double>::R : PairShape<float>::R;
+    return pair_blocks(g, esize, zlen) * (g.nx == 1 ? kRowWaves : R + 4);
+}
+
+// Longest segments that still give every CU a block (every segment starts
+// with four steps that write nothing).
+int plan_pair_zlen(const Geometry& g, int esize, int num_cus) {
+    const int want = g.nx == 1 ? 3 * num_cus : num_cus;
+    int zlen = g.nz;
+    while (zlen > 8 && pair_blocks(g, esize, zlen) < want) zlen = (zlen + 1) / 2;
+    while (zlen > 128 && pair_blocks(g, esize, zlen) < 8 * want) zlen = (zlen + 1) / 2;
+    return zlen;
+}
+
+template <typename T>
+hipError_t launch_pair(int pair, const Geometry& g, const Physics& ph, int zlen, const PairBuffers& b, double dt,
+                       hipStream_t s) {
+    if (!pair_capable(g) || zlen < 1 || g.lpr != 64) return hipErrorInvalidValue;
+    const PairArgs<T> a = pair_args<T>(g, ph, zlen, pair, b, dt);
+    const dim3 grid((unsigned)pair_blocks(g, sizeof(T), zlen));
+    if (g.nx == 1) {
+        if (pair == 1) hipLaunchKernelGGL((k_pair_row<T, 1>), grid, dim3(64 * kRowWaves), 0, s, a);
+        else hipLaunchKernelGGL((k_pair_row<T, 2>), grid, dim3(64 * kRowWaves), 0, s, a);
+    } else {
+        const dim3 block(64 * (PairShape<T>::R + 4));
+        if (pair == 1) hipLaunchKernelGGL((k_pair<T, 1>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_pair<T, 2>), grid, block, 0, s, a);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_pair_predict(int pair, const Geometry& g, const Physics& ph, const PairBuffers& b, double dt,
+                               hipStream_t s) {
+    const PredictArgs p = predict_args(g, ph, pair, b, dt);
+    hipLaunchKernelGGL(k_pair_predict, dim3(blocks_of((long long)g.nx * g.nz * kMomStride)), dim3(256), 0, s, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_pair_totals(const Geometry& g, bool compensated, const PairBuffers& b, hipStream_t s) {
+    const long long nsites = (long long)g.nx * g.nz;
+    const dim3 grid(blocks_of(nsites * kPairRec));
+    if (compensated) hipLaunchKernelGGL((k_pair_totals<true>), grid, dim3(256), 0, s, b.part, g.nch, nsites, b.tot);
+    else hipLaunchKernelGGL((k_pair_totals<false>), grid, dim3(256), 0, s, b.part, g.nch, nsites, b.tot);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_pair_sums(const Geometry& g, const T* y, double* part, hipStream_t s) {
+    const long long runs = ((long long)g.nx * g.nz + kSumSites - 1) / kSumSites;
+    hipLaunchKernelGGL((k_pair_sums<T>), dim3((unsigned)((runs * 2 * g.nch + 3) / 4)), dim3(256), 0, s, g, y, part);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// batched runs: the launches of a step for every member run; the runs keep
+// their own buffers, segments and physics.  All tables live in one device
+// buffer, [pairs 1, 2] x [flips 0, 1] of arguments and the block maps, and a
+// rebuild (a member joins or leaves) reuses it.
+// ---------------------------------------------------------------------------
+namespace {
+
+template <typename T>
+hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hipStream_t s) {
+    const int n = (int)ms.size();
+    std::vector<char> host;
+    auto put = [&](const void* p, size_t bytes) {
+        const size_t at = (host.size() + 255) / 256 * 256;
+        host.resize(at + bytes);
+        std::memcpy(host.data() + at, p, bytes);
+        return at;
+    };
+    // pair, totals and predict blocks -> (member, block of member)
+    std::vector<long long> count[3];
+    for (const BatchMember& m : ms) {
+        const Geometry& g = m.g;
+        const long long sites = (long long)g.nx * g.nz, nseg = (g.nz + m.zlen - 1) / m.zlen;
+        // (the box form for every member, one-row grids included)
+        count[0].push_back(nseg * 2 * g.nch * ((g.nx + PairShape<T>::R - 1) / PairShape<T>::R));
+        count[1].push_back((sites * kPairRec + 255) / 256);
+        count[2].push_back((sites * kMomStride + 255) / 256);
+    }
+    auto put_map = [&](const std::vector<long long>& c, int& blocks) {
+        long long total = 0;
+        for (long long k : c) total += k;
+        blocks = (int)total;
+        const size_t at = (host.size() + 255) / 256 * 256;
+        host.resize(at + total * 2 * sizeof(int));
+        int* p = (int*)(host.data() + at);
+        for (int r = 0; r < n; ++r)
+            for (int b = 0; b < (int)c[r]; ++b) {
+                *p++ = r;
+                *p++ = b;
+            }
+        return at;
+    };
+    size_t off_args[2][2], off_pre[2][2], off_map[3];
+    for (int flip = 0; flip < 2; ++flip)
+        for (int pair = 1; pair <= 2; ++pair) {
+            std::vector<PairArgs<T>> pa(n);
+            std::vector<PredictArgs> pp(n);
+            for (int r = 0; r < n; ++r) {
+                PairBuffers b = ms[r].b;
+                if (flip) {
+                    const void* u = b.u;
+                    b.u = b.unew;
+                    b.unew = const_cast<void*>(u);
+                }
+                pa[r] = pair_args<T>(ms[r].g, ms[r].ph, ms[r].zlen, pair, b, ms[r].dt);
+                pp[r] = predict_args(ms[r].g, ms[r].ph, pair, b, ms[r].dt);
+            }
+            off_args[pair - 1][flip] = put(pa.data(), n * sizeof(PairArgs<T>));
+            off_pre[pair - 1][flip] = put(pp.data(), n * sizeof(PredictArgs));
+        }
+    std::vector<SumArgs> sa(n);
+    for (int r = 0; r < n; ++r)
+        sa[r] = SumArgs{ms[r].b.part, ms[r].b.tot, ms[r].g.nch, (long long)ms[r].g.nx * ms[r].g.nz};
+    const size_t off_sum = put(sa.data(), n * sizeof(SumArgs));
+    int blocks[3];
+    for (int k = 0; k < 3; ++k) off_map[k] = put_map(count[k], blocks[k]);
+    const std::vector<int> zeros(kBatchCounters, 0);
+    const size_t off_ctr = put(zeros.data(), kBatchCounters * sizeof(int));
+    hipError_t e;
+    if (t.bytes < host.size()) {
+        batch_free(t);
+        if ((e = hipMalloc(&t.buf, host.size())) != hipSuccess) return e;
+        t.bytes = host.size();
+    }
+    char* d = static_cast<char*>(t.buf);
+    for (int p = 0; p < 2; ++p)
+        for (int flip = 0; flip < 2; ++flip) {
+            t.args[p][flip] = d + off_args[p][flip];
+            t.pre[p][flip] = d + off_pre[p][flip];
+        }
+    t.sum = d + off_sum;
+    t.bmap = (int*)(d + off_map[0]);
+    t.tmap = (int*)(d + off_map[1]);
+    t.pmap = (int*)(d + off_map[2]);
+    t.ctr = (int*)(d + off_ctr);
+    t.nblocks = blocks[0];
+    t.tblocks = blocks[1];
+    t.pblocks = blocks[2];
+    // persistent launch: a grid of as many blocks as the GPU holds at once
+    {
+        int dev = 0, cus = 0, bpc = 0;
+        if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
+        if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
+        if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_pair_batch_q<T, 2>, 64 * (PairShape<T>::R + 4), 0)) !=
+            hipSuccess)
+            return e;
+        t.pgrid = std::max(8, (cus * std::max(bpc, 1) + 7) / 8 * 8);
+    }
+    if ((e = hipMemcpyAsync(t.buf, host.data(), host.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return e;
+    return hipStreamSynchronize(s);
+}
+
+template <typename T>
+hipError_t batch_pair_t(const BatchTables& t, int pair, int flip, hipStream_t s) {
+    const dim3 block(64 * (PairShape<T>::R + 4));
+    const PairArgs<T>* a = (const PairArgs<T>*)t.args[pair - 1][flip];
+    if (t.launch == kBatchPersistent) {
+        int* c = t.ctr + 8 * (pair - 1);
+        hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, c, 8);   // a kernel node, not a memset, in graphs
+        const dim3 pg(t.pgrid);
+        if (pair == 1) hipLaunchKernelGGL((k_pair_batch_q<T, 1>), pg, block, 0, s, a, t.bmap, c, t.nblocks);
+        else hipLaunchKernelGGL((k_pair_batch_q<T, 2>), pg, block, 0, s, a, t.bmap, c, t.nblocks);
+        return hipGetLastError();
+    }
+    if (pair == 1) hipLaunchKernelGGL((k_pair_batch<T, 1>), dim3(t.nblocks), block, 0, s, a, t.bmap);
+    else hipLaunchKernelGGL((k_pair_batch<T, 2>), dim3(t.nblocks), block, 0, s, a, t.bmap);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t batch_build(BatchTables& t, const std::vector<BatchMember>& ms, int esize, int launch, hipStream_t s) {
+    t.esize = esize;
+    t.launch = launch;
+    t.nblocks = 0;
+    if (ms.empty()) return hipSuccess;
+    for (const auto& m : ms)
+        if (!pair_capable(m.g) || m.zlen < 1 || m.g.lpr != 64) return hipErrorInvalidValue;
+    return esize == 8 ? batch_build_t<double>(t, ms, s) : batch_build_t<float>(t, ms, s);
+}
+
+void batch_free(BatchTables& t) {
+    if (t.buf) (void)hipFree(t.buf);
+    t.buf = nullptr;
+    t.bytes = 0;
+    t.nblocks = 0;
+}
+
+hipError_t batch_pair(const BatchTables& t, int pair, int flip, hipStream_t s) {
+    if (t.nblocks == 0) return hipSuccess;
+    return t.esize == 8 ? batch_pair_t<double>(t, pair, flip, s) : batch_pair_t<float>(t, pair, flip, s);
+}
+
+hipError_t batch_step(const BatchTables& t, int flip, hipStream_t s) {
+    if (t.nblocks == 0) return hipSuccess;
+    for (int pair = 1; pair <= 2; ++pair) {
+        hipLaunchKernelGGL(k_pair_predict_batch, dim3(t.pblocks), dim3(256), 0, s,
+                           (const PredictArgs*)t.pre[pair - 1][flip], t.pmap);
+        const hipError_t e = batch_pair(t, pair, flip, s);
+        if (e != hipSuccess) return e;
+        const dim3 tg(t.tblocks), tb(256);
+        if (t.esize == 4) hipLaunchKernelGGL((k_pair_totals_batch<true>), tg, tb, 0, s, (const SumArgs*)t.sum, t.tmap);
+        else hipLaunchKernelGGL((k_pair_totals_batch<false>), tg, tb, 0, s, (const SumArgs*)t.sum, t.tmap);
+    }
+    return hipGetLastError();
+}
+
+#define NUOSC_PAIR_INST(T)                                                                                        \
+    template hipError_t launch_pair<T>(int, const Geometry&, const Physics&, int, const PairBuffers&, double,     \
+                                       hipStream_t);                                                              \
+    template hipError_t launch_pair_sums<T>(const Geometry&, const T*, double*, hipStream_t);
+NUOSC_PAIR_INST(double)
+NUOSC_PAIR_INST(float)
+#undef NUOSC_PAIR_INST
+
+}  // namespace nuosc
