@@ -221,6 +221,9 @@ int nuosc_renormalize(nuosc_sim* sim);
  * upload_field: one field from the interior layout.  After uploading all the
  *   fields call nuosc_state_updated to refresh the velocity moments. */
 int nuosc_download_field(nuosc_sim* sim, int field, double* host);
+/* several fields at once, [field][nx][nz][nv]: f0, f0 + 1, ..., nf of them */
+int nuosc_download_fields(nuosc_sim* sim, int f0, int nf, double* host);
+int nuosc_upload_fields(nuosc_sim* sim, int f0, int nf, const double* host);
 int nuosc_download_field_ghosted(nuosc_sim* sim, int field, double* host);
 int nuosc_upload_field(nuosc_sim* sim, int field, const double* host);
 int nuosc_state_updated(nuosc_sim* sim);

@@ -123,6 +123,8 @@ SIGNATURES = {
     "nuosc_analysis": ([_vp, C.POINTER(Analysis)], C.c_int),
     "nuosc_renormalize": ([_vp], C.c_int),
     "nuosc_download_field": ([_vp, C.c_int, _dp], C.c_int),
+    "nuosc_download_fields": ([_vp, C.c_int, C.c_int, _dp], C.c_int),
+    "nuosc_upload_fields": ([_vp, C.c_int, C.c_int, _dp], C.c_int),
     "nuosc_download_field_ghosted": ([_vp, C.c_int, _dp], C.c_int),
     "nuosc_upload_field": ([_vp, C.c_int, _dp], C.c_int),
     "nuosc_state_updated": ([_vp], C.c_int),
@@ -343,7 +345,7 @@ class NuOsc:
         """RHS of an interior state array (nvar, nx, nz, nv) -> (nvar, nx, nz, nv)."""
         a = np.ascontiguousarray(state, dtype=np.float64)
         assert a.shape == (self.nvar, self.nx, self.nz, self.nv)
-        out = np.zeros_like(a)
+        out = np.empty_like(a)
         self._check(lib().nuosc_calrhs(self._h, _ptr(a), _ptr(out)))
         return out
 
@@ -359,12 +361,14 @@ class NuOsc:
 
     # -- state transfer ---------------------------------------------------
     def get_field(self, f):
-        out = np.zeros(self.nx * self.nz * self.nv)
+        out = np.empty((self.nx, self.nz, self.nv))
         self._check(lib().nuosc_download_field(self._h, int(f), _ptr(out)))
-        return out.reshape(self.nx, self.nz, self.nv)
+        return out
 
     def get_state(self):
-        return np.stack([self.get_field(f) for f in range(self.nvar)])
+        out = np.empty((self.nvar, self.nx, self.nz, self.nv))
+        self._check(lib().nuosc_download_fields(self._h, 0, self.nvar, _ptr(out)))
+        return out
 
     def get_field_ghosted(self, f):
         shp = (self.nx + 2 * self.gx, self.nz + 2 * self.gz, self.nv)
@@ -375,8 +379,7 @@ class NuOsc:
     def set_state(self, state):
         a = np.asarray(state, dtype=np.float64)
         assert a.shape == (self.nvar, self.nx, self.nz, self.nv)
-        for f in range(self.nvar):
-            self._check(lib().nuosc_upload_field(self._h, f, _ptr(np.ascontiguousarray(a[f]).reshape(-1))))
+        self._check(lib().nuosc_upload_fields(self._h, 0, self.nvar, _ptr(np.ascontiguousarray(a))))
         self._check(lib().nuosc_state_updated(self._h))
 
     def p3_slice(self, xidx, vidx, noalloc=False):
@@ -385,7 +388,7 @@ class NuOsc:
         slice size is bounded)."""
         xi = np.ascontiguousarray(xidx, dtype=np.int32)
         vi = np.ascontiguousarray(vidx, dtype=np.int32)
-        out = np.zeros(len(xi) * self.nz * len(vi))
+        out = np.empty(len(xi) * self.nz * len(vi))
         fn = lib().nuosc_p3_slice_noalloc if noalloc else lib().nuosc_p3_slice
         self._check(fn(self._h, xi.ctypes.data_as(_ip), len(xi), vi.ctypes.data_as(_ip), len(vi), _ptr(out)))
         return out.reshape(len(xi), self.nz, len(vi))

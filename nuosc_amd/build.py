@@ -37,7 +37,7 @@ HOST_FLAGS = [
 ]
 
 KERNEL_SRCS = ["nuosc_kernels.hip", "nuosc_pair.hip", "nuosc_flavor3.hip", "nuosc_noalloc.hip"]
-HOST_SRCS = ["nuosc_capi.cpp", "vgrid.cpp", "nuosc_serve.cpp"]
+HOST_SRCS = ["nuosc_capi.cpp", "nuosc_xfer.cpp", "vgrid.cpp", "nuosc_serve.cpp"]
 CLI_SRCS = ["NuOsc.cpp", "nuosc_main.cpp"]
 
 

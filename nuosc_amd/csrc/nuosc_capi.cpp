@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "nuosc_dev.h"
+#include "nuosc_xfer.h"
 #include "vgrid.h"
 
 using namespace nuosc;
@@ -514,6 +515,42 @@ int fill_state_ghosts(nuosc_sim* s, void* y) {
     return NUOSC_OK;
 }
 
+// total doubles in chunks of at most a slot, through pinned slots: down fills
+// host from kernel launches, up the other way round; at(n0, cnt, slot)
+// launches the kernel of elements [n0, n0 + cnt).  Pieces small enough that
+// the threads share even a transfer of a few MB.
+template <typename F>
+int transfer(nuosc_sim* s, bool down, double* host, long long total, F at) {
+    const long long most = kSlotBytes / sizeof(double);
+    const long long chunk = std::min(most, std::max(most / 8, (total + kXferThreads - 1) / kXferThreads));
+    auto count = [&](long long c) { return std::min(chunk, total - c * chunk); };
+    const hipError_t e = xfer_run(
+        s->cfg.device, s->stream, (total + chunk - 1) / chunk, down,
+        [&](long long c, void* slot) { return at(c * chunk, count(c), static_cast<double*>(slot)); },
+        [&](long long c, void* slot) {
+            double* h = host + c * chunk;
+            std::memcpy(down ? h : slot, down ? slot : h, sizeof(double) * (size_t)count(c));
+        });
+    if (e == hipErrorOutOfMemory) return fail(s, NUOSC_ENOMEM, "staging buffer allocation failed");
+    HIPCK(s, e);
+    return NUOSC_OK;
+}
+
+// fields f0 .. f0 + nf - 1 of the state copy y <-> host [f][nx][nz][nv]
+int fields_down(nuosc_sim* s, const void* y, int f0, int nf, double* host) {
+    return transfer(s, true, host, (long long)nf * s->nx * s->nz * s->nv, [&](long long n0, long long cnt, double* slot) {
+        return is64(s) ? launch_pack<double>(s->geo, (const double*)y, f0, n0, cnt, slot, s->stream)
+                       : launch_pack<float>(s->geo, (const float*)y, f0, n0, cnt, slot, s->stream);
+    });
+}
+int fields_up(nuosc_sim* s, void* y, int f0, int nf, const double* host) {
+    return transfer(s, false, const_cast<double*>(host), (long long)nf * s->nx * s->nz * s->nv,
+                    [&](long long n0, long long cnt, double* slot) {
+                        return is64(s) ? launch_unpack<double>(s->geo, slot, (double*)y, f0, n0, cnt, s->stream)
+                                       : launch_unpack<float>(s->geo, slot, (float*)y, f0, n0, cnt, s->stream);
+                    });
+}
+
 int set_device_time(nuosc_sim* s) {
     if (!s->d_time) return NUOSC_OK;
     HIPCK(s, hipMemcpyAsync(s->d_time, &s->phy_time, sizeof(double), hipMemcpyHostToDevice, s->stream));
@@ -625,17 +662,18 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
     if (c.device < 0 || c.device >= ndev) return fail(nullptr, NUOSC_EINVAL, "device ordinal out of range");
 
     nuosc_sim* s = new nuosc_sim();
+    xfer_retain();
     s->cfg = c;
     s->nf = (c.nflavor == 3) ? kNVar3 : kNVar;
     // CartGrid.cpp:197-201
     s->nx = int((c.x1 - c.x0) / c.dx);
     s->nz = int((c.z1 - c.z0) / c.dz);
     if (s->nx < 1 || s->nz < 1) {
-        delete s;
+        nuosc_destroy(s);
         return fail(nullptr, NUOSC_EINVAL, "empty grid");
     }
     if (c.bc == NUOSC_BC_OPEN_Z && s->nz < 3) {
-        delete s;
+        nuosc_destroy(s);
         return fail(nullptr, NUOSC_EINVAL, "the open z boundary needs nz >= 3 (quadratic outflow extrapolation)");
     }
     const int zoff = (c.bc == NUOSC_BC_OPEN_Z) ? c.gz : 0;
@@ -654,7 +692,7 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
     {
         const CopyLayout L = copy_layout(s->nx, s->nz, nzs, s->nvp, s->nch, (int)s->esize, s->nf);
         if (!L.ok) {
-            delete s;
+            nuosc_destroy(s);
             return fail(nullptr, NUOSC_EINVAL,
                         "grid too large for one GPU handle: a few stored x rows (nz * nv) or the moment records "
                         "(nx * nz * nv) exceed 4 GiB");
@@ -784,6 +822,7 @@ int nuosc_destroy(nuosc_sim* s) {
     if (s->ev0) (void)hipEventDestroy(s->ev0);
     if (s->ev1) (void)hipEventDestroy(s->ev1);
     if (s->stream) (void)hipStreamDestroy(s->stream);
+    xfer_release();
     delete s;
     return NUOSC_OK;
 }
@@ -1092,15 +1131,8 @@ int nuosc_autotune(nuosc_sim* s, int trials, int* best_zlen, double* best_ms) {
 
 int nuosc_calrhs(nuosc_sim* s, const double* in, double* out) {
     if (!s || !in || !out) return NUOSC_EINVAL;
-    const size_t fbytes = sizeof(double) * (size_t)s->nx * s->nz * s->nv;
-    int rc = ensure_tmp(s, fbytes);
+    int rc = fields_up(s, s->st_ya, 0, s->nf, in);
     if (rc) return rc;
-    const size_t fe = (size_t)s->nx * s->nz * s->nv;
-    for (int f = 0; f < s->nf; ++f) {
-        HIPCK(s, hipMemcpyAsync(s->d_tmp, in + f * fe, fbytes, hipMemcpyHostToDevice, s->stream));
-        if (is64(s)) HIPCK(s, launch_unpack<double>(s->geo, s->d_tmp, (double*)s->st_ya, f, s->stream));
-        else HIPCK(s, launch_unpack<float>(s->geo, s->d_tmp, (float*)s->st_ya, f, s->stream));
-    }
     rc = fill_state_ghosts(s, s->st_ya);
     if (rc) return rc;
     if (s->nf == kNVar3) {
@@ -1124,13 +1156,7 @@ int nuosc_calrhs(nuosc_sim* s, const double* in, double* out) {
         HIPCK(s, launch_stage<float>(0, s->geo, s->ph, s->plan, (float*)s->st_ya, nullptr, nullptr,
                                      (float*)s->st_yb, s->mom_a, nullptr, 0.0, 0.0, s->stream));
     }
-    for (int f = 0; f < s->nf; ++f) {
-        if (is64(s)) HIPCK(s, launch_pack<double>(s->geo, (double*)s->st_yb, f, s->d_tmp, s->stream));
-        else HIPCK(s, launch_pack<float>(s->geo, (float*)s->st_yb, f, s->d_tmp, s->stream));
-        HIPCK(s, hipMemcpyAsync(out + f * fe, s->d_tmp, fbytes, hipMemcpyDeviceToHost, s->stream));
-    }
-    HIPCK(s, hipStreamSynchronize(s->stream));
-    return NUOSC_OK;
+    return fields_down(s, s->st_yb, 0, s->nf, out);
 }
 
 int nuosc_analysis(nuosc_sim* s, nuosc_analysis_t* o) {
@@ -1167,18 +1193,12 @@ int nuosc_renormalize(nuosc_sim* s) {
     return refresh_rk4(s);
 }
 
-int nuosc_download_field(nuosc_sim* s, int f, double* host) {
+int nuosc_download_field(nuosc_sim* s, int f, double* host) { return nuosc_download_fields(s, f, 1, host); }
+
+int nuosc_download_fields(nuosc_sim* s, int f0, int nf, double* host) {
     if (!s || !host) return NUOSC_EINVAL;
-    int rc = check_field(s, f);
-    if (rc) return rc;
-    const size_t bytes = sizeof(double) * (size_t)s->nx * s->nz * s->nv;
-    rc = ensure_tmp(s, bytes);
-    if (rc) return rc;
-    if (is64(s)) HIPCK(s, launch_pack<double>(s->geo, (double*)s->st_u, f, s->d_tmp, s->stream));
-    else HIPCK(s, launch_pack<float>(s->geo, (float*)s->st_u, f, s->d_tmp, s->stream));
-    HIPCK(s, hipMemcpyAsync(host, s->d_tmp, bytes, hipMemcpyDeviceToHost, s->stream));
-    HIPCK(s, hipStreamSynchronize(s->stream));
-    return NUOSC_OK;
+    if (f0 < 0 || nf < 1 || f0 > s->nf - nf) return fail(s, NUOSC_EINVAL, "field index out of range");
+    return fields_down(s, s->st_u, f0, nf, host);
 }
 
 int nuosc_download_field_ghosted(nuosc_sim* s, int f, double* host) {
@@ -1202,19 +1222,13 @@ int nuosc_download_field_ghosted(nuosc_sim* s, int f, double* host) {
     return NUOSC_OK;
 }
 
-int nuosc_upload_field(nuosc_sim* s, int f, const double* host) {
+int nuosc_upload_field(nuosc_sim* s, int f, const double* host) { return nuosc_upload_fields(s, f, 1, host); }
+
+int nuosc_upload_fields(nuosc_sim* s, int f0, int nf, const double* host) {
     if (!s || !host) return NUOSC_EINVAL;
-    int rc = check_field(s, f);
-    if (rc) return rc;
-    const size_t bytes = sizeof(double) * (size_t)s->nx * s->nz * s->nv;
-    rc = ensure_tmp(s, bytes);
-    if (rc) return rc;
-    HIPCK(s, hipMemcpyAsync(s->d_tmp, host, bytes, hipMemcpyHostToDevice, s->stream));
-    if (is64(s)) HIPCK(s, launch_unpack<double>(s->geo, s->d_tmp, (double*)s->st_u, f, s->stream));
-    else HIPCK(s, launch_unpack<float>(s->geo, s->d_tmp, (float*)s->st_u, f, s->stream));
-    HIPCK(s, hipStreamSynchronize(s->stream));
+    if (f0 < 0 || nf < 1 || f0 > s->nf - nf) return fail(s, NUOSC_EINVAL, "field index out of range");
     s->have_moments = s->have_sums = false;
-    return NUOSC_OK;
+    return fields_up(s, s->st_u, f0, nf, host);
 }
 
 int nuosc_state_updated(nuosc_sim* s) {
@@ -1235,19 +1249,16 @@ int nuosc_p3_slice(nuosc_sim* s, const int* xidx, int sx, const int* vidx, int s
     const size_t n = (size_t)sx * s->nz * sv;
     if (n == 0) return NUOSC_OK;
     const size_t ibytes = sizeof(int) * (size_t)(sx + sv);
-    const size_t ibytes_al = (ibytes + 255) / 256 * 256;
-    int rc = ensure_tmp(s, ibytes_al + sizeof(double) * n);
+    int rc = ensure_tmp(s, ibytes);
     if (rc) return rc;
     int* di = reinterpret_cast<int*>(s->d_tmp);
-    double* dd = reinterpret_cast<double*>(reinterpret_cast<char*>(s->d_tmp) + ibytes_al);
     std::vector<int> idx(xidx, xidx + sx);
     idx.insert(idx.end(), vidx, vidx + sv);
     HIPCK(s, hipMemcpyAsync(di, idx.data(), ibytes, hipMemcpyHostToDevice, s->stream));
-    if (is64(s)) HIPCK(s, launch_p3_slice<double>(s->geo, (double*)s->st_u, s->d_g0, di, sx, di + sx, sv, dd, s->stream));
-    else HIPCK(s, launch_p3_slice<float>(s->geo, (float*)s->st_u, s->d_g0, di, sx, di + sx, sv, dd, s->stream));
-    HIPCK(s, hipMemcpyAsync(dst, dd, sizeof(double) * n, hipMemcpyDeviceToHost, s->stream));
-    HIPCK(s, hipStreamSynchronize(s->stream));
-    return NUOSC_OK;
+    return transfer(s, true, dst, (long long)n, [&](long long n0, long long cnt, double* slot) {
+        return is64(s) ? launch_p3_slice<double>(s->geo, (double*)s->st_u, s->d_g0, di, di + sx, sv, n0, cnt, slot, s->stream)
+                       : launch_p3_slice<float>(s->geo, (float*)s->st_u, s->d_g0, di, di + sx, sv, n0, cnt, slot, s->stream);
+    });
 }
 
 }  // extern "C"

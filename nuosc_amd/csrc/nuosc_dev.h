@@ -201,16 +201,19 @@ template <typename T>
 hipError_t launch_ghosted(const Geometry& g, int gx, int gz, const T* y, int f, double* dst,
                           hipStream_t s);
 
-// Interior of field f of state y <-> FP64 dense [nx][nz][nv].
+// Elements [n0, n0 + cnt) of the interior of fields f0, f0 + 1, ... of state y
+// in FP64, dense [f][nx][nz][nv] <-> a buffer of cnt doubles.
 template <typename T>
-hipError_t launch_pack(const Geometry& g, const T* y, int f, double* dst, hipStream_t s);
+hipError_t launch_pack(const Geometry& g, const T* y, int f0, long long n0, long long cnt, double* dst, hipStream_t s);
 template <typename T>
-hipError_t launch_unpack(const Geometry& g, const double* src, T* y, int f, hipStream_t s);
+hipError_t launch_unpack(const Geometry& g, const double* src, T* y, int f0, long long n0, long long cnt,
+                         hipStream_t s);
 
-// P3 = (ee-mm)/G0 at x indices xi[sx] and v indices vi[sv]: dst[sx][nz][sv].
+// P3 = (ee-mm)/G0 at x indices xi[] and v indices vi[sv]: elements
+// [n0, n0 + cnt) of [x index][nz][sv].
 template <typename T>
-hipError_t launch_p3_slice(const Geometry& g, const T* y, const double* G0, const int* xi, int sx,
-                           const int* vi, int sv, double* dst, hipStream_t s);
+hipError_t launch_p3_slice(const Geometry& g, const T* y, const double* G0, const int* xi, const int* vi, int sv,
+                           long long n0, long long cnt, double* dst, hipStream_t s);
 
 // Stage pairs (nuosc_pair.hip): RK4 stages 1+2 and 3+4 in one pass each, for
 // 2-flavour periodic boxes with the default discretisation.  A step is

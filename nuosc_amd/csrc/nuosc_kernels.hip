@@ -1293,63 +1293,65 @@ hipError_t launch_ghosted(const Geometry& g, int gx, int gz, const T* y, int f, 
     return hipGetLastError();
 }
 
+// elements [n0, n0 + cnt) of fields f0.. laid out [f][site][v], to or from a
+// buffer (pinned host memory: nuosc_xfer.h) that holds just those
 template <typename T>
-__global__ void k_pack(const Geometry g, const T* __restrict__ y, int f, double* __restrict__ dst) {
-    const long long n = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long total = (long long)g.nx * g.nz * g.nv;
-    if (n >= total) return;
-    const long long s = n / g.nv;
-    const int v = (int)(n % g.nv);
-    dst[n] = (double)y[site_off(g, s) + f * g.nvp + v];
+__global__ __launch_bounds__(256) void k_pack(const Geometry g, const T* __restrict__ y, int f0, long long n0,
+                                              long long cnt, double* __restrict__ dst) {
+    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= cnt) return;
+    const long long n = n0 + k, r = n / g.nv, sites = (long long)g.nx * g.nz;
+    const int f = f0 + (int)(r / sites);
+    dst[k] = (double)y[site_off(g, r % sites) + (long long)f * g.nvp + n % g.nv];
 }
 
 template <typename T>
-__global__ void k_unpack(const Geometry g, const double* __restrict__ src, T* __restrict__ y, int f) {
-    const long long n = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long total = (long long)g.nx * g.nz * g.nvp;
-    if (n >= total) return;
-    const long long s = n / g.nvp;
-    const int v = (int)(n % g.nvp);
-    y[site_off(g, s) + f * g.nvp + v] = (v < g.nv) ? (T)src[s * g.nv + v] : (T)0;
+__global__ __launch_bounds__(256) void k_unpack(const Geometry g, const double* __restrict__ src, T* __restrict__ y,
+                                                int f0, long long n0, long long cnt) {
+    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= cnt) return;
+    const long long n = n0 + k, r = n / g.nv, sites = (long long)g.nx * g.nz;
+    const int f = f0 + (int)(r / sites);
+    y[site_off(g, r % sites) + (long long)f * g.nvp + n % g.nv] = (T)src[k];
 }
 
 template <typename T>
-hipError_t launch_pack(const Geometry& g, const T* y, int f, double* dst, hipStream_t s) {
-    const long long total = (long long)g.nx * g.nz * g.nv;
-    hipLaunchKernelGGL((k_pack<T>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, g, y, f, dst);
+hipError_t launch_pack(const Geometry& g, const T* y, int f0, long long n0, long long cnt, double* dst, hipStream_t s) {
+    hipLaunchKernelGGL((k_pack<T>), dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, g, y, f0, n0, cnt, dst);
     return hipGetLastError();
 }
 
 template <typename T>
-hipError_t launch_unpack(const Geometry& g, const double* src, T* y, int f, hipStream_t s) {
-    const long long total = (long long)g.nx * g.nz * g.nvp;
-    hipLaunchKernelGGL((k_unpack<T>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, g, src, y, f);
+hipError_t launch_unpack(const Geometry& g, const double* src, T* y, int f0, long long n0, long long cnt,
+                         hipStream_t s) {
+    hipLaunchKernelGGL((k_unpack<T>), dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, g, src, y, f0, n0, cnt);
     return hipGetLastError();
 }
 
+// elements [n0, n0 + cnt) of the slice dst[sx][nz][sv]
 template <typename T>
-__global__ void k_p3_slice(const Geometry g, const T* __restrict__ y, const double* __restrict__ G0,
-                           const int* __restrict__ xi, int sx, const int* __restrict__ vi, int sv,
-                           double* __restrict__ dst) {
-    const long long n = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long total = (long long)sx * g.nz * sv;
-    if (n >= total) return;
+__global__ __launch_bounds__(256) void k_p3_slice(const Geometry g, const T* __restrict__ y,
+                                                  const double* __restrict__ G0, const int* __restrict__ xi,
+                                                  const int* __restrict__ vi, int sv, long long n0, long long cnt,
+                                                  double* __restrict__ dst) {
+    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= cnt) return;
+    const long long n = n0 + k;
     const int b = (int)(n % sv);
     const long long r = n / sv;
     const int j = (int)(r % g.nz), a = (int)(r / g.nz);
     const int v = vi[b];
     const long long o = elem_off(g, xi[a], j + g.zoff, 0) + v;
     const double iG = 1.0 / G0[v];  // nuosc_ana.cpp:10,14
-    dst[n] = ((double)y[o + 0 * g.nvp] - (double)y[o + 1 * g.nvp]) * iG;
+    dst[k] = ((double)y[o + 0 * g.nvp] - (double)y[o + 1 * g.nvp]) * iG;
 }
 
 template <typename T>
-hipError_t launch_p3_slice(const Geometry& g, const T* y, const double* G0, const int* xi, int sx,
-                           const int* vi, int sv, double* dst, hipStream_t s) {
-    const long long total = (long long)sx * g.nz * sv;
-    if (total == 0) return hipSuccess;
-    hipLaunchKernelGGL((k_p3_slice<T>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, g, y, G0,
-                       xi, sx, vi, sv, dst);
+hipError_t launch_p3_slice(const Geometry& g, const T* y, const double* G0, const int* xi, const int* vi, int sv,
+                           long long n0, long long cnt, double* dst, hipStream_t s) {
+    if (cnt == 0) return hipSuccess;
+    hipLaunchKernelGGL((k_p3_slice<T>), dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, g, y, G0, xi, vi, sv, n0,
+                       cnt, dst);
     return hipGetLastError();
 }
 
@@ -1477,11 +1479,13 @@ hipError_t launch_advance_time(double* t_dev, double dt, hipStream_t s) {
     template hipError_t launch_analysis<T>(const Geometry&, const T*, const double*, const double*,      \
                                            double*, double*, hipStream_t);                               \
     template hipError_t launch_ghosted<T>(const Geometry&, int, int, const T*, int, double*, hipStream_t); \
-    template hipError_t launch_pack<T>(const Geometry&, const T*, int, double*, hipStream_t);            \
-    template hipError_t launch_unpack<T>(const Geometry&, const double*, T*, int, hipStream_t);          \
+    template hipError_t launch_pack<T>(const Geometry&, const T*, int, long long, long long, double*,    \
+                                       hipStream_t);                                                     \
+    template hipError_t launch_unpack<T>(const Geometry&, const double*, T*, int, long long, long long,  \
+                                         hipStream_t);                                                   \
     template hipError_t launch_xghosts<T>(const Geometry&, T*, hipStream_t);                              \
-    template hipError_t launch_p3_slice<T>(const Geometry&, const T*, const double*, const int*, int,    \
-                                           const int*, int, double*, hipStream_t);                       \
+    template hipError_t launch_p3_slice<T>(const Geometry&, const T*, const double*, const int*,         \
+                                           const int*, int, long long, long long, double*, hipStream_t); \
     template hipError_t launch_renorm<T>(const Geometry&, T*, const double*, const double*, hipStream_t); \
     template hipError_t launch_open_ghosts<T>(const Geometry&, T*, const double*, const double*, const Inflow&, \
                                               const double*, double, hipStream_t);

@@ -85,10 +85,10 @@ extern "C" int nuosc_p3_slice_noalloc(nuosc_sim* s, const int* xidx, int sx, con
     if (sx) e = hipMemcpyAsync(di, xidx, sizeof(int) * sx, hipMemcpyHostToDevice, v.stream);
     if (e == hipSuccess && sv) e = hipMemcpyAsync(di + sx, vidx, sizeof(int) * sv, hipMemcpyHostToDevice, v.stream);
     if (e == hipSuccess)
-        e = v.esize == 8 ? launch_p3_slice<double>(v.geo, static_cast<const double*>(v.state), v.g0, di, sx, di + sx,
-                                                   sv, dd, v.stream)
-                         : launch_p3_slice<float>(v.geo, static_cast<const float*>(v.state), v.g0, di, sx, di + sx,
-                                                  sv, dd, v.stream);
+        e = v.esize == 8 ? launch_p3_slice<double>(v.geo, static_cast<const double*>(v.state), v.g0, di, di + sx, sv, 0,
+                                                   (long long)n, dd, v.stream)
+                         : launch_p3_slice<float>(v.geo, static_cast<const float*>(v.state), v.g0, di, di + sx, sv, 0,
+                                                  (long long)n, dd, v.stream);
     if (e == hipSuccess) e = hipMemcpyAsync(dst, dd, sizeof(double) * n, hipMemcpyDeviceToHost, v.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
     if (e != hipSuccess)
