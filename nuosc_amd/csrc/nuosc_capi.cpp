@@ -54,7 +54,6 @@ struct nuosc_sim {
     double* d_vgrid = nullptr;  // vx | vy | vz | vw
     double* d_g0 = nullptr;     // G0 | G0b
     double* d_part = nullptr;
-    double* d_ana = nullptr;
     double* d_tmp = nullptr;    // FP64 staging (interior or ghosted field)
     double* d_time = nullptr;   // device copy of phy_time (open boundary data)
     Inflow inflow{};
@@ -486,16 +485,21 @@ int run_steps(nuosc_sim* s, StepKind kind, int nsteps) {
     return NUOSC_OK;
 }
 
-// Device analysis sums -> host (kNAna doubles).
+// Device analysis sums -> host (kNAna doubles), written to a pinned slot by
+// the last kernel.
 int analysis_sums(nuosc_sim* s, double* h) {
-    if (is64(s))
-        HIPCK(s, launch_analysis<double>(s->geo, (double*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->d_part, s->d_ana,
-                                         s->stream));
-    else
-        HIPCK(s, launch_analysis<float>(s->geo, (float*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->d_part, s->d_ana,
-                                        s->stream));
-    HIPCK(s, hipMemcpyAsync(h, s->d_ana, sizeof(double) * kNAna, hipMemcpyDeviceToHost, s->stream));
-    HIPCK(s, hipStreamSynchronize(s->stream));
+    const hipError_t e = xfer_run(
+        s->cfg.device, s->stream, 1, true,
+        [&](long long, void* slot) {
+            double* out = static_cast<double*>(slot);
+            return is64(s) ? launch_analysis<double>(s->geo, (double*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->d_part, out,
+                                                     s->stream)
+                           : launch_analysis<float>(s->geo, (float*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->d_part, out,
+                                                    s->stream);
+        },
+        [&](long long, void* slot) { std::memcpy(h, slot, sizeof(double) * kNAna); });
+    if (e == hipErrorOutOfMemory) return fail(s, NUOSC_ENOMEM, "staging buffer allocation failed");
+    HIPCK(s, e);
     return NUOSC_OK;
 }
 
@@ -783,8 +787,7 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
         if (hipMemsetAsync(s->d_time, 0, sizeof(double), s->stream) != hipSuccess) return bail(NUOSC_EHIP, "memset failed");
     }
     const int nb = ana_blocks(s->geo);
-    if (hipMalloc((void**)&s->d_part, (size_t)nb * kNAna * 2 * sizeof(double)) != hipSuccess ||
-        hipMalloc((void**)&s->d_ana, kNAna * sizeof(double)) != hipSuccess)
+    if (hipMalloc((void**)&s->d_part, (size_t)nb * kNAna * 2 * sizeof(double)) != hipSuccess)
         return bail(NUOSC_ENOMEM, "allocation failed");
     std::vector<double> hv(4 * (size_t)s->nv);
     for (int k = 0; k < s->nv; ++k) {
@@ -816,7 +819,7 @@ int nuosc_destroy(nuosc_sim* s) {
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     drop_graph(s);
     void* bufs[] = {s->st_u, s->st_w, s->st_ya, s->st_yb, s->mom_part, s->mom_u, s->mom_a, s->mom_b,
-                    s->pair_tot, s->d_vgrid, s->d_g0, s->d_part, s->d_ana, s->d_tmp, s->d_time};
+                    s->pair_tot, s->d_vgrid, s->d_g0, s->d_part, s->d_tmp, s->d_time};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
     if (s->ev0) (void)hipEventDestroy(s->ev0);
@@ -1530,7 +1533,7 @@ int nuosc_estimate_device_bytes(const nuosc_config* c, long long* bytes) {
     const bool pairs = steps_in_pairs(*c);
     b += part_doubles(nx, nz, nv, nch, nf, pairs) * 8;                 // moments: partials, totals
     b += (nf == kNVar3 ? 2ll * kNMom3 : 3ll * kMomStride + (pairs ? kPairRec : 0)) * nx * nz * 8;
-    b += 4 * nv * 8 + 2 * nv * 8 + 2048ll * kNAna * 16 + kNAna * 8;    // v-grid, G0, analysis
+    b += 4 * nv * 8 + 2 * nv * 8 + 2048ll * kNAna * 16;                // v-grid, G0, analysis
     b += 2 * nz * 8;                                                   // init tables
     *bytes = b;
     return NUOSC_OK;

@@ -1143,10 +1143,40 @@ constexpr int kAnaThreads = 256;
 
 int ana_blocks(const Geometry& g) {
     const long long pts = (long long)g.nx * g.nz * g.nv;
-    long long nb = (pts + kAnaThreads * 16 - 1) / (kAnaThreads * 16);
-    if (nb > 2048) nb = 2048;
-    if (nb < 1) nb = 1;
-    return (int)nb;
+    // a point per thread up to 2048 blocks (8 per CU): a small grid is latency,
+    // 16 points per thread on a few CUs took 20-33 us there
+    const long long nb = (pts + kAnaThreads - 1) / kAnaThreads;
+    return (int)std::min<long long>(nb, 2048);
+}
+
+// One more addend of a compensated sum, or of the maximum (a NaN never
+// replaces it: std::max semantics of nuosc_ana.cpp:64)
+__device__ __forceinline__ void ana_add(int q, double& s, double& e, double ps, double pe) {
+    if (q == ANA_MAXDP) {
+        s = (s < ps) ? ps : s;
+    } else {
+        double s2, err;
+        two_sum(s, ps, s2, err);
+        s = s2;
+        e = e + pe + err;
+    }
+}
+// (s, e) joined over the wave, in every lane: lanes l ^ 32, l ^ 16 by permlane
+// swaps, then rotations by 8 and 4 within a row and quad permutations, none of
+// which goes through LDS
+__device__ __forceinline__ void ana_wave(int q, double& s, double& e) {
+    double s1 = s, e1 = e;
+    swap_halves(s, s1);
+    swap_halves(e, e1);
+    ana_add(q, s, e, s1, e1);
+    s1 = s, e1 = e;
+    swap_rows(s, s1);
+    swap_rows(e, e1);
+    ana_add(q, s, e, s1, e1);
+    ana_add(q, s, e, dpp_f64<kDppRowRor8, 0xF>(s, s), dpp_f64<kDppRowRor8, 0xF>(e, e));
+    ana_add(q, s, e, dpp_f64<kDppRowRor4, 0xF>(s, s), dpp_f64<kDppRowRor4, 0xF>(e, e));
+    ana_add(q, s, e, dpp_f64<kDppXor2, 0xF>(s, s), dpp_f64<kDppXor2, 0xF>(e, e));
+    ana_add(q, s, e, dpp_f64<kDppXor1, 0xF>(s, s), dpp_f64<kDppXor1, 0xF>(e, e));
 }
 
 template <typename T>
@@ -1160,11 +1190,15 @@ __global__ __launch_bounds__(kAnaThreads) void k_analysis(const Geometry g, cons
 #pragma unroll
     for (int q = 0; q < kNAna; ++q) { S[q] = 0.0; E[q] = 0.0; }
     const long long pts = (long long)g.nx * g.nz * g.nv;
-    const long long stride = (long long)gridDim.x * blockDim.x;
-    for (long long n = (long long)blockIdx.x * blockDim.x + threadIdx.x; n < pts; n += stride) {
-        const long long site = n / g.nv;
-        const int v = (int)(n % g.nv);
-        const long long o = site_off(g, site) + v;
+    const long long stride = (long long)gridDim.x * blockDim.x, n0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    // (x row i, z j, direction v) of point n, carried along instead of divided
+    // out for every point (64-bit divisions: the FP32 form was bound by them)
+    int v = (int)(n0 % g.nv), j = (int)(n0 / g.nv % g.nz);
+    long long i = n0 / g.nv / g.nz;
+    const int dv = (int)(stride % g.nv), dj = (int)(stride / g.nv % g.nz);
+    const long long di = stride / g.nv / g.nz;
+    for (long long n = n0; n < pts; n += stride) {
+        const long long o = elem_off(g, i, j + g.zoff, 0) + v;
         double f[kNVar];
         bool finite = true;
 #pragma unroll
@@ -1200,59 +1234,39 @@ __global__ __launch_bounds__(kAnaThreads) void k_analysis(const Geometry g, cons
         const double m = (dP < dPb) ? dPb : dP;
         S[ANA_MAXDP] = (S[ANA_MAXDP] < m) ? m : S[ANA_MAXDP];
         if (!finite) S[ANA_BAD] += 1.0;
+        i += di;
+        j += dj;
+        v += dv;
+        if (v >= g.nv) v -= g.nv, ++j;
+        if (j >= g.nz) j -= g.nz, ++i;
     }
     // wave then block reduction in a fixed order
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
     for (int q = 0; q < kNAna; ++q) {
-        for (int m = 32; m >= 1; m >>= 1) {
-            const double os = __shfl_xor(S[q], m), oe = __shfl_xor(E[q], m);
-            if (q == ANA_MAXDP) {
-                S[q] = (S[q] < os) ? os : S[q];
-            } else {
-                double s2, err;
-                two_sum(S[q], os, s2, err);
-                S[q] = s2;
-                E[q] = E[q] + oe + err;
-            }
-        }
+        ana_wave(q, S[q], E[q]);
         if (lane == 0) { sh_s[wv][q] = S[q]; sh_e[wv][q] = E[q]; }
     }
     __syncthreads();
     if (threadIdx.x < kNAna) {
         const int q = threadIdx.x;
         double s = sh_s[0][q], e = sh_e[0][q];
-        for (int k = 1; k < kAnaThreads / kWave; ++k) {
-            if (q == ANA_MAXDP) {
-                s = (s < sh_s[k][q]) ? sh_s[k][q] : s;
-            } else {
-                double s2, err;
-                two_sum(s, sh_s[k][q], s2, err);
-                s = s2;
-                e = e + sh_e[k][q] + err;
-            }
-        }
+        for (int k = 1; k < kAnaThreads / kWave; ++k) ana_add(q, s, e, sh_s[k][q], sh_e[k][q]);
         part[(long long)blockIdx.x * kNAna * 2 + q] = s;
         part[(long long)blockIdx.x * kNAna * 2 + kNAna + q] = e;
     }
 }
 
-__global__ void k_analysis_final(const double* __restrict__ part, int nb, double* __restrict__ out) {
-    const int q = threadIdx.x;
-    if (q >= kNAna) return;
-    double s = part[q], e = part[kNAna + q];
-    for (int b = 1; b < nb; ++b) {
-        const double ps = part[(long long)b * kNAna * 2 + q], pe = part[(long long)b * kNAna * 2 + kNAna + q];
-        if (q == ANA_MAXDP) {
-            s = (s < ps) ? ps : s;
-        } else {
-            double s2, err;
-            two_sum(s, ps, s2, err);
-            s = s2;
-            e = e + pe + err;
-        }
-    }
-    out[q] = (q == ANA_MAXDP) ? s : s + e;
+// A wave per quantity: the blocks' partials, every 64th to a lane (one thread
+// adding 2048 of them took 0.7 ms, more than the pass over a 10^7-point state)
+__global__ __launch_bounds__(kNAna * kWave) void k_analysis_final(const double* __restrict__ part, int nb,
+                                                                  double* __restrict__ out) {
+    const int q = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    double s = 0.0, e = 0.0;
+    for (int b = lane; b < nb; b += kWave)
+        ana_add(q, s, e, part[(long long)b * kNAna * 2 + q], part[(long long)b * kNAna * 2 + kNAna + q]);
+    ana_wave(q, s, e);
+    if (lane == 0) out[q] = (q == ANA_MAXDP) ? s : s + e;
 }
 
 template <typename T>
@@ -1260,7 +1274,7 @@ hipError_t launch_analysis(const Geometry& g, const T* y, const double* G0, cons
                            double* part, double* out, hipStream_t s) {
     const int nb = ana_blocks(g);
     hipLaunchKernelGGL((k_analysis<T>), dim3(nb), dim3(kAnaThreads), 0, s, g, y, G0, G0b, part);
-    hipLaunchKernelGGL(k_analysis_final, dim3(1), dim3(64), 0, s, part, nb, out);
+    hipLaunchKernelGGL(k_analysis_final, dim3(1), dim3(kNAna * kWave), 0, s, part, nb, out);
     return hipGetLastError();
 }
 

@@ -65,7 +65,7 @@ __device__ __forceinline__ double dpp_f64(double old, double src) {
     return f64_of(lo, hi);
 }
 
-constexpr int kDppRowRor8 = 0x128, kDppRowShl4 = 0x104, kDppRowShr4 = 0x114;
+constexpr int kDppRowRor8 = 0x128, kDppRowRor4 = 0x124, kDppRowShl4 = 0x104, kDppRowShr4 = 0x114;
 constexpr int kDppXor2 = 0x4E, kDppXor1 = 0xB1;   // quad_perm [2,3,0,1], [1,0,3,2]
 
 // Wave total of 16 per-lane values: lane l ends with the total of value l >> 2.

@@ -121,7 +121,7 @@ __device__ __forceinline__ void fill_table(const Geometry& g, SumTable& t, int c
 
 __device__ __forceinline__ double dpp_add_ror(double x, bool eight) {
     // x + x of lane +-8 / +-4 within the 16-lane row
-    return eight ? x + dpp_f64<kDppRowRor8, 0xF>(x, x) : x + dpp_f64<0x124, 0xF>(x, x);
+    return eight ? x + dpp_f64<kDppRowRor8, 0xF>(x, x) : x + dpp_f64<kDppRowRor4, 0xF>(x, x);
 }
 
 // Direction sums of (c0, c1, c2) over the chunk, stored as one record of 27
