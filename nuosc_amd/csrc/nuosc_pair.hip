@@ -612,15 +612,15 @@ __global__ __launch_bounds__(256) void k_pair_sums(const Geometry g, const T* __
 }
 
 // ---------------------------------------------------------------------------
-// totals of a site's partial sums in chunk order, and the moments they give
+// totals of a site's partial sums in chunk order, and the moments they give.
+// Totals are stored as the combinations the moments are made of, per monomial
+//   D = (bemr - emr, bemi + emi, (bee - bmm) - (ee - mm))   [site][kMono][3]
+//   Q = (bemr + emr, bemi - emi, (bee - bmm) + (ee - mm))   after all D's
 // ---------------------------------------------------------------------------
 template <bool COMP>
-__device__ __forceinline__ void pair_totals_body(const double* __restrict__ part, int nch, long long nsites,
-                                                 double* __restrict__ tot, long long n) {
-    if (n >= nsites * kPairRec) return;
-    const long long site = n / kPairRec;
-    const double* rec = part + site * nch * kPairRec + n % kPairRec;
+__device__ __forceinline__ double chunk_sum(const double* __restrict__ rec, int nch) {
     double sum = rec[0], err = 0.0;
+#pragma unroll 4
     for (int c = 1; c < nch; ++c) {
         const double x = rec[(long long)c * kPairRec];
         if constexpr (COMP) {   // (FP32 form: as k_moment_totals)
@@ -631,11 +631,30 @@ __device__ __forceinline__ void pair_totals_body(const double* __restrict__ part
             sum += x;
         }
     }
-    tot[n] = sum + err;
+    return sum + err;
+}
+// A block adds the records of kTotSites sites, a thread per sum (the reads are
+// the whole pass: 1.25 GB at 512 x 512 x 642), and combines them through LDS.
+constexpr int kTotSites = 8, kTotThreads = 448;
+static_assert(kTotSites * kPairRec <= kTotThreads, "a thread per sum");
+template <bool COMP>
+__device__ __forceinline__ void pair_totals_body(const double* __restrict__ part, int nch, long long nsites,
+                                                 double* __restrict__ tot, long long blk, double (&sums)[kTotSites * kPairRec]) {
+    const long long s0 = blk * kTotSites;
+    const int n = (int)min((long long)kTotSites, nsites - s0), tid = threadIdx.x;
+    if (tid < n * kPairRec)
+        sums[tid] = chunk_sum<COMP>(part + (s0 + tid / kPairRec) * nch * kPairRec + tid % kPairRec, nch);
+    __syncthreads();
+    if (tid < n * kPairRec) {
+        const int k = tid < n * kRec ? tid : tid - n * kRec;   // entry of D, then of Q
+        const double nu = sums[k / kRec * kPairRec + k % kRec], bar = sums[k / kRec * kPairRec + kRec + k % kRec];
+        const bool plus = (k % 3 == 1) == (tid < n * kRec);
+        tot[(tid < n * kRec ? 0 : nsites * kRec) + s0 * kRec + k] = plus ? bar + nu : bar - nu;
+    }
 }
 
 struct PredictArgs {
-    const double* tot;    // [site][2][kMono][3]
+    const double* tot;    // D, then Q
     const double* base;   // what the prediction starts from (an m, or null: that of tot's state)
     double* m;            // mu times the moments of tot's state
     double* inner;        // mu times the moments of base + c k
@@ -645,79 +664,94 @@ struct PredictArgs {
     int nx, nz;
 };
 
-// index of u_a u_b among the monomials; yy (a = b = 2) is 1 - xx - zz
+// A block predicts kPredZ sites of one x row, 16 threads a site: thread
+// (site, s) moment component a = s % 4 of vector s / 4 (A: bemr - emr,
+// B: bemi + emi, C: bee - bmm - ee + mm).  The totals it needs (the row's
+// sites and two more at each end, the same sites of the four neighbouring
+// rows) are staged in LDS with coalesced loads: read from L2 by each thread
+// where needed, the pass took 0.29 ms at 512 x 512, a third of it index
+// arithmetic.  The moments of k follow nuosc_class.cpp:115-287 summed over
+// directions with w u_a.
+constexpr int kPredZ = 16;
+struct PredictLds {
+    double d[kPredZ + 4][kRec];       // own row, z - 2 .. z + 17
+    double x[4][kPredZ][kRec];        // x - 2, x - 1, x + 1, x + 2
+    double q[kPredZ][kRec];
+};
+// monomial of u_a u_b, a <= b (0: yy, which is 1 - xx - zz)
+__device__ __forceinline__ int mono_of(int lo, int hi) { return lo == 0 ? hi : (lo == 1 ? 3 + hi : 5 + lo); }
 __device__ __forceinline__ double second(const double* t, int a, int b, int c) {
-    const int lo = min(a, b), hi = max(a, b);
-    if (lo == 0) return t[hi * 3 + c];
-    if (lo == 2 && hi == 2) return t[c] - t[4 * 3 + c] - t[8 * 3 + c];
-    return t[(lo == 1 ? 3 + hi : 5 + lo) * 3 + c];   // xx, xy, xz; yz, zz
+    if (a == 2 && b == 2) return t[c] - t[4 * 3 + c] - t[8 * 3 + c];
+    return t[mono_of(min(a, b), max(a, b)) * 3 + c];
 }
 
-// Thread (site, s): moment component a = s % 4 of vector s / 4 (A: bemr - emr,
-// B: bemi + emi, C: bee - bmm - ee + mm).  The moments of k follow
-// nuosc_class.cpp:115-287 summed over directions with w u_a.
-__device__ __forceinline__ void predict_body(const PredictArgs& p, long long n) {
-    const long long nsites = (long long)p.nx * p.nz;
-    const long long site = n / kMomStride;
-    const int s = (int)(n % kMomStride);
-    if (site >= nsites) return;
+// blocks of one run
+__host__ __device__ inline long long predict_blocks(int nx, int nz) { return (long long)nx * ((nz + kPredZ - 1) / kPredZ); }
+
+__device__ __forceinline__ void predict_body(const PredictArgs& p, int blk, PredictLds& l) {
+    const int tiles = (p.nz + kPredZ - 1) / kPredZ;
+    const int i = blk / tiles, z0 = (blk % tiles) * kPredZ, nz = p.nz;
+    const int n = min(kPredZ, nz - z0), tid = threadIdx.x;
+    const long long row = (long long)i * nz, nsites = (long long)p.nx * nz;
+    for (int k = tid; k < (n + 4) * kRec; k += 256)
+        l.d[k / kRec][k % kRec] = p.tot[(row + wrapi(z0 - 2 + k / kRec, nz)) * kRec + k % kRec];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const double* t = p.tot + ((long long)wrapi(i + (q < 2 ? q - 2 : q - 1), p.nx) * nz + z0) * kRec;
+        for (int k = tid; k < n * kRec; k += 256) (&l.x[q][0][0])[k] = t[k];
+    }
+    for (int k = tid; k < n * kRec; k += 256) (&l.q[0][0])[k] = p.tot[(nsites + row + z0) * kRec + k];
+    __syncthreads();
+    const int zl = tid / kMomStride, s = tid % kMomStride;
+    if (zl >= n) return;
+    const long long o = (row + z0 + zl) * kMomStride + s;
     if (s >= kNMom) {
-        p.m[n] = p.inner[n] = 0.0;
+        p.m[o] = p.inner[o] = 0.0;
         return;
     }
     const int a = s & 3, v = s >> 2;
-    const int i = (int)(site / p.nz), j = (int)(site % p.nz);
-    const double* t = p.tot + site * kPairRec;
-    const double* tb = t + kRec;
-    // the vector's combination of the two halves: bar - nu, bar + nu, bar - nu
-    const double sg = v == 1 ? 1.0 : -1.0;
-    auto comb = [&](const double* q, int b) { return second(q + kRec, a, b, v) + sg * second(q, a, b, v); };
-    const double m0 = t[kRec + a * 3 + v] + sg * t[a * 3 + v];
+    const double *d = l.d[zl + 2], *q = l.q[zl];
+    const double m0 = d[a * 3 + v];
     // transport: advection multiplies by vx or vz, Kreiss-Oliger by nothing
     double kt = 0.0;
 #pragma unroll
     for (int ax = 0; ax < 2; ++ax) {
-        double d[4], e[4];
-        const int b = ax ? 3 : 1;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int o = q < 2 ? q - 2 : q - 1;
-            const long long ns = ax ? (long long)i * p.nz + wrapi(j + o, p.nz) : (long long)wrapi(i + o, p.nx) * p.nz + j;
-            const double* tn = p.tot + ns * kPairRec;
-            d[q] = comb(tn, b);
-            e[q] = tn[kRec + a * 3 + v] + sg * tn[a * 3 + v];
-        }
-        kt += -((d[0] - d[3]) - 8.0 * (d[1] - d[2])) / (ax ? p.twelve_dz : p.twelve_dx);
-        kt += (ax ? p.ko_z : p.ko_x) * (e[0] + e[3] - 4 * (e[1] + e[2]) + 6 * m0);
+        const int b = ax ? 3 : 1, second_ab = mono_of(min(a, b), max(a, b)) * 3 + v, first = a * 3 + v;
+        auto at = [&](int k) { return ax ? l.d[zl + (k < 2 ? k : k + 1)] : l.x[k][zl]; };
+        const double adv = (at(0)[second_ab] - at(3)[second_ab]) - 8.0 * (at(1)[second_ab] - at(2)[second_ab]);
+        const double ko = at(0)[first] + at(3)[first] - 4 * (at(1)[first] + at(2)[first]) + 6 * m0;
+        kt += (ax ? p.ko_z : p.ko_x) * ko - adv / (ax ? p.twelve_dz : p.twelve_dx);
     }
     // interaction: sum over b of s_b (moment b) (second moment a b), s = (1, -1, -1, -1)
     double loc = 0.0;
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-        const double Ab = tb[b * 3] - t[b * 3], Bb = tb[b * 3 + 1] + t[b * 3 + 1], Cb = tb[b * 3 + 2] - t[b * 3 + 2];
+        const double Ab = d[b * 3], Bb = d[b * 3 + 1], Cb = d[b * 3 + 2];
         double x;
         if (v == 0)        // k_emr of bar minus nu: -mu [ d3 B + (bemi - emi) C ]
-            x = -p.mu * ((second(tb, a, b, 2) - second(t, a, b, 2)) * Bb + Cb * (second(tb, a, b, 1) - second(t, a, b, 1)));
-        else if (v == 1)   // k_emi: mu [ -(bee - bmm + ee - mm) A + (bemr + emr) C ]
-            x = p.mu * (Cb * (second(tb, a, b, 0) + second(t, a, b, 0)) - (second(tb, a, b, 2) + second(t, a, b, 2)) * Ab);
+            x = -p.mu * (second(d, a, b, 2) * Bb + Cb * second(q, a, b, 1));
+        else if (v == 1)   // k_emi of bar plus nu: mu [ -(bee - bmm + ee - mm) A + (bemr + emr) C ]
+            x = p.mu * (Cb * second(q, a, b, 0) - second(q, a, b, 2) * Ab);
         else               // k_ee - k_mm = 2 k_ee: 2 mu2 [ (bemi - emi) A + (bemr - emr) B ]
-            x = 2 * p.mu2 * ((second(tb, a, b, 1) - second(t, a, b, 1)) * Ab + (second(tb, a, b, 0) - second(t, a, b, 0)) * Bb);
+            x = 2 * p.mu2 * (second(q, a, b, 1) * Ab + second(d, a, b, 0) * Bb);
         loc += b == 0 ? x : -x;
     }
-    const double r1 = tb[a * 3] + t[a * 3], i1 = tb[a * 3 + 1] - t[a * 3 + 1], e1 = tb[a * 3 + 2] + t[a * 3 + 2];
+    const double r1 = q[a * 3], i1 = q[a * 3 + 1], e1 = q[a * 3 + 2];
     const double vac = v == 0 ? -p.p2ct * i1 : (v == 1 ? p.pmo * (p.ct2 * r1 + p.st * e1) : -2 * p.p2st * i1);
     const double mm = p.mu * m0;
-    p.m[n] = mm;
-    p.inner[n] = (p.base ? p.base[n] : mm) + p.mu * (p.c * (loc + kt + vac));
+    p.m[o] = mm;
+    p.inner[o] = (p.base ? p.base[o] : mm) + p.mu * (p.c * (loc + kt + vac));
 }
 
 template <bool COMP>
-__global__ __launch_bounds__(256) void k_pair_totals(const double* __restrict__ part, int nch, long long nsites,
-                                                     double* __restrict__ tot) {
-    pair_totals_body<COMP>(part, nch, nsites, tot, (long long)blockIdx.x * 256 + threadIdx.x);
+__global__ __launch_bounds__(kTotThreads) void k_pair_totals(const double* __restrict__ part, int nch, long long nsites,
+                                                             double* __restrict__ tot) {
+    __shared__ double sums[kTotSites * kPairRec];
+    pair_totals_body<COMP>(part, nch, nsites, tot, blockIdx.x, sums);
 }
 __global__ __launch_bounds__(256) void k_pair_predict(const PredictArgs p) {
-    predict_body(p, (long long)blockIdx.x * 256 + threadIdx.x);
+    __shared__ PredictLds lds;
+    predict_body(p, blockIdx.x, lds);
 }
 
 struct SumArgs {
@@ -727,15 +761,17 @@ struct SumArgs {
     long long nsites;
 };
 template <bool COMP>
-__global__ __launch_bounds__(256) void k_pair_totals_batch(const SumArgs* __restrict__ runs, const int* __restrict__ map) {
+__global__ __launch_bounds__(kTotThreads) void k_pair_totals_batch(const SumArgs* __restrict__ runs, const int* __restrict__ map) {
     const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)map;
     const SumArgs a = runs[cm[2 * blockIdx.x]];
-    pair_totals_body<COMP>(a.part, a.nch, a.nsites, a.tot, (long long)cm[2 * blockIdx.x + 1] * 256 + threadIdx.x);
+    __shared__ double sums[kTotSites * kPairRec];
+    pair_totals_body<COMP>(a.part, a.nch, a.nsites, a.tot, cm[2 * blockIdx.x + 1], sums);
 }
 __global__ __launch_bounds__(256) void k_pair_predict_batch(const PredictArgs* __restrict__ runs, const int* __restrict__ map) {
     const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)map;
+    __shared__ PredictLds lds;
     const PredictArgs p = runs[cm[2 * blockIdx.x]];
-    predict_body(p, (long long)cm[2 * blockIdx.x + 1] * 256 + threadIdx.x);
+    predict_body(p, cm[2 * blockIdx.x + 1], lds);
 }
 
 template <typename T>
@@ -782,8 +818,6 @@ PredictArgs predict_args(const Geometry& g, const Physics& ph, int pair, const P
     p.nz = g.nz;
     return p;
 }
-
-unsigned blocks_of(long long n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
 
@@ -832,15 +866,15 @@ hipError_t launch_pair(int pair, const Geometry& g, const Physics& ph, int zlen,
 hipError_t launch_pair_predict(int pair, const Geometry& g, const Physics& ph, const PairBuffers& b, double dt,
                                hipStream_t s) {
     const PredictArgs p = predict_args(g, ph, pair, b, dt);
-    hipLaunchKernelGGL(k_pair_predict, dim3(blocks_of((long long)g.nx * g.nz * kMomStride)), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(k_pair_predict, dim3((unsigned)predict_blocks(g.nx, g.nz)), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 
 hipError_t launch_pair_totals(const Geometry& g, bool compensated, const PairBuffers& b, hipStream_t s) {
     const long long nsites = (long long)g.nx * g.nz;
-    const dim3 grid(blocks_of(nsites * kPairRec));
-    if (compensated) hipLaunchKernelGGL((k_pair_totals<true>), grid, dim3(256), 0, s, b.part, g.nch, nsites, b.tot);
-    else hipLaunchKernelGGL((k_pair_totals<false>), grid, dim3(256), 0, s, b.part, g.nch, nsites, b.tot);
+    const dim3 grid((unsigned)((nsites + kTotSites - 1) / kTotSites));
+    if (compensated) hipLaunchKernelGGL((k_pair_totals<true>), grid, dim3(kTotThreads), 0, s, b.part, g.nch, nsites, b.tot);
+    else hipLaunchKernelGGL((k_pair_totals<false>), grid, dim3(kTotThreads), 0, s, b.part, g.nch, nsites, b.tot);
     return hipGetLastError();
 }
 
@@ -876,8 +910,8 @@ hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hip
         const long long sites = (long long)g.nx * g.nz, nseg = (g.nz + m.zlen - 1) / m.zlen;
         // (the box form for every member, one-row grids included)
         count[0].push_back(nseg * 2 * g.nch * ((g.nx + PairShape<T>::R - 1) / PairShape<T>::R));
-        count[1].push_back((sites * kPairRec + 255) / 256);
-        count[2].push_back((sites * kMomStride + 255) / 256);
+        count[1].push_back((sites + kTotSites - 1) / kTotSites);
+        count[2].push_back(predict_blocks(g.nx, g.nz));
     }
     auto put_map = [&](const std::vector<long long>& c, int& blocks) {
         long long total = 0;
@@ -1001,7 +1035,7 @@ hipError_t batch_step(const BatchTables& t, int flip, hipStream_t s) {
                            (const PredictArgs*)t.pre[pair - 1][flip], t.pmap);
         const hipError_t e = batch_pair(t, pair, flip, s);
         if (e != hipSuccess) return e;
-        const dim3 tg(t.tblocks), tb(256);
+        const dim3 tg(t.tblocks), tb(kTotThreads);
         if (t.esize == 4) hipLaunchKernelGGL((k_pair_totals_batch<true>), tg, tb, 0, s, (const SumArgs*)t.sum, t.tmap);
         else hipLaunchKernelGGL((k_pair_totals_batch<false>), tg, tb, 0, s, (const SumArgs*)t.sum, t.tmap);
     }
