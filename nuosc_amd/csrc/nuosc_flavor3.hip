@@ -455,7 +455,11 @@ __device__ __forceinline__ void stage3z_body(const F3ZArgs<T>& a, ZSlab<T>& sl, 
     };
     const unsigned dof = (unsigned)pv * esz;
     const unsigned vo = (unsigned)min(wr + kXg, spare) * xrowb + dof;
-    const unsigned vos = (unsigned)(row_ok && live ? wr + kXg : spare) * xrowb + dof;
+    // lanes past nv and rows past nx store nothing: an offset past the range.
+    // (Their spare row lies within reach of 32 bits for the last blocks only:
+    // from the others its offset wrapped, into a row of a box of more than
+    // 4 GiB.)
+    const unsigned vos = row_ok && live ? (unsigned)(wr + kXg) * xrowb + dof : wbytes;
     // edge rows: wave wr of each group loads block row -2, -1, 4, 5 (slots 0, 1, 6, 7)
     const int eb = wr < 2 ? wr - 2 : kZRows + wr - 2;
     const unsigned vh = (unsigned)min(eb + kXg, spare) * xrowb + dof;

@@ -310,3 +310,22 @@ def test_flavor3_fp32_tracks_fp64_open_srk3(nuosc_mod, case):
     assert np.max(np.abs(sa - sb)) <= bound * np.max(np.abs(sa)), np.max(np.abs(sa - sb)) / np.max(np.abs(sa))
     a.close()
     b.close()
+
+
+def test_flavor3_wide_box_beyond_4gib(nuosc_mod):
+    """A state copy of more than 4 GiB (512 x 4096 x 12 directions: 52 lanes of
+    every wave past the last direction store nothing).  The ipt-0 pulse depends
+    on z only, so every x row stays bitwise the row of a narrow box."""
+    N = nuosc_mod
+    init = dict(ipt=0, alpha=0.9, eps0=1e-1, sigma=20.0, lnue=0.6, lnueb=0.5)
+    sims = []
+    for nx in (512, 4):
+        g = N.NuOsc(nflavor=3, **cfg_for(nx, 4096, 1, dx=0.125))
+        g.fillInitValue(**init)
+        g.step_rk4(2)
+        sims.append(g)
+    wide, narrow = sims
+    assert wide.shape == (512, 4096, 12)
+    for f in (2, 8, 17):
+        a, b = wide.get_field(f), narrow.get_field(f)
+        assert np.array_equal(a, np.broadcast_to(b[:1], a.shape)), f
