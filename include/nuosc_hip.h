@@ -290,9 +290,10 @@ int nuosc_batch_size(const nuosc_batch* batch);
  * returns after the device work completed. */
 int nuosc_batch_step(nuosc_batch* batch, int nsteps);
 const char* nuosc_batch_last_error(const nuosc_batch* batch);
-/* z-segment length of the batched stage kernels, shared by every member
- * (default 64, capped at each member's nz; 0 = each member's own plan).  A
- * common length gives every block of a batched launch the same work.
+/* z-segment length of the batched stage-pair kernels, shared by every member
+ * and capped at each member's nz (0 = each member's own plan; the default is
+ * planned for the members).  A common length gives every block of a batched
+ * launch the same work.
  * batch_autotune times the batched stages-1+2 kernel for zlen in {16, ..., 256}
  * and both launch forms (trials launches each, the fastest kept; only the
  * RK4 scratch copies are written) and keeps the best pair (the launch form

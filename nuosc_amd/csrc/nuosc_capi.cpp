@@ -1282,10 +1282,12 @@ struct nuosc_batch {
     std::vector<std::array<const void*, 2>> copies;
     hipGraph_t graph[2] = {};
     hipGraphExec_t graph_exec[2] = {};
-    // z-segment length shared by all members (0: each member's own plan).
-    // One length gives every block of the batched launch the same amount of
-    // work, so the contiguous block ranges of the 8 XCDs stay balanced.
-    int zlen = 64;
+    // z-segment length shared by all members (0: each member's own plan, -1:
+    // planned for the members).  One length gives every block of the batched
+    // launch the same amount of work, so the contiguous block ranges of the 8
+    // XCDs stay balanced.
+    int zlen = -1;
+    int num_cus = 0;
     int launch = kBatchGrid;   // NUOSC_BATCH_GRID or NUOSC_BATCH_PERSISTENT
     std::string err;
 };
@@ -1323,8 +1325,14 @@ int batch_tables(nuosc_batch* b) {
     std::vector<BatchMember> ms;
     b->copies.clear();
     b->flip = 0;
+    int shared = b->zlen;
+    if (shared < 0) {
+        std::vector<Geometry> grids;
+        for (nuosc_sim* m : b->members) grids.push_back(m->geo);
+        shared = plan_batch_zlen(grids, is64(b->members[0]) ? 8 : 4, b->num_cus);
+    }
     for (nuosc_sim* m : b->members) {
-        const int zlen = b->zlen > 0 ? std::min(b->zlen, m->nz) : m->pair_zlen;
+        const int zlen = shared > 0 ? std::min(shared, m->nz) : m->pair_zlen;
         ms.push_back(BatchMember{m->geo, m->ph, zlen, pair_buffers(m), m->dt});
         b->copies.push_back({m->st_u, m->st_ya});
     }
@@ -1356,6 +1364,10 @@ int nuosc_batch_create(int device, int precision, nuosc_batch** out) {
     nuosc_batch* b = new nuosc_batch();
     b->device = device;
     b->precision = precision;
+    if (hipDeviceGetAttribute(&b->num_cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
+        delete b;
+        return fail(nullptr, NUOSC_EHIP, "device query failed");
+    }
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) {
         delete b;
         return fail(nullptr, NUOSC_EHIP, "stream creation failed");

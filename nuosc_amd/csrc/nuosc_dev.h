@@ -223,15 +223,16 @@ hipError_t launch_p3_slice(const Geometry& g, const T* y, const double* G0, cons
 struct PairBuffers {
     const void* u;
     void *a, *y3, *unew;        // A = Y2 + u + dt k2, Y3, the new state
-    double *mu, *m3, *min;      // mu times the moments of u, Y3 and the inner input (Y2, then Y4), [site][kMomStride]
+    double *mu, *m3, *min;      // moment records of u, Y3 and the inner input (Y2, then Y4), [site][kMomStride]
     double *part, *tot;         // direction sums: [site][chunk][kPairRec] partial, [site][kPairRec] total
 };
 bool pair_capable(const Geometry& g);
 // blocks and wavefronts of one pair kernel with z segments of zlen sites
 int pair_blocks(const Geometry& g, int esize, int zlen);
 int pair_waves(const Geometry& g, int esize, int zlen);
-// z-segment length the pair kernels start with
+// z-segment length the pair kernels start with, alone and for a batch of grids
 int plan_pair_zlen(const Geometry& g, int esize, int num_cus);
+int plan_batch_zlen(const std::vector<Geometry>& grids, int esize, int num_cus);
 template <typename T>
 hipError_t launch_pair(int pair, const Geometry& g, const Physics& ph, int zlen, const PairBuffers& b, double dt,
                        hipStream_t s);

@@ -170,10 +170,9 @@ struct PairArgs {
     unsigned long long u;      // pair 2: u
     unsigned long long a;      // A: written by pair 1, read by pair 2
     unsigned long long out;    // Y3 (pair 1), u' (pair 2); no input of the pass
-    unsigned long long m1, m2; // moments of y and of the inner input, times mu: [site][kMomStride]
+    unsigned long long m1, m2; // moment records of y and of the inner input: [site][kMomStride]
     unsigned long long part;   // partial sums of out: [site][chunk][2][kRec]
     double c1, c2, cA;         // inner input u + c1 k; output factor c2; A's factor cA
-    double pst, p2ct;          // pmo st, 2 pmo ct
     int zlen, xgroups, nunits;
 };
 
@@ -203,25 +202,25 @@ struct PairConst {
     double vx, vy, vz;
     T fx, fz;          // -v / (12 h)
     T kx, kz, k6;      // -ko / (16 h) per axis; 6 (kx + kz)
-    double pst, p2ct;
 };
 
 // Interaction and vacuum terms as one precession: with the projections A, B, C
-// of the site's moments (INP, nuosc_class.cpp:187), here times mu,
+// of the site's moments (INP, nuosc_class.cpp:187),
 //   k_ee = 2 (q emi + b emr), k_mm = -k_ee, k_emr = -(b d + c emi),
-//   k_emi = c emr - q d,  d = ee - mm,  q = A - pmo st, b = B, c = C + 2 pmo ct
+//   k_emi = c emr - q d,  d = ee - mm,
+//   q = mu A - pmo st, b = mu B, c = mu C + 2 pmo ct
+// (the records of the pair kernels hold mu times the moments, with the vacuum
+// terms added to the first of A and of C: k_pair_predict)
 // (the terms of nuosc_class.cpp:193-200, 280-287 collected).
 template <typename T>
 struct Precession {
-    T q2, b2, q, b, c;
+    T q, b, c;
 };
 template <typename T>
 __device__ __forceinline__ Precession<T> precession(const PairConst<T>& k, const double (&m)[kNMom]) {
-    const double A = m[0] - m[1] * k.vx - m[2] * k.vy - m[3] * k.vz;
-    const double B = m[4] - m[5] * k.vx - m[6] * k.vy - m[7] * k.vz;
-    const double C = m[8] - m[9] * k.vx - m[10] * k.vy - m[11] * k.vz;
-    const double q = A - k.pst, c = C + k.p2ct;
-    return Precession<T>{(T)(2 * q), (T)(2 * B), (T)q, (T)B, (T)c};
+    return Precession<T>{(T)(m[0] - m[1] * k.vx - m[2] * k.vy - m[3] * k.vz),
+                         (T)(m[4] - m[5] * k.vx - m[6] * k.vy - m[7] * k.vz),
+                         (T)(m[8] - m[9] * k.vx - m[10] * k.vy - m[11] * k.vz)};
 }
 
 __device__ __forceinline__ void load_moments(unsigned long long site, double (&m)[kNMom]) {
@@ -238,7 +237,7 @@ template <typename T, typename XN>
 __device__ __forceinline__ void rhs_unit(const PairConst<T>& k, const Precession<T>& r, const T (&c)[kF],
                                          const T (&zm2)[kF], const T (&zm1)[kF], const T (&zp1)[kF],
                                          const T (&zp2)[kF], XN xn, T (&out)[kF]) {
-    const T d = c[0] - c[1], ee = r.q2 * c[3] + r.b2 * c[2];
+    const T d = c[0] - c[1], ee = (T)2 * (r.q * c[3] + r.b * c[2]);
     const T loc[kF] = {ee, -ee, -(r.b * d + r.c * c[3]), r.c * c[2] - r.q * d};
 #pragma unroll
     for (int f = 0; f < kF; ++f) {
@@ -302,8 +301,6 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
     k.kx = (T)g.ko_x;
     k.kz = (T)g.ko_z;
     k.k6 = (T)(6 * (g.ko_x + g.ko_z));
-    k.pst = a.pst;
-    k.p2ct = a.p2ct;
     const T c1 = (T)a.c1, c2 = (T)a.c2, cA = (T)a.cA;
 
     T U[6][kF];    // y of the own row, z = j .. j+4, and j+5 on its way: slot (phase + z - j) % 6
@@ -656,8 +653,8 @@ __device__ __forceinline__ void pair_totals_body(const double* __restrict__ part
 struct PredictArgs {
     const double* tot;    // D, then Q
     const double* base;   // what the prediction starts from (an m, or null: that of tot's state)
-    double* m;            // mu times the moments of tot's state
-    double* inner;        // mu times the moments of base + c k
+    double* m;            // record of tot's state: mu times its moments, with the vacuum terms
+    double* inner;        // the same of base + c k
     double c;
     double mu, mu2, p2st, p2ct, pmo, ct2, st;
     double twelve_dx, twelve_dz, ko_x, ko_z;
@@ -738,7 +735,8 @@ __device__ __forceinline__ void predict_body(const PredictArgs& p, int blk, Pred
     }
     const double r1 = q[a * 3], i1 = q[a * 3 + 1], e1 = q[a * 3 + 2];
     const double vac = v == 0 ? -p.p2ct * i1 : (v == 1 ? p.pmo * (p.ct2 * r1 + p.st * e1) : -2 * p.p2st * i1);
-    const double mm = p.mu * m0;
+    // (the record's offset: see precession())
+    const double mm = p.mu * m0 + (s == 0 ? -p.pmo * p.st : (s == 8 ? p.p2ct : 0.0));
     p.m[o] = mm;
     p.inner[o] = (p.base ? p.base[o] : mm) + p.mu * (p.c * (loc + kt + vac));
 }
@@ -788,8 +786,6 @@ PairArgs<T> pair_args(const Geometry& g, const Physics& ph, int zlen, int pair, 
     a.c1 = pair == 1 ? 0.5 * dt : dt;
     a.c2 = pair == 1 ? 0.5 * dt : 1.0 / 6.0 * dt;
     a.cA = dt;
-    a.pst = ph.pmo * ph.st;
-    a.p2ct = ph.pmo * 2 * ph.ct;
     a.zlen = zlen;
     a.xgroups = g.nx == 1 ? 1 : (g.nx + PairShape<T>::R - 1) / PairShape<T>::R;
     a.nunits = 2 * g.nch;
@@ -825,10 +821,17 @@ bool pair_capable(const Geometry& g) {
     return g.nf == kNVar && g.bc == 0 && !g.ko5 && g.adv == kAdvCfd4;
 }
 
-int pair_blocks(const Geometry& g, int esize, int zlen) {
-    const long long nseg = (g.nz + zlen - 1) / zlen, nu = 2ll * g.nch;
+namespace {
+// blocks of the box form (batches take it for one-row grids too)
+long long pair_box_blocks(const Geometry& g, int esize, int zlen) {
     const int R = esize == 8 ? PairShape<double>::R : PairShape<float>::R;
-    return (int)(nseg * (g.nx == 1 ? (nu + kRowWaves - 1) / kRowWaves : nu * ((g.nx + R - 1) / R)));
+    return (long long)((g.nz + zlen - 1) / zlen) * 2 * g.nch * ((g.nx + R - 1) / R);
+}
+}  // namespace
+
+int pair_blocks(const Geometry& g, int esize, int zlen) {
+    if (g.nx > 1) return (int)pair_box_blocks(g, esize, zlen);
+    return (g.nz + zlen - 1) / zlen * ((2 * g.nch + kRowWaves - 1) / kRowWaves);
 }
 
 int pair_waves(const Geometry& g, int esize, int zlen) {
@@ -836,14 +839,47 @@ int pair_waves(const Geometry& g, int esize, int zlen) {
     return pair_blocks(g, esize, zlen) * (g.nx == 1 ? kRowWaves : R + 4);
 }
 
-// Longest segments that still give every CU a block (every segment starts
-// with four steps that write nothing).
+// Time of a pair kernel's blocks in steps of the z march: rounds of as many
+// blocks as the GPU holds at once (one per CU in the box form, counted as
+// three in the one-row form, of which FP32 holds five: 3001 x 492 in FP32 takes
+// 110-113 us in segments of 24 or 16 sites, 130 in 10), each of zlen steps and
+// about eight more: four that write nothing, the rest the block's start.  At 512 x 512 x
+// 642 the model orders segments of 64 .. 512 sites as they measure in both
+// precisions (FP64: 256 best, 19.5 ms, 64 worst, 20.5 ms; FP32: 128 best, 11.5,
+// 171 worst, 12.0); 20 x 200 x 162: segments of 13 sites are two rounds (75 us
+// a kernel), 15 one.
+double pair_march_steps(long long blocks, int zlen, bool one_row, int num_cus) {
+    const long long slots = (long long)num_cus * (one_row ? 3 : 1);
+    return (double)((blocks + slots - 1) / slots) * (zlen + 8);
+}
+
 int plan_pair_zlen(const Geometry& g, int esize, int num_cus) {
-    const int want = g.nx == 1 ? 3 * num_cus : num_cus;
-    int zlen = g.nz;
-    while (zlen > 8 && pair_blocks(g, esize, zlen) < want) zlen = (zlen + 1) / 2;
-    while (zlen > 128 && pair_blocks(g, esize, zlen) < 8 * want) zlen = (zlen + 1) / 2;
-    return zlen;
+    int best = g.nz;
+    double least = 1e300;
+    for (int most = std::min(g.nz, 1024); most >= 1; --most) {
+        const int nseg = (g.nz + most - 1) / most, zlen = (g.nz + nseg - 1) / nseg;   // equal segments
+        const double t = pair_march_steps(pair_blocks(g, esize, zlen), zlen, g.nx == 1, num_cus);
+        if (t < least) {
+            least = t;
+            best = zlen;
+        }
+    }
+    return best;
+}
+
+int plan_batch_zlen(const std::vector<Geometry>& gs, int esize, int num_cus) {
+    int best = 64;
+    double least = 1e300;
+    for (int zlen : {4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256}) {
+        long long blocks = 0;
+        for (const Geometry& g : gs) blocks += pair_box_blocks(g, esize, std::min(zlen, g.nz));
+        const double t = pair_march_steps(blocks, zlen, false, num_cus);
+        if (t < least) {
+            least = t;
+            best = zlen;
+        }
+    }
+    return best;
 }
 
 template <typename T>
@@ -907,9 +943,8 @@ hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hip
     std::vector<long long> count[3];
     for (const BatchMember& m : ms) {
         const Geometry& g = m.g;
-        const long long sites = (long long)g.nx * g.nz, nseg = (g.nz + m.zlen - 1) / m.zlen;
-        // (the box form for every member, one-row grids included)
-        count[0].push_back(nseg * 2 * g.nch * ((g.nx + PairShape<T>::R - 1) / PairShape<T>::R));
+        const long long sites = (long long)g.nx * g.nz;
+        count[0].push_back(pair_box_blocks(g, sizeof(T), m.zlen));
         count[1].push_back((sites + kTotSites - 1) / kTotSites);
         count[2].push_back(predict_blocks(g.nx, g.nz));
     }
