@@ -282,19 +282,21 @@ hipError_t enqueue_sums(nuosc_sim* s, const T* y) {
     return e != hipSuccess ? e : launch_pair_totals(s->geo, sizeof(T) == 4, pair_buffers(s), s->stream);
 }
 
-// One RK4 step in two stage pairs (nuosc_pair.hip) from st_u into st_ya; the
-// caller exchanges the two.  Events ev[0], ev[1] bracket the first pair's
-// kernel alone, ev[4], ev[5] the second's.
+// One RK4 step in two stage pairs, or one SSP-RK3 step in a pair and a lone
+// stage (nuosc_pair.hip), from st_u into st_ya; the caller exchanges the two.
+// Events ev[0], ev[1] bracket the first kernel alone, ev[4], ev[5] the second.
+enum StepKind { kRk4 = 0, kSrk3 = 1 };
 template <typename T>
-int enqueue_step_pairs(nuosc_sim* s, hipEvent_t* ev = nullptr) {
+int enqueue_step_pairs(nuosc_sim* s, StepKind kind, hipEvent_t* ev = nullptr) {
     const PairBuffers b = pair_buffers(s);
     const bool comp = sizeof(T) == 4;
-    for (int pair = 1; pair <= 2; ++pair) {
+    for (int half = 0; half < 2; ++half) {
+        const int pair = kind == kRk4 ? 1 + half : (half ? kLone : 3);
         HIPCK(s, launch_pair_predict(pair, s->geo, s->ph, b, s->dt, s->stream));
-        if (ev) HIPCK(s, hipEventRecord(ev[4 * pair - 4], s->stream));
+        if (ev) HIPCK(s, hipEventRecord(ev[4 * half], s->stream));
         HIPCK(s, launch_pair<T>(pair, s->geo, s->ph, s->pair_zlen, b, s->dt, s->stream));
-        if (ev) HIPCK(s, hipEventRecord(ev[4 * pair - 3], s->stream));
-        if (pair == 2 && s->cfg.renorm) {
+        if (ev) HIPCK(s, hipEventRecord(ev[4 * half + 1], s->stream));
+        if (half && s->cfg.renorm) {
             T* u = static_cast<T*>(b.unew);
             HIPCK(s, launch_renorm<T>(s->geo, u, s->d_g0, s->d_g0 + s->nv, s->stream));
             HIPCK(s, launch_pair_sums<T>(s->geo, u, b.part, s->stream));
@@ -426,16 +428,16 @@ void set_plan(nuosc_sim* s, int zlen) {
     if (s->pairs) s->pair_zlen = s->plan.zlen;
 }
 
-// what an RK4 step needs of the state u: its direction sums (stage pairs) or
-// its moments
-int refresh_rk4(nuosc_sim* s) {
+// what a step needs of the state u: its direction sums (stage pairs) or its
+// moments
+int refresh_step(nuosc_sim* s) {
     if (!s->pairs) return refresh_moments(s);
     if (is64(s)) HIPCK(s, enqueue_sums<double>(s, (double*)s->st_u));
     else HIPCK(s, enqueue_sums<float>(s, (float*)s->st_u));
     s->have_sums = true;
     return NUOSC_OK;
 }
-bool rk4_ready(const nuosc_sim* s) { return s->pairs ? s->have_sums : s->have_moments; }
+bool step_ready(const nuosc_sim* s) { return s->pairs ? s->have_sums : s->have_moments; }
 
 // the stage pairs leave the new state in st_ya
 void state_stepped(nuosc_sim* s) {
@@ -446,14 +448,18 @@ void state_stepped(nuosc_sim* s) {
 
 // nsteps steps on the handle's stream, replayed from a captured graph if the
 // handle uses them
-enum StepKind { kRk4 = 0, kSrk3 = 1 };
 int run_steps(nuosc_sim* s, StepKind kind, int nsteps) {
-    const bool pairs = kind == kRk4 && s->pairs;
+    const bool pairs = s->pairs;
     auto enqueue = [&] {
-        if (pairs) return is64(s) ? enqueue_step_pairs<double>(s) : enqueue_step_pairs<float>(s);
+        if (pairs) return is64(s) ? enqueue_step_pairs<double>(s, kind) : enqueue_step_pairs<float>(s, kind);
         if (kind == kRk4) return is64(s) ? enqueue_step<double>(s) : enqueue_step<float>(s);
         return is64(s) ? enqueue_step_srk3<double>(s) : enqueue_step_srk3<float>(s);
     };
+    if (nsteps < 0) return fail(s, NUOSC_EINVAL, "negative step count");
+    if (!step_ready(s)) {
+        const int rc = refresh_step(s);
+        if (rc) return rc;
+    }
     HIPCK(s, hipEventRecord(s->ev0, s->stream));
     for (int n = 0; n < nsteps; ++n) {
         if (s->cfg.use_graph) {
@@ -957,31 +963,15 @@ int nuosc_fill_init(nuosc_sim* s, int ipt, double alpha, double eps0, double sig
     rc = set_device_time(s);
     if (rc) return rc;
     s->have_moments = false;
-    rc = refresh_rk4(s);
+    rc = refresh_step(s);
     if (rc) return rc;
     HIPCK(s, hipStreamSynchronize(s->stream));
     return NUOSC_OK;
 }
 
-int nuosc_step_rk4(nuosc_sim* s, int nsteps) {
-    if (!s) return NUOSC_EINVAL;
-    if (nsteps < 0) return fail(s, NUOSC_EINVAL, "negative step count");
-    if (!rk4_ready(s)) {
-        int rc = refresh_rk4(s);
-        if (rc) return rc;
-    }
-    return run_steps(s, kRk4, nsteps);
-}
+int nuosc_step_rk4(nuosc_sim* s, int nsteps) { return s ? run_steps(s, kRk4, nsteps) : NUOSC_EINVAL; }
 
-int nuosc_step_srk3(nuosc_sim* s, int nsteps) {
-    if (!s) return NUOSC_EINVAL;
-    if (nsteps < 0) return fail(s, NUOSC_EINVAL, "negative step count");
-    if (!s->have_moments) {
-        int rc = refresh_moments(s);
-        if (rc) return rc;
-    }
-    return run_steps(s, kSrk3, nsteps);
-}
+int nuosc_step_srk3(nuosc_sim* s, int nsteps) { return s ? run_steps(s, kSrk3, nsteps) : NUOSC_EINVAL; }
 
 int nuosc_synchronize(nuosc_sim* s) {
     if (!s) return NUOSC_EINVAL;
@@ -1000,8 +990,8 @@ int nuosc_last_step_ms(nuosc_sim* s, double* ms) {
 
 int nuosc_profile_stages(nuosc_sim* s, int nsteps, double* stage_ms) {
     if (!s || !stage_ms || nsteps < 1) return NUOSC_EINVAL;
-    if (!rk4_ready(s)) {
-        int rc = refresh_rk4(s);
+    if (!step_ready(s)) {
+        int rc = refresh_step(s);
         if (rc) return rc;
     }
     hipEvent_t ev[8] = {};
@@ -1010,7 +1000,7 @@ int nuosc_profile_stages(nuosc_sim* s, int nsteps, double* stage_ms) {
     double acc[4] = {0, 0, 0, 0};
     int rc = NUOSC_OK;
     for (int n = 0; n < nsteps && rc == NUOSC_OK; ++n) {
-        if (s->pairs) rc = is64(s) ? enqueue_step_pairs<double>(s, ev) : enqueue_step_pairs<float>(s, ev);
+        if (s->pairs) rc = is64(s) ? enqueue_step_pairs<double>(s, kRk4, ev) : enqueue_step_pairs<float>(s, kRk4, ev);
         else rc = is64(s) ? enqueue_step<double>(s, ev) : enqueue_step<float>(s, ev);
         if (rc) break;
         if (s->pairs) state_stepped(s);
@@ -1077,8 +1067,8 @@ int nuosc_autotune(nuosc_sim* s, int trials, int* best_zlen, double* best_ms) {
             return NUOSC_OK;
         }
     }
-    if (!rk4_ready(s)) {
-        int rc = refresh_rk4(s);
+    if (!step_ready(s)) {
+        int rc = refresh_step(s);
         if (rc) return rc;
     }
     hipEvent_t e0, e1;
@@ -1193,7 +1183,7 @@ int nuosc_renormalize(nuosc_sim* s) {
     if (is64(s)) HIPCK(s, launch_renorm<double>(s->geo, (double*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->stream));
     else HIPCK(s, launch_renorm<float>(s->geo, (float*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->stream));
     s->have_moments = false;
-    return refresh_rk4(s);
+    return refresh_step(s);
 }
 
 int nuosc_download_field(nuosc_sim* s, int f, double* host) { return nuosc_download_fields(s, f, 1, host); }
@@ -1237,7 +1227,7 @@ int nuosc_upload_fields(nuosc_sim* s, int f0, int nf, const double* host) {
 int nuosc_state_updated(nuosc_sim* s) {
     if (!s) return NUOSC_EINVAL;
     s->have_moments = false;
-    int rc = refresh_rk4(s);
+    int rc = refresh_step(s);
     if (rc) return rc;
     HIPCK(s, hipStreamSynchronize(s->stream));
     return NUOSC_OK;
@@ -1345,7 +1335,7 @@ int batch_tables(nuosc_batch* b) {
 int batch_sync_members(nuosc_batch* b) {
     for (nuosc_sim* m : b->members) {
         if (m->cfg.renorm) return bfail(b, NUOSC_EINVAL, "renormalising runs cannot be batched");
-        if (!rk4_ready(m) && refresh_rk4(m) != NUOSC_OK) return bfail(b, NUOSC_EHIP, m->err);
+        if (!step_ready(m) && refresh_step(m) != NUOSC_OK) return bfail(b, NUOSC_EHIP, m->err);
         if (hipStreamSynchronize(m->stream) != hipSuccess) return bfail(b, NUOSC_EHIP, "member stream sync failed");
     }
     return NUOSC_OK;

@@ -215,14 +215,16 @@ template <typename T>
 hipError_t launch_p3_slice(const Geometry& g, const T* y, const double* G0, const int* xi, const int* vi, int sv,
                            long long n0, long long cnt, double* dst, hipStream_t s);
 
-// Stage pairs (nuosc_pair.hip): RK4 stages 1+2 and 3+4 in one pass each, for
-// 2-flavour periodic boxes with the default discretisation.  A step is
-//   predict(1), pair(1), totals, predict(2), pair(2), totals
-// and needs the direction sums tot of u; it leaves those of unew, and the new
-// state in unew (u is not touched).
+// Stage pairs (nuosc_pair.hip): RK4 stages 1+2 and 3+4 (pairs 1 and 2) or
+// SSP-RK3 stages 1+2 (pair 3) in one pass each and SSP-RK3 stage 3 (kLone),
+// for 2-flavour periodic boxes with the default discretisation.  A step is
+//   predict(p), pair(p), totals, predict(q), pair(q), totals
+// with (p, q) = (1, 2) or (3, kLone) and needs the direction sums tot of u; it
+// leaves those of unew, and the new state in unew (u is not touched).
+constexpr int kLone = 4;
 struct PairBuffers {
     const void* u;
-    void *a, *y3, *unew;        // A = Y2 + u + dt k2, Y3, the new state
+    void *a, *y3, *unew;        // A = Y2 + u + dt k2, Y3 (SSP-RK3: u2), the new state
     double *mu, *m3, *min;      // moment records of u, Y3 and the inner input (Y2, then Y4), [site][kMomStride]
     double *part, *tot;         // direction sums: [site][chunk][kPairRec] partial, [site][kPairRec] total
 };

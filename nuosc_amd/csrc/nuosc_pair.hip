@@ -7,7 +7,10 @@
 // registers and LDS:
 //   pair 1: read u       -> Y2 (on chip) -> Y3 = u + dt/2 k2, A = Y2 + u + dt k2
 //   pair 2: read Y3, u, A -> Y4 (on chip) -> u' = (A + Y4)/3 + dt/6 k4
-// 3 + 4 = 7 passes (448 B per FP64 update instead of 768).
+// 3 + 4 = 7 passes (448 B per FP64 update instead of 768).  An SSP-RK3 step is
+// a pair and a single stage, 2 + 3 = 5 passes instead of 8:
+//   pair 3: read u       -> u1 = u + dt k (on chip) -> u2 = 3/4 u + 1/4 (u1 + dt k)
+//   k_lone: read u2, u   -> u' = 1/3 u + 2/3 (u2 + dt k)
 //
 // What made the passes separate is the interaction term of the inner input Y:
 // it needs the velocity moments of Y at each site, a sum over all directions,
@@ -166,13 +169,14 @@ __device__ __forceinline__ unsigned sum_offset(int lane, unsigned past) {
 template <typename T>
 struct PairArgs {
     Geometry g;
-    unsigned long long y;      // stencil input (stored x row 0): u (pair 1), Y3 (pair 2)
-    unsigned long long u;      // pair 2: u
+    unsigned long long y;      // stencil input (stored x row 0): u (pairs 1, 3), Y3 (pair 2), u2 (lone stage)
+    unsigned long long u;      // pair 2, lone stage: u
     unsigned long long a;      // A: written by pair 1, read by pair 2
-    unsigned long long out;    // Y3 (pair 1), u' (pair 2); no input of the pass
+    unsigned long long out;    // Y3 (pair 1), u2 (pair 3), u' (pair 2, lone stage); no input of the pass
     unsigned long long m1, m2; // moment records of y and of the inner input: [site][kMomStride]
     unsigned long long part;   // partial sums of out: [site][chunk][2][kRec]
-    double c1, c2, cA;         // inner input u + c1 k; output factor c2; A's factor cA
+    double c1, c2, cA;         // inner input u + c1 k; output's and A's factors of k (pair 3, lone stage:
+                               // output c2 u + cA (y + c1 k))
     int zlen, xgroups, nunits;
 };
 
@@ -203,6 +207,20 @@ struct PairConst {
     T fx, fz;          // -v / (12 h)
     T kx, kz, k6;      // -ko / (16 h) per axis; 6 (kx + kz)
 };
+
+template <typename T>
+__device__ __forceinline__ PairConst<T> pair_const(const Geometry& g, int pv) {
+    PairConst<T> k;
+    k.vx = g.vx[pv];
+    k.vy = g.vy[pv];
+    k.vz = g.vz[pv];
+    k.fx = (T)(-k.vx / g.twelve_dx);
+    k.fz = (T)(-k.vz / g.twelve_dz);
+    k.kx = (T)g.ko_x;
+    k.kz = (T)g.ko_z;
+    k.k6 = (T)(6 * (g.ko_x + g.ko_z));
+    return k;
+}
 
 // Interaction and vacuum terms as one precession: with the projections A, B, C
 // of the site's moments (INP, nuosc_class.cpp:187),
@@ -292,15 +310,7 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
     const unsigned vrec = sum_offset(lane, pbytes);
     const unsigned long long mrow = (unsigned long long)row * nz * (kMomStride * 8);
     const unsigned mbytes = (unsigned)nz * (kMomStride * 8), vm = (unsigned)(lane & 15) * 8;
-    PairConst<T> k;
-    k.vx = g.vx[pv];
-    k.vy = g.vy[pv];
-    k.vz = g.vz[pv];
-    k.fx = (T)(-k.vx / g.twelve_dx);
-    k.fz = (T)(-k.vz / g.twelve_dz);
-    k.kx = (T)g.ko_x;
-    k.kz = (T)g.ko_z;
-    k.k6 = (T)(6 * (g.ko_x + g.ko_z));
+    const PairConst<T> k = pair_const<T>(g, pv);
     const T c1 = (T)a.c1, c2 = (T)a.c2, cA = (T)a.cA;
 
     T U[6][kF];    // y of the own row, z = j .. j+4, and j+5 on its way: slot (phase + z - j) % 6
@@ -395,7 +405,7 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
                         kk);
 #pragma unroll
             for (int f = 0; f < kF; ++f) {
-                Y4[f] = (PAIR == 1 ? U2[f] : uc[f]) + c1 * kk[f];
+                Y4[f] = (PAIR != 2 ? U2[f] : uc[f]) + c1 * kk[f];
                 // (not OUT: computed here, not sunk to its use two steps on,
                 // which kept every operand alive and spilled)
                 if constexpr (!OUT) asm volatile("" : "+v"(Y4[f]));
@@ -429,6 +439,9 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
                     yo[f] = U0[f] + c2 * kk[f];
                     pst<T>((Y2[f] + U0[f]) + cA * kk[f], ra, vo, so + f * rowb);
                 }
+            } else if constexpr (PAIR == 3) {   // u2 = 3/4 u + 1/4 (u1 + dt k)
+#pragma unroll
+                for (int f = 0; f < kF; ++f) yo[f] = c2 * U0[f] + cA * (Y2[f] + c1 * kk[f]);
             } else {                     // u' = (A + Y4) / 3 + dt/6 k4
                 // (1/3 in two parts: a third rounded to T alone grows u by
                 // 3e-8 (FP32) or 6e-17 of itself every step)
@@ -468,6 +481,120 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
         step(integral_constant<int, 2>{}, std::true_type{});
         if (j == j1) break;
         step(integral_constant<int, 3>{}, std::true_type{});
+        if (j == j1) break;
+    }
+}
+
+// A wavefront of a lone stage (SSP-RK3's last): the output at z = j from y at
+// z = j-2 .. j+2 and u at z = j, with the loads, the slab of y rows and the ring
+// of phases of pair_wave.  All R + 4 rows of a block are output rows (put:
+// inside the grid); its first and last two waves also load the rows beyond.
+template <typename T, bool NOX, typename LDS>
+__device__ __forceinline__ void lone_wave(const PairArgs<T>& a, int row, bool put, int ch, int grp, int j0, int j1,
+                                          int slot, int erow, int slot_e, SumTable& tab, SumStage& sst, LDS* lds) {
+    const Geometry& g = a.g;
+    const int lane = threadIdx.x & 63, nz = g.nz;
+    const unsigned rowb = (unsigned)g.nvp * (unsigned)sizeof(T);
+    const unsigned siteb = (unsigned)(g.srec * (long long)sizeof(T));
+    const unsigned long long xrowb = (unsigned long long)g.xrow * sizeof(T);
+    const unsigned gofs = (unsigned)(grp * kF) * rowb;
+    const unsigned long long rbase = (unsigned long long)(row + kXg) * xrowb + gofs;
+    const unsigned long long ebase = (unsigned long long)(max(erow, 0) + kXg) * xrowb + gofs;
+    const unsigned rbytes = (unsigned)xrowb - gofs;
+    const int pv = min(ch * 64 + lane, g.nv - 1);
+    const unsigned vo = (unsigned)pv * (unsigned)sizeof(T);
+    const unsigned ve = erow >= 0 ? vo : rbytes, vs = put ? vo : rbytes;
+    const unsigned zrec = (unsigned)(g.nch * kPairRec * 8);
+    const unsigned rec0 = (unsigned)(ch * kPairRec + grp * kRec) * 8;
+    const unsigned long long prow = a.part + (unsigned long long)row * nz * zrec + rec0;
+    const unsigned pbytes = (unsigned)nz * zrec - rec0;
+    const unsigned vrec = put ? sum_offset(lane, pbytes) : pbytes;
+    const unsigned long long mrow = (unsigned long long)row * nz * (kMomStride * 8);
+    const unsigned mbytes = (unsigned)nz * (kMomStride * 8), vm = (unsigned)(lane & 15) * 8;
+    const PairConst<T> k = pair_const<T>(g, pv);
+    const T c1 = (T)a.c1, c2 = (T)a.c2, cA = (T)a.cA;
+
+    T U[6][kF];   // y of the own row, z = j-2 .. j+2, and j+3 on its way: slot (phase + 2 + z - j) % 6
+    T E[6][kF];   // edge row of y, z = j .. j+3, in the slots of U
+    auto next = [&](int z) { return z + 1 == nz ? 0 : z + 1; };
+    auto load = [&](unsigned long long base, unsigned v, int z, T (&x)[kF]) {
+        const __amdgpu_buffer_rsrc_t r = prs(base, rbytes);
+#pragma unroll
+        for (int f = 0; f < kF; ++f) x[f] = pld<T>(r, v, (unsigned)z * siteb + f * rowb);
+    };
+    int j = j0;
+    int z3 = uniform(wrapi(j + 3, nz)), z1 = uniform(wrapi(j + 1, nz));
+#pragma unroll
+    for (int q = 0; q < 5; ++q) load(a.y + rbase, vo, uniform(wrapi(j - 2 + q, nz)), U[q]);
+    if constexpr (!NOX) {
+#pragma unroll
+        for (int q = 2; q < 5; ++q) load(a.y + ebase, ve, uniform(wrapi(j - 2 + q, nz)), E[q]);
+    }
+    auto step = [&](auto phase) {
+        constexpr int P = decltype(phase)::value;
+        constexpr int b = P & 1;
+        const auto& U2 = U[(P + 2) % 6];
+        load(a.y + rbase, vo, z3, U[(P + 5) % 6]);
+        if constexpr (!NOX) load(a.y + ebase, ve, z3, E[(P + 5) % 6]);
+        T uc[kF];
+        {
+            const __amdgpu_buffer_rsrc_t ru = prs(a.u + rbase, rbytes);
+#pragma unroll
+            for (int f = 0; f < kF; ++f) uc[f] = pld<T, 2>(ru, vo, (unsigned)j * siteb + f * rowb);
+        }
+        const unsigned w1 = __builtin_amdgcn_raw_buffer_load_b32(prs(a.m1 + mrow, mbytes), vm, (unsigned)z1 * (kMomStride * 8), 0);
+        double m1[kNMom];
+        load_moments(a.m1 + mrow + (unsigned)j * (kMomStride * 8), m1);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!NOX) {
+#pragma unroll
+            for (int f = 0; f < kF; ++f) lds->y[b][slot + 2][f][lane] = U2[f];
+#pragma unroll
+            for (int f = 0; f < kF; ++f) lds->y[b][slot_e][f][lane] = E[(P + 2) % 6][f];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        }
+        const Precession<T> r1 = precession(k, m1);
+        T kk[kF], yo[kF];
+        rhs_unit<T>(k, r1, U2, U[P % 6], U[(P + 1) % 6], U[(P + 3) % 6], U[(P + 4) % 6],
+                    [&](int f, T& xm2, T& xm1, T& xp1, T& xp2) {
+                        if constexpr (NOX) {
+                            xm2 = xm1 = xp1 = xp2 = U2[f];
+                        } else {
+                            xm2 = lds->y[b][slot][f][lane];
+                            xm1 = lds->y[b][slot + 1][f][lane];
+                            xp1 = lds->y[b][slot + 3][f][lane];
+                            xp2 = lds->y[b][slot + 4][f][lane];
+                        }
+                    },
+                    kk);
+        const __amdgpu_buffer_rsrc_t ro = prs(a.out + rbase, rbytes);
+#pragma unroll
+        for (int f = 0; f < kF; ++f) {
+            yo[f] = c2 * uc[f] + cA * (U2[f] + c1 * kk[f]);
+            pst<T>(yo[f], ro, vs, (unsigned)j * siteb + f * rowb);
+        }
+        direction_sums((double)yo[2], (double)yo[3], (double)yo[0] - (double)yo[1], sst, tab, lane, prs(prow, pbytes),
+                       vrec, (unsigned)j * zrec);
+        asm volatile("" ::"v"(w1));
+        ++j;
+        z3 = next(z3);
+        z1 = next(z1);
+    };
+    using std::integral_constant;
+    for (;;) {
+        step(integral_constant<int, 0>{});
+        if (j == j1) break;
+        step(integral_constant<int, 1>{});
+        if (j == j1) break;
+        step(integral_constant<int, 2>{});
+        if (j == j1) break;
+        step(integral_constant<int, 3>{});
+        if (j == j1) break;
+        step(integral_constant<int, 4>{});
+        if (j == j1) break;
+        step(integral_constant<int, 5>{});
         if (j == j1) break;
     }
 }
@@ -567,6 +694,45 @@ __global__ void k_zero_ints(int* __restrict__ p, int n) {
 
 constexpr int kRowWaves = 4;   // waves per block of the one-row form, a unit each
 
+template <typename T, int R>
+struct LoneSlab {
+    T y[2][R + 9][kF][64];   // rows -2 .. R+5 of y, and a slot idle lanes write
+    SumTable tab;
+    SumStage st[R + 4];
+};
+
+template <typename T>
+__global__ __launch_bounds__(64 * (PairShape<T>::R + 4)) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
+void k_lone(const PairArgs<T> a) {
+    constexpr int R = PairShape<T>::R, NW = R + 4;
+    __shared__ LoneSlab<T, R> lds;
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lb = xcd_remap(blockIdx.x, gridDim.x);
+    const int xg = uniform(lb % a.xgroups), rest = uniform(lb / a.xgroups);
+    const int un = uniform(rest % a.nunits), j0 = uniform(rest / a.nunits) * a.zlen;
+    const int nx = a.g.nx, ib = xg * NW, r = ib + wib;
+    if (wib == 0) fill_table(a.g, lds.tab, un >> 1, threadIdx.x & 63);   // (read after the first barrier)
+    const bool lo = wib < 2, hi = wib >= NW - 2;
+    const int er = lo ? ib - 2 + wib : ib + wib + 2;
+    lone_wave<T, false>(a, uniform(wrapi(r, nx)), r < nx, un >> 1, un & 1, j0, min(a.g.nz, j0 + a.zlen), wib,
+                        lo || hi ? uniform(wrapi(er, nx)) : -1, lo ? wib : (hi ? wib + 4 : R + 8), lds.tab,
+                        lds.st[wib], &lds);
+}
+
+template <typename T>
+__global__ __launch_bounds__(64 * kRowWaves) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
+void k_lone_row(const PairArgs<T> a) {
+    __shared__ PairRowLds<kRowWaves> lds;
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lb = xcd_remap(blockIdx.x, gridDim.x);
+    const int groups = (a.nunits + kRowWaves - 1) / kRowWaves;
+    const int un = uniform(lb % groups) * kRowWaves + wib, j0 = uniform(lb / groups) * a.zlen;
+    if (un >= a.nunits) return;
+    fill_table(a.g, lds.tab[wib], un >> 1, threadIdx.x & 63);
+    lone_wave<T, true>(a, 0, true, un >> 1, un & 1, j0, min(a.g.nz, j0 + a.zlen), 0, -1, 0, lds.tab[wib], lds.st[wib],
+                       (LoneSlab<T, 1>*)nullptr);
+}
+
 template <typename T, int PAIR>
 __global__ __launch_bounds__(64 * kRowWaves) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
 void k_pair_row(const PairArgs<T> a) {
@@ -654,7 +820,7 @@ struct PredictArgs {
     const double* tot;    // D, then Q
     const double* base;   // what the prediction starts from (an m, or null: that of tot's state)
     double* m;            // record of tot's state: mu times its moments, with the vacuum terms
-    double* inner;        // the same of base + c k
+    double* inner;        // the same of base + c k (null: not wanted)
     double c;
     double mu, mu2, p2st, p2ct, pmo, ct2, st;
     double twelve_dx, twelve_dz, ko_x, ko_z;
@@ -703,12 +869,17 @@ __device__ __forceinline__ void predict_body(const PredictArgs& p, int blk, Pred
     if (zl >= n) return;
     const long long o = (row + z0 + zl) * kMomStride + s;
     if (s >= kNMom) {
-        p.m[o] = p.inner[o] = 0.0;
+        p.m[o] = 0.0;
+        if (p.inner) p.inner[o] = 0.0;
         return;
     }
     const int a = s & 3, v = s >> 2;
     const double *d = l.d[zl + 2], *q = l.q[zl];
     const double m0 = d[a * 3 + v];
+    // (the record's offset: see precession())
+    const double mm = p.mu * m0 + (s == 0 ? -p.pmo * p.st : (s == 8 ? p.p2ct : 0.0));
+    p.m[o] = mm;
+    if (!p.inner) return;
     // transport: advection multiplies by vx or vz, Kreiss-Oliger by nothing
     double kt = 0.0;
 #pragma unroll
@@ -735,9 +906,6 @@ __device__ __forceinline__ void predict_body(const PredictArgs& p, int blk, Pred
     }
     const double r1 = q[a * 3], i1 = q[a * 3 + 1], e1 = q[a * 3 + 2];
     const double vac = v == 0 ? -p.p2ct * i1 : (v == 1 ? p.pmo * (p.ct2 * r1 + p.st * e1) : -2 * p.p2st * i1);
-    // (the record's offset: see precession())
-    const double mm = p.mu * m0 + (s == 0 ? -p.pmo * p.st : (s == 8 ? p.p2ct : 0.0));
-    p.m[o] = mm;
     p.inner[o] = (p.base ? p.base[o] : mm) + p.mu * (p.c * (loc + kt + vac));
 }
 
@@ -776,18 +944,23 @@ template <typename T>
 PairArgs<T> pair_args(const Geometry& g, const Physics& ph, int zlen, int pair, const PairBuffers& b, double dt) {
     PairArgs<T> a{};
     a.g = g;
-    a.y = (unsigned long long)(pair == 1 ? b.u : b.y3);
+    const bool first = pair == 1 || pair == 3;   // u is the stencil input
+    a.y = (unsigned long long)(first ? b.u : b.y3);
     a.u = (unsigned long long)b.u;
     a.a = (unsigned long long)b.a;
-    a.out = (unsigned long long)(pair == 1 ? b.y3 : b.unew);
-    a.m1 = (unsigned long long)(pair == 1 ? b.mu : b.m3);
+    a.out = (unsigned long long)(first ? b.y3 : b.unew);
+    a.m1 = (unsigned long long)(first ? b.mu : b.m3);
     a.m2 = (unsigned long long)b.min;
     a.part = (unsigned long long)b.part;
-    a.c1 = pair == 1 ? 0.5 * dt : dt;
-    a.c2 = pair == 1 ? 0.5 * dt : 1.0 / 6.0 * dt;
-    a.cA = dt;
+    switch (pair) {
+        case 1: a.c1 = a.c2 = 0.5 * dt; a.cA = dt; break;
+        case 2: a.c1 = dt; a.c2 = 1.0 / 6.0 * dt; break;
+        case 3: a.c1 = dt; a.c2 = 3.0 / 4.0; a.cA = 1.0 / 4.0; break;
+        default: a.c1 = dt; a.c2 = 1.0 / 3.0; a.cA = 2.0 / 3.0; break;
+    }
     a.zlen = zlen;
-    a.xgroups = g.nx == 1 ? 1 : (g.nx + PairShape<T>::R - 1) / PairShape<T>::R;
+    const int rows = PairShape<T>::R + (pair == kLone ? 4 : 0);
+    a.xgroups = g.nx == 1 ? 1 : (g.nx + rows - 1) / rows;
     a.nunits = 2 * g.nch;
     return a;
 }
@@ -795,9 +968,9 @@ PairArgs<T> pair_args(const Geometry& g, const Physics& ph, int zlen, int pair, 
 PredictArgs predict_args(const Geometry& g, const Physics& ph, int pair, const PairBuffers& b, double dt) {
     PredictArgs p{};
     p.tot = b.tot;
-    p.base = pair == 1 ? nullptr : b.mu;
-    p.m = pair == 1 ? b.mu : b.m3;
-    p.inner = b.min;
+    p.base = pair == 2 ? b.mu : nullptr;
+    p.m = pair == 1 || pair == 3 ? b.mu : b.m3;
+    p.inner = pair == kLone ? nullptr : b.min;
     p.c = pair == 1 ? 0.5 * dt : dt;
     p.mu = ph.mu;
     p.mu2 = 2 * ph.mu;
@@ -887,14 +1060,19 @@ hipError_t launch_pair(int pair, const Geometry& g, const Physics& ph, int zlen,
                        hipStream_t s) {
     if (!pair_capable(g) || zlen < 1 || g.lpr != 64) return hipErrorInvalidValue;
     const PairArgs<T> a = pair_args<T>(g, ph, zlen, pair, b, dt);
-    const dim3 grid((unsigned)pair_blocks(g, sizeof(T), zlen));
+    const unsigned nseg = (unsigned)((g.nz + zlen - 1) / zlen);
     if (g.nx == 1) {
-        if (pair == 1) hipLaunchKernelGGL((k_pair_row<T, 1>), grid, dim3(64 * kRowWaves), 0, s, a);
-        else hipLaunchKernelGGL((k_pair_row<T, 2>), grid, dim3(64 * kRowWaves), 0, s, a);
+        const dim3 grid(nseg * ((a.nunits + kRowWaves - 1) / kRowWaves)), block(64 * kRowWaves);
+        if (pair == 1) hipLaunchKernelGGL((k_pair_row<T, 1>), grid, block, 0, s, a);
+        else if (pair == 2) hipLaunchKernelGGL((k_pair_row<T, 2>), grid, block, 0, s, a);
+        else if (pair == 3) hipLaunchKernelGGL((k_pair_row<T, 3>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_lone_row<T>), grid, block, 0, s, a);
     } else {
-        const dim3 block(64 * (PairShape<T>::R + 4));
+        const dim3 grid(nseg * (unsigned)(a.xgroups * a.nunits)), block(64 * (PairShape<T>::R + 4));
         if (pair == 1) hipLaunchKernelGGL((k_pair<T, 1>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((k_pair<T, 2>), grid, block, 0, s, a);
+        else if (pair == 2) hipLaunchKernelGGL((k_pair<T, 2>), grid, block, 0, s, a);
+        else if (pair == 3) hipLaunchKernelGGL((k_pair<T, 3>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_lone<T>), grid, block, 0, s, a);
     }
     return hipGetLastError();
 }

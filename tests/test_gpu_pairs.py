@@ -1,5 +1,5 @@
-"""RK4 in stage pairs (2-flavour periodic boxes): against the oracle at shapes
-that leave the x groups (8 rows in FP64, 12 in FP32), the z segments and the
+"""RK4 and SSP-RK3 in stage pairs (2-flavour periodic boxes): against the oracle at
+shapes that leave the x groups (8 to 16 rows), the z segments and the
 last direction chunk partly filled, boxes narrower than the stencils' reach,
 and mixed with the paths that keep other records of the state."""
 import numpy as np
@@ -29,7 +29,8 @@ def make(N, nx, nz, nn, **kw):
 
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("precision", [64, 32])
-def test_pairs_match_oracle(nuosc_mod, oracle_mod, shape, precision):
+@pytest.mark.parametrize("scheme", ["rk4", "srk3"])
+def test_pairs_match_oracle(nuosc_mod, oracle_mod, shape, precision, scheme):
     """FP64: 1e-12 per field over 9 steps (a few roundings each).  FP32: one
     rounding (2^-24) per store of Y3, A and u' and about four per stage update,
     grown by at most e^(gamma t) < 2: 9 steps x 8 x 2^-24 x 2 = 8.6e-6."""
@@ -40,8 +41,8 @@ def test_pairs_match_oracle(nuosc_mod, oracle_mod, shape, precision):
     if zlen:
         g.set_zlen(zlen)
     for n in (1, 2, 6):     # odd and even numbers of exchanges of the state copies
-        g.step_rk4(n)
-        o.step(n)
+        (g.step_rk4 if scheme == "rk4" else g.step_srk3)(n)
+        (o.step if scheme == "rk4" else o.step_srk3)(n)
     a, b = g.get_state(), o.get_state()
     tol = 1e-12 if precision == 64 else 9 * 8 * 2.0 ** -24 * 2
     for f in range(8):
