@@ -12,11 +12,11 @@ from a hipGraph) over the whole state, which stays resident in HBM.
 Prints one JSON line:
   value          site*dir RK4 updates/s = nx*nz*nv*K / wall(K steps)
   roofline       for the dominant kernel (RK4 stages 3+4; stage 2 where a step
-                 is not made of stage pairs): algorithmic bytes per launch (4
-                 state passes x 8 fields x sizeof(real) per update) / its
-                 average duration from HIP events, against 8 TB/s
-  step_roofline  the same for a whole step (7 passes: 448 B per update in
-                 FP64; 12 where it is not made of stage pairs), plus vs_16pass_ceiling = updates/s over 8 TB/s / 1024 B
+                 is not made of stage pairs): algorithmic bytes per launch (3
+                 state passes in FP64, 4 in FP32 and in stage 2, x 8 fields x
+                 sizeof(real) per update) / its average duration from HIP events, against 8 TB/s
+  step_roofline  the same for a whole step (FP64 5 passes: 320 B per update;
+                 FP32 7 passes: 224 B; 12 passes where it is not made of stage pairs), plus vs_16pass_ceiling = updates/s over 8 TB/s / 1024 B
                  (FP64; 512 B FP32), the ceiling of the 16-pass RK4 streaming
                  in which the per-update targets are stated
   fp32           (default box run) the same workload in the FP32 form: value,
@@ -56,8 +56,9 @@ HBM_PEAK_GBS = 8000.0
 # state passes per update of each stage (read + write of the 8 fields):
 # S1 u -> Y2; S2 Y2, u -> Y3, A; S3 Y3, u -> Y4; S4 Y4, A -> u'
 STAGE_PASSES = (2, 4, 3, 3)
-# the same in stage pairs: u -> Y3, A; Y3, u, A -> u'
-PAIR_PASSES = (3, 0, 4, 0)
+# the same in stage pairs, by bytes per number; FP64: u -> Y3; Y3, u -> u'
+# FP32: u -> Y3, A; Y3, u, A -> u'
+PAIR_PASSES = {8: (2, 0, 3, 0), 4: (3, 0, 4, 0)}
 
 
 def parse():
@@ -488,7 +489,7 @@ def measure_box(N, a, precision):
     value = upd * a.steps / wall
     # the largest kernel: stages 3+4 where a step is two stage pairs, else stage 2
     pairs = stage_ms[1] == 0
-    passes = PAIR_PASSES if pairs else STAGE_PASSES
+    passes = PAIR_PASSES[esize] if pairs else STAGE_PASSES
     main = 2 if pairs else 1
     s2_bytes = passes[main] * nvar * esize * upd
     s2_gbs = s2_bytes / (stage_ms[main] * 1e-3) / 1e9
@@ -584,7 +585,7 @@ def batched_leg(N, a, runs=64, steps=20):
     b.close()
     for g in sims:
         g.close()
-    bpu = sum(PAIR_PASSES) * 8 * 4
+    bpu = sum(PAIR_PASSES[4]) * 8 * 4
     v_bat, v_seq = upd * steps / t_bat, upd * steps / t_seq
     return {
         "value": v_bat, "unit": "updates/s", "sequential_value": v_seq, "speedup_vs_sequential": t_seq / t_bat,

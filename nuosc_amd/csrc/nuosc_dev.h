@@ -224,13 +224,12 @@ hipError_t launch_p3_slice(const Geometry& g, const T* y, const double* G0, cons
 constexpr int kLone = 4;
 struct PairBuffers {
     const void* u;
-    void *a, *y3, *unew;        // A = Y2 + u + dt k2, Y3 (SSP-RK3: u2), the new state
+    void *a, *y3, *unew;        // A = Y2 + u + dt k2 (FP32), Y3 (SSP-RK3: u2), the new state
     double *mu, *m3, *min;      // moment records of u, Y3 and the inner input (Y2, then Y4), [site][kMomStride]
     double *part, *tot;         // direction sums: [site][chunk][kPairRec] partial, [site][kPairRec] total
 };
 bool pair_capable(const Geometry& g);
-// blocks and wavefronts of one pair kernel with z segments of zlen sites
-int pair_blocks(const Geometry& g, int esize, int zlen);
+// wavefronts of the first pair kernel with z segments of zlen sites
 int pair_waves(const Geometry& g, int esize, int zlen);
 // z-segment length the pair kernels start with, alone and for a batch of grids
 int plan_pair_zlen(const Geometry& g, int esize, int num_cus);
@@ -268,10 +267,10 @@ struct BatchTables {
     void* args[2][2] = {};   // [pair][flip] PairArgs arrays
     void* pre[2][2] = {};    // [pair][flip] PredictArgs arrays
     void* sum = nullptr;     // totals arguments
-    int *bmap = nullptr, *tmap = nullptr, *pmap = nullptr;   // logical block -> (member, block of member)
+    int *bmap[2] = {}, *tmap = nullptr, *pmap = nullptr;   // logical block -> (member, block of member)
     int* ctr = nullptr;      // work-queue counters of the persistent launch
-    int nblocks = 0, tblocks = 0, pblocks = 0, esize = 8;
-    int launch = kBatchGrid, pgrid = 0;   // launch form; resident blocks of the persistent grid
+    int nblocks[2] = {0, 0}, tblocks = 0, pblocks = 0, esize = 8;
+    int launch = kBatchGrid, pgrid[2] = {0, 0};   // launch form; resident blocks of the persistent grids
 };
 hipError_t batch_build(BatchTables& t, const std::vector<BatchMember>& members, int esize, int launch,
                        hipStream_t s);

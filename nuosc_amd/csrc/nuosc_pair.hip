@@ -7,7 +7,16 @@
 // registers and LDS:
 //   pair 1: read u       -> Y2 (on chip) -> Y3 = u + dt/2 k2, A = Y2 + u + dt k2
 //   pair 2: read Y3, u, A -> Y4 (on chip) -> u' = (A + Y4)/3 + dt/6 k4
-// 3 + 4 = 7 passes (448 B per FP64 update instead of 768).  An SSP-RK3 step is
+// 3 + 4 = 7 passes instead of 12.  In FP64, which is bound by the passes, A is
+// not kept either: A = Y2 + 2 Y3 - u and Y2 = u + dt/2 k1, so pair 2 forms k1
+// again from the u it reads anyway:
+//   pair 1: read u     -> Y2 (on chip) -> Y3
+//   pair 2: read Y3, u -> Y4 (on chip) -> u' = (2 Y3 + Y4)/3 + dt/6 (k1 + k4)
+// 2 + 3 = 5 passes (320 B per update instead of 768; 512 x 512 x 642: 28.9 ms
+// a step stage by stage, 19.3 in 7 passes, 18.1 in 5: pair 1 is bound by HBM,
+// 7.3 ms, pair 2 by its waits at 2 waves per SIMD, 10.5-11).  FP32 is bound by
+// its vector instructions in both pairs (5.2 and 5.5 ms, 75% busy), so there A
+// is kept.  An SSP-RK3 step is
 // a pair and a single stage, 2 + 3 = 5 passes instead of 8:
 //   pair 3: read u       -> u1 = u + dt k (on chip) -> u2 = 3/4 u + 1/4 (u1 + dt k)
 //   k_lone: read u2, u   -> u' = 1/3 u + 2/3 (u2 + dt k)
@@ -74,8 +83,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t prs(unsigned long long base, u
     return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, kPairRsrc3);
 }
 
-// constant address space: uniform loads from it become scalar loads
-typedef const __attribute__((address_space(4))) double pcdouble;
 // the compiler divides integers in vector registers and may then keep what is
 // derived from the quotient there; this puts a wave-uniform value back
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
@@ -171,25 +178,37 @@ struct PairArgs {
     Geometry g;
     unsigned long long y;      // stencil input (stored x row 0): u (pairs 1, 3), Y3 (pair 2), u2 (lone stage)
     unsigned long long u;      // pair 2, lone stage: u
-    unsigned long long a;      // A: written by pair 1, read by pair 2
+    unsigned long long a;      // A (FP32): written by pair 1, read by pair 2
     unsigned long long out;    // Y3 (pair 1), u2 (pair 3), u' (pair 2, lone stage); no input of the pass
     unsigned long long m1, m2; // moment records of y and of the inner input: [site][kMomStride]
+    unsigned long long m0;     // pair 2: of u
     unsigned long long part;   // partial sums of out: [site][chunk][2][kRec]
     double c1, c2, cA;         // inner input u + c1 k; output's and A's factors of k (pair 3, lone stage:
                                // output c2 u + cA (y + c1 k))
     int zlen, xgroups, nunits;
 };
 
-// x rows a block writes: R, from R + 4 rows of the inner input and R + 8 of y
-template <typename T>
+// FP64: pair 2 forms k1 again instead of reading A
+template <typename T, int PAIR>
+constexpr bool kAgain = sizeof(T) == 8 && PAIR == 2;
+
+// x rows a block writes: R, from R + 4 rows of the inner input (a wavefront
+// each) and R + 8 of y; and the waves per SIMD its registers allow.  FP64: 12
+// waves (3 per SIMD, 168 VGPRs) with a slab of 137 KB; pair 2 holds a z window
+// of u as well (230 VGPRs, so 8 waves, 2 per SIMD; 131 KB).  FP32: 16 waves (4 per SIMD): fewer
+// edge rows for the row (12 waves at 5 per SIMD took 14.6 instead of 11.5 ms
+// per step at 512 x 512 x 642).
+template <typename T, int PAIR>
 struct PairShape {
-    static constexpr int R = sizeof(T) == 8 ? 8 : 12;
+    static constexpr int R = sizeof(T) == 4 ? 12 : (kAgain<T, PAIR> ? 4 : 8);
+    static constexpr int SimdWaves = sizeof(T) == 4 ? 4 : (kAgain<T, PAIR> ? 2 : 3);
 };
 
-template <typename T, int R>
+template <typename T, int R, bool AGAIN>
 struct PairSlab {
     T y[2][R + 9][kF][64];   // rows -4 .. R+3 of y at the inner input's z, and a slot idle lanes write
     T m[2][R + 4][kF][64];   // rows -2 .. R+1 of the inner input
+    T u[AGAIN ? 2 : 0][R + 4][kF][64];   // the same rows of u
     SumTable tab;
     SumStage st[R];
 };
@@ -203,7 +222,7 @@ struct PairRowLds {
 // Per-direction and physics factors of k(y)
 template <typename T>
 struct PairConst {
-    double vx, vy, vz;
+    double nvx, nvy, nvz;   // minus the direction
     T fx, fz;          // -v / (12 h)
     T kx, kz, k6;      // -ko / (16 h) per axis; 6 (kx + kz)
 };
@@ -211,11 +230,11 @@ struct PairConst {
 template <typename T>
 __device__ __forceinline__ PairConst<T> pair_const(const Geometry& g, int pv) {
     PairConst<T> k;
-    k.vx = g.vx[pv];
-    k.vy = g.vy[pv];
-    k.vz = g.vz[pv];
-    k.fx = (T)(-k.vx / g.twelve_dx);
-    k.fz = (T)(-k.vz / g.twelve_dz);
+    k.nvx = -g.vx[pv];
+    k.nvy = -g.vy[pv];
+    k.nvz = -g.vz[pv];
+    k.fx = (T)(k.nvx / g.twelve_dx);
+    k.fz = (T)(k.nvz / g.twelve_dz);
     k.kx = (T)g.ko_x;
     k.kz = (T)g.ko_z;
     k.k6 = (T)(6 * (g.ko_x + g.ko_z));
@@ -234,18 +253,34 @@ template <typename T>
 struct Precession {
     T q, b, c;
 };
+// x: the site's record, value n in lane n of every 16-lane row.  The products
+// take it by DPP row_newbcast (64-bit operations have that control), four
+// instructions a projection; the compiler forms a broadcast as two moves
+// instead (24 per stage), and records in scalar registers (three moves) cost a
+// scalar load that no register is free to prefetch.  (The s_nop covers a DPP
+// read of x behind the instruction that wrote it.)
+#define NUOSC_BC(n) " row_newbcast:" #n " row_mask:0xf bank_mask:0xf\n\t"
 template <typename T>
-__device__ __forceinline__ Precession<T> precession(const PairConst<T>& k, const double (&m)[kNMom]) {
-    return Precession<T>{(T)(m[0] - m[1] * k.vx - m[2] * k.vy - m[3] * k.vz),
-                         (T)(m[4] - m[5] * k.vx - m[6] * k.vy - m[7] * k.vz),
-                         (T)(m[8] - m[9] * k.vx - m[10] * k.vy - m[11] * k.vz)};
+__device__ __forceinline__ Precession<T> precession(const PairConst<T>& k, double x) {
+    double A, B, C;
+    asm("s_nop 1\n\t"
+        "v_mov_b64_dpp %0, %3" NUOSC_BC(0)
+        "v_mov_b64_dpp %1, %3" NUOSC_BC(4)
+        "v_mov_b64_dpp %2, %3" NUOSC_BC(8)
+        "v_fmac_f64_dpp %0, %3, %4" NUOSC_BC(1)
+        "v_fmac_f64_dpp %1, %3, %4" NUOSC_BC(5)
+        "v_fmac_f64_dpp %2, %3, %4" NUOSC_BC(9)
+        "v_fmac_f64_dpp %0, %3, %5" NUOSC_BC(2)
+        "v_fmac_f64_dpp %1, %3, %5" NUOSC_BC(6)
+        "v_fmac_f64_dpp %2, %3, %5" NUOSC_BC(10)
+        "v_fmac_f64_dpp %0, %3, %6" NUOSC_BC(3)
+        "v_fmac_f64_dpp %1, %3, %6" NUOSC_BC(7)
+        "v_fmac_f64_dpp %2, %3, %6" NUOSC_BC(11)
+        : "=&v"(A), "=&v"(B), "=&v"(C)
+        : "v"(x), "v"(k.nvx), "v"(k.nvy), "v"(k.nvz));
+    return Precession<T>{(T)A, (T)B, (T)C};
 }
-
-__device__ __forceinline__ void load_moments(unsigned long long site, double (&m)[kNMom]) {
-    pcdouble* p = (pcdouble*)site;
-#pragma unroll
-    for (int q = 0; q < kNMom; ++q) m[q] = p[q];
-}
+#undef NUOSC_BC
 
 // k(y) of the 4 fields: c centre values, z neighbours, x neighbours through
 // the callable.  The stencils (nuosc_class.cpp:122-123, 182-183) are taken on
@@ -316,23 +351,34 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
     T U[6][kF];    // y of the own row, z = j .. j+4, and j+5 on its way: slot (phase + z - j) % 6
     T Y[6][kF];    // inner input, z = j-2 .. j+2: slot (phase + 2 + z - j) % 6 (not OUT: from j on)
     T E[6][kF];    // not OUT: edge row of y, z = j+2 .. j+5, in the slots of U
-    T uc[kF];      // pair 2: u at z = j+2 (of the next step, once used)
+    T uc[kF];      // pair 2 (FP32): u at z = j+2 (of the next step, once used)
+    T W[6][kF];    // pair 2 (FP64): u of the own row, z = j-2 .. j+2, and j+3 on its way: the slots of Y
     auto next = [&](int z) { return z + 1 == nz ? 0 : z + 1; };
     auto load = [&](unsigned long long base, unsigned v, int z, T (&x)[kF]) {
         const __amdgpu_buffer_rsrc_t r = prs(base, rbytes);
 #pragma unroll
         for (int f = 0; f < kF; ++f) x[f] = pld<T>(r, v, (unsigned)z * siteb + f * rowb);
     };
-    int j = j0 - 4;   // the step; z5, z3, z2: wrapped j+5, j+3, j+2
-    int z5 = uniform(wrapi(j + 5, nz)), z3 = uniform(wrapi(j + 3, nz)), z2 = uniform(wrapi(j + 2, nz));
-    int z1 = uniform(wrapi(j + 1, nz));
+    int j = j0 - 4;   // the step; z5, z3, z1: wrapped j+5, j+3, j+1
+    int z5 = uniform(wrapi(j + 5, nz)), z3 = uniform(wrapi(j + 3, nz)), z1 = uniform(wrapi(j + 1, nz));
+    const int z2 = uniform(wrapi(j + 2, nz));
 #pragma unroll
     for (int q = 0; q < 5; ++q) load(a.y + rbase, vo, wrapi(j + q, nz), U[q]);
     if constexpr (!OUT && !NOX) {
 #pragma unroll
         for (int q = 2; q < 5; ++q) load(a.y + ebase, ve, wrapi(j + q, nz), E[q]);
     }
-    if constexpr (PAIR == 2) load(a.u + rbase, vo, z2, uc);
+    constexpr bool AGAIN = kAgain<T, PAIR>;
+    // moment records of this step and the next: of y at z = j+2, of the inner
+    // input and (FP64 pair 2) of u at z = j
+    auto moment = [&](unsigned long long m, int z) {
+        return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(prs(m + mrow, mbytes), vm,
+                                                                               (unsigned)z * (kMomStride * 8), 0));
+    };
+    double M1[2], M2[2] = {0.0, 0.0}, M0[2] = {0.0, 0.0};
+    M1[0] = moment(a.m1, z2);
+    if constexpr (AGAIN) load(a.u + rbase, vo, z2, W[4]);
+    else if constexpr (PAIR == 2) load(a.u + rbase, vo, z2, uc);
 #pragma unroll
     for (int q = 0; q < 6; ++q)
 #pragma unroll
@@ -356,27 +402,27 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
         // ---- loads for the next steps (A: for the end of this one)
         load(a.y + rbase, vo, z5, U[(P + 5) % 6]);
         if constexpr (!OUT && !NOX) load(a.y + ebase, ve, z5, E[(P + 5) % 6]);
+        if constexpr (AGAIN) load(a.u + rbase, vo, z3, W[(P + 5) % 6]);
         T ac[kF];
-        if constexpr (PAIR == 2 && WRITE) {
+        if constexpr (PAIR == 2 && !AGAIN && WRITE) {
             const __amdgpu_buffer_rsrc_t ra = prs(a.a + rbase, rbytes);
 #pragma unroll
             for (int f = 0; f < kF; ++f) ac[f] = pld<T, 2>(ra, vo, (unsigned)j * siteb + f * rowb);
         }
-        // the moment records of the next step: into L2, for the scalar loads
-        const __amdgpu_buffer_rsrc_t rm1 = prs(a.m1 + mrow, mbytes), rm2 = prs(a.m2 + mrow, mbytes);
-        const unsigned w1 = __builtin_amdgcn_raw_buffer_load_b32(rm1, vm, (unsigned)z3 * (kMomStride * 8), 0);
-        unsigned w2 = 0;
-        if constexpr (OUT) w2 = __builtin_amdgcn_raw_buffer_load_b32(rm2, vm, (unsigned)z1 * (kMomStride * 8), 0);
-        // moments of y at z = j + 2 (uniform: scalar loads, which arrive with the
-        // barrier)
-        double m1[kNMom], m2[kNMom];
-        load_moments(a.m1 + mrow + (unsigned)z2 * (kMomStride * 8), m1);
+        // moment records of the next step
+        M1[b ^ 1] = moment(a.m1, z3);
+        if constexpr (OUT) M2[b ^ 1] = moment(a.m2, z1);
+        if constexpr (OUT && AGAIN) M0[b ^ 1] = moment(a.m0, z1);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (!NOX) {
 #pragma unroll
             for (int f = 0; f < kF; ++f) lds->y[b][slot_m + 2][f][lane] = U2[f];
 #pragma unroll
             for (int f = 0; f < kF; ++f) lds->m[b][slot_m][f][lane] = Y2[f];
+            if constexpr (AGAIN && WRITE) {
+#pragma unroll
+                for (int f = 0; f < kF; ++f) lds->u[b][slot_m][f][lane] = W[(P + 2) % 6][f];
+            }
             if constexpr (!OUT) {
 #pragma unroll
                 for (int f = 0; f < kF; ++f) lds->y[b][slot_e][f][lane] = E[(P + 2) % 6][f];
@@ -386,10 +432,7 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
         }
         {   // ---- the inner input at z = j + 2
-            const Precession<T> r1 = precession(k, m1);
-            // (and the inner input's moments at z = j, for the output)
-            if constexpr (OUT && WRITE) load_moments(a.m2 + mrow + (unsigned)j * (kMomStride * 8), m2);
-            __builtin_amdgcn_sched_barrier(0);
+            const Precession<T> r1 = precession(k, M1[b]);
             T kk[kF];
             rhs_unit<T>(k, r1, U2, U0, U1, U3, U4,
                         [&](int f, T& xm2, T& xm1, T& xp1, T& xp2) {
@@ -405,18 +448,18 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
                         kk);
 #pragma unroll
             for (int f = 0; f < kF; ++f) {
-                Y4[f] = (PAIR != 2 ? U2[f] : uc[f]) + c1 * kk[f];
+                Y4[f] = (PAIR != 2 ? U2[f] : (AGAIN ? W[(P + 4) % 6][f] : uc[f])) + c1 * kk[f];
                 // (not OUT: computed here, not sunk to its use two steps on,
                 // which kept every operand alive and spilled)
                 if constexpr (!OUT) asm volatile("" : "+v"(Y4[f]));
             }
         }
-        if constexpr (PAIR == 2) {
+        if constexpr (PAIR == 2 && !AGAIN) {
             load(a.u + rbase, vo, z3, uc);
             __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (OUT && WRITE) {   // ---- the output at z = j
-            const Precession<T> r2 = precession(k, m2);
+            const Precession<T> r2 = precession(k, M2[b]);
             T kk[kF], yo[kF];
             rhs_unit<T>(k, r2, Y2, Y0, Y1, Y3, Y4,
                         [&](int f, T& xm2, T& xm1, T& xp1, T& xp2) {
@@ -432,20 +475,41 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
                         kk);
             const unsigned so = (unsigned)j * siteb;
             const __amdgpu_buffer_rsrc_t ro = prs(a.out + rbase, rbytes);
-            if constexpr (PAIR == 1) {   // A = Y2 + u + dt k2, Y3 = u + dt/2 k2
+            // (1/3 in two parts: a third rounded to T alone grows u by 3e-8 (FP32)
+            // or 6e-17 of itself every step)
+            const T third = (T)(1.0 / 3.0), rest = sizeof(T) == 4 ? (T)(1.0 / 3.0 - (double)third) : (T)kThirdRest;
+            if constexpr (PAIR == 1) {   // Y3 = u + dt/2 k2, A = Y2 + u + dt k2
                 const __amdgpu_buffer_rsrc_t ra = prs(a.a + rbase, rbytes);
 #pragma unroll
                 for (int f = 0; f < kF; ++f) {
                     yo[f] = U0[f] + c2 * kk[f];
-                    pst<T>((Y2[f] + U0[f]) + cA * kk[f], ra, vo, so + f * rowb);
+                    if constexpr (!kAgain<T, 2>) pst<T>((Y2[f] + U0[f]) + cA * kk[f], ra, vo, so + f * rowb);
+                }
+            } else if constexpr (AGAIN) {   // u' = (2 Y3 + Y4) / 3 + dt/6 (k1 + k4)
+                const Precession<T> r0 = precession(k, M0[b]);
+                const auto& W2 = W[(P + 2) % 6];
+                T k1[kF];
+                rhs_unit<T>(k, r0, W2, W[P % 6], W[(P + 1) % 6], W[(P + 3) % 6], W[(P + 4) % 6],
+                            [&](int f, T& xm2, T& xm1, T& xp1, T& xp2) {
+                                if constexpr (NOX) {
+                                    xm2 = xm1 = xp1 = xp2 = W2[f];
+                                } else {
+                                    xm2 = lds->u[b][slot_m - 2][f][lane];
+                                    xm1 = lds->u[b][slot_m - 1][f][lane];
+                                    xp1 = lds->u[b][slot_m + 1][f][lane];
+                                    xp2 = lds->u[b][slot_m + 2][f][lane];
+                                }
+                            },
+                            k1);
+#pragma unroll
+                for (int f = 0; f < kF; ++f) {
+                    const T s = (T)2 * U0[f] + Y2[f];
+                    yo[f] = s * third + (s * rest + c2 * (k1[f] + kk[f]));
                 }
             } else if constexpr (PAIR == 3) {   // u2 = 3/4 u + 1/4 (u1 + dt k)
 #pragma unroll
                 for (int f = 0; f < kF; ++f) yo[f] = c2 * U0[f] + cA * (Y2[f] + c1 * kk[f]);
             } else {                     // u' = (A + Y4) / 3 + dt/6 k4
-                // (1/3 in two parts: a third rounded to T alone grows u by
-                // 3e-8 (FP32) or 6e-17 of itself every step)
-                const T third = (T)(1.0 / 3.0), rest = sizeof(T) == 4 ? (T)(1.0 / 3.0 - (double)third) : (T)kThirdRest;
 #pragma unroll
                 for (int f = 0; f < kF; ++f) {
                     const T s = ac[f] + Y2[f];
@@ -457,11 +521,9 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
             direction_sums((double)yo[2], (double)yo[3], (double)yo[0] - (double)yo[1], sst, tab, lane,
                            prs(prow, pbytes), vrec, (unsigned)j * zrec);
         }
-        asm volatile("" ::"v"(w1), "v"(w2));
         ++j;
         z5 = next(z5);
         z3 = next(z3);
-        z2 = next(z2);
         z1 = next(z1);
     };
     using std::integral_constant;
@@ -524,6 +586,11 @@ __device__ __forceinline__ void lone_wave(const PairArgs<T>& a, int row, bool pu
     };
     int j = j0;
     int z3 = uniform(wrapi(j + 3, nz)), z1 = uniform(wrapi(j + 1, nz));
+    auto moment = [&](int z) {
+        return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(prs(a.m1 + mrow, mbytes), vm,
+                                                                               (unsigned)z * (kMomStride * 8), 0));
+    };
+    double M1[2] = {moment(j), 0.0};
 #pragma unroll
     for (int q = 0; q < 5; ++q) load(a.y + rbase, vo, uniform(wrapi(j - 2 + q, nz)), U[q]);
     if constexpr (!NOX) {
@@ -542,9 +609,7 @@ __device__ __forceinline__ void lone_wave(const PairArgs<T>& a, int row, bool pu
 #pragma unroll
             for (int f = 0; f < kF; ++f) uc[f] = pld<T, 2>(ru, vo, (unsigned)j * siteb + f * rowb);
         }
-        const unsigned w1 = __builtin_amdgcn_raw_buffer_load_b32(prs(a.m1 + mrow, mbytes), vm, (unsigned)z1 * (kMomStride * 8), 0);
-        double m1[kNMom];
-        load_moments(a.m1 + mrow + (unsigned)j * (kMomStride * 8), m1);
+        M1[b ^ 1] = moment(z1);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (!NOX) {
 #pragma unroll
@@ -555,7 +620,7 @@ __device__ __forceinline__ void lone_wave(const PairArgs<T>& a, int row, bool pu
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
         }
-        const Precession<T> r1 = precession(k, m1);
+        const Precession<T> r1 = precession(k, M1[b]);
         T kk[kF], yo[kF];
         rhs_unit<T>(k, r1, U2, U[P % 6], U[(P + 1) % 6], U[(P + 3) % 6], U[(P + 4) % 6],
                     [&](int f, T& xm2, T& xm1, T& xp1, T& xp2) {
@@ -577,7 +642,6 @@ __device__ __forceinline__ void lone_wave(const PairArgs<T>& a, int row, bool pu
         }
         direction_sums((double)yo[2], (double)yo[3], (double)yo[0] - (double)yo[1], sst, tab, lane, prs(prow, pbytes),
                        vrec, (unsigned)j * zrec);
-        asm volatile("" ::"v"(w1));
         ++j;
         z3 = next(z3);
         z1 = next(z1);
@@ -602,7 +666,7 @@ __device__ __forceinline__ void lone_wave(const PairArgs<T>& a, int row, bool pu
 // logical block -> (x group fastest, unit, z segment): neighbouring blocks,
 // which share edge rows, run on one XCD at about the same time
 template <typename T, int PAIR, int R>
-__device__ __forceinline__ void pair_block(const PairArgs<T>& a, int lb, int wib, PairSlab<T, R>& lds) {
+__device__ __forceinline__ void pair_block(const PairArgs<T>& a, int lb, int wib, PairSlab<T, R, kAgain<T, PAIR>>& lds) {
     const int xg = uniform(lb % a.xgroups), rest = uniform(lb / a.xgroups);
     const int un = uniform(rest % a.nunits), j0 = uniform(rest / a.nunits) * a.zlen;
     const int ch = un >> 1, grp = un & 1;
@@ -622,18 +686,11 @@ __device__ __forceinline__ void pair_block(const PairArgs<T>& a, int lb, int wib
     }
 }
 
-// Waves per SIMD the register allocation aims at: 12 waves of one block per
-// CU (FP64: its slab takes 137 KB), two blocks in FP32.
-template <typename T>
-constexpr int pair_simd_waves() {
-    return sizeof(T) == 8 ? 3 : 4;
-}
-
 template <typename T, int PAIR>
-__global__ __launch_bounds__(64 * (PairShape<T>::R + 4)) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
+__global__ __launch_bounds__(64 * (PairShape<T, PAIR>::R + 4)) __attribute__((amdgpu_waves_per_eu(PairShape<T, PAIR>::SimdWaves)))
 void k_pair(const PairArgs<T> a) {
-    constexpr int R = PairShape<T>::R;
-    __shared__ PairSlab<T, R> lds;
+    constexpr int R = PairShape<T, PAIR>::R;
+    __shared__ PairSlab<T, R, kAgain<T, PAIR>> lds;
     const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     pair_block<T, PAIR, R>(a, xcd_remap(blockIdx.x, gridDim.x), wib, lds);
 }
@@ -641,10 +698,10 @@ void k_pair(const PairArgs<T> a) {
 // Many independent runs in one launch: logical block -> (run, block of run)
 // from bmap; each run's arguments from the runs table (read with scalar loads).
 template <typename T, int PAIR>
-__global__ __launch_bounds__(64 * (PairShape<T>::R + 4)) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
+__global__ __launch_bounds__(64 * (PairShape<T, PAIR>::R + 4)) __attribute__((amdgpu_waves_per_eu(PairShape<T, PAIR>::SimdWaves)))
 void k_pair_batch(const PairArgs<T>* __restrict__ runs, const int* __restrict__ bmap) {
-    constexpr int R = PairShape<T>::R;
-    __shared__ PairSlab<T, R> lds;
+    constexpr int R = PairShape<T, PAIR>::R;
+    __shared__ PairSlab<T, R, kAgain<T, PAIR>> lds;
     const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lb = xcd_remap(blockIdx.x, gridDim.x);
     const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)bmap;
@@ -662,11 +719,11 @@ void k_pair_batch(const PairArgs<T>* __restrict__ runs, const int* __restrict__ 
 // counter passes the range (the exit every wave reaches); the counters are
 // zeroed by k_zero_ints before each launch.
 template <typename T, int PAIR>
-__global__ __launch_bounds__(64 * (PairShape<T>::R + 4)) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
+__global__ __launch_bounds__(64 * (PairShape<T, PAIR>::R + 4)) __attribute__((amdgpu_waves_per_eu(PairShape<T, PAIR>::SimdWaves)))
 void k_pair_batch_q(const PairArgs<T>* __restrict__ runs, const int* __restrict__ bmap, int* __restrict__ ctr,
                     int nitems) {
-    constexpr int R = PairShape<T>::R;
-    __shared__ PairSlab<T, R> lds;
+    constexpr int R = PairShape<T, PAIR>::R;
+    __shared__ PairSlab<T, R, kAgain<T, PAIR>> lds;
     __shared__ int next;
     const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int x = blockIdx.x % 8;
@@ -702,9 +759,9 @@ struct LoneSlab {
 };
 
 template <typename T>
-__global__ __launch_bounds__(64 * (PairShape<T>::R + 4)) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
+__global__ __launch_bounds__(64 * (PairShape<T, 3>::R + 4)) __attribute__((amdgpu_waves_per_eu(PairShape<T, 3>::SimdWaves)))
 void k_lone(const PairArgs<T> a) {
-    constexpr int R = PairShape<T>::R, NW = R + 4;
+    constexpr int R = PairShape<T, 3>::R, NW = R + 4;
     __shared__ LoneSlab<T, R> lds;
     const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lb = xcd_remap(blockIdx.x, gridDim.x);
@@ -720,7 +777,7 @@ void k_lone(const PairArgs<T> a) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(64 * kRowWaves) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
+__global__ __launch_bounds__(64 * kRowWaves) __attribute__((amdgpu_waves_per_eu(PairShape<T, 3>::SimdWaves)))
 void k_lone_row(const PairArgs<T> a) {
     __shared__ PairRowLds<kRowWaves> lds;
     const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -734,7 +791,7 @@ void k_lone_row(const PairArgs<T> a) {
 }
 
 template <typename T, int PAIR>
-__global__ __launch_bounds__(64 * kRowWaves) __attribute__((amdgpu_waves_per_eu(pair_simd_waves<T>())))
+__global__ __launch_bounds__(64 * kRowWaves) __attribute__((amdgpu_waves_per_eu(PairShape<T, PAIR>::SimdWaves)))
 void k_pair_row(const PairArgs<T> a) {
     __shared__ PairRowLds<kRowWaves> lds;
     const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -940,6 +997,12 @@ __global__ __launch_bounds__(256) void k_pair_predict_batch(const PredictArgs* _
     predict_body(p, cm[2 * blockIdx.x + 1], lds);
 }
 
+// x rows a block of a pair (or of the lone stage) writes
+int pair_rows(int esize, int pair) {
+    if (esize == 4) return PairShape<float, 1>::R + (pair == kLone ? 4 : 0);
+    return pair == 2 ? PairShape<double, 2>::R : PairShape<double, 1>::R + (pair == kLone ? 4 : 0);
+}
+
 template <typename T>
 PairArgs<T> pair_args(const Geometry& g, const Physics& ph, int zlen, int pair, const PairBuffers& b, double dt) {
     PairArgs<T> a{};
@@ -951,6 +1014,7 @@ PairArgs<T> pair_args(const Geometry& g, const Physics& ph, int zlen, int pair, 
     a.out = (unsigned long long)(first ? b.y3 : b.unew);
     a.m1 = (unsigned long long)(first ? b.mu : b.m3);
     a.m2 = (unsigned long long)b.min;
+    a.m0 = (unsigned long long)b.mu;
     a.part = (unsigned long long)b.part;
     switch (pair) {
         case 1: a.c1 = a.c2 = 0.5 * dt; a.cA = dt; break;
@@ -959,7 +1023,7 @@ PairArgs<T> pair_args(const Geometry& g, const Physics& ph, int zlen, int pair, 
         default: a.c1 = dt; a.c2 = 1.0 / 3.0; a.cA = 2.0 / 3.0; break;
     }
     a.zlen = zlen;
-    const int rows = PairShape<T>::R + (pair == kLone ? 4 : 0);
+    const int rows = pair_rows(sizeof(T), pair);
     a.xgroups = g.nx == 1 ? 1 : (g.nx + rows - 1) / rows;
     a.nunits = 2 * g.nch;
     return a;
@@ -996,34 +1060,31 @@ bool pair_capable(const Geometry& g) {
 
 namespace {
 // blocks of the box form (batches take it for one-row grids too)
-long long pair_box_blocks(const Geometry& g, int esize, int zlen) {
-    const int R = esize == 8 ? PairShape<double>::R : PairShape<float>::R;
+long long pair_box_blocks(const Geometry& g, int esize, int pair, int zlen) {
+    const int R = pair_rows(esize, pair);
     return (long long)((g.nz + zlen - 1) / zlen) * 2 * g.nch * ((g.nx + R - 1) / R);
 }
-}  // namespace
-
-int pair_blocks(const Geometry& g, int esize, int zlen) {
-    if (g.nx > 1) return (int)pair_box_blocks(g, esize, zlen);
+long long pair_blocks(const Geometry& g, int esize, int pair, int zlen) {
+    if (g.nx > 1) return pair_box_blocks(g, esize, pair, zlen);
     return (g.nz + zlen - 1) / zlen * ((2 * g.nch + kRowWaves - 1) / kRowWaves);
-}
-
-int pair_waves(const Geometry& g, int esize, int zlen) {
-    const int R = esize == 8 ? PairShape<double>::R : PairShape<float>::R;
-    return pair_blocks(g, esize, zlen) * (g.nx == 1 ? kRowWaves : R + 4);
 }
 
 // Time of a pair kernel's blocks in steps of the z march: rounds of as many
 // blocks as the GPU holds at once (one per CU in the box form, counted as
 // three in the one-row form, of which FP32 holds five: 3001 x 492 in FP32 takes
 // 110-113 us in segments of 24 or 16 sites, 130 in 10), each of zlen steps and
-// about eight more: four that write nothing, the rest the block's start.  At 512 x 512 x
-// 642 the model orders segments of 64 .. 512 sites as they measure in both
-// precisions (FP64: 256 best, 19.5 ms, 64 worst, 20.5 ms; FP32: 128 best, 11.5,
-// 171 worst, 12.0); 20 x 200 x 162: segments of 13 sites are two rounds (75 us
-// a kernel), 15 one.
+// about eight more: four that write nothing, the rest the block's start.  At
+// 512 x 512 x 642 the model orders segments of 64 .. 512 sites as they measure
+// in both precisions; 20 x 200 x 162: segments of 13 sites are two rounds
+// (75 us a kernel), 15 one.
 double pair_march_steps(long long blocks, int zlen, bool one_row, int num_cus) {
     const long long slots = (long long)num_cus * (one_row ? 3 : 1);
     return (double)((blocks + slots - 1) / slots) * (zlen + 8);
+}
+}  // namespace
+
+int pair_waves(const Geometry& g, int esize, int zlen) {
+    return (int)(pair_blocks(g, esize, 1, zlen) * (g.nx == 1 ? kRowWaves : pair_rows(esize, 1) + 4));
 }
 
 int plan_pair_zlen(const Geometry& g, int esize, int num_cus) {
@@ -1031,7 +1092,8 @@ int plan_pair_zlen(const Geometry& g, int esize, int num_cus) {
     double least = 1e300;
     for (int most = std::min(g.nz, 1024); most >= 1; --most) {
         const int nseg = (g.nz + most - 1) / most, zlen = (g.nz + nseg - 1) / nseg;   // equal segments
-        const double t = pair_march_steps(pair_blocks(g, esize, zlen), zlen, g.nx == 1, num_cus);
+        double t = 0.0;
+        for (int pair : {1, 2}) t += pair_march_steps(pair_blocks(g, esize, pair, zlen), zlen, g.nx == 1, num_cus);
         if (t < least) {
             least = t;
             best = zlen;
@@ -1044,9 +1106,12 @@ int plan_batch_zlen(const std::vector<Geometry>& gs, int esize, int num_cus) {
     int best = 64;
     double least = 1e300;
     for (int zlen : {4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256}) {
-        long long blocks = 0;
-        for (const Geometry& g : gs) blocks += pair_box_blocks(g, esize, std::min(zlen, g.nz));
-        const double t = pair_march_steps(blocks, zlen, false, num_cus);
+        double t = 0.0;
+        for (int pair : {1, 2}) {
+            long long blocks = 0;
+            for (const Geometry& g : gs) blocks += pair_box_blocks(g, esize, pair, std::min(zlen, g.nz));
+            t += pair_march_steps(blocks, zlen, false, num_cus);
+        }
         if (t < least) {
             least = t;
             best = zlen;
@@ -1068,7 +1133,8 @@ hipError_t launch_pair(int pair, const Geometry& g, const Physics& ph, int zlen,
         else if (pair == 3) hipLaunchKernelGGL((k_pair_row<T, 3>), grid, block, 0, s, a);
         else hipLaunchKernelGGL((k_lone_row<T>), grid, block, 0, s, a);
     } else {
-        const dim3 grid(nseg * (unsigned)(a.xgroups * a.nunits)), block(64 * (PairShape<T>::R + 4));
+        const dim3 grid(nseg * (unsigned)(a.xgroups * a.nunits));
+        const dim3 block(64 * (pair_rows(sizeof(T), pair) + (pair == kLone ? 0 : 4)));
         if (pair == 1) hipLaunchKernelGGL((k_pair<T, 1>), grid, block, 0, s, a);
         else if (pair == 2) hipLaunchKernelGGL((k_pair<T, 2>), grid, block, 0, s, a);
         else if (pair == 3) hipLaunchKernelGGL((k_pair<T, 3>), grid, block, 0, s, a);
@@ -1117,14 +1183,15 @@ hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hip
         std::memcpy(host.data() + at, p, bytes);
         return at;
     };
-    // pair, totals and predict blocks -> (member, block of member)
-    std::vector<long long> count[3];
+    // blocks of the two pairs, the totals and the prediction -> (member, block of member)
+    std::vector<long long> count[4];
     for (const BatchMember& m : ms) {
         const Geometry& g = m.g;
         const long long sites = (long long)g.nx * g.nz;
-        count[0].push_back(pair_box_blocks(g, sizeof(T), m.zlen));
-        count[1].push_back((sites + kTotSites - 1) / kTotSites);
-        count[2].push_back(predict_blocks(g.nx, g.nz));
+        // (the box form for every member, one-row grids included)
+        for (int pair : {1, 2}) count[pair - 1].push_back(pair_box_blocks(g, sizeof(T), pair, m.zlen));
+        count[2].push_back((sites + kTotSites - 1) / kTotSites);
+        count[3].push_back(predict_blocks(g.nx, g.nz));
     }
     auto put_map = [&](const std::vector<long long>& c, int& blocks) {
         long long total = 0;
@@ -1140,7 +1207,7 @@ hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hip
             }
         return at;
     };
-    size_t off_args[2][2], off_pre[2][2], off_map[3];
+    size_t off_args[2][2], off_pre[2][2], off_map[4];
     for (int flip = 0; flip < 2; ++flip)
         for (int pair = 1; pair <= 2; ++pair) {
             std::vector<PairArgs<T>> pa(n);
@@ -1162,8 +1229,8 @@ hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hip
     for (int r = 0; r < n; ++r)
         sa[r] = SumArgs{ms[r].b.part, ms[r].b.tot, ms[r].g.nch, (long long)ms[r].g.nx * ms[r].g.nz};
     const size_t off_sum = put(sa.data(), n * sizeof(SumArgs));
-    int blocks[3];
-    for (int k = 0; k < 3; ++k) off_map[k] = put_map(count[k], blocks[k]);
+    int blocks[4];
+    for (int k = 0; k < 4; ++k) off_map[k] = put_map(count[k], blocks[k]);
     const std::vector<int> zeros(kBatchCounters, 0);
     const size_t off_ctr = put(zeros.data(), kBatchCounters * sizeof(int));
     hipError_t e;
@@ -1179,41 +1246,44 @@ hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hip
             t.pre[p][flip] = d + off_pre[p][flip];
         }
     t.sum = d + off_sum;
-    t.bmap = (int*)(d + off_map[0]);
-    t.tmap = (int*)(d + off_map[1]);
-    t.pmap = (int*)(d + off_map[2]);
+    for (int p = 0; p < 2; ++p) {
+        t.bmap[p] = (int*)(d + off_map[p]);
+        t.nblocks[p] = blocks[p];
+    }
+    t.tmap = (int*)(d + off_map[2]);
+    t.pmap = (int*)(d + off_map[3]);
     t.ctr = (int*)(d + off_ctr);
-    t.nblocks = blocks[0];
-    t.tblocks = blocks[1];
-    t.pblocks = blocks[2];
+    t.tblocks = blocks[2];
+    t.pblocks = blocks[3];
     // persistent launch: a grid of as many blocks as the GPU holds at once
     {
-        int dev = 0, cus = 0, bpc = 0;
+        int dev = 0, cus = 0, bpc[2] = {0, 0};
         if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
         if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
-        if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, k_pair_batch_q<T, 2>, 64 * (PairShape<T>::R + 4), 0)) !=
-            hipSuccess)
+        if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc[0], k_pair_batch_q<T, 1>,
+                                                              64 * (PairShape<T, 1>::R + 4), 0)) != hipSuccess)
             return e;
-        t.pgrid = std::max(8, (cus * std::max(bpc, 1) + 7) / 8 * 8);
+        if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc[1], k_pair_batch_q<T, 2>,
+                                                              64 * (PairShape<T, 2>::R + 4), 0)) != hipSuccess)
+            return e;
+        for (int p = 0; p < 2; ++p) t.pgrid[p] = std::max(8, (cus * std::max(bpc[p], 1) + 7) / 8 * 8);
     }
     if ((e = hipMemcpyAsync(t.buf, host.data(), host.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return e;
     return hipStreamSynchronize(s);
 }
 
-template <typename T>
-hipError_t batch_pair_t(const BatchTables& t, int pair, int flip, hipStream_t s) {
-    const dim3 block(64 * (PairShape<T>::R + 4));
-    const PairArgs<T>* a = (const PairArgs<T>*)t.args[pair - 1][flip];
+template <typename T, int PAIR>
+hipError_t batch_pair_t(const BatchTables& t, int flip, hipStream_t s) {
+    const dim3 block(64 * (PairShape<T, PAIR>::R + 4));
+    const PairArgs<T>* a = (const PairArgs<T>*)t.args[PAIR - 1][flip];
+    const int n = t.nblocks[PAIR - 1];
     if (t.launch == kBatchPersistent) {
-        int* c = t.ctr + 8 * (pair - 1);
+        int* c = t.ctr + 8 * (PAIR - 1);
         hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, c, 8);   // a kernel node, not a memset, in graphs
-        const dim3 pg(t.pgrid);
-        if (pair == 1) hipLaunchKernelGGL((k_pair_batch_q<T, 1>), pg, block, 0, s, a, t.bmap, c, t.nblocks);
-        else hipLaunchKernelGGL((k_pair_batch_q<T, 2>), pg, block, 0, s, a, t.bmap, c, t.nblocks);
-        return hipGetLastError();
+        hipLaunchKernelGGL((k_pair_batch_q<T, PAIR>), dim3(t.pgrid[PAIR - 1]), block, 0, s, a, t.bmap[PAIR - 1], c, n);
+    } else {
+        hipLaunchKernelGGL((k_pair_batch<T, PAIR>), dim3(n), block, 0, s, a, t.bmap[PAIR - 1]);
     }
-    if (pair == 1) hipLaunchKernelGGL((k_pair_batch<T, 1>), dim3(t.nblocks), block, 0, s, a, t.bmap);
-    else hipLaunchKernelGGL((k_pair_batch<T, 2>), dim3(t.nblocks), block, 0, s, a, t.bmap);
     return hipGetLastError();
 }
 
@@ -1222,7 +1292,7 @@ hipError_t batch_pair_t(const BatchTables& t, int pair, int flip, hipStream_t s)
 hipError_t batch_build(BatchTables& t, const std::vector<BatchMember>& ms, int esize, int launch, hipStream_t s) {
     t.esize = esize;
     t.launch = launch;
-    t.nblocks = 0;
+    t.nblocks[0] = t.nblocks[1] = 0;
     if (ms.empty()) return hipSuccess;
     for (const auto& m : ms)
         if (!pair_capable(m.g) || m.zlen < 1 || m.g.lpr != 64) return hipErrorInvalidValue;
@@ -1233,16 +1303,17 @@ void batch_free(BatchTables& t) {
     if (t.buf) (void)hipFree(t.buf);
     t.buf = nullptr;
     t.bytes = 0;
-    t.nblocks = 0;
+    t.nblocks[0] = t.nblocks[1] = 0;
 }
 
 hipError_t batch_pair(const BatchTables& t, int pair, int flip, hipStream_t s) {
-    if (t.nblocks == 0) return hipSuccess;
-    return t.esize == 8 ? batch_pair_t<double>(t, pair, flip, s) : batch_pair_t<float>(t, pair, flip, s);
+    if (t.nblocks[0] == 0) return hipSuccess;
+    if (t.esize == 8) return pair == 1 ? batch_pair_t<double, 1>(t, flip, s) : batch_pair_t<double, 2>(t, flip, s);
+    return pair == 1 ? batch_pair_t<float, 1>(t, flip, s) : batch_pair_t<float, 2>(t, flip, s);
 }
 
 hipError_t batch_step(const BatchTables& t, int flip, hipStream_t s) {
-    if (t.nblocks == 0) return hipSuccess;
+    if (t.nblocks[0] == 0) return hipSuccess;
     for (int pair = 1; pair <= 2; ++pair) {
         hipLaunchKernelGGL(k_pair_predict_batch, dim3(t.pblocks), dim3(256), 0, s,
                            (const PredictArgs*)t.pre[pair - 1][flip], t.pmap);
