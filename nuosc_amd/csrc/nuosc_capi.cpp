@@ -51,6 +51,7 @@ struct nuosc_sim {
     double* mom_a = nullptr;
     double* mom_b = nullptr;
     double* pair_tot = nullptr;  // direction sums of u (handles that step in stage pairs)
+    double* pair_open = nullptr; // open z: PairBuffers' gpart and gin
     double* d_vgrid = nullptr;  // vx | vy | vz | vw
     double* d_g0 = nullptr;     // G0 | G0b
     double* d_part = nullptr;
@@ -124,9 +125,11 @@ CopyLayout copy_layout(int nx, int nz, int nzs, int nvp, int nch, int esize, int
     return CopyLayout{gq.srec, gq.xrow, 4 * copy_elems(gq), true};
 }
 
-// RK4 in stage pairs: 2 flavours, periodic box, the default discretisation
+// RK4 in stage pairs: 2 flavours, the default discretisation.  (Open z too: a
+// step of 1 x 4096 x 642 takes 0.28 ms instead of 0.44-0.47 stage by stage, 128 x 512 x
+// 642 5.0 instead of 7.7, FP32 2.8 instead of 4.1, 1 x 500 x 92 0.06 instead of 0.08.)
 bool steps_in_pairs(const nuosc_config& c) {
-    return c.nflavor != 3 && c.bc == NUOSC_BC_PERIODIC && c.ko_order != 5 && c.adv == NUOSC_ADV_CFD4;
+    return c.nflavor != 3 && c.ko_order != 5 && c.adv == NUOSC_ADV_CFD4;
 }
 // doubles of the partial moment records (with the spare x row's) and of the
 // partial direction sums, which share one buffer
@@ -272,7 +275,8 @@ int enqueue_step3_srk3(nuosc_sim* s) {
 
 PairBuffers pair_buffers(const nuosc_sim* s) {
     return PairBuffers{s->st_u, s->st_w,   s->st_yb,  s->st_ya,   s->mom_u,
-                       s->mom_b, s->mom_a, s->mom_part, s->pair_tot};
+                       s->mom_b, s->mom_a, s->mom_part, s->pair_tot,
+                       s->pair_open, s->pair_open ? s->pair_open + 4ll * s->nx * s->nch * kPairRec : nullptr};
 }
 
 // direction sums of the state y (partial records, then totals)
@@ -292,6 +296,9 @@ int enqueue_step_pairs(nuosc_sim* s, StepKind kind, hipEvent_t* ev = nullptr) {
     const bool comp = sizeof(T) == 4;
     for (int half = 0; half < 2; ++half) {
         const int pair = kind == kRk4 ? 1 + half : (half ? kLone : 3);
+        if (s->geo.bc == NUOSC_BC_OPEN_Z)
+            HIPCK(s, launch_pair_ghosts<T>(pair, s->geo, b, s->d_g0, s->d_g0 + s->nv, s->inflow, s->d_time, s->dt,
+                                           s->stream));
         HIPCK(s, launch_pair_predict(pair, s->geo, s->ph, b, s->dt, s->stream));
         if (ev) HIPCK(s, hipEventRecord(ev[4 * half], s->stream));
         HIPCK(s, launch_pair<T>(pair, s->geo, s->ph, s->pair_zlen, b, s->dt, s->stream));
@@ -303,6 +310,7 @@ int enqueue_step_pairs(nuosc_sim* s, StepKind kind, hipEvent_t* ev = nullptr) {
         }
         HIPCK(s, launch_pair_totals(s->geo, comp, b, s->stream));
     }
+    if (s->geo.bc == NUOSC_BC_OPEN_Z) HIPCK(s, launch_advance_time(s->d_time, s->dt, s->stream));
     return NUOSC_OK;
 }
 
@@ -791,6 +799,12 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
     if (c.bc == NUOSC_BC_OPEN_Z) {
         if (hipMalloc((void**)&s->d_time, sizeof(double)) != hipSuccess) return bail(NUOSC_ENOMEM, "allocation failed");
         if (hipMemsetAsync(s->d_time, 0, sizeof(double), s->stream) != hipSuccess) return bail(NUOSC_EHIP, "memset failed");
+        if (s->pairs) {
+            const size_t b = (size_t)pair_open_doubles(s->nx, s->nch, s->nvp) * sizeof(double);
+            if (hipMalloc((void**)&s->pair_open, b) != hipSuccess) return bail(NUOSC_ENOMEM, "moment allocation failed");
+            s->device_bytes += (long long)b;
+            if (hipMemsetAsync(s->pair_open, 0, b, s->stream) != hipSuccess) return bail(NUOSC_EHIP, "memset failed");
+        }
     }
     const int nb = ana_blocks(s->geo);
     if (hipMalloc((void**)&s->d_part, (size_t)nb * kNAna * 2 * sizeof(double)) != hipSuccess)
@@ -825,7 +839,7 @@ int nuosc_destroy(nuosc_sim* s) {
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     drop_graph(s);
     void* bufs[] = {s->st_u, s->st_w, s->st_ya, s->st_yb, s->mom_part, s->mom_u, s->mom_a, s->mom_b,
-                    s->pair_tot, s->d_vgrid, s->d_g0, s->d_part, s->d_tmp, s->d_time};
+                    s->pair_tot, s->pair_open, s->d_vgrid, s->d_g0, s->d_part, s->d_tmp, s->d_time};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
     if (s->ev0) (void)hipEventDestroy(s->ev0);
@@ -1535,6 +1549,7 @@ int nuosc_estimate_device_bytes(const nuosc_config* c, long long* bytes) {
     const bool pairs = steps_in_pairs(*c);
     b += part_doubles(nx, nz, nv, nch, nf, pairs) * 8;                 // moments: partials, totals
     b += (nf == kNVar3 ? 2ll * kNMom3 : 3ll * kMomStride + (pairs ? kPairRec : 0)) * nx * nz * 8;
+    if (pairs && c->bc == NUOSC_BC_OPEN_Z) b += pair_open_doubles(nx, nch, nvp) * 8;   // ghost sites
     b += 4 * nv * 8 + 2 * nv * 8 + 2048ll * kNAna * 16;                // v-grid, G0, analysis
     b += 2 * nz * 8;                                                   // init tables
     *bytes = b;

@@ -217,16 +217,19 @@ hipError_t launch_p3_slice(const Geometry& g, const T* y, const double* G0, cons
 
 // Stage pairs (nuosc_pair.hip): RK4 stages 1+2 and 3+4 (pairs 1 and 2) or
 // SSP-RK3 stages 1+2 (pair 3) in one pass each and SSP-RK3 stage 3 (kLone),
-// for 2-flavour periodic boxes with the default discretisation.  A step is
+// for 2-flavour boxes with the default discretisation.  A step is
 //   predict(p), pair(p), totals, predict(q), pair(q), totals
+// (open z: with ghosts(p) and ghosts(q) ahead of the predictions)
 // with (p, q) = (1, 2) or (3, kLone) and needs the direction sums tot of u; it
 // leaves those of unew, and the new state in unew (u is not touched).
 constexpr int kLone = 4;
 struct PairBuffers {
-    const void* u;
+    void* u;                    // (open z: its ghost sites are written)
     void *a, *y3, *unew;        // A = Y2 + u + dt k2 (FP32), Y3 (SSP-RK3: u2), the new state
     double *mu, *m3, *min;      // moment records of u, Y3 and the inner input (Y2, then Y4), [site][kMomStride]
     double *part, *tot;         // direction sums: [site][chunk][kPairRec] partial, [site][kPairRec] total
+    double* gpart;              // open z: partial direction sums of the ghost sites, [nx][end][depth][chunk][kPairRec]
+    void* gin;                  // and inflow values of the inner input there, [end][depth][kNVar][nvp]
 };
 bool pair_capable(const Geometry& g);
 // wavefronts of the first pair kernel with z segments of zlen sites
@@ -240,6 +243,15 @@ hipError_t launch_pair(int pair, const Geometry& g, const Physics& ph, int zlen,
 hipError_t launch_pair_predict(int pair, const Geometry& g, const Physics& ph, const PairBuffers& b, double dt,
                                hipStream_t s);
 hipError_t launch_pair_totals(const Geometry& g, bool compensated, const PairBuffers& b, hipStream_t s);
+// open z: the two ghost sites past each end of the pair's stencil input, their
+// direction sums, and the inflow values of the inner input; t_dev: the time of u
+template <typename T>
+hipError_t launch_pair_ghosts(int pair, const Geometry& g, const PairBuffers& b, const double* G0, const double* G0b,
+                              const Inflow& in, const double* t_dev, double dt, hipStream_t s);
+// doubles of gpart and gin together
+inline long long pair_open_doubles(long long nx, long long nch, long long nvp) {
+    return nx * 4 * nch * kPairRec + 4 * kNVar * nvp;
+}
 // partial direction sums of a state
 template <typename T>
 hipError_t launch_pair_sums(const Geometry& g, const T* y, double* part, hipStream_t s);

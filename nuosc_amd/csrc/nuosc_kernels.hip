@@ -1430,35 +1430,20 @@ __global__ __launch_bounds__(256) void k_open_ghosts(const Geometry g, T* __rest
     const double vz = g.vz[v];
     const bool inflow = side == 0 ? (vz > 0.0) : (vz < 0.0);
     if (inflow) {
-        double a = 0.0;
-        if (in.on) {
-            const double t = t_dev[0] + cdt;
-            const double z = in.z0 + (j + 0.5) * in.dz;
-            const double zz = z - vz * t - in.zc;
-            a = in.eps0 * exp(-zz * zz / (2.0 * in.sigma * in.sigma));
+        double x[4];
+        for (int grp = 0; grp < 2; ++grp) {
+            open_inflow(in, vz, j, t_dev[0] + cdt, 0.5 * (grp ? G0b : G0)[v], x);
+            for (int f = 0; f < 4; ++f) y[o + (grp * 4 + f) * g.nvp] = (T)x[f];
         }
-        const double p3o = sqrt(1.0 - a * a);
-        const double hg = 0.5 * G0[v], hgb = 0.5 * G0b[v];
-        y[o + 0 * g.nvp] = (T)(hg * (1.0 + p3o));
-        y[o + 1 * g.nvp] = (T)(hg * (1.0 - p3o));
-        y[o + 2 * g.nvp] = (T)(hg * a);
-        y[o + 3 * g.nvp] = (T)0.0;
-        y[o + 4 * g.nvp] = (T)(hgb * (1.0 + p3o));
-        y[o + 5 * g.nvp] = (T)(hgb * (1.0 - p3o));
-        y[o + 6 * g.nvp] = (T)(hgb * a);
-        y[o + 7 * g.nvp] = (T)0.0;
         for (int f = kNVar; f < g.nf; ++f) y[o + f * g.nvp] = (T)0.0;
     } else {
         // quadratic extrapolation through the three edge cells
-        const double w0 = q == 1 ? 3.0 : (q == 2 ? 6.0 : 10.0);
-        const double w1 = q == 1 ? -3.0 : (q == 2 ? -8.0 : -15.0);
-        const double w2 = q == 1 ? 1.0 : (q == 2 ? 3.0 : 6.0);
         const int e0 = side == 0 ? 0 : g.nz - 1, dir = side == 0 ? 1 : -1;
         const long long c0 = elem_off(g, i, e0 + g.zoff, 0) + v;
         const long long step = (long long)dir * g.srec;   // one site record along z
         for (int f = 0; f < g.nf; ++f) {
             const T* p = y + c0 + f * g.nvp;
-            y[o + f * g.nvp] = (T)(w0 * (double)p[0] + w1 * (double)p[step] + w2 * (double)p[2 * step]);
+            y[o + f * g.nvp] = (T)open_extrapolate(q, (double)p[0], (double)p[step], (double)p[2 * step]);
         }
     }
 }

@@ -1,5 +1,6 @@
 // nuosc_lanes.h -- cross-lane sums of FP64 values over a 64-lane wavefront
-// (gfx950): the moment reductions of the stage kernels.
+// (gfx950): the moment reductions of the stage kernels; and the values of the
+// open z boundary.
 //
 // wave_sum16 adds 16 per-lane values over the wave as a halving tree:
 // level 1 pairs lane l with l ^ 32, level 2 with l ^ 16, level 3 with l ^ 8,
@@ -28,6 +29,8 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include "nuosc_dev.h"
 
 namespace nuosc {
 
@@ -121,6 +124,32 @@ __device__ __forceinline__ double wave_sum32(const double (&a)[32], int lane) {
     double f = keep + dpp_f64<kDppXor2, 0xF>(send, send);
     f = f + dpp_f64<kDppXor1, 0xF>(f, f);
     return f;
+}
+
+// Open z boundary: quadratic extrapolation from the edge sites e0, e1, e2 to the
+// ghost site of depth q = 1, 2, 3.
+__device__ __forceinline__ double open_extrapolate(int q, double e0, double e1, double e2) {
+#pragma clang fp contract(off)
+    const double w0 = q == 1 ? 3.0 : (q == 2 ? 6.0 : 10.0);
+    const double w1 = q == 1 ? -3.0 : (q == 2 ? -8.0 : -15.0);
+    const double w2 = q == 1 ? 1.0 : (q == 2 ? 3.0 : 6.0);
+    return w0 * e0 + w1 * e1 + w2 * e2;
+}
+// ... and the inflow values (ee, mm, emr, emi) of direction vz at site j, time
+// t; hg: half the direction's weight G0 (antineutrinos: G0b).
+__device__ __forceinline__ void open_inflow(const Inflow& in, double vz, int j, double t, double hg, double (&x)[4]) {
+#pragma clang fp contract(off)
+    double a = 0.0;
+    if (in.on) {
+        const double z = in.z0 + (j + 0.5) * in.dz;
+        const double zz = z - vz * t - in.zc;
+        a = in.eps0 * exp(-zz * zz / (2.0 * in.sigma * in.sigma));
+    }
+    const double p3o = sqrt(1.0 - a * a);
+    x[0] = hg * (1.0 + p3o);
+    x[1] = hg * (1.0 - p3o);
+    x[2] = hg * a;
+    x[3] = 0.0;
 }
 
 }  // namespace nuosc

@@ -1,5 +1,9 @@
 // nuosc_pair.hip -- CDNA4 (gfx950) kernels that advance two RK4 stages in one
-// pass over the state (2 flavours, periodic box, the default discretisation).
+// pass over the state (2 flavours, the default discretisation).
+//
+// Open z: the ghost sites of the stencil input are filled by k_pair_ghosts, and
+// those of the inner input, which never leaves the chip, by the rule itself (in
+// the first step of a segment at the lower end and the last two at the upper).
 //
 // The stage-by-stage form (k_stage, nuosc_kernels.hip) writes and re-reads
 // every stage input: 12 passes over the state per step.  k_pair does stages
@@ -13,11 +17,12 @@
 //   pair 1: read u     -> Y2 (on chip) -> Y3
 //   pair 2: read Y3, u -> Y4 (on chip) -> u' = (2 Y3 + Y4)/3 + dt/6 (k1 + k4)
 // 2 + 3 = 5 passes (320 B per update instead of 768; 512 x 512 x 642: 28.9 ms
-// a step stage by stage, 19.3 in 7 passes, 18.1 in 5: pair 1 is bound by HBM,
-// 7.3 ms, pair 2 by its waits at 2 waves per SIMD, 10.5-11).  FP32 is bound by
-// its vector instructions in both pairs (5.2 and 5.5 ms, 75% busy), so there A
-// is kept.  An SSP-RK3 step is
-// a pair and a single stage, 2 + 3 = 5 passes instead of 8:
+// a step stage by stage, 19.3 in 7 passes, 18.1 in 5).  Pair 1 takes 7.0 ms (24
+// GB moved, 3.4 TB/s), pair 2 11.0 (36 GB); with every load from one z and
+// nothing stored they take 5.4 and 9.0, so pair 2 is bound by issuing its
+// instructions at 2 waves per SIMD and memory adds a part.  FP32 takes 5.2 and
+// 5.5 ms, 3.9 each without memory traffic: a third k in pair 2 would cost more
+// than the 2 passes, so there A is kept.  An SSP-RK3 step is a pair and a single stage, 2 + 3 = 5 passes instead of 8:
 //   pair 3: read u       -> u1 = u + dt k (on chip) -> u2 = 3/4 u + 1/4 (u1 + dt k)
 //   k_lone: read u2, u   -> u' = 1/3 u + 2/3 (u2 + dt k)
 //
@@ -183,6 +188,7 @@ struct PairArgs {
     unsigned long long m1, m2; // moment records of y and of the inner input: [site][kMomStride]
     unsigned long long m0;     // pair 2: of u
     unsigned long long part;   // partial sums of out: [site][chunk][2][kRec]
+    unsigned long long gin;    // open z: inflow values of the inner input's ghost sites, [end][depth][8][nvp]
     double c1, c2, cA;         // inner input u + c1 k; output's and A's factors of k (pair 3, lone stage:
                                // output c2 u + cA (y + c1 k))
     int zlen, xgroups, nunits;
@@ -305,6 +311,36 @@ __device__ __forceinline__ void rhs_unit(const PairConst<T>& k, const Precession
     }
 }
 
+// Open z: inflow values of the inner input at the ghost site of this depth past
+// one end; those past the upper end are kept in LDS (glds): a load in the z
+// loop that only its last steps need would have to be waited for in each.
+template <typename T>
+__device__ __forceinline__ void inflow_values(const PairArgs<T>& a, int ch, int grp, int end, int depth, T (&v)[kF]) {
+    const int pv = min(ch * 64 + (int)(threadIdx.x & 63), a.g.nv - 1);
+    const T* p = (const T*)a.gin + (long long)((end * 2 + depth - 1) * kNVar + grp * kF) * a.g.nvp + pv;
+#pragma unroll
+    for (int f = 0; f < kF; ++f) v[f] = p[(long long)f * a.g.nvp];
+}
+template <typename T, bool OPEN, int W>
+struct GhostLds {
+    T v[W][2][kF][64];
+    __device__ __forceinline__ const T (*get(int w) const)[kF][64] { return v[w]; }
+    __device__ __forceinline__ void fill(const PairArgs<T>& a, int ch, int grp, int w) {
+        T x[kF];
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            inflow_values(a, ch, grp, 1, d + 1, x);
+#pragma unroll
+            for (int f = 0; f < kF; ++f) v[w][d][f][threadIdx.x & 63] = x[f];
+        }
+    }
+};
+template <typename T, int W>
+struct GhostLds<T, false, W> {
+    __device__ __forceinline__ const T (*get(int) const)[kF][64] { return nullptr; }
+    __device__ __forceinline__ void fill(const PairArgs<T>&, int, int, int) {}
+};
+
 // One wavefront of a pair: x row `row`, unit (chunk ch, neutrinos grp = 0 or
 // antineutrinos 1), z segment [j0, j1).  Step j forms the inner input at
 // z = j + 2 and, from step j0 on, the output at z = j; the four steps before
@@ -312,6 +348,7 @@ __device__ __forceinline__ void rhs_unit(const PairConst<T>& k, const Precession
 //   OUT   the wave writes its row; otherwise the row only feeds neighbours
 //         (and the wave loads an edge row of y)
 //   NOX   one x row: x neighbours are the point itself, no slab, no barrier
+//   OPEN  open z (a form of its own: the periodic one has no branch in its steps)
 // Per step each wave puts its row of y at z = j + 2 and of the inner input at
 // z = j into the slab of the step's parity, passes the one barrier, and reads
 // its x neighbours; the other parity's slab is rewritten only after the next
@@ -323,11 +360,12 @@ __device__ __forceinline__ void rhs_unit(const PairConst<T>& k, const Precession
 // The z windows are rings of six slots and a step is compiled for each of the
 // six phases, so that no register is moved to shift a window (54 of 354
 // vector instructions per step before).
-template <typename T, int PAIR, bool OUT, bool NOX, typename LDS>
+template <typename T, int PAIR, bool OUT, bool NOX, bool OPEN, typename LDS>
 __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch, int grp, int j0, int j1, int slot_m,
-                                          int erow, int slot_e, SumTable& tab, SumStage& sst, LDS* lds) {
+                                          int erow, int slot_e, SumTable& tab, SumStage& sst, LDS* lds,
+                                          const T (*glds)[kF][64]) {
     const Geometry& g = a.g;
-    const int lane = threadIdx.x & 63, nz = g.nz;
+    const int lane = threadIdx.x & 63, nz = g.nz, zo = OPEN ? g.zoff : 0;
     const unsigned rowb = (unsigned)g.nvp * (unsigned)sizeof(T);
     const unsigned siteb = (unsigned)(g.srec * (long long)sizeof(T));
     const unsigned long long xrowb = (unsigned long long)g.xrow * sizeof(T);
@@ -353,25 +391,29 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
     T E[6][kF];    // not OUT: edge row of y, z = j+2 .. j+5, in the slots of U
     T uc[kF];      // pair 2 (FP32): u at z = j+2 (of the next step, once used)
     T W[6][kF];    // pair 2 (FP64): u of the own row, z = j-2 .. j+2, and j+3 on its way: the slots of Y
-    auto next = [&](int z) { return z + 1 == nz ? 0 : z + 1; };
+    // step j's site j + q: wrapped, or (open z) within the two ghost sites at
+    // each end (those of the first and last steps that lie further out are not used)
+    auto at = [&](int jj, int q) { return OPEN ? max(-2, min(jj + q, nz + 1)) : wrapi(jj + q, nz); };
+    auto next = [&](int z, int jj, int q) { return OPEN ? at(jj, q) : (z + 1 == nz ? 0 : z + 1); };
     auto load = [&](unsigned long long base, unsigned v, int z, T (&x)[kF]) {
         const __amdgpu_buffer_rsrc_t r = prs(base, rbytes);
 #pragma unroll
-        for (int f = 0; f < kF; ++f) x[f] = pld<T>(r, v, (unsigned)z * siteb + f * rowb);
+        for (int f = 0; f < kF; ++f) x[f] = pld<T>(r, v, (unsigned)(z + zo) * siteb + f * rowb);
     };
     int j = j0 - 4;   // the step; z5, z3, z1: wrapped j+5, j+3, j+1
-    int z5 = uniform(wrapi(j + 5, nz)), z3 = uniform(wrapi(j + 3, nz)), z1 = uniform(wrapi(j + 1, nz));
-    const int z2 = uniform(wrapi(j + 2, nz));
+    int z5 = uniform(at(j, 5)), z3 = uniform(at(j, 3)), z1 = uniform(at(j, 1));
+    const int z2 = uniform(at(j, 2));
 #pragma unroll
-    for (int q = 0; q < 5; ++q) load(a.y + rbase, vo, wrapi(j + q, nz), U[q]);
+    for (int q = 0; q < 5; ++q) load(a.y + rbase, vo, at(j, q), U[q]);
     if constexpr (!OUT && !NOX) {
 #pragma unroll
-        for (int q = 2; q < 5; ++q) load(a.y + ebase, ve, wrapi(j + q, nz), E[q]);
+        for (int q = 2; q < 5; ++q) load(a.y + ebase, ve, at(j, q), E[q]);
     }
     constexpr bool AGAIN = kAgain<T, PAIR>;
     // moment records of this step and the next: of y at z = j+2, of the inner
     // input and (FP64 pair 2) of u at z = j
     auto moment = [&](unsigned long long m, int z) {
+        if constexpr (OPEN) z = max(0, min(z, nz - 1));   // (no k is wanted at a ghost site)
         return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(prs(m + mrow, mbytes), vm,
                                                                                (unsigned)z * (kMomStride * 8), 0));
     };
@@ -384,18 +426,24 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
 #pragma unroll
         for (int f = 0; f < kF; ++f) Y[q][f] = (T)0;
 
-    // phase P: the step's number modulo 6; WRITE: step j0 or later
+    // open z: the inner input at the ghost site of this depth past one end: the
+    // inflow value v, or extrapolated from the edge sites e0, e1, e2
+    auto ghost = [&](int end, int depth, T v, T e0, T e1, T e2) {
+        const bool in = end == 0 ? k.nvz < 0.0 : k.nvz > 0.0;
+        return in ? v : (T)open_extrapolate(depth, (double)e0, (double)e1, (double)e2);
+    };
+    // phase P: the step's number modulo 6; WRITE: step j0 or later; BEGIN: step j0 (open z)
     auto step = [&](auto phase, auto write) {
         constexpr int P = decltype(phase)::value;
-        constexpr bool WRITE = decltype(write)::value;
+        constexpr bool WRITE = decltype(write)::value != 0, BEGIN = decltype(write)::value == 2;
         constexpr int b = P & 1;
         const auto& U0 = U[P % 6];
         const auto& U1 = U[(P + 1) % 6];
         const auto& U2 = U[(P + 2) % 6];
         const auto& U3 = U[(P + 3) % 6];
         const auto& U4 = U[(P + 4) % 6];
-        const auto& Y0 = Y[P % 6];
-        const auto& Y1 = Y[(P + 1) % 6];
+        auto& Y0 = Y[P % 6];
+        auto& Y1 = Y[(P + 1) % 6];
         const auto& Y2 = Y[(P + 2) % 6];
         const auto& Y3 = Y[(P + 3) % 6];
         auto& Y4 = Y[(P + 4) % 6];
@@ -407,7 +455,7 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
         if constexpr (PAIR == 2 && !AGAIN && WRITE) {
             const __amdgpu_buffer_rsrc_t ra = prs(a.a + rbase, rbytes);
 #pragma unroll
-            for (int f = 0; f < kF; ++f) ac[f] = pld<T, 2>(ra, vo, (unsigned)j * siteb + f * rowb);
+            for (int f = 0; f < kF; ++f) ac[f] = pld<T, 2>(ra, vo, (unsigned)(j + zo) * siteb + f * rowb);
         }
         // moment records of the next step
         M1[b ^ 1] = moment(a.m1, z3);
@@ -454,9 +502,31 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
                 if constexpr (!OUT) asm volatile("" : "+v"(Y4[f]));
             }
         }
+        if constexpr (OPEN && OUT) {   // ghost sites past the upper end
+            if (j + 2 >= nz) {
+                const int past = j + 2 - nz;
+#pragma unroll
+                for (int f = 0; f < kF; ++f)
+                    Y4[f] = ghost(1, past + 1, glds[past][f][lane], past ? Y2[f] : Y3[f], past ? Y1[f] : Y2[f],
+                                  past ? Y0[f] : Y1[f]);
+            }
+        }
         if constexpr (PAIR == 2 && !AGAIN) {
             load(a.u + rbase, vo, z3, uc);
             __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (OPEN && OUT && BEGIN) {   // and below the lower one
+            if (j < 2) {
+                T gv1[kF], gv2[kF];
+                inflow_values(a, ch, grp, 0, 1, gv1);
+                inflow_values(a, ch, grp, 0, 2, gv2);
+#pragma unroll
+                for (int f = 0; f < kF; ++f) {
+                    const T y1 = j == 0 ? ghost(0, 1, gv1[f], Y2[f], Y3[f], Y4[f]) : Y1[f];
+                    Y0[f] = j == 0 ? ghost(0, 2, gv2[f], Y2[f], Y3[f], Y4[f]) : ghost(0, 1, gv1[f], Y1[f], Y2[f], Y3[f]);
+                    Y1[f] = y1;
+                }
+            }
         }
         if constexpr (OUT && WRITE) {   // ---- the output at z = j
             const Precession<T> r2 = precession(k, M2[b]);
@@ -473,7 +543,7 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
                             }
                         },
                         kk);
-            const unsigned so = (unsigned)j * siteb;
+            const unsigned so = (unsigned)(j + zo) * siteb;
             const __amdgpu_buffer_rsrc_t ro = prs(a.out + rbase, rbytes);
             // (1/3 in two parts: a third rounded to T alone grows u by 3e-8 (FP32)
             // or 6e-17 of itself every step)
@@ -522,27 +592,44 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
                            prs(prow, pbytes), vrec, (unsigned)j * zrec);
         }
         ++j;
-        z5 = next(z5);
-        z3 = next(z3);
-        z1 = next(z1);
+        z5 = next(z5, j, 5);
+        z3 = next(z3, j, 3);
+        z1 = next(z1, j, 1);
     };
     using std::integral_constant;
-    step(integral_constant<int, 0>{}, std::false_type{});
-    step(integral_constant<int, 1>{}, std::false_type{});
-    step(integral_constant<int, 2>{}, std::false_type{});
-    step(integral_constant<int, 3>{}, std::false_type{});
+    step(integral_constant<int, 0>{}, integral_constant<int, 0>{});
+    step(integral_constant<int, 1>{}, integral_constant<int, 0>{});
+    step(integral_constant<int, 2>{}, integral_constant<int, 0>{});
+    step(integral_constant<int, 3>{}, integral_constant<int, 0>{});
+    if constexpr (OPEN) {   // (step j0 by itself: only there can the lower end lie in the window)
+        step(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+        while (j != j1) {
+            step(integral_constant<int, 5>{}, integral_constant<int, 1>{});
+            if (j == j1) break;
+            step(integral_constant<int, 0>{}, integral_constant<int, 1>{});
+            if (j == j1) break;
+            step(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+            if (j == j1) break;
+            step(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+            if (j == j1) break;
+            step(integral_constant<int, 3>{}, integral_constant<int, 1>{});
+            if (j == j1) break;
+            step(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+        }
+        return;
+    }
     for (;;) {
-        step(integral_constant<int, 4>{}, std::true_type{});
+        step(integral_constant<int, 4>{}, integral_constant<int, 1>{});
         if (j == j1) break;
-        step(integral_constant<int, 5>{}, std::true_type{});
+        step(integral_constant<int, 5>{}, integral_constant<int, 1>{});
         if (j == j1) break;
-        step(integral_constant<int, 0>{}, std::true_type{});
+        step(integral_constant<int, 0>{}, integral_constant<int, 1>{});
         if (j == j1) break;
-        step(integral_constant<int, 1>{}, std::true_type{});
+        step(integral_constant<int, 1>{}, integral_constant<int, 1>{});
         if (j == j1) break;
-        step(integral_constant<int, 2>{}, std::true_type{});
+        step(integral_constant<int, 2>{}, integral_constant<int, 1>{});
         if (j == j1) break;
-        step(integral_constant<int, 3>{}, std::true_type{});
+        step(integral_constant<int, 3>{}, integral_constant<int, 1>{});
         if (j == j1) break;
     }
 }
@@ -551,11 +638,11 @@ __device__ __forceinline__ void pair_wave(const PairArgs<T>& a, int row, int ch,
 // z = j-2 .. j+2 and u at z = j, with the loads, the slab of y rows and the ring
 // of phases of pair_wave.  All R + 4 rows of a block are output rows (put:
 // inside the grid); its first and last two waves also load the rows beyond.
-template <typename T, bool NOX, typename LDS>
+template <typename T, bool NOX, bool OPEN, typename LDS>
 __device__ __forceinline__ void lone_wave(const PairArgs<T>& a, int row, bool put, int ch, int grp, int j0, int j1,
                                           int slot, int erow, int slot_e, SumTable& tab, SumStage& sst, LDS* lds) {
     const Geometry& g = a.g;
-    const int lane = threadIdx.x & 63, nz = g.nz;
+    const int lane = threadIdx.x & 63, nz = g.nz, zo = OPEN ? g.zoff : 0;
     const unsigned rowb = (unsigned)g.nvp * (unsigned)sizeof(T);
     const unsigned siteb = (unsigned)(g.srec * (long long)sizeof(T));
     const unsigned long long xrowb = (unsigned long long)g.xrow * sizeof(T);
@@ -578,24 +665,26 @@ __device__ __forceinline__ void lone_wave(const PairArgs<T>& a, int row, bool pu
 
     T U[6][kF];   // y of the own row, z = j-2 .. j+2, and j+3 on its way: slot (phase + 2 + z - j) % 6
     T E[6][kF];   // edge row of y, z = j .. j+3, in the slots of U
-    auto next = [&](int z) { return z + 1 == nz ? 0 : z + 1; };
+    auto at = [&](int jj, int q) { return OPEN ? max(-2, min(jj + q, nz + 1)) : wrapi(jj + q, nz); };   // as pair_wave
+    auto next = [&](int z, int jj, int q) { return OPEN ? at(jj, q) : (z + 1 == nz ? 0 : z + 1); };
     auto load = [&](unsigned long long base, unsigned v, int z, T (&x)[kF]) {
         const __amdgpu_buffer_rsrc_t r = prs(base, rbytes);
 #pragma unroll
-        for (int f = 0; f < kF; ++f) x[f] = pld<T>(r, v, (unsigned)z * siteb + f * rowb);
+        for (int f = 0; f < kF; ++f) x[f] = pld<T>(r, v, (unsigned)(z + zo) * siteb + f * rowb);
     };
     int j = j0;
-    int z3 = uniform(wrapi(j + 3, nz)), z1 = uniform(wrapi(j + 1, nz));
+    int z3 = uniform(at(j, 3)), z1 = uniform(at(j, 1));
     auto moment = [&](int z) {
+        if constexpr (OPEN) z = min(z, nz - 1);
         return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(prs(a.m1 + mrow, mbytes), vm,
                                                                                (unsigned)z * (kMomStride * 8), 0));
     };
     double M1[2] = {moment(j), 0.0};
 #pragma unroll
-    for (int q = 0; q < 5; ++q) load(a.y + rbase, vo, uniform(wrapi(j - 2 + q, nz)), U[q]);
+    for (int q = 0; q < 5; ++q) load(a.y + rbase, vo, uniform(at(j, q - 2)), U[q]);
     if constexpr (!NOX) {
 #pragma unroll
-        for (int q = 2; q < 5; ++q) load(a.y + ebase, ve, uniform(wrapi(j - 2 + q, nz)), E[q]);
+        for (int q = 2; q < 5; ++q) load(a.y + ebase, ve, uniform(at(j, q - 2)), E[q]);
     }
     auto step = [&](auto phase) {
         constexpr int P = decltype(phase)::value;
@@ -607,7 +696,7 @@ __device__ __forceinline__ void lone_wave(const PairArgs<T>& a, int row, bool pu
         {
             const __amdgpu_buffer_rsrc_t ru = prs(a.u + rbase, rbytes);
 #pragma unroll
-            for (int f = 0; f < kF; ++f) uc[f] = pld<T, 2>(ru, vo, (unsigned)j * siteb + f * rowb);
+            for (int f = 0; f < kF; ++f) uc[f] = pld<T, 2>(ru, vo, (unsigned)(j + zo) * siteb + f * rowb);
         }
         M1[b ^ 1] = moment(z1);
         __builtin_amdgcn_sched_barrier(0);
@@ -638,13 +727,13 @@ __device__ __forceinline__ void lone_wave(const PairArgs<T>& a, int row, bool pu
 #pragma unroll
         for (int f = 0; f < kF; ++f) {
             yo[f] = c2 * uc[f] + cA * (U2[f] + c1 * kk[f]);
-            pst<T>(yo[f], ro, vs, (unsigned)j * siteb + f * rowb);
+            pst<T>(yo[f], ro, vs, (unsigned)(j + zo) * siteb + f * rowb);
         }
         direction_sums((double)yo[2], (double)yo[3], (double)yo[0] - (double)yo[1], sst, tab, lane, prs(prow, pbytes),
                        vrec, (unsigned)j * zrec);
         ++j;
-        z3 = next(z3);
-        z1 = next(z1);
+        z3 = next(z3, j, 3);
+        z1 = next(z1, j, 1);
     };
     using std::integral_constant;
     for (;;) {
@@ -665,34 +754,40 @@ __device__ __forceinline__ void lone_wave(const PairArgs<T>& a, int row, bool pu
 
 // logical block -> (x group fastest, unit, z segment): neighbouring blocks,
 // which share edge rows, run on one XCD at about the same time
-template <typename T, int PAIR, int R>
-__device__ __forceinline__ void pair_block(const PairArgs<T>& a, int lb, int wib, PairSlab<T, R, kAgain<T, PAIR>>& lds) {
+template <typename T, int PAIR, bool OPEN, int R>
+__device__ __forceinline__ void pair_block(const PairArgs<T>& a, int lb, int wib, PairSlab<T, R, kAgain<T, PAIR>>& lds,
+                                           GhostLds<T, OPEN, 1>& gl) {
     const int xg = uniform(lb % a.xgroups), rest = uniform(lb / a.xgroups);
     const int un = uniform(rest % a.nunits), j0 = uniform(rest / a.nunits) * a.zlen;
     const int ch = un >> 1, grp = un & 1;
     const int nx = a.g.nx, j1 = min(a.g.nz, j0 + a.zlen), ib = xg * R;
-    if (wib == 0) fill_table(a.g, lds.tab, ch, threadIdx.x & 63);   // (read after the first barriers)
+    if (wib == 0) {   // (read after the first barriers)
+        fill_table(a.g, lds.tab, ch, threadIdx.x & 63);
+        gl.fill(a, ch, grp, 0);
+    }
     // wave wib works on x row ib - 2 + wib; rows past either end wrap (the box
     // is periodic), and rows past the last one write nothing
     const int r = ib - 2 + wib, row = uniform(wrapi(r, nx));
     if (wib >= 2 && wib < R + 2 && r < nx) {
-        pair_wave<T, PAIR, true, false>(a, row, ch, grp, j0, j1, wib, -1, 0, lds.tab, lds.st[wib - 2], &lds);
+        pair_wave<T, PAIR, true, false, OPEN>(a, row, ch, grp, j0, j1, wib, -1, 0, lds.tab, lds.st[wib - 2], &lds,
+                                              gl.get(0));
     } else {
         // the first and last two waves also load the rows beyond: -4, -3, R+2, R+3
         const bool lo = wib < 2, hi = wib >= R + 2;
         const int er = lo ? ib - 4 + wib : ib + wib;
-        pair_wave<T, PAIR, false, false>(a, row, ch, grp, j0, j1, wib, lo || hi ? uniform(wrapi(er, nx)) : -1,
-                                         lo ? wib : (hi ? wib + 4 : R + 8), lds.tab, lds.st[0], &lds);
+        pair_wave<T, PAIR, false, false, OPEN>(a, row, ch, grp, j0, j1, wib, lo || hi ? uniform(wrapi(er, nx)) : -1,
+                                         lo ? wib : (hi ? wib + 4 : R + 8), lds.tab, lds.st[0], &lds, gl.get(0));
     }
 }
 
-template <typename T, int PAIR>
+template <typename T, int PAIR, bool OPEN>
 __global__ __launch_bounds__(64 * (PairShape<T, PAIR>::R + 4)) __attribute__((amdgpu_waves_per_eu(PairShape<T, PAIR>::SimdWaves)))
 void k_pair(const PairArgs<T> a) {
     constexpr int R = PairShape<T, PAIR>::R;
     __shared__ PairSlab<T, R, kAgain<T, PAIR>> lds;
     const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    pair_block<T, PAIR, R>(a, xcd_remap(blockIdx.x, gridDim.x), wib, lds);
+    __shared__ GhostLds<T, OPEN, 1> gl;
+    pair_block<T, PAIR, OPEN, R>(a, xcd_remap(blockIdx.x, gridDim.x), wib, lds, gl);
 }
 
 // Many independent runs in one launch: logical block -> (run, block of run)
@@ -702,12 +797,13 @@ __global__ __launch_bounds__(64 * (PairShape<T, PAIR>::R + 4)) __attribute__((am
 void k_pair_batch(const PairArgs<T>* __restrict__ runs, const int* __restrict__ bmap) {
     constexpr int R = PairShape<T, PAIR>::R;
     __shared__ PairSlab<T, R, kAgain<T, PAIR>> lds;
+    GhostLds<T, false, 1> gl;
     const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lb = xcd_remap(blockIdx.x, gridDim.x);
     const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)bmap;
     const int run = cm[2 * lb], blk = cm[2 * lb + 1];
     const PairArgs<T> a = runs[run];   // uniform, read-only: scalar loads
-    pair_block<T, PAIR, R>(a, blk, wib, lds);
+    pair_block<T, PAIR, false, R>(a, blk, wib, lds, gl);
 }
 
 // The same work as a persistent kernel: a grid of resident blocks takes
@@ -725,6 +821,7 @@ void k_pair_batch_q(const PairArgs<T>* __restrict__ runs, const int* __restrict_
     constexpr int R = PairShape<T, PAIR>::R;
     __shared__ PairSlab<T, R, kAgain<T, PAIR>> lds;
     __shared__ int next;
+    GhostLds<T, false, 1> gl;
     const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int x = blockIdx.x % 8;
     const int per = nitems / 8, rem = nitems % 8;
@@ -740,7 +837,7 @@ void k_pair_batch_q(const PairArgs<T>* __restrict__ runs, const int* __restrict_
         const int lb = start + k;
         const int run = cm[2 * lb], blk = cm[2 * lb + 1];
         const PairArgs<T> a = runs[run];   // uniform, read-only: scalar loads
-        pair_block<T, PAIR, R>(a, blk, wib, lds);
+        pair_block<T, PAIR, false, R>(a, blk, wib, lds, gl);
     }
 }
 
@@ -758,7 +855,7 @@ struct LoneSlab {
     SumStage st[R + 4];
 };
 
-template <typename T>
+template <typename T, bool OPEN>
 __global__ __launch_bounds__(64 * (PairShape<T, 3>::R + 4)) __attribute__((amdgpu_waves_per_eu(PairShape<T, 3>::SimdWaves)))
 void k_lone(const PairArgs<T> a) {
     constexpr int R = PairShape<T, 3>::R, NW = R + 4;
@@ -771,12 +868,12 @@ void k_lone(const PairArgs<T> a) {
     if (wib == 0) fill_table(a.g, lds.tab, un >> 1, threadIdx.x & 63);   // (read after the first barrier)
     const bool lo = wib < 2, hi = wib >= NW - 2;
     const int er = lo ? ib - 2 + wib : ib + wib + 2;
-    lone_wave<T, false>(a, uniform(wrapi(r, nx)), r < nx, un >> 1, un & 1, j0, min(a.g.nz, j0 + a.zlen), wib,
+    lone_wave<T, false, OPEN>(a, uniform(wrapi(r, nx)), r < nx, un >> 1, un & 1, j0, min(a.g.nz, j0 + a.zlen), wib,
                         lo || hi ? uniform(wrapi(er, nx)) : -1, lo ? wib : (hi ? wib + 4 : R + 8), lds.tab,
                         lds.st[wib], &lds);
 }
 
-template <typename T>
+template <typename T, bool OPEN>
 __global__ __launch_bounds__(64 * kRowWaves) __attribute__((amdgpu_waves_per_eu(PairShape<T, 3>::SimdWaves)))
 void k_lone_row(const PairArgs<T> a) {
     __shared__ PairRowLds<kRowWaves> lds;
@@ -786,11 +883,11 @@ void k_lone_row(const PairArgs<T> a) {
     const int un = uniform(lb % groups) * kRowWaves + wib, j0 = uniform(lb / groups) * a.zlen;
     if (un >= a.nunits) return;
     fill_table(a.g, lds.tab[wib], un >> 1, threadIdx.x & 63);
-    lone_wave<T, true>(a, 0, true, un >> 1, un & 1, j0, min(a.g.nz, j0 + a.zlen), 0, -1, 0, lds.tab[wib], lds.st[wib],
+    lone_wave<T, true, OPEN>(a, 0, true, un >> 1, un & 1, j0, min(a.g.nz, j0 + a.zlen), 0, -1, 0, lds.tab[wib], lds.st[wib],
                        (LoneSlab<T, 1>*)nullptr);
 }
 
-template <typename T, int PAIR>
+template <typename T, int PAIR, bool OPEN>
 __global__ __launch_bounds__(64 * kRowWaves) __attribute__((amdgpu_waves_per_eu(PairShape<T, PAIR>::SimdWaves)))
 void k_pair_row(const PairArgs<T> a) {
     __shared__ PairRowLds<kRowWaves> lds;
@@ -800,8 +897,10 @@ void k_pair_row(const PairArgs<T> a) {
     const int un = uniform(lb % groups) * kRowWaves + wib, j0 = uniform(lb / groups) * a.zlen;
     if (un >= a.nunits) return;
     fill_table(a.g, lds.tab[wib], un >> 1, threadIdx.x & 63);   // (the wave's own: its LDS accesses stay in order)
-    pair_wave<T, PAIR, true, true>(a, 0, un >> 1, un & 1, j0, min(a.g.nz, j0 + a.zlen), 0, -1, 0, lds.tab[wib],
-                                   lds.st[wib], (PairRowLds<kRowWaves>*)nullptr);
+    __shared__ GhostLds<T, OPEN, kRowWaves> gl;
+    gl.fill(a, un >> 1, un & 1, wib);
+    pair_wave<T, PAIR, true, true, OPEN>(a, 0, un >> 1, un & 1, j0, min(a.g.nz, j0 + a.zlen), 0, -1, 0, lds.tab[wib],
+                                   lds.st[wib], (PairRowLds<kRowWaves>*)nullptr, gl.get(wib));
 }
 
 // ---------------------------------------------------------------------------
@@ -853,6 +952,62 @@ __device__ __forceinline__ double chunk_sum(const double* __restrict__ rec, int 
     }
     return sum + err;
 }
+// Open z: the two ghost sites past each end of the stencil input y, and their
+// partial direction sums (which the prediction adds).  A wave per (x row, end,
+// depth) and chunk: at 1 x 4096 x 642 it is the latency of one wave's work (a
+// block per site, its waves sharing the chunks, took 24 us).  The waves of row
+// 0 also write the inflow values the inner input has there (gin: they are the
+// same in every x row).
+constexpr int kGhostWaves = 4;
+struct OpenArgs {
+    unsigned long long y;             // u, Y3 or u2
+    const double *G0, *G0b, *t_dev;
+    Inflow in;
+    double cdt, cdt_inner;            // times of y and of the inner input, from t_dev
+    double* part;                     // records [nx][end][depth][chunk]
+    unsigned long long gin;
+};
+template <typename T>
+__global__ __launch_bounds__(64 * kGhostWaves) void k_pair_ghosts(const Geometry g, const OpenArgs a) {
+    __shared__ PairRowLds<kGhostWaves> lds;
+    const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int groups = (g.nch + kGhostWaves - 1) / kGhostWaves;
+    const int site = uniform(blockIdx.x / groups), ch = uniform(blockIdx.x % groups) * kGhostWaves + wib;
+    if (ch >= g.nch) return;
+    const int i = site / 4, end = site / 2 % 2, depth = site % 2 + 1;
+    const int j = end == 0 ? -depth : g.nz - 1 + depth, e0 = end == 0 ? 0 : g.nz - 1;
+    T* const y = (T*)a.y;
+    fill_table(g, lds.tab[wib], ch, lane);
+    const unsigned vrec = sum_offset(lane, kRec * 8);
+    const long long dz = end == 0 ? g.srec : -g.srec;
+    const int pv = min(ch * 64 + lane, g.nv - 1);
+    const double vz = g.vz[pv];
+    const bool in = end == 0 ? vz > 0.0 : vz < 0.0;
+#pragma unroll
+    for (int grp = 0; grp < 2; ++grp) {
+        double h[kF], x[kF];
+        T* const p = y + elem_off(g, i, j + g.zoff, grp * kF) + pv;
+        const T* const e = y + elem_off(g, i, e0 + g.zoff, grp * kF) + pv;
+        const double hg = 0.5 * (grp ? a.G0b : a.G0)[pv];
+        if (in) open_inflow(a.in, vz, j, a.t_dev[0] + a.cdt, hg, h);
+#pragma unroll
+        for (int f = 0; f < kF; ++f) {
+            const long long o = (long long)f * g.nvp;
+            const T v = in ? (T)h[f] : (T)open_extrapolate(depth, (double)e[o], (double)e[o + dz], (double)e[o + 2 * dz]);
+            if (ch * 64 + lane < g.nv) p[o] = v;
+            x[f] = (double)v;
+        }
+        direction_sums(x[2], x[3], x[0] - x[1], lds.st[wib], lds.tab[wib], lane,
+                       prs((unsigned long long)(a.part + ((long long)site * g.nch + ch) * kPairRec + grp * kRec), kRec * 8),
+                       vrec, 0);
+        if (i == 0 && in) {
+            T* const q = (T*)a.gin + (long long)((end * 2 + depth - 1) * kNVar + grp * kF) * g.nvp + pv;
+            open_inflow(a.in, vz, j, a.t_dev[0] + a.cdt_inner, hg, h);
+#pragma unroll
+            for (int f = 0; f < kF; ++f) q[(long long)f * g.nvp] = (T)h[f];
+        }
+    }
+}
 // A block adds the records of kTotSites sites, a thread per sum (the reads are
 // the whole pass: 1.25 GB at 512 x 512 x 642), and combines them through LDS.
 constexpr int kTotSites = 8, kTotThreads = 448;
@@ -878,6 +1033,8 @@ struct PredictArgs {
     const double* base;   // what the prediction starts from (an m, or null: that of tot's state)
     double* m;            // record of tot's state: mu times its moments, with the vacuum terms
     double* inner;        // the same of base + c k (null: not wanted)
+    const double* gpart;  // open z: records of the two ghost sites at each end, [nx][end][depth][chunk] (null: periodic)
+    int nch;
     double c;
     double mu, mu2, p2st, p2ct, pmo, ct2, st;
     double twelve_dx, twelve_dz, ko_x, ko_z;
@@ -913,8 +1070,16 @@ __device__ __forceinline__ void predict_body(const PredictArgs& p, int blk, Pred
     const int i = blk / tiles, z0 = (blk % tiles) * kPredZ, nz = p.nz;
     const int n = min(kPredZ, nz - z0), tid = threadIdx.x;
     const long long row = (long long)i * nz, nsites = (long long)p.nx * nz;
-    for (int k = tid; k < (n + 4) * kRec; k += 256)
-        l.d[k / kRec][k % kRec] = p.tot[(row + wrapi(z0 - 2 + k / kRec, nz)) * kRec + k % kRec];
+    for (int k = tid; k < (n + 4) * kRec; k += 256) {
+        const int z = z0 - 2 + k / kRec;
+        if (p.gpart && (z < 0 || z >= nz)) {
+            const double* t = p.gpart + (i * 4ll + (z < 0 ? -1 - z : 2 + z - nz)) * p.nch * kPairRec + k % kRec;
+            const double nu = chunk_sum<true>(t, p.nch), bar = chunk_sum<true>(t + kRec, p.nch);
+            l.d[k / kRec][k % kRec] = k % kRec % 3 == 1 ? bar + nu : bar - nu;
+        } else {
+            l.d[k / kRec][k % kRec] = p.tot[(row + wrapi(z, nz)) * kRec + k % kRec];
+        }
+    }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const double* t = p.tot + ((long long)wrapi(i + (q < 2 ? q - 2 : q - 1), p.nx) * nz + z0) * kRec;
@@ -1016,6 +1181,7 @@ PairArgs<T> pair_args(const Geometry& g, const Physics& ph, int zlen, int pair, 
     a.m2 = (unsigned long long)b.min;
     a.m0 = (unsigned long long)b.mu;
     a.part = (unsigned long long)b.part;
+    a.gin = (unsigned long long)b.gin;
     switch (pair) {
         case 1: a.c1 = a.c2 = 0.5 * dt; a.cA = dt; break;
         case 2: a.c1 = dt; a.c2 = 1.0 / 6.0 * dt; break;
@@ -1035,6 +1201,8 @@ PredictArgs predict_args(const Geometry& g, const Physics& ph, int pair, const P
     p.base = pair == 2 ? b.mu : nullptr;
     p.m = pair == 1 || pair == 3 ? b.mu : b.m3;
     p.inner = pair == kLone ? nullptr : b.min;
+    p.gpart = g.bc ? b.gpart : nullptr;
+    p.nch = g.nch;
     p.c = pair == 1 ? 0.5 * dt : dt;
     p.mu = ph.mu;
     p.mu2 = 2 * ph.mu;
@@ -1055,7 +1223,7 @@ PredictArgs predict_args(const Geometry& g, const Physics& ph, int pair, const P
 }  // namespace
 
 bool pair_capable(const Geometry& g) {
-    return g.nf == kNVar && g.bc == 0 && !g.ko5 && g.adv == kAdvCfd4;
+    return g.nf == kNVar && (g.bc == 0 || (g.zoff >= 2 && g.nz >= 3)) && !g.ko5 && g.adv == kAdvCfd4;
 }
 
 namespace {
@@ -1120,26 +1288,34 @@ int plan_batch_zlen(const std::vector<Geometry>& gs, int esize, int num_cus) {
     return best;
 }
 
+namespace {
+template <typename T, bool OPEN>
+void launch_pair_form(int pair, const PairArgs<T>& a, unsigned nseg, hipStream_t s) {
+    if (a.g.nx == 1) {
+        const dim3 grid(nseg * ((a.nunits + kRowWaves - 1) / kRowWaves)), block(64 * kRowWaves);
+        if (pair == 1) hipLaunchKernelGGL((k_pair_row<T, 1, OPEN>), grid, block, 0, s, a);
+        else if (pair == 2) hipLaunchKernelGGL((k_pair_row<T, 2, OPEN>), grid, block, 0, s, a);
+        else if (pair == 3) hipLaunchKernelGGL((k_pair_row<T, 3, OPEN>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_lone_row<T, OPEN>), grid, block, 0, s, a);
+    } else {
+        const dim3 grid(nseg * (unsigned)(a.xgroups * a.nunits));
+        const dim3 block(64 * (pair_rows(sizeof(T), pair) + (pair == kLone ? 0 : 4)));
+        if (pair == 1) hipLaunchKernelGGL((k_pair<T, 1, OPEN>), grid, block, 0, s, a);
+        else if (pair == 2) hipLaunchKernelGGL((k_pair<T, 2, OPEN>), grid, block, 0, s, a);
+        else if (pair == 3) hipLaunchKernelGGL((k_pair<T, 3, OPEN>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_lone<T, OPEN>), grid, block, 0, s, a);
+    }
+}
+}  // namespace
+
 template <typename T>
 hipError_t launch_pair(int pair, const Geometry& g, const Physics& ph, int zlen, const PairBuffers& b, double dt,
                        hipStream_t s) {
     if (!pair_capable(g) || zlen < 1 || g.lpr != 64) return hipErrorInvalidValue;
     const PairArgs<T> a = pair_args<T>(g, ph, zlen, pair, b, dt);
     const unsigned nseg = (unsigned)((g.nz + zlen - 1) / zlen);
-    if (g.nx == 1) {
-        const dim3 grid(nseg * ((a.nunits + kRowWaves - 1) / kRowWaves)), block(64 * kRowWaves);
-        if (pair == 1) hipLaunchKernelGGL((k_pair_row<T, 1>), grid, block, 0, s, a);
-        else if (pair == 2) hipLaunchKernelGGL((k_pair_row<T, 2>), grid, block, 0, s, a);
-        else if (pair == 3) hipLaunchKernelGGL((k_pair_row<T, 3>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((k_lone_row<T>), grid, block, 0, s, a);
-    } else {
-        const dim3 grid(nseg * (unsigned)(a.xgroups * a.nunits));
-        const dim3 block(64 * (pair_rows(sizeof(T), pair) + (pair == kLone ? 0 : 4)));
-        if (pair == 1) hipLaunchKernelGGL((k_pair<T, 1>), grid, block, 0, s, a);
-        else if (pair == 2) hipLaunchKernelGGL((k_pair<T, 2>), grid, block, 0, s, a);
-        else if (pair == 3) hipLaunchKernelGGL((k_pair<T, 3>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((k_lone<T>), grid, block, 0, s, a);
-    }
+    if (g.bc) launch_pair_form<T, true>(pair, a, nseg, s);
+    else launch_pair_form<T, false>(pair, a, nseg, s);
     return hipGetLastError();
 }
 
@@ -1155,6 +1331,18 @@ hipError_t launch_pair_totals(const Geometry& g, bool compensated, const PairBuf
     const dim3 grid((unsigned)((nsites + kTotSites - 1) / kTotSites));
     if (compensated) hipLaunchKernelGGL((k_pair_totals<true>), grid, dim3(kTotThreads), 0, s, b.part, g.nch, nsites, b.tot);
     else hipLaunchKernelGGL((k_pair_totals<false>), grid, dim3(kTotThreads), 0, s, b.part, g.nch, nsites, b.tot);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_pair_ghosts(int pair, const Geometry& g, const PairBuffers& b, const double* G0, const double* G0b,
+                              const Inflow& in, const double* t_dev, double dt, hipStream_t s) {
+    if (!pair_capable(g)) return hipErrorInvalidValue;
+    const bool first = pair == 1 || pair == 3;
+    const OpenArgs a{(unsigned long long)(first ? b.u : b.y3), G0, G0b, t_dev, in, first ? 0.0 : 0.5 * dt,
+                     pair == 1 ? 0.5 * dt : dt, b.gpart, (unsigned long long)b.gin};
+    const unsigned groups = (unsigned)((g.nch + kGhostWaves - 1) / kGhostWaves);
+    hipLaunchKernelGGL((k_pair_ghosts<T>), dim3((unsigned)g.nx * 4 * groups), dim3(64 * kGhostWaves), 0, s, g, a);
     return hipGetLastError();
 }
 
@@ -1329,6 +1517,8 @@ hipError_t batch_step(const BatchTables& t, int flip, hipStream_t s) {
 #define NUOSC_PAIR_INST(T)                                                                                        \
     template hipError_t launch_pair<T>(int, const Geometry&, const Physics&, int, const PairBuffers&, double,     \
                                        hipStream_t);                                                              \
+    template hipError_t launch_pair_ghosts<T>(int, const Geometry&, const PairBuffers&, const double*, const double*, \
+                                              const Inflow&, const double*, double, hipStream_t);                 \
     template hipError_t launch_pair_sums<T>(const Geometry&, const T*, double*, hipStream_t);
 NUOSC_PAIR_INST(double)
 NUOSC_PAIR_INST(float)

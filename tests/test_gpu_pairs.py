@@ -1,4 +1,4 @@
-"""RK4 and SSP-RK3 in stage pairs (2-flavour periodic boxes): against the oracle at
+"""RK4 and SSP-RK3 in stage pairs (2-flavour boxes, periodic and open in z): against the oracle at
 shapes that leave the x groups (8 to 16 rows), the z segments and the
 last direction chunk partly filled, boxes narrower than the stencils' reach,
 and mixed with the paths that keep other records of the state."""
@@ -96,3 +96,55 @@ def test_pairs_mixed_with_other_paths(nuosc_mod, oracle_mod):
     o.step(3)
     a, b = g.get_state(), o.get_state()
     assert np.max(np.abs(a - b)) <= 1e-12 * np.max(np.abs(b))
+
+
+# open z: nx, nz, refinement, ghost sites, z-segment length (segments that begin
+# at the second site or end at the last but one, boxes of three sites)
+OPEN_SHAPES = [(1, 3, 1, 2, 1), (1, 4, 4, 2, 3), (1, 40, 2, 3, 7), (2, 3, 2, 2, 2), (3, 5, 1, 2, 1), (5, 33, 3, 2, 0),
+               (9, 20, 2, 3, 32), (13, 29, 2, 2, 7)]
+
+
+@pytest.mark.parametrize("shape", OPEN_SHAPES)
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("scheme", ["rk4", "srk3"])
+def test_open_pairs_match_oracle(nuosc_mod, oracle_mod, shape, precision, scheme):
+    """A pulse entering through z0, all couplings on.  FP64: 1e-12 per field as
+    above.  FP32: besides the 8 roundings a step of the periodic box, the
+    extrapolated ghost values (weights 7 and 17 in sum) reach the edge sites'
+    stages through the stencil (8/12 and 1/12) times dt/h = 0.4, 2.4 more a
+    stage at most: 9 steps x 18 x 2^-24 x 2 = 1.9e-5."""
+    nx, nz, nn, gz, zlen = shape
+    zc = -nz * H / 2 - 0.3
+    init = dict(ipt=0, alpha=0.85, eps0=0.3, sigma=0.5, lnue=0.6, lnueb=0.5)
+    g = nuosc_mod.NuOsc(nv=nn, CFL=0.4, gz=gz, bc=nuosc_mod.BC_OPEN_Z, zc=zc, precision=precision, **geo(nx, nz), **PHYS)
+    o = oracle_mod.OracleSim(nn=nn, cfl=0.4, gz=gz, bc=1, zc=zc, **geo(nx, nz), **PHYS)
+    g.fillInitValue(**init)
+    o.fill_init(**init)
+    if zlen:
+        g.set_zlen(zlen)
+    for n in (1, 2, 6):
+        (g.step_rk4 if scheme == "rk4" else g.step_srk3)(n)
+        (o.step if scheme == "rk4" else o.step_srk3)(n)
+    a, b = g.get_state(), o.get_state()
+    tol = 1e-12 if precision == 64 else 9 * 18 * 2.0 ** -24 * 2
+    for f in range(8):
+        assert np.max(np.abs(a[f] - b[f])) <= tol * np.max(np.abs(b[:4] if f < 4 else b[4:])), f
+    assert g.phy_time == pytest.approx(o.phy_time, rel=1e-14)
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+def test_open_pairs_segments_bitwise(nuosc_mod, precision):
+    """The state does not depend on the z segments, on graph replay or on how
+    the steps are split into calls."""
+    runs = []
+    for use_graph, zlen, calls in ((True, 0, (7,)), (False, 1, (1, 2, 1, 3)), (True, 5, (3, 4)), (True, 64, (5, 2))):
+        g = nuosc_mod.NuOsc(nv=3, CFL=0.4, bc=nuosc_mod.BC_OPEN_Z, zc=-3.0, precision=precision, use_graph=use_graph,
+                            **geo(11, 37), **PHYS)
+        g.fillInitValue(ipt=0, alpha=0.85, eps0=0.3, sigma=0.5, lnue=0.6, lnueb=0.5)
+        if zlen:
+            g.set_zlen(zlen)
+        for n in calls:
+            g.step_rk4(n)
+        runs.append(g.get_state())
+    for r in runs[1:]:
+        assert np.array_equal(r, runs[0])
