@@ -20,8 +20,8 @@
 // a step stage by stage, 19.3 in 7 passes, 18.1 in 5).  Pair 1 takes 7.0 ms (24
 // GB moved, 3.4 TB/s), pair 2 11.0 (36 GB); with every load from one z and
 // nothing stored they take 5.4 and 9.0, so pair 2 is bound by issuing its
-// instructions at 2 waves per SIMD and memory adds a part.  FP32 takes 5.2 and
-// 5.5 ms, 3.9 each without memory traffic: a third k in pair 2 would cost more
+// instructions at 2 waves per SIMD and memory adds a part.  FP32 takes 4.9 and
+// 5.2 ms, 3.9 each without memory traffic: a third k in pair 2 would cost more
 // than the 2 passes, so there A is kept.  An SSP-RK3 step is a pair and a single stage, 2 + 3 = 5 passes instead of 8:
 //   pair 3: read u       -> u1 = u + dt k (on chip) -> u2 = 3/4 u + 1/4 (u1 + dt k)
 //   k_lone: read u2, u   -> u' = 1/3 u + 2/3 (u2 + dt k)
@@ -752,15 +752,26 @@ __device__ __forceinline__ void lone_wave(const PairArgs<T>& a, int row, bool pu
     }
 }
 
-// logical block -> (x group fastest, unit, z segment): neighbouring blocks,
-// which share edge rows, run on one XCD at about the same time
+// logical block -> (neutrinos or antineutrinos fastest, x group, chunk, z
+// segment): neighbouring blocks, which share the sites' records and edge rows,
+// run on one XCD at about the same time.  (With the x group fastest the FP32
+// pairs took 5.07 and 5.60 ms at 512 x 512 x 642 instead of 4.94 and 5.16, FP64
+// pair 1 7.00 instead of 6.88, pair 2 the same 11.0; tiles of 4, 8 or all units
+// gain no more, and all units lose the edge rows: FP64 12.0 ms.)
+struct BlockPlace {
+    int xg, ch, grp, seg;
+};
+template <typename T>
+__device__ __forceinline__ BlockPlace block_place(const PairArgs<T>& a, int lb) {
+    const int h = lb >> 1, xg = uniform(h % a.xgroups), rest = uniform(h / a.xgroups);
+    return BlockPlace{xg, uniform(rest % a.g.nch), lb & 1, uniform(rest / a.g.nch)};
+}
 template <typename T, int PAIR, bool OPEN, int R>
 __device__ __forceinline__ void pair_block(const PairArgs<T>& a, int lb, int wib, PairSlab<T, R, kAgain<T, PAIR>>& lds,
                                            GhostLds<T, OPEN, 1>& gl) {
-    const int xg = uniform(lb % a.xgroups), rest = uniform(lb / a.xgroups);
-    const int un = uniform(rest % a.nunits), j0 = uniform(rest / a.nunits) * a.zlen;
-    const int ch = un >> 1, grp = un & 1;
-    const int nx = a.g.nx, j1 = min(a.g.nz, j0 + a.zlen), ib = xg * R;
+    const BlockPlace p = block_place(a, lb);
+    const int ch = p.ch, grp = p.grp, j0 = p.seg * a.zlen;
+    const int nx = a.g.nx, j1 = min(a.g.nz, j0 + a.zlen), ib = p.xg * R;
     if (wib == 0) {   // (read after the first barriers)
         fill_table(a.g, lds.tab, ch, threadIdx.x & 63);
         gl.fill(a, ch, grp, 0);
@@ -861,14 +872,12 @@ void k_lone(const PairArgs<T> a) {
     constexpr int R = PairShape<T, 3>::R, NW = R + 4;
     __shared__ LoneSlab<T, R> lds;
     const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int lb = xcd_remap(blockIdx.x, gridDim.x);
-    const int xg = uniform(lb % a.xgroups), rest = uniform(lb / a.xgroups);
-    const int un = uniform(rest % a.nunits), j0 = uniform(rest / a.nunits) * a.zlen;
-    const int nx = a.g.nx, ib = xg * NW, r = ib + wib;
-    if (wib == 0) fill_table(a.g, lds.tab, un >> 1, threadIdx.x & 63);   // (read after the first barrier)
+    const BlockPlace p = block_place(a, xcd_remap(blockIdx.x, gridDim.x));
+    const int nx = a.g.nx, ib = p.xg * NW, r = ib + wib, j0 = p.seg * a.zlen;
+    if (wib == 0) fill_table(a.g, lds.tab, p.ch, threadIdx.x & 63);   // (read after the first barrier)
     const bool lo = wib < 2, hi = wib >= NW - 2;
     const int er = lo ? ib - 2 + wib : ib + wib + 2;
-    lone_wave<T, false, OPEN>(a, uniform(wrapi(r, nx)), r < nx, un >> 1, un & 1, j0, min(a.g.nz, j0 + a.zlen), wib,
+    lone_wave<T, false, OPEN>(a, uniform(wrapi(r, nx)), r < nx, p.ch, p.grp, j0, min(a.g.nz, j0 + a.zlen), wib,
                         lo || hi ? uniform(wrapi(er, nx)) : -1, lo ? wib : (hi ? wib + 4 : R + 8), lds.tab,
                         lds.st[wib], &lds);
 }
