@@ -421,6 +421,34 @@ struct F3ZArgs {
     int quads, nch, zlen;
 };
 
+// projections p[q] = x[4q] + nvx x[4q+1] + nvy x[4q+2] + nvz x[4q+3] of a half
+// record, q < 4, with value n of it in lane n of every 16-lane row: the products
+// take it by DPP row_newbcast.  (The s_nop covers a DPP read of x behind the
+// instruction that wrote it.)
+#define NUOSC_BC(n) " row_newbcast:" #n " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void project4(double x, double nvx, double nvy, double nvz, double* p) {
+    asm("s_nop 1\n\t"
+        "v_mov_b64_dpp %0, %4" NUOSC_BC(0)
+        "v_mov_b64_dpp %1, %4" NUOSC_BC(4)
+        "v_mov_b64_dpp %2, %4" NUOSC_BC(8)
+        "v_mov_b64_dpp %3, %4" NUOSC_BC(12)
+        "v_fmac_f64_dpp %0, %4, %5" NUOSC_BC(1)
+        "v_fmac_f64_dpp %1, %4, %5" NUOSC_BC(5)
+        "v_fmac_f64_dpp %2, %4, %5" NUOSC_BC(9)
+        "v_fmac_f64_dpp %3, %4, %5" NUOSC_BC(13)
+        "v_fmac_f64_dpp %0, %4, %6" NUOSC_BC(2)
+        "v_fmac_f64_dpp %1, %4, %6" NUOSC_BC(6)
+        "v_fmac_f64_dpp %2, %4, %6" NUOSC_BC(10)
+        "v_fmac_f64_dpp %3, %4, %6" NUOSC_BC(14)
+        "v_fmac_f64_dpp %0, %4, %7" NUOSC_BC(3)
+        "v_fmac_f64_dpp %1, %4, %7" NUOSC_BC(7)
+        "v_fmac_f64_dpp %2, %4, %7" NUOSC_BC(11)
+        "v_fmac_f64_dpp %3, %4, %7" NUOSC_BC(15)
+        : "=&v"(p[0]), "=&v"(p[1]), "=&v"(p[2]), "=&v"(p[3])
+        : "v"(x), "v"(nvx), "v"(nvy), "v"(nvz));
+}
+#undef NUOSC_BC
+
 template <typename T, int STAGE, int GRP>
 __device__ __forceinline__ void stage3z_body(const F3ZArgs<T>& a, ZSlab<T>& sl, int lb, int wr) {
     constexpr int grp = GRP;
@@ -475,9 +503,16 @@ __device__ __forceinline__ void stage3z_body(const F3ZArgs<T>& a, ZSlab<T>& sl, 
     for (int q = 0; q < 9; ++q) h[q] = (T)a.h[q];
     const double wv = live ? g.vw[pv] : 0.0;
     const double q4[4] = {wv, vxd * wv, vyd * wv, vzd * wv};
-    // the site's moment totals are wave-uniform: scalar loads
+    // The site's moment totals.  FP64: loaded a step ahead, value n of a half
+    // record in lane n of every 16-lane row (with scalar loads in the step, which
+    // went to HBM each time, stages 1-4 of 192 x 192 x 642 took 2.60, 3.90, 3.03
+    // and 3.00 ms instead of 2.29, 3.77, 2.95 and 2.98).  FP32 has no registers
+    // left for that (6-16 spilled VGPRs) and keeps the scalar loads.
+    constexpr bool kAhead = sizeof(T) == 8;
+    const double* const mtot = a.mom + (long long)min(i, nx - 1) * nz * kNMom3;
     typedef const __attribute__((address_space(4))) double cdz;
-    cdz* mrow = (cdz*)(a.mom + (long long)min(i, nx - 1) * nz * kNMom3);
+    cdz* mrow = (cdz*)mtot;
+    const double* const mlane = mtot + (lane & 15);
 
     const int j0 = zs * a.zlen;
     const int j1 = min(nz, j0 + a.zlen);
@@ -493,6 +528,11 @@ __device__ __forceinline__ void stage3z_body(const F3ZArgs<T>& a, ZSlab<T>& sl, 
     // step; the same in FP64 was 4.5% slower).
     constexpr bool kEdgeAtEnd = sizeof(T) == 4;
     T hreg[NF];     // at the top of step j: the edge row of z+1
+    double m0 = 0.0, m1 = 0.0;
+    if constexpr (kAhead) {
+        m0 = mlane[(long long)j0 * kNMom3];
+        m1 = mlane[(long long)j0 * kNMom3 + 16];
+    }
     {
         const __amdgpu_buffer_rsrc_t ry = rs(a.yin);
 #pragma unroll
@@ -518,6 +558,12 @@ __device__ __forceinline__ void stage3z_body(const F3ZArgs<T>& a, ZSlab<T>& sl, 
 #pragma unroll
         for (int q = 0; q < NF; ++q)
             win[q][4] = zld<T>(ry, vo, s2 + (unsigned)kGroupField[grp][q] * rowb);
+        double m0n = 0.0, m1n = 0.0;
+        if constexpr (kAhead) {
+            const long long mn = (long long)min(j + 1, nz - 1) * kNMom3;
+            m0n = mlane[mn];
+            m1n = mlane[mn + 16];
+        }
         __builtin_amdgcn_sched_barrier(0);
         // ---- LDS: own centre values of z (the edge rows of z are there)
         T (*X)[kZSlots][64] = sl.x[j & 1];
@@ -545,16 +591,29 @@ __device__ __forceinline__ void stage3z_body(const F3ZArgs<T>& a, ZSlab<T>& sl, 
         for (int f = 0; f < kNVar3; ++f) c[f] = X[f][slot_c][lane];
         T P[8];
         {
-            const long long mo = (long long)j * kNMom3;
+            // INP, nuosc_class.cpp:187
+            if constexpr (kAhead) {
+                double p[8];
+                project4(m0, -vxd, -vyd, -vzd, p);
+                project4(m1, -vxd, -vyd, -vzd, p + 4);
 #pragma unroll
-            for (int q = 0; q < 8; ++q)   // INP, nuosc_class.cpp:187
-                P[q] = (T)(mrow[mo + 4 * q] - mrow[mo + 4 * q + 1] * vxd - mrow[mo + 4 * q + 2] * vyd -
-                           mrow[mo + 4 * q + 3] * vzd);
+                for (int q = 0; q < 8; ++q) P[q] = (T)p[q];
+            } else {
+                const long long mo = (long long)j * kNMom3;
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    P[q] = (T)(mrow[mo + 4 * q] - mrow[mo + 4 * q + 1] * vxd - mrow[mo + 4 * q + 2] * vyd -
+                               mrow[mo + 4 * q + 3] * vzd);
+            }
         }
+        m0 = m0n;
+        m1 = m1n;
         T I[kNVar3], V[kNVar3];
         local_terms3<T>(c, P, (T)a.mu, (T)a.pmo, h, I, V);
         // (u and A are read once per stage: loaded with the non-temporal hint,
-        // 1.5-1.8% faster per step in both precisions, medians of 4 runs)
+        // 1.5-1.8% faster per step in both precisions, medians of 4 runs; loaded
+        // at the top of the step FP64 stages 3 and 4 took 3.03 and 3.06 ms
+        // instead of 2.95 and 2.98 at 192 x 192 x 642)
         T uc[NF];
         if constexpr (STAGE == 2 || STAGE == 3 || STAGE == 6 || STAGE == 7 || STAGE == 4) {
             const __amdgpu_buffer_rsrc_t ru = rs(STAGE == 4 ? a.w : a.u);
