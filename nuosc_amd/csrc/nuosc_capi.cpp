@@ -503,7 +503,7 @@ int run_steps(nuosc_sim* s, StepKind kind, int nsteps) {
 // the last kernel.
 int analysis_sums(nuosc_sim* s, double* h) {
     const hipError_t e = xfer_run(
-        s->cfg.device, s->stream, 1, true,
+        s->cfg.device, s->stream, 1, 1, true,
         [&](long long, void* slot) {
             double* out = static_cast<double*>(slot);
             return is64(s) ? launch_analysis<double>(s->geo, (double*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->d_part, out,
@@ -535,15 +535,16 @@ int fill_state_ghosts(nuosc_sim* s, void* y) {
 
 // total doubles in chunks of at most a slot, through pinned slots: down fills
 // host from kernel launches, up the other way round; at(n0, cnt, slot)
-// launches the kernel of elements [n0, n0 + cnt).  Pieces small enough that
-// the threads share even a transfer of a few MB.
+// launches the kernel of elements [n0, n0 + cnt).  Pieces of an eighth where
+// threads share a transfer of a few MB.
 template <typename F>
 int transfer(nuosc_sim* s, bool down, double* host, long long total, F at) {
     const long long most = kSlotBytes / sizeof(double);
-    const long long chunk = std::min(most, std::max(most / 8, (total + kXferThreads - 1) / kXferThreads));
+    const int nthreads = xfer_threads(total * (long long)sizeof(double));
+    const long long chunk = nthreads == 1 ? most : std::min(most, std::max(most / 8, (total + 7) / 8));
     auto count = [&](long long c) { return std::min(chunk, total - c * chunk); };
     const hipError_t e = xfer_run(
-        s->cfg.device, s->stream, (total + chunk - 1) / chunk, down,
+        s->cfg.device, s->stream, (total + chunk - 1) / chunk, nthreads, down,
         [&](long long c, void* slot) { return at(c * chunk, count(c), static_cast<double*>(slot)); },
         [&](long long c, void* slot) {
             double* h = host + c * chunk;

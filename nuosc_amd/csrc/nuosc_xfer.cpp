@@ -89,11 +89,11 @@ void xfer_release() {
     }
 }
 
-hipError_t xfer_run(int device, hipStream_t s, long long nchunks, bool down,
+hipError_t xfer_run(int device, hipStream_t s, long long nchunks, int nthreads, bool down,
                     const std::function<hipError_t(long long, void*)>& enqueue,
                     const std::function<void(long long, void*)>& host) {
     if (nchunks <= 0) return hipSuccess;
-    const int want = (int)std::min<long long>(nchunks, kXferThreads);
+    const int want = (int)std::min<long long>(nchunks, nthreads);
     std::vector<Slot> slots;
     std::vector<std::thread> threads;
     try {

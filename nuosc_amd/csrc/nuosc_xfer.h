@@ -22,12 +22,21 @@ constexpr int kXferThreads = 8;   // of the 16 slots a device may hold: two larg
 void xfer_retain();
 void xfer_release();
 
-// Moves nchunks chunks.  down: enqueue(c, slot) queues work on s that fills
+// Threads for a transfer of this many bytes, the caller's included.  Each one
+// more may have to wait its turn of the scheduler (about 3 ms) where the caller's
+// program keeps every core busy, and the transfer ends with its last thread:
+// 8 MB into a new array with the workers of a thread pool spinning took 2.8 ms
+// with four or eight threads, 0.48 with one or two (0.69 by the runtime's copy).
+// 92 MB: 10.5 ms with one, 7.3 with two, 4.3 with eight; 3 MB: 0.20 with one,
+// 0.24 with two, 0.67 with eight.
+inline int xfer_threads(long long bytes) { return bytes < (4 << 20) ? 1 : (bytes < (32 << 20) ? 2 : kXferThreads); }
+
+// Moves nchunks chunks, on up to this many threads.  down: enqueue(c, slot) queues work on s that fills
 // slot, then host(c, slot) runs once it is done; up: host(c, slot) fills the
 // slot, then enqueue(c, slot) queues the work that reads it.  Returns when
 // all of it is done; an error (also of a chunk not started because of it) is
 // returned, hipErrorOutOfMemory if no slot can be had.
-hipError_t xfer_run(int device, hipStream_t s, long long nchunks, bool down,
+hipError_t xfer_run(int device, hipStream_t s, long long nchunks, int nthreads, bool down,
                     const std::function<hipError_t(long long, void*)>& enqueue,
                     const std::function<void(long long, void*)>& host);
 
