@@ -76,7 +76,7 @@ struct Geometry {
     int bc;                // 0 periodic, 1 open in z
     int nzs, zoff;         // stored z rows per x row, stored row of interior z = 0
     int nf;                // fields per site record: 8 (2 flavours) or 18 (3 flavours)
-    int nox;               // one x row (nx = 1) and the default discretisation: the stage
+    int nox;               // one x row (nx = 1) and the default discretisation: the RHS
                            // kernel's NOX form (x neighbours are the point itself)
 };
 

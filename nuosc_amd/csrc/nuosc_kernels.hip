@@ -14,8 +14,9 @@
 // per-(site, chunk) partial sums, so no separate pass over the state is
 // needed; the consumer adds the partials of a site in chunk order.
 //
-// RK4 is streamed with four state copies u, A, yA, yB in 12 passes over the
-// 8 fields per step.  With the stage inputs Y2 = u + dt/2 k1,
+// The default discretisation steps in stage pairs (nuosc_pair.hip); the stage
+// kernel serves its RHS and the other schemes, whose RK4 is streamed with four
+// state copies u, A, yA, yB in 12 passes over the 8 fields per step.  With the stage inputs Y2 = u + dt/2 k1,
 // Y3 = u + dt/2 k2, Y4 = u + dt k3, the new state is
 //   u + dt/6 (k1 + 2k2 + 2k3 + k4) = (A + Y4) / 3 + dt/6 k4,
 //   A = Y2 + 2 Y3 - u = Y2 + u + dt k2,
@@ -437,9 +438,7 @@ __device__ __forceinline__ void stage_body(const StageArgs<T>& a, int lblock, in
     // stores the same bits to the same address as that direction's lane, so
     // the padding columns are never written.
     // (NOX: lanes of chunks past the last one sit in other waves than the
-    // owner of direction nv-1 and store into the spare row: the SSP-RK3
-    // stage 7 rewrites u in place, so a duplicate store could reach u before
-    // the owner has read it)
+    // owner of direction nv-1 and store into the spare row)
     const unsigned vos = (unsigned)(row_ok && (!NOX || ch < nch) ? own + kXg : spare) * xrowb + dof;
     // Edge rows: edge e = wib + W g (row group g < LG of wave wib, e < 2 RAD)
     // loads block row e - RAD (e < RAD) or WR + e - RAD with its L lanes.  The
@@ -772,19 +771,18 @@ __device__ __forceinline__ void stage_body(const StageArgs<T>& a, int lblock, in
     }
 }
 
-// Waves per SIMD the register allocation aims at: the FP64 slab kernels are
-// held to 2 by their LDS (two 73.7 KB blocks of 4 waves per CU); the FP64
-// one-row (NOX) stages 0-5 fit 168 VGPRs (3 waves), the SSP-RK3 stages 6 and
-// 7 would spill there (2 waves); the FP32 stages fit 128 (4 waves).
-template <typename T, int STAGE, int RAD = 2, bool NOX = false>
+// Waves per SIMD the register allocation aims at: the FP64 slab kernel of
+// radius 2 is held to 2 by its LDS (two 73.7 KB blocks of 4 waves per CU); its
+// one-row (NOX) form fits 168 VGPRs (3 waves); FP32 fits 128 (4 waves).
+template <typename T, int RAD = 2, bool NOX = false>
 constexpr int stage_waves() {
-    return RAD == 3 ? (sizeof(T) == 4 ? 2 : 1) : (sizeof(T) == 4 ? 4 : (STAGE <= 5 && NOX ? 3 : 2));
+    return RAD == 3 ? (sizeof(T) == 4 ? 2 : 1) : (sizeof(T) == 4 ? 4 : (NOX ? 3 : 2));
 }
 
-// RAD = 2: the reference's default discretisation; RAD = 3: any of the
-// schemes, chosen at run time (Geometry::ko5, Geometry::adv)
+// RAD = 2: the reference's default discretisation (stage 0 only); RAD = 3: any
+// of the schemes, chosen at run time (Geometry::ko5, Geometry::adv)
 template <typename T, int R, int STAGE, bool COMP, int RAD = 2, bool NOX = false>
-__global__ __launch_bounds__(64 * StageShape<T>::W) __attribute__((amdgpu_waves_per_eu(stage_waves<T, STAGE, RAD, NOX>()))) void k_stage(const StageArgs<T> a) {
+__global__ __launch_bounds__(64 * StageShape<T>::W) __attribute__((amdgpu_waves_per_eu(stage_waves<T, RAD, NOX>()))) void k_stage(const StageArgs<T> a) {
     constexpr int W = StageShape<T>::W;
     __shared__ Slab<T, R, W, RAD> slab;   // (never touched by NOX, which the compiler then leaves unallocated)
     const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -883,30 +881,11 @@ hipError_t launch_stage(int stage, const Geometry& g, const Physics& ph, const S
     constexpr int R = StageShape<T>::R;
     if (g.lpr != dirs_per_chunk((int)sizeof(T)) || g.wpb != StageShape<T>::W) return hipErrorInvalidValue;
     dim3 grid(pl.nblocks), block(64 * StageShape<T>::W);
-    if (g.nox) {   // one x row, default discretisation
-        switch (stage) {
-            case 0: hipLaunchKernelGGL((k_stage<T, R, 0, COMP, 2, true>), grid, block, 0, s, a); break;
-            case 1: hipLaunchKernelGGL((k_stage<T, R, 1, COMP, 2, true>), grid, block, 0, s, a); break;
-            case 2: hipLaunchKernelGGL((k_stage<T, R, 2, COMP, 2, true>), grid, block, 0, s, a); break;
-            case 3: hipLaunchKernelGGL((k_stage<T, R, 3, COMP, 2, true>), grid, block, 0, s, a); break;
-            case 4: hipLaunchKernelGGL((k_stage<T, R, 4, COMP, 2, true>), grid, block, 0, s, a); break;
-            case 5: hipLaunchKernelGGL((k_stage<T, R, 5, COMP, 2, true>), grid, block, 0, s, a); break;
-            case 6: hipLaunchKernelGGL((k_stage<T, R, 6, COMP, 2, true>), grid, block, 0, s, a); break;
-            case 7: hipLaunchKernelGGL((k_stage<T, R, 7, COMP, 2, true>), grid, block, 0, s, a); break;
-            default: return hipErrorInvalidValue;
-        }
-    } else if (scheme_radius(g.ko5, g.adv) == 2 && g.adv == kAdvCfd4) {
-        switch (stage) {
-            case 0: hipLaunchKernelGGL((k_stage<T, R, 0, COMP>), grid, block, 0, s, a); break;
-            case 1: hipLaunchKernelGGL((k_stage<T, R, 1, COMP>), grid, block, 0, s, a); break;
-            case 2: hipLaunchKernelGGL((k_stage<T, R, 2, COMP>), grid, block, 0, s, a); break;
-            case 3: hipLaunchKernelGGL((k_stage<T, R, 3, COMP>), grid, block, 0, s, a); break;
-            case 4: hipLaunchKernelGGL((k_stage<T, R, 4, COMP>), grid, block, 0, s, a); break;
-            case 5: hipLaunchKernelGGL((k_stage<T, R, 5, COMP>), grid, block, 0, s, a); break;
-            case 6: hipLaunchKernelGGL((k_stage<T, R, 6, COMP>), grid, block, 0, s, a); break;
-            case 7: hipLaunchKernelGGL((k_stage<T, R, 7, COMP>), grid, block, 0, s, a); break;
-            default: return hipErrorInvalidValue;
-        }
+    // the default discretisation steps in stage pairs (nuosc_pair.hip): RHS only
+    if (scheme_radius(g.ko5, g.adv) == 2 && g.adv == kAdvCfd4) {
+        if (stage != 0) return hipErrorInvalidValue;
+        if (g.nox) hipLaunchKernelGGL((k_stage<T, R, 0, COMP, 2, true>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_stage<T, R, 0, COMP>), grid, block, 0, s, a);
     } else {
         switch (stage) {
             case 0: hipLaunchKernelGGL((k_stage<T, R, 0, COMP, 3>), grid, block, 0, s, a); break;
