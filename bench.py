@@ -20,7 +20,7 @@ Prints one JSON line:
                  (FP64; 512 B FP32), the ceiling of the 16-pass RK4 streaming
                  in which the per-update targets are stated
   fp32           (default box run) the same workload in the FP32 form: value,
-                 speed-up over FP64, its stage-2 roofline
+                 speed-up over FP64, its stages-3+4 roofline
   batched        (default box run) the 64-run batched scan (FP32), 20 steps:
                  aggregate updates/s together and one after another, the
                  speed-up, and each mode's HBM fraction at 224 B per update

@@ -17,8 +17,8 @@
 //   pair 1: read u     -> Y2 (on chip) -> Y3
 //   pair 2: read Y3, u -> Y4 (on chip) -> u' = (2 Y3 + Y4)/3 + dt/6 (k1 + k4)
 // 2 + 3 = 5 passes (320 B per update instead of 768; 512 x 512 x 642: 28.9 ms
-// a step stage by stage, 19.3 in 7 passes, 18.1 in 5).  Pair 1 takes 7.0 ms (24
-// GB moved, 3.4 TB/s), pair 2 11.0 (36 GB); with every load from one z and
+// a step stage by stage, 19.3 in 7 passes, 18.1 in 5).  Pair 1 takes 6.8 ms (25
+// GB moved, 3.7 TB/s), pair 2 10.8 (38 GB); with every load from one z and
 // nothing stored they take 5.4 and 9.0, so pair 2 is bound by issuing its
 // instructions at 2 waves per SIMD and memory adds a part.  FP32 takes 4.9 and
 // 5.2 ms, 3.9 each without memory traffic: a third k in pair 2 would cost more
