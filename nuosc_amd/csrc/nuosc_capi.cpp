@@ -11,6 +11,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <iterator>
 #include <map>
 #include <mutex>
 #include <string>
@@ -71,7 +72,7 @@ struct nuosc_sim {
     // st_u; flip counts those exchanges (mod 2)
     bool pairs = false;
     int flip = 0;
-    int pair_zlen = 0;                    // z-segment length of the pair kernels
+    int pair_zlen[kLone + 1] = {};        // z-segment length of each pair kernel (the lone stage's last)
     int steps_in_last_call = 0;
     Geometry geo{};
     Physics ph{};
@@ -301,7 +302,7 @@ int enqueue_step_pairs(nuosc_sim* s, StepKind kind, hipEvent_t* ev = nullptr) {
                                            s->stream));
         HIPCK(s, launch_pair_predict(pair, s->geo, s->ph, b, s->dt, s->stream));
         if (ev) HIPCK(s, hipEventRecord(ev[4 * half], s->stream));
-        HIPCK(s, launch_pair<T>(pair, s->geo, s->ph, s->pair_zlen, b, s->dt, s->stream));
+        HIPCK(s, launch_pair<T>(pair, s->geo, s->ph, s->pair_zlen[pair], b, s->dt, s->stream));
         if (ev) HIPCK(s, hipEventRecord(ev[4 * half + 1], s->stream));
         if (half && s->cfg.renorm) {
             T* u = static_cast<T*>(b.unew);
@@ -431,7 +432,7 @@ int refresh_moments(nuosc_sim* s) {
 // z-segment length of the stage kernels (of the stage pairs too)
 void set_plan(nuosc_sim* s, int zlen) {
     s->plan = plan_stage_zlen(s->geo, zlen);
-    if (s->pairs) s->pair_zlen = s->plan.zlen;
+    for (int& z : s->pair_zlen) z = s->plan.zlen;
 }
 
 // what a step needs of the state u: its direction sums (stage pairs) or its
@@ -588,8 +589,8 @@ template <typename T>
 hipError_t enqueue_scratch_stages(nuosc_sim* s) {
     if (s->pairs) {
         const PairBuffers b = pair_buffers(s);
-        const hipError_t e1 = launch_pair<T>(1, s->geo, s->ph, s->pair_zlen, b, s->dt, s->stream);
-        return e1 != hipSuccess ? e1 : launch_pair<T>(2, s->geo, s->ph, s->pair_zlen, b, s->dt, s->stream);
+        const hipError_t e1 = launch_pair<T>(1, s->geo, s->ph, s->pair_zlen[1], b, s->dt, s->stream);
+        return e1 != hipSuccess ? e1 : launch_pair<T>(2, s->geo, s->ph, s->pair_zlen[2], b, s->dt, s->stream);
     }
     const double dt = s->dt, c2 = dt / 2;
     const Geometry& g = s->geo;
@@ -820,7 +821,8 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, c.device) != hipSuccess) return bail(NUOSC_EHIP, "device query failed");
     s->plan = plan_stage(s->geo, prop.multiProcessorCount);
-    if (s->pairs) s->pair_zlen = plan_pair_zlen(s->geo, (int)s->esize, prop.multiProcessorCount);
+    for (int pair = 1; s->pairs && pair <= kLone; ++pair)
+        s->pair_zlen[pair] = plan_pair_zlen(s->geo, (int)s->esize, pair, prop.multiProcessorCount);
     if (hipStreamSynchronize(s->stream) != hipSuccess) return bail(NUOSC_EHIP, "stream sync failed");
     s->G0h.assign(s->nv, 0.0);
     s->G0bh.assign(s->nv, 0.0);
@@ -1036,8 +1038,8 @@ int nuosc_profile_stages(nuosc_sim* s, int nsteps, double* stage_ms) {
 
 int nuosc_get_plan(const nuosc_sim* s, int* zlen, int* waves) {
     if (!s) return NUOSC_EINVAL;
-    if (zlen) *zlen = s->pairs ? s->pair_zlen : s->plan.zlen;
-    if (waves) *waves = s->pairs ? pair_waves(s->geo, (int)s->esize, s->pair_zlen) : s->plan.ntask;
+    if (zlen) *zlen = s->pairs ? s->pair_zlen[1] : s->plan.zlen;
+    if (waves) *waves = s->pairs ? pair_waves(s->geo, (int)s->esize, s->pair_zlen[1]) : s->plan.ntask;
     return NUOSC_OK;
 }
 
@@ -1071,7 +1073,7 @@ int nuosc_autotune(nuosc_sim* s, int trials, int* best_zlen, double* best_ms) {
         auto it = g_tune_cache.find(key);
         if (it != g_tune_cache.end()) {
             HIPCK(s, hipStreamSynchronize(s->stream));
-            if (s->pairs) s->pair_zlen = std::min(it->second, s->nz);
+            if (s->pairs) s->pair_zlen[1] = s->pair_zlen[2] = std::min(it->second, s->nz);
             else s->plan = plan_stage_zlen(s->geo, it->second);
             drop_graph(s);
             if (s->batch) batch_member_changed(s->batch);
@@ -1088,7 +1090,8 @@ int nuosc_autotune(nuosc_sim* s, int trials, int* best_zlen, double* best_ms) {
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
         return fail(s, NUOSC_EHIP, "event creation failed");
     const StagePlan keep = s->plan;
-    const int keep_pair = s->pair_zlen;
+    int keep_pair[kLone + 1];
+    std::copy(std::begin(s->pair_zlen), std::end(s->pair_zlen), keep_pair);
     std::vector<int> cand;
     for (int zl = 8; zl <= 256; zl *= 2) {
         if (zl > s->nz && zl != 8) break;
@@ -1116,13 +1119,13 @@ int nuosc_autotune(nuosc_sim* s, int trials, int* best_zlen, double* best_ms) {
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     s->plan = keep;
-    s->pair_zlen = keep_pair;
+    std::copy(std::begin(keep_pair), std::end(keep_pair), s->pair_zlen);
     if (rc) return rc;
     size_t kb = 0;
     for (size_t k = 1; k < cand.size(); ++k)
         if (tmin[k] < tmin[kb]) kb = k;
     const int best = cand[kb];
-    if (s->pairs) s->pair_zlen = std::min(best, s->nz);   // (RK4 only: the SSP-RK3 stages keep their plan)
+    if (s->pairs) s->pair_zlen[1] = s->pair_zlen[2] = std::min(best, s->nz);   // (RK4 only: the SSP-RK3 stages keep their plan)
     else s->plan = plan_stage_zlen(s->geo, best);
     drop_graph(s);
     if (s->batch) batch_member_changed(s->batch);
@@ -1335,7 +1338,7 @@ int batch_tables(nuosc_batch* b) {
         shared = plan_batch_zlen(grids, is64(b->members[0]) ? 8 : 4, b->num_cus);
     }
     for (nuosc_sim* m : b->members) {
-        const int zlen = shared > 0 ? std::min(shared, m->nz) : m->pair_zlen;
+        const int zlen = shared > 0 ? std::min(shared, m->nz) : m->pair_zlen[1];
         ms.push_back(BatchMember{m->geo, m->ph, zlen, pair_buffers(m), m->dt});
         b->copies.push_back({m->st_u, m->st_ya});
     }

@@ -234,8 +234,8 @@ struct PairBuffers {
 bool pair_capable(const Geometry& g);
 // wavefronts of the first pair kernel with z segments of zlen sites
 int pair_waves(const Geometry& g, int esize, int zlen);
-// z-segment length the pair kernels start with, alone and for a batch of grids
-int plan_pair_zlen(const Geometry& g, int esize, int num_cus);
+// z-segment length a pair kernel starts with alone, and both pairs of a batch of grids
+int plan_pair_zlen(const Geometry& g, int esize, int pair, int num_cus);
 int plan_batch_zlen(const std::vector<Geometry>& grids, int esize, int num_cus);
 template <typename T>
 hipError_t launch_pair(int pair, const Geometry& g, const Physics& ph, int zlen, const PairBuffers& b, double dt,
