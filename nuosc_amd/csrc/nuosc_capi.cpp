@@ -534,13 +534,11 @@ int fill_state_ghosts(nuosc_sim* s, void* y) {
 
 // total doubles in chunks of at most a slot, through pinned slots: down fills
 // host from kernel launches, up the other way round; at(n0, cnt, slot)
-// launches the kernel of elements [n0, n0 + cnt).  Pieces of an eighth where
-// threads share a transfer of a few MB.
+// launches the kernel of elements [n0, n0 + cnt).
 template <typename F>
 int transfer(nuosc_sim* s, bool down, double* host, long long total, F at) {
-    const long long most = kSlotBytes / sizeof(double);
+    const long long chunk = kSlotBytes / sizeof(double);
     const int nthreads = xfer_threads(total * (long long)sizeof(double));
-    const long long chunk = nthreads == 1 ? most : std::min(most, std::max(most / 8, (total + 7) / 8));
     auto count = [&](long long c) { return std::min(chunk, total - c * chunk); };
     const hipError_t e = xfer_run(
         s->cfg.device, s->stream, (total + chunk - 1) / chunk, nthreads, down,

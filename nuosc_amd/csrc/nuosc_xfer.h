@@ -24,12 +24,12 @@ void xfer_release();
 
 // Threads for a transfer of this many bytes, the caller's included.  Each one
 // more may have to wait its turn of the scheduler (about 3 ms) where the caller's
-// program keeps every core busy, and the transfer ends with its last thread:
-// 8 MB into a new array with the workers of a thread pool spinning took 2.8 ms
-// with four or eight threads, 0.48 with one or two (0.69 by the runtime's copy).
-// 92 MB: 10.5 ms with one, 7.3 with two, 4.3 with eight; 3 MB: 0.20 with one,
-// 0.24 with two, 0.67 with eight.
-inline int xfer_threads(long long bytes) { return bytes < (4 << 20) ? 1 : (bytes < (32 << 20) ? 2 : kXferThreads); }
+// program keeps every core busy, and the transfer ends with its last thread; into
+// new pages they also get in each other's way.  8 MB with the workers of a thread
+// pool spinning: 2.8 ms with eight threads, 0.60 with two, 0.47 with one (0.69 by
+// the runtime's copy); nine of 3-8 MB into new arrays: 8.6 ms with two, 2.9 with
+// one (5.9).  92 MB: 10.5 ms with one, 7.3 with two, 4.3 with eight.
+inline int xfer_threads(long long bytes) { return bytes < (32 << 20) ? 1 : kXferThreads; }
 
 // Moves nchunks chunks, on up to this many threads.  down: enqueue(c, slot) queues work on s that fills
 // slot, then host(c, slot) runs once it is done; up: host(c, slot) fills the
