@@ -964,9 +964,12 @@ __device__ __forceinline__ double chunk_sum(const double* __restrict__ rec, int 
 // Open z: the two ghost sites past each end of the stencil input y, and their
 // partial direction sums (which the prediction adds).  A wave per (x row, end,
 // depth) and chunk: at 1 x 4096 x 642 it is the latency of one wave's work (a
-// block per site, its waves sharing the chunks, took 24 us).  The waves of row
-// 0 also write the inflow values the inner input has there (gin: they are the
-// same in every x row).
+// block per site, its waves sharing the chunks, took 24 us).  The waves are
+// numbered through: with blocks of four chunks of one site, three of four waves
+// idle at 12-42 directions, a step took 529 us instead of 375 at 4096 x 12 x 12
+// and 354 instead of 283 at 2048 x 16 x 42 (FP32).  The waves of row 0 also write
+// the inflow values the inner input has there (gin: they are the same in every
+// x row).
 constexpr int kGhostWaves = 4;
 struct OpenArgs {
     unsigned long long y;             // u, Y3 or u2
@@ -980,9 +983,8 @@ template <typename T>
 __global__ __launch_bounds__(64 * kGhostWaves) void k_pair_ghosts(const Geometry g, const OpenArgs a) {
     __shared__ PairRowLds<kGhostWaves> lds;
     const int wib = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-    const int groups = (g.nch + kGhostWaves - 1) / kGhostWaves;
-    const int site = uniform(blockIdx.x / groups), ch = uniform(blockIdx.x % groups) * kGhostWaves + wib;
-    if (ch >= g.nch) return;
+    const int id = uniform((int)blockIdx.x * kGhostWaves + wib), site = uniform(id / g.nch), ch = uniform(id % g.nch);
+    if (site >= 4 * g.nx) return;
     const int i = site / 4, end = site / 2 % 2, depth = site % 2 + 1;
     const int j = end == 0 ? -depth : g.nz - 1 + depth, e0 = end == 0 ? 0 : g.nz - 1;
     T* const y = (T*)a.y;
@@ -1370,8 +1372,9 @@ hipError_t launch_pair_ghosts(int pair, const Geometry& g, const PairBuffers& b,
     const bool first = pair == 1 || pair == 3;
     const OpenArgs a{(unsigned long long)(first ? b.u : b.y3), G0, G0b, t_dev, in, first ? 0.0 : 0.5 * dt,
                      pair == 1 ? 0.5 * dt : dt, b.gpart, (unsigned long long)b.gin};
-    const unsigned groups = (unsigned)((g.nch + kGhostWaves - 1) / kGhostWaves);
-    hipLaunchKernelGGL((k_pair_ghosts<T>), dim3((unsigned)g.nx * 4 * groups), dim3(64 * kGhostWaves), 0, s, g, a);
+    const long long waves = 4ll * g.nx * g.nch;
+    const dim3 grid((unsigned)((waves + kGhostWaves - 1) / kGhostWaves));
+    hipLaunchKernelGGL((k_pair_ghosts<T>), grid, dim3(64 * kGhostWaves), 0, s, g, a);
     return hipGetLastError();
 }
 

@@ -148,3 +148,24 @@ def test_open_pairs_segments_bitwise(nuosc_mod, precision):
         runs.append(g.get_state())
     for r in runs[1:]:
         assert np.array_equal(r, runs[0])
+
+
+@pytest.mark.parametrize("nx,nn", [(1, 5), (2, 6), (3, 4), (5, 8), (7, 1)])
+@pytest.mark.parametrize("precision", [64, 32])
+def test_open_ghost_waves(nuosc_mod, oracle_mod, nx, nn, precision):
+    """4 nx ghost sites of 1 to 11 direction chunks, four waves to a block: blocks
+    within one site, over several, and a partly filled last one.  Tolerances of
+    test_open_pairs_match_oracle, for 3 steps."""
+    nz = 9
+    zc = -nz * H / 2 - 0.3
+    init = dict(ipt=0, alpha=0.85, eps0=0.3, sigma=0.5, lnue=0.6, lnueb=0.5)
+    g = nuosc_mod.NuOsc(nv=nn, CFL=0.4, gz=2, bc=nuosc_mod.BC_OPEN_Z, zc=zc, precision=precision, **geo(nx, nz), **PHYS)
+    o = oracle_mod.OracleSim(nn=nn, cfl=0.4, gz=2, bc=1, zc=zc, **geo(nx, nz), **PHYS)
+    g.fillInitValue(**init)
+    o.fill_init(**init)
+    g.step_rk4(3)
+    o.step(3)
+    a, b = g.get_state(), o.get_state()
+    tol = 1e-12 if precision == 64 else 3 * 18 * 2.0 ** -24 * 2
+    for f in range(8):
+        assert np.max(np.abs(a[f] - b[f])) <= tol * np.max(np.abs(b[:4] if f < 4 else b[4:])), f
