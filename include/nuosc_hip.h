@@ -249,9 +249,10 @@ int nuosc_last_step_ms(nuosc_sim* sim, double* ms);
 /* Measurement helper: run nsteps RK4 steps eagerly with a pair of HIP events
  * around each of the four stage kernels (on the handle's stream) and return
  * the average duration of each stage kernel in stage_ms[4] (ms).  Handles
- * that step in stage pairs (2 flavours, periodic, the default discretisation)
- * report the kernel of stages 1+2 in stage_ms[0], that of stages 3+4 in
- * stage_ms[2] and zeros.  Advances the state and phy_time like
+ * that step in stage pairs (2 flavours and the default discretisation, with
+ * either z boundary, unless the box is so shallow in z or has so few directions
+ * that stage by stage is faster) report the kernel of stages 1+2 in
+ * stage_ms[0], that of stages 3+4 in stage_ms[2] and zeros.  Advances the state and phy_time like
  * nuosc_step_rk4. */
 int nuosc_profile_stages(nuosc_sim* sim, int nsteps, double* stage_ms);
 

@@ -28,6 +28,9 @@ namespace {
 thread_local std::string g_create_error;
 }
 
+// RK4 or SSP-RK3 step
+enum StepKind { kRk4 = 0, kSrk3 = 1 };
+
 struct nuosc_sim {
     nuosc_config cfg{};
     // geometry (CartGrid.cpp:191-208)
@@ -68,9 +71,9 @@ struct nuosc_sim {
     hipGraphExec_t graph_exec[2][2] = {};
     bool have_moments = false;            // mom_u holds the moments of u
     bool have_sums = false;               // pair_tot holds the direction sums of u
-    // RK4 in stage pairs: the new state goes to st_ya, which then becomes
-    // st_u; flip counts those exchanges (mod 2)
-    bool pairs = false;
+    // RK4, SSP-RK3 in stage pairs: the new state goes to st_ya, which then
+    // becomes st_u; flip counts those exchanges (mod 2)
+    bool pairs[2] = {false, false};
     int flip = 0;
     int pair_zlen[kLone + 1] = {};        // z-segment length of each pair kernel (the lone stage's last)
     int steps_in_last_call = 0;
@@ -126,11 +129,42 @@ CopyLayout copy_layout(int nx, int nz, int nzs, int nvp, int nch, int esize, int
     return CopyLayout{gq.srec, gq.xrow, 4 * copy_elems(gq), true};
 }
 
-// RK4 in stage pairs: 2 flavours, the default discretisation.  (Open z too: a
-// step of 1 x 4096 x 642 takes 0.28 ms instead of 0.44-0.47 stage by stage, 128 x 512 x
-// 642 5.0 instead of 7.7, FP32 2.8 instead of 4.1, 1 x 500 x 92 0.06 instead of 0.08.)
-bool steps_in_pairs(const nuosc_config& c) {
-    return c.nflavor != 3 && c.ko_order != 5 && c.adv == NUOSC_ADV_CFD4;
+// Steps in stage pairs: 2 flavours, the default discretisation, unless stage by
+// stage is faster.  A pair's march takes four more z steps than it writes and its
+// blocks are three to four times as large, which shallow boxes do not make up for
+// once they fill the GPU (below that the fewer launches count); and a pair moves
+// 864 B of direction sums a site and chunk, more than an FP32 pass over the fields
+// of 12 directions.  us a step, stage by stage / in pairs:
+//   RK4, 642 directions   FP64 40 x 1 56 / 43, 1000 x 1 206 / 370, x 4 525 / 560,
+//     x 6 749 / 702; FP32 1000 x 3 233 / 247, x 8 495 / 428
+//   RK4, 42               FP64 400 x 1 42 / 41, FP32 open 3000 x 4 198 / 206, x 8 258 / 250
+//   SSP-RK3, 642          FP64 1000 x 2 222 / 260; FP32 1000 x 6 270 / 287, x 11 489 / 433,
+//     open x 8 645 / 691, x 11 812 / 789
+//   SSP-RK3, 42           FP64 3000 x 8 189 / 167, open x 4 216 / 228, x 8 304 / 292;
+//     FP32 12 x 1 30 / 33, x 3 39 / 34, open 1000 x 24 154 / 161, x 40 210 / 207
+//   RK4, 12               FP64 3000 x 8 214 / 236, x 11 302 / 285, open x 24 625 / 652,
+//     x 40 991 / 955; FP32 open 400 x 40 144 / 132, 3000 x 40 521 / 558
+//   SSP-RK3, 12           FP64 open 1000 x 24 182 / 200, 3000 x 40 715 / 707; FP32
+//     400 x 40 87 / 82, x 200 245 / 261; 2 x 4096 FP64 124 / 145, FP32 99 / 125
+// (The shallow limits allow for a last round of blocks that is nearly empty: FP32
+// RK4 at 162 directions 1000 x 6 1.23 times faster in pairs, 1024 x 6 0.95.)  One x
+// row has no slab to fill and takes pairs; at up to five sites they cost an
+// SSP-RK3 step of it 3-9 us of 20-58.
+bool steps_in_pairs(const nuosc_config& c, StepKind kind, long long nx, long long nz) {
+    if (c.nflavor == 3 || c.ko_order == 5 || c.adv != NUOSC_ADV_CFD4) return false;
+    if (nx == 1) return true;
+    const bool f32 = c.precision == NUOSC_PREC_FP32, open = c.bc == NUOSC_BC_OPEN_Z, srk3 = kind == kSrk3;
+    const int nv = 10 * c.nn * c.nn + 2, nch = (nv + 63) / 64;
+    if (srk3 && nz < 2) return false;
+    if (nv < 32) {
+        if (srk3 && nx < 8 && nz > 1000) return false;
+        if (f32) return nx <= 500 && nx * nz <= (srk3 && open ? 12000 : 20000);
+        return nx <= 500 || nz >= (open ? 40 : 12);
+    }
+    if (nx * nch <= 700) return true;
+    if (!srk3) return nz >= (f32 ? 8 : (open ? 3 : 6));
+    if (!f32) return nz >= 8;
+    return nz >= (open && nv < 256 ? 32 : 12);
 }
 // doubles of the partial moment records (with the spare x row's) and of the
 // partial direction sums, which share one buffer
@@ -290,7 +324,6 @@ hipError_t enqueue_sums(nuosc_sim* s, const T* y) {
 // One RK4 step in two stage pairs, or one SSP-RK3 step in a pair and a lone
 // stage (nuosc_pair.hip), from st_u into st_ya; the caller exchanges the two.
 // Events ev[0], ev[1] bracket the first kernel alone, ev[4], ev[5] the second.
-enum StepKind { kRk4 = 0, kSrk3 = 1 };
 template <typename T>
 int enqueue_step_pairs(nuosc_sim* s, StepKind kind, hipEvent_t* ev = nullptr) {
     const PairBuffers b = pair_buffers(s);
@@ -437,14 +470,14 @@ void set_plan(nuosc_sim* s, int zlen) {
 
 // what a step needs of the state u: its direction sums (stage pairs) or its
 // moments
-int refresh_step(nuosc_sim* s) {
-    if (!s->pairs) return refresh_moments(s);
+int refresh_step(nuosc_sim* s, StepKind kind = kRk4) {
+    if (!s->pairs[kind]) return refresh_moments(s);
     if (is64(s)) HIPCK(s, enqueue_sums<double>(s, (double*)s->st_u));
     else HIPCK(s, enqueue_sums<float>(s, (float*)s->st_u));
     s->have_sums = true;
     return NUOSC_OK;
 }
-bool step_ready(const nuosc_sim* s) { return s->pairs ? s->have_sums : s->have_moments; }
+bool step_ready(const nuosc_sim* s, StepKind kind = kRk4) { return s->pairs[kind] ? s->have_sums : s->have_moments; }
 
 // the stage pairs leave the new state in st_ya
 void state_stepped(nuosc_sim* s) {
@@ -456,15 +489,15 @@ void state_stepped(nuosc_sim* s) {
 // nsteps steps on the handle's stream, replayed from a captured graph if the
 // handle uses them
 int run_steps(nuosc_sim* s, StepKind kind, int nsteps) {
-    const bool pairs = s->pairs;
+    const bool pairs = s->pairs[kind];
     auto enqueue = [&] {
         if (pairs) return is64(s) ? enqueue_step_pairs<double>(s, kind) : enqueue_step_pairs<float>(s, kind);
         if (kind == kRk4) return is64(s) ? enqueue_step<double>(s) : enqueue_step<float>(s);
         return is64(s) ? enqueue_step_srk3<double>(s) : enqueue_step_srk3<float>(s);
     };
     if (nsteps < 0) return fail(s, NUOSC_EINVAL, "negative step count");
-    if (!step_ready(s)) {
-        const int rc = refresh_step(s);
+    if (!step_ready(s, kind)) {
+        const int rc = refresh_step(s, kind);
         if (rc) return rc;
     }
     HIPCK(s, hipEventRecord(s->ev0, s->stream));
@@ -585,7 +618,7 @@ int check_field(nuosc_sim* s, int f) {
 // only, with whatever the inner moments hold: their values do not matter here.)
 template <typename T>
 hipError_t enqueue_scratch_stages(nuosc_sim* s) {
-    if (s->pairs) {
+    if (s->pairs[kRk4]) {
         const PairBuffers b = pair_buffers(s);
         const hipError_t e1 = launch_pair<T>(1, s->geo, s->ph, s->pair_zlen[1], b, s->dt, s->stream);
         return e1 != hipSuccess ? e1 : launch_pair<T>(2, s->geo, s->ph, s->pair_zlen[2], b, s->dt, s->stream);
@@ -739,8 +772,9 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
 
     const size_t state_bytes = (size_t)s->state_elems * s->esize;
     const bool three = s->nf == kNVar3;
-    s->pairs = steps_in_pairs(c);
-    const size_t part_bytes = (size_t)part_doubles(s->nx, s->nz, s->nv, s->nch, s->nf, s->pairs) * sizeof(double);
+    for (StepKind k : {kRk4, kSrk3}) s->pairs[k] = steps_in_pairs(c, k, s->nx, s->nz);
+    const bool pairs = s->pairs[kRk4] || s->pairs[kSrk3];
+    const size_t part_bytes = (size_t)part_doubles(s->nx, s->nz, s->nv, s->nch, s->nf, pairs) * sizeof(double);
     const size_t mom_bytes = (size_t)s->nx * s->nz * (three ? kNMom3 : kMomStride) * sizeof(double);
     void** states[4] = {&s->st_u, &s->st_w, &s->st_ya, &s->st_yb};
     {
@@ -754,7 +788,7 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
     double** moms[5] = {&s->mom_part, &s->mom_u, &s->mom_a, &s->mom_b, &s->pair_tot};
     for (double** p : moms) {
         if (three && p == &s->mom_b) continue;   // 3 flavours: totals of the stage input and a calRHS scratch
-        if (!s->pairs && p == &s->pair_tot) continue;
+        if (!pairs && p == &s->pair_tot) continue;
         const size_t b = (p == &s->mom_part) ? part_bytes : (p == &s->pair_tot ? (size_t)s->nx * s->nz * kPairRec * sizeof(double) : mom_bytes);
         if (hipMalloc((void**)p, b) != hipSuccess) return bail(NUOSC_ENOMEM, "moment allocation failed");
         s->device_bytes += (long long)b;
@@ -797,7 +831,7 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
     if (c.bc == NUOSC_BC_OPEN_Z) {
         if (hipMalloc((void**)&s->d_time, sizeof(double)) != hipSuccess) return bail(NUOSC_ENOMEM, "allocation failed");
         if (hipMemsetAsync(s->d_time, 0, sizeof(double), s->stream) != hipSuccess) return bail(NUOSC_EHIP, "memset failed");
-        if (s->pairs) {
+        if (pairs) {
             const size_t b = (size_t)pair_open_doubles(s->nx, s->nch, s->nvp) * sizeof(double);
             if (hipMalloc((void**)&s->pair_open, b) != hipSuccess) return bail(NUOSC_ENOMEM, "moment allocation failed");
             s->device_bytes += (long long)b;
@@ -819,7 +853,7 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, c.device) != hipSuccess) return bail(NUOSC_EHIP, "device query failed");
     s->plan = plan_stage(s->geo, prop.multiProcessorCount);
-    for (int pair = 1; s->pairs && pair <= kLone; ++pair)
+    for (int pair = 1; pairs && pair <= kLone; ++pair)
         s->pair_zlen[pair] = plan_pair_zlen(s->geo, (int)s->esize, pair, prop.multiProcessorCount);
     if (hipStreamSynchronize(s->stream) != hipSuccess) return bail(NUOSC_EHIP, "stream sync failed");
     s->G0h.assign(s->nv, 0.0);
@@ -975,7 +1009,7 @@ int nuosc_fill_init(nuosc_sim* s, int ipt, double alpha, double eps0, double sig
     drop_graph(s);
     rc = set_device_time(s);
     if (rc) return rc;
-    s->have_moments = false;
+    s->have_moments = s->have_sums = false;
     rc = refresh_step(s);
     if (rc) return rc;
     HIPCK(s, hipStreamSynchronize(s->stream));
@@ -1007,22 +1041,24 @@ int nuosc_profile_stages(nuosc_sim* s, int nsteps, double* stage_ms) {
         int rc = refresh_step(s);
         if (rc) return rc;
     }
+    const bool pairs = s->pairs[kRk4];
     hipEvent_t ev[8] = {};
     for (auto& e : ev)
         if (hipEventCreate(&e) != hipSuccess) return fail(s, NUOSC_EHIP, "event creation failed");
     double acc[4] = {0, 0, 0, 0};
     int rc = NUOSC_OK;
     for (int n = 0; n < nsteps && rc == NUOSC_OK; ++n) {
-        if (s->pairs) rc = is64(s) ? enqueue_step_pairs<double>(s, kRk4, ev) : enqueue_step_pairs<float>(s, kRk4, ev);
+        if (pairs) rc = is64(s) ? enqueue_step_pairs<double>(s, kRk4, ev) : enqueue_step_pairs<float>(s, kRk4, ev);
         else rc = is64(s) ? enqueue_step<double>(s, ev) : enqueue_step<float>(s, ev);
         if (rc) break;
-        if (s->pairs) state_stepped(s);
+        if (pairs) state_stepped(s);
+        else s->have_sums = false;
         s->phy_time += s->dt;
-        if (hipEventSynchronize(ev[s->pairs ? 5 : 7]) != hipSuccess) {
+        if (hipEventSynchronize(ev[pairs ? 5 : 7]) != hipSuccess) {
             rc = fail(s, NUOSC_EHIP, "event sync failed");
             break;
         }
-        for (int k = 0; k < 4 && rc == NUOSC_OK; k += s->pairs ? 2 : 1) {
+        for (int k = 0; k < 4 && rc == NUOSC_OK; k += pairs ? 2 : 1) {
             float f = 0;
             if (hipEventElapsedTime(&f, ev[2 * k], ev[2 * k + 1]) != hipSuccess)
                 rc = fail(s, NUOSC_EHIP, "event timing failed");
@@ -1036,8 +1072,8 @@ int nuosc_profile_stages(nuosc_sim* s, int nsteps, double* stage_ms) {
 
 int nuosc_get_plan(const nuosc_sim* s, int* zlen, int* waves) {
     if (!s) return NUOSC_EINVAL;
-    if (zlen) *zlen = s->pairs ? s->pair_zlen[1] : s->plan.zlen;
-    if (waves) *waves = s->pairs ? pair_waves(s->geo, (int)s->esize, s->pair_zlen[1]) : s->plan.ntask;
+    if (zlen) *zlen = s->pairs[kRk4] ? s->pair_zlen[1] : s->plan.zlen;
+    if (waves) *waves = s->pairs[kRk4] ? pair_waves(s->geo, (int)s->esize, s->pair_zlen[1]) : s->plan.ntask;
     return NUOSC_OK;
 }
 
@@ -1071,7 +1107,7 @@ int nuosc_autotune(nuosc_sim* s, int trials, int* best_zlen, double* best_ms) {
         auto it = g_tune_cache.find(key);
         if (it != g_tune_cache.end()) {
             HIPCK(s, hipStreamSynchronize(s->stream));
-            if (s->pairs) s->pair_zlen[1] = s->pair_zlen[2] = std::min(it->second, s->nz);
+            if (s->pairs[kRk4]) s->pair_zlen[1] = s->pair_zlen[2] = std::min(it->second, s->nz);
             else s->plan = plan_stage_zlen(s->geo, it->second);
             drop_graph(s);
             if (s->batch) batch_member_changed(s->batch);
@@ -1123,7 +1159,7 @@ int nuosc_autotune(nuosc_sim* s, int trials, int* best_zlen, double* best_ms) {
     for (size_t k = 1; k < cand.size(); ++k)
         if (tmin[k] < tmin[kb]) kb = k;
     const int best = cand[kb];
-    if (s->pairs) s->pair_zlen[1] = s->pair_zlen[2] = std::min(best, s->nz);   // (RK4 only: the SSP-RK3 stages keep their plan)
+    if (s->pairs[kRk4]) s->pair_zlen[1] = s->pair_zlen[2] = std::min(best, s->nz);   // (RK4 only: the SSP-RK3 stages keep their plan)
     else s->plan = plan_stage_zlen(s->geo, best);
     drop_graph(s);
     if (s->batch) batch_member_changed(s->batch);
@@ -1196,7 +1232,7 @@ int nuosc_renormalize(nuosc_sim* s) {
     if (!s) return NUOSC_EINVAL;
     if (is64(s)) HIPCK(s, launch_renorm<double>(s->geo, (double*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->stream));
     else HIPCK(s, launch_renorm<float>(s->geo, (float*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->stream));
-    s->have_moments = false;
+    s->have_moments = s->have_sums = false;
     return refresh_step(s);
 }
 
@@ -1240,7 +1276,7 @@ int nuosc_upload_fields(nuosc_sim* s, int f0, int nf, const double* host) {
 
 int nuosc_state_updated(nuosc_sim* s) {
     if (!s) return NUOSC_EINVAL;
-    s->have_moments = false;
+    s->have_moments = s->have_sums = false;
     int rc = refresh_step(s);
     if (rc) return rc;
     HIPCK(s, hipStreamSynchronize(s->stream));
@@ -1278,10 +1314,11 @@ struct nuosc_batch {
     int precision = NUOSC_PREC_FP64;
     std::vector<nuosc_sim*> members;
     hipStream_t stream = nullptr;
-    BatchTables tables;
+    BatchTables tables;    // members that step in stage pairs
+    StageBatch stages;     // members that step stage by stage
     bool dirty = true;
     // the tables hold both exchanges of the members' state copies: at flip f
-    // member k's state is in copies[k][f]
+    // member k's state is in copies[k][f] (stage by stage: the same copy)
     int flip = 0;
     std::vector<std::array<const void*, 2>> copies;
     hipGraph_t graph[2] = {};
@@ -1327,20 +1364,31 @@ namespace {
 // (re)build the device tables of the batched launches from the members
 int batch_tables(nuosc_batch* b) {
     std::vector<BatchMember> ms;
+    std::vector<StageMember> st;
+    const int esize = is64(b->members[0]) ? 8 : 4;
     b->copies.clear();
     b->flip = 0;
     int shared = b->zlen;
     if (shared < 0) {
         std::vector<Geometry> grids;
-        for (nuosc_sim* m : b->members) grids.push_back(m->geo);
-        shared = plan_batch_zlen(grids, is64(b->members[0]) ? 8 : 4, b->num_cus);
+        for (nuosc_sim* m : b->members)
+            if (m->pairs[kRk4]) grids.push_back(m->geo);
+        shared = plan_batch_zlen(grids, esize, b->num_cus);
     }
     for (nuosc_sim* m : b->members) {
-        const int zlen = shared > 0 ? std::min(shared, m->nz) : m->pair_zlen[1];
-        ms.push_back(BatchMember{m->geo, m->ph, zlen, pair_buffers(m), m->dt});
-        b->copies.push_back({m->st_u, m->st_ya});
+        if (m->pairs[kRk4]) {
+            const int zlen = shared > 0 ? std::min(shared, m->nz) : m->pair_zlen[1];
+            ms.push_back(BatchMember{m->geo, m->ph, zlen, pair_buffers(m), m->dt});
+            b->copies.push_back({m->st_u, m->st_ya});
+        } else {
+            const int zlen = b->zlen < 0 ? 64 : (b->zlen ? b->zlen : m->plan.zlen);
+            st.push_back(StageMember{m->geo, m->ph, plan_stage_zlen(m->geo, zlen), m->st_u, m->st_w, m->st_ya, m->st_yb,
+                                     m->mom_part, m->mom_u, m->mom_a, m->mom_b, m->dt});
+            b->copies.push_back({m->st_u, m->st_u});
+        }
     }
-    hipError_t e = batch_build(b->tables, ms, is64(b->members[0]) ? 8 : 4, b->launch, b->stream);
+    hipError_t e = batch_build(b->tables, ms, esize, b->launch, b->stream);
+    if (e == hipSuccess) e = stage_batch_build(b->stages, st, esize, b->launch, b->stream);
     if (e != hipSuccess) return bfail(b, NUOSC_EHIP, std::string("batch tables: ") + hipGetErrorString(e));
     return NUOSC_OK;
 }
@@ -1386,6 +1434,7 @@ int nuosc_batch_destroy(nuosc_batch* b) {
     for (nuosc_sim* m : b->members) m->batch = nullptr;
     batch_drop_graph(b);
     batch_free(b->tables);
+    stage_batch_free(b->stages);
     (void)hipStreamDestroy(b->stream);
     delete b;
     return NUOSC_OK;
@@ -1442,6 +1491,7 @@ int nuosc_batch_step(nuosc_batch* b, int nsteps) {
             if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
                 return bfail(b, NUOSC_EHIP, "capture failed");
             hipError_t le = batch_step(b->tables, b->flip, b->stream);
+            if (le == hipSuccess) le = stage_batch_step(b->stages, 4, b->stream);
             hipGraph_t gr = nullptr;
             hipError_t ce = hipStreamEndCapture(b->stream, &gr);
             if (le != hipSuccess || ce != hipSuccess) {
@@ -1455,7 +1505,8 @@ int nuosc_batch_step(nuosc_batch* b, int nsteps) {
         if (hipGraphLaunch(exec, b->stream) != hipSuccess) return bfail(b, NUOSC_EHIP, "graph launch failed");
         b->flip ^= 1;
         for (nuosc_sim* m : b->members) {
-            state_stepped(m);
+            if (m->pairs[kRk4]) state_stepped(m);
+            else m->have_sums = false;
             m->phy_time += m->dt;
         }
     }
@@ -1504,8 +1555,9 @@ int nuosc_batch_autotune(nuosc_batch* b, int trials, int* best_zlen, double* bes
             rc = batch_tables(b);
             if (rc) break;
             (void)hipEventRecord(e0, b->stream);
-            // pair 1 writes only the RK4 scratch copies (A, Y3) and records, never the state
+            // pair 1 and stages 1-3 write only the RK4 scratch copies and records, never the state
             hipError_t le = batch_pair(b->tables, 1, 0, b->stream);
+            if (le == hipSuccess) le = stage_batch_step(b->stages, 3, b->stream);
             (void)hipEventRecord(e1, b->stream);
             if (le != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
                 rc = bfail(b, NUOSC_EHIP, "autotune launch failed");
@@ -1546,7 +1598,7 @@ int nuosc_estimate_device_bytes(const nuosc_config* c, long long* bytes) {
     const CopyLayout L = copy_layout((int)nx, (int)nz, (int)nzs, (int)nvp, (int)nch, esize, nf);
     if (!L.ok) return NUOSC_EINVAL;
     long long b = L.elems * esize;                                     // u, w, yA, yB
-    const bool pairs = steps_in_pairs(*c);
+    const bool pairs = steps_in_pairs(*c, kRk4, nx, nz) || steps_in_pairs(*c, kSrk3, nx, nz);
     b += part_doubles(nx, nz, nv, nch, nf, pairs) * 8;                 // moments: partials, totals
     b += (nf == kNVar3 ? 2ll * kNMom3 : 3ll * kMomStride + (pairs ? kPairRec : 0)) * nx * nz * 8;
     if (pairs && c->bc == NUOSC_BC_OPEN_Z) b += pair_open_doubles(nx, nch, nvp) * 8;   // ghost sites

@@ -257,9 +257,24 @@ template <typename T>
 hipError_t launch_pair_sums(const Geometry& g, const T* y, double* part, hipStream_t s);
 
 // Batched runs: every member run advances one RK4 step per batch_step call
-// with one launch of each kernel of a step for all members.  Members keep
-// their own buffers, segments and physics; all share the precision (esize) of
-// the tables.
+// (and stage_batch_step call: members that step stage by stage) with one
+// launch of each kernel of a step for all members.  Members keep their own
+// buffers, segments and physics; all share the precision (esize) of the tables.
+
+// host image of a device buffer of tables
+struct TableImage {
+    std::vector<char> host;
+    size_t put(const void* p, size_t bytes);   // returns the offset
+    // counts[r] blocks of member r -> (member, block of member) of every block
+    size_t put_map(const std::vector<long long>& counts, int& blocks);
+    // into buf, which is kept if it is large enough
+    hipError_t upload(void*& buf, size_t& bytes, hipStream_t s) const;
+};
+// as many blocks of this kernel as the current device holds at once
+hipError_t resident_blocks(const void* kernel, int threads, int& blocks);
+// (a kernel, not a memset, for captured graphs)
+hipError_t launch_zero_ints(int* p, int n, hipStream_t s);
+
 struct BatchMember {
     Geometry g;
     Physics ph;
@@ -274,7 +289,7 @@ constexpr int kBatchGrid = 0, kBatchPersistent = 1;
 constexpr int kBatchCounters = 16;   // 8 XCD counters for each of the 2 pairs
 
 struct BatchTables {
-    void* buf = nullptr;   // one device buffer holds all of the following
+    void* buf = nullptr;   // a TableImage: all of the following
     size_t bytes = 0;
     void* args[2][2] = {};   // [pair][flip] PairArgs arrays
     void* pre[2][2] = {};    // [pair][flip] PredictArgs arrays
@@ -291,6 +306,30 @@ void batch_free(BatchTables& t);
 hipError_t batch_step(const BatchTables& t, int flip, hipStream_t s);
 // one pair kernel of every member alone (autotuner timing)
 hipError_t batch_pair(const BatchTables& t, int pair, int flip, hipStream_t s);
+
+// The same for members that step stage by stage
+struct StageMember {
+    Geometry g;
+    Physics ph;
+    StagePlan pl;
+    void *u, *w, *ya, *yb;          // state copies
+    double *mpart, *mu, *ma, *mb;   // partial records; totals of u, yA, yB
+    double dt;
+};
+struct StageBatch {
+    void* buf = nullptr;
+    size_t bytes = 0;
+    void *args[4] = {}, *tot[4] = {}, *xg[4] = {};   // per stage: kernel arguments, totals, x-ghost refresh
+    int *bmap = nullptr, *tmap = nullptr, *xmap = nullptr;
+    int* ctr = nullptr;   // 8 XCD counters for each stage
+    int nblocks = 0, tblocks = 0, xblocks = 0, esize = 8;
+    int launch = kBatchGrid, pgrid = 0;
+};
+hipError_t stage_batch_build(StageBatch& t, const std::vector<StageMember>& members, int esize, int launch,
+                             hipStream_t s);
+void stage_batch_free(StageBatch& t);
+// the first nstages stages of a step of every member (3: only the scratch copies are written)
+hipError_t stage_batch_step(const StageBatch& t, int nstages, hipStream_t s);
 
 // Open z boundary: fill the zoff ghost rows at both z ends of state y for
 // time t = *t_dev + cdt (inflow directions: the Inflow pulse state;

@@ -14,9 +14,10 @@
 // per-(site, chunk) partial sums, so no separate pass over the state is
 // needed; the consumer adds the partials of a site in chunk order.
 //
-// The default discretisation steps in stage pairs (nuosc_pair.hip); the stage
-// kernel serves its RHS and the other schemes, whose RK4 is streamed with four
-// state copies u, A, yA, yB in 12 passes over the 8 fields per step.  With the stage inputs Y2 = u + dt/2 k1,
+// Boxes deep enough in z step in stage pairs (nuosc_pair.hip) in the default
+// discretisation; the stage kernel serves its RHS, the other boxes and the other
+// schemes.  There RK4 is streamed with four state copies u, A, yA, yB in 12
+// passes over the 8 fields per step.  With the stage inputs Y2 = u + dt/2 k1,
 // Y3 = u + dt/2 k2, Y4 = u + dt k3, the new state is
 //   u + dt/6 (k1 + 2k2 + 2k3 + k4) = (A + Y4) / 3 + dt/6 k4,
 //   A = Y2 + 2 Y3 - u = Y2 + u + dt k2,
@@ -39,6 +40,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <cstring>
 #include <vector>
 
 namespace nuosc {
@@ -771,22 +773,80 @@ __device__ __forceinline__ void stage_body(const StageArgs<T>& a, int lblock, in
     }
 }
 
-// Waves per SIMD the register allocation aims at: the FP64 slab kernel of
-// radius 2 is held to 2 by its LDS (two 73.7 KB blocks of 4 waves per CU); its
-// one-row (NOX) form fits 168 VGPRs (3 waves); FP32 fits 128 (4 waves).
+// Waves per SIMD the register allocation aims at: the FP64 slab kernels of
+// radius 2 are held to 2 by their LDS (two 73.7 KB blocks of 4 waves per CU); the
+// one-row (NOX) form of the RHS fits 168 VGPRs (3 waves); FP32 fits 128 (4 waves).
 template <typename T, int RAD = 2, bool NOX = false>
 constexpr int stage_waves() {
     return RAD == 3 ? (sizeof(T) == 4 ? 2 : 1) : (sizeof(T) == 4 ? 4 : (NOX ? 3 : 2));
 }
 
-// RAD = 2: the reference's default discretisation (stage 0 only); RAD = 3: any
-// of the schemes, chosen at run time (Geometry::ko5, Geometry::adv)
+// RAD = 2: the reference's default discretisation (NOX: stage 0 only); RAD = 3:
+// any of the schemes, chosen at run time (Geometry::ko5, Geometry::adv)
 template <typename T, int R, int STAGE, bool COMP, int RAD = 2, bool NOX = false>
 __global__ __launch_bounds__(64 * StageShape<T>::W) __attribute__((amdgpu_waves_per_eu(stage_waves<T, RAD, NOX>()))) void k_stage(const StageArgs<T> a) {
     constexpr int W = StageShape<T>::W;
     __shared__ Slab<T, R, W, RAD> slab;   // (never touched by NOX, which the compiler then leaves unallocated)
     const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     stage_body<T, R, W, RAD, STAGE, COMP, NOX>(a, xcd_remap(blockIdx.x, gridDim.x), wib, slab);
+}
+
+// Many independent runs in one launch: logical block -> (run, block of run)
+// from bmap; each run's arguments from the runs table (read with scalar loads).
+template <typename T, int R, int STAGE, bool COMP>
+__global__ __launch_bounds__(64 * StageShape<T>::W) __attribute__((amdgpu_waves_per_eu(stage_waves<T>()))) void k_stage_batch(
+    const StageArgs<T>* __restrict__ runs, const int* __restrict__ bmap) {
+    constexpr int W = StageShape<T>::W;
+    __shared__ Slab<T, R, W, 2> slab;
+    const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lb = xcd_remap(blockIdx.x, gridDim.x);
+    const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)bmap;
+    const int run = cm[2 * lb], blk = cm[2 * lb + 1];
+    const StageArgs<T> a = runs[run];   // uniform, read-only: scalar loads
+    stage_body<T, R, W, 2, STAGE, COMP>(a, blk, wib, slab);
+}
+
+// The same work as a persistent kernel: a grid of resident blocks takes
+// logical blocks from a work queue until it is empty.  Logical blocks keep
+// the split of xcd_remap (one contiguous range per XCD, block b of the grid
+// runs on XCD b % 8), and each XCD's blocks draw from their range through
+// their own counter ctr[x], so neighbouring logical blocks still run on one
+// XCD at about the same time.  Every block leaves the loop once its XCD's
+// counter passes the range (the exit every wave reaches); the counters are
+// zeroed by k_zero_ints before each launch.
+template <typename T, int R, int STAGE, bool COMP>
+__global__ __launch_bounds__(64 * StageShape<T>::W) __attribute__((amdgpu_waves_per_eu(stage_waves<T>()))) void k_stage_batch_q(
+    const StageArgs<T>* __restrict__ runs, const int* __restrict__ bmap, int* __restrict__ ctr, int nitems) {
+    constexpr int W = StageShape<T>::W;
+    __shared__ Slab<T, R, W, 2> slab;
+    __shared__ int next;
+    const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x = blockIdx.x % 8;
+    const int per = nitems / 8, rem = nitems % 8;
+    const int start = x < rem ? x * (per + 1) : rem * (per + 1) + (x - rem) * per;
+    const int count = per + (x < rem ? 1 : 0);
+    const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)bmap;
+    for (;;) {
+        if (threadIdx.x == 0) next = atomicAdd(&ctr[x], 1);
+        __syncthreads();
+        const int k = __builtin_amdgcn_readfirstlane(next);
+        __syncthreads();   // every wave has read next before thread 0 rewrites it
+        if (k >= count) break;
+        const int lb = start + k;
+        const int run = cm[2 * lb], blk = cm[2 * lb + 1];
+        const StageArgs<T> a = runs[run];   // uniform, read-only: scalar loads
+        stage_body<T, R, W, 2, STAGE, COMP>(a, blk, wib, slab);
+    }
+}
+
+__global__ void k_zero_ints(int* __restrict__ p, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = 0;
+}
+
+hipError_t launch_zero_ints(int* p, int n, hipStream_t s) {
+    hipLaunchKernelGGL(k_zero_ints, dim3((n + 63) / 64), dim3(64), 0, s, p, n);
+    return hipGetLastError();
 }
 
 int rows_per_wave(int esize) { return esize == 8 ? StageShape<double>::R : StageShape<float>::R; }
@@ -881,11 +941,21 @@ hipError_t launch_stage(int stage, const Geometry& g, const Physics& ph, const S
     constexpr int R = StageShape<T>::R;
     if (g.lpr != dirs_per_chunk((int)sizeof(T)) || g.wpb != StageShape<T>::W) return hipErrorInvalidValue;
     dim3 grid(pl.nblocks), block(64 * StageShape<T>::W);
-    // the default discretisation steps in stage pairs (nuosc_pair.hip): RHS only
-    if (scheme_radius(g.ko5, g.adv) == 2 && g.adv == kAdvCfd4) {
+    if (g.nox) {   // one x row, default discretisation: steps in stage pairs
         if (stage != 0) return hipErrorInvalidValue;
-        if (g.nox) hipLaunchKernelGGL((k_stage<T, R, 0, COMP, 2, true>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((k_stage<T, R, 0, COMP>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((k_stage<T, R, 0, COMP, 2, true>), grid, block, 0, s, a);
+    } else if (scheme_radius(g.ko5, g.adv) == 2 && g.adv == kAdvCfd4) {
+        switch (stage) {
+            case 0: hipLaunchKernelGGL((k_stage<T, R, 0, COMP>), grid, block, 0, s, a); break;
+            case 1: hipLaunchKernelGGL((k_stage<T, R, 1, COMP>), grid, block, 0, s, a); break;
+            case 2: hipLaunchKernelGGL((k_stage<T, R, 2, COMP>), grid, block, 0, s, a); break;
+            case 3: hipLaunchKernelGGL((k_stage<T, R, 3, COMP>), grid, block, 0, s, a); break;
+            case 4: hipLaunchKernelGGL((k_stage<T, R, 4, COMP>), grid, block, 0, s, a); break;
+            case 5: hipLaunchKernelGGL((k_stage<T, R, 5, COMP>), grid, block, 0, s, a); break;
+            case 6: hipLaunchKernelGGL((k_stage<T, R, 6, COMP>), grid, block, 0, s, a); break;
+            case 7: hipLaunchKernelGGL((k_stage<T, R, 7, COMP>), grid, block, 0, s, a); break;
+            default: return hipErrorInvalidValue;
+        }
     } else {
         switch (stage) {
             case 0: hipLaunchKernelGGL((k_stage<T, R, 0, COMP, 3>), grid, block, 0, s, a); break;
@@ -949,12 +1019,26 @@ __device__ __forceinline__ void xg_body(const XgArgs& a, long long blk) {
 
 __global__ __launch_bounds__(256) void k_xghosts(const XgArgs a) { xg_body(a, blockIdx.x); }
 
+__global__ __launch_bounds__(256) void k_xghosts_batch(const XgArgs* __restrict__ runs, const int* __restrict__ xmap) {
+    const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)xmap;
+    const int run = cm[2 * blockIdx.x], blk = cm[2 * blockIdx.x + 1];
+    const XgArgs a = runs[run];
+    xg_body(a, blk);
+}
+
 template <typename T>
 hipError_t launch_xghosts(const Geometry& g, T* y, hipStream_t s) {
     const XgArgs a = xg_args(g, y, sizeof(T));
     hipLaunchKernelGGL(k_xghosts, dim3((unsigned)xg_blocks(a.words)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
+
+struct TotArgs {
+    const double* part;
+    double* tot;
+    int nch;
+    long long nsites;
+};
 
 template <bool COMP>
 __device__ __forceinline__ void totals_body(const double* __restrict__ part, int nch, long long nsites,
@@ -997,6 +1081,176 @@ hipError_t launch_moment_totals(const Geometry& g, bool compensated, const doubl
     if (compensated) hipLaunchKernelGGL((k_moment_totals<true>), grid, block, 0, s, part, g.nch, nsites, tot);
     else hipLaunchKernelGGL((k_moment_totals<false>), grid, block, 0, s, part, g.nch, nsites, tot);
     return hipGetLastError();
+}
+
+size_t TableImage::put(const void* p, size_t bytes) {
+    const size_t at = (host.size() + 255) / 256 * 256;
+    host.resize(at + bytes);
+    if (p) std::memcpy(host.data() + at, p, bytes);
+    return at;
+}
+size_t TableImage::put_map(const std::vector<long long>& counts, int& blocks) {
+    long long total = 0;
+    for (long long k : counts) total += k;
+    blocks = (int)total;
+    const size_t at = put(nullptr, total * 2 * sizeof(int));
+    int* p = (int*)(host.data() + at);
+    for (int r = 0; r < (int)counts.size(); ++r)
+        for (int b = 0; b < (int)counts[r]; ++b) {
+            *p++ = r;
+            *p++ = b;
+        }
+    return at;
+}
+hipError_t TableImage::upload(void*& buf, size_t& bytes, hipStream_t s) const {
+    hipError_t e;
+    if (bytes < host.size()) {
+        if (buf) (void)hipFree(buf);
+        buf = nullptr;
+        bytes = 0;
+        if ((e = hipMalloc(&buf, host.size())) != hipSuccess) return e;
+        bytes = host.size();
+    }
+    if ((e = hipMemcpyAsync(buf, host.data(), host.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return e;
+    return hipStreamSynchronize(s);
+}
+hipError_t resident_blocks(const void* kernel, int threads, int& blocks) {
+    hipError_t e;
+    int dev = 0, cus = 0, per = 0;
+    if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
+    if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
+    if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0)) != hipSuccess) return e;
+    blocks = std::max(8, (cus * std::max(per, 1) + 7) / 8 * 8);
+    return hipSuccess;
+}
+
+// ---------------------------------------------------------------------------
+// batched runs that step stage by stage: one launch per stage, per refresh of
+// x ghost rows and per moment-total pass for every member
+// ---------------------------------------------------------------------------
+template <bool COMP>
+__global__ __launch_bounds__(256) void k_moment_totals_batch(const TotArgs* __restrict__ runs,
+                                                             const int* __restrict__ bmap) {
+    const __attribute__((address_space(4))) int* cm = (const __attribute__((address_space(4))) int*)bmap;
+    const int run = cm[2 * blockIdx.x], blk = cm[2 * blockIdx.x + 1];
+    const TotArgs ta = runs[run];
+    totals_body<COMP>(ta.part, ta.nch, ta.nsites, ta.tot, (long long)blk * 256 + threadIdx.x);
+}
+
+
+template <typename T>
+static hipError_t stage_batch_build_t(StageBatch& t, const std::vector<StageMember>& ms, hipStream_t s) {
+    const int n = (int)ms.size();
+    TableImage im;
+    std::vector<long long> count[3];   // stage, totals and ghost-row blocks
+    for (const StageMember& m : ms) {
+        count[0].push_back(m.pl.nblocks);
+        count[1].push_back(((long long)m.g.nx * m.g.nz * kMomStride + 255) / 256);
+        count[2].push_back(xg_blocks(xg_args(m.g, nullptr, sizeof(T)).words));
+    }
+    size_t off[4][3], off_map[3];
+    for (int st = 1; st <= 4; ++st) {
+        std::vector<StageArgs<T>> args(n);
+        std::vector<TotArgs> tots(n);
+        std::vector<XgArgs> xgs(n);
+        for (int r = 0; r < n; ++r) {
+            const StageMember& m = ms[r];
+            const double dt = m.dt, c6 = 1.0 / 6.0 * dt, c2 = 0.5 * dt;
+            T *u = (T*)m.u, *w = (T*)m.w, *ya = (T*)m.ya, *yb = (T*)m.yb;
+            T* yin;
+            const T* uu;
+            T* yout;
+            const double* mt;
+            double* mo;
+            double cw, cy;
+            switch (st) {   // (as enqueue_step)
+                case 1: yin = u; uu = u; yout = ya; mt = m.mu; mo = m.ma; cw = 0.0; cy = c2; break;
+                case 2: yin = ya; uu = u; yout = yb; mt = m.ma; mo = m.mb; cw = dt; cy = c2; break;
+                case 3: yin = yb; uu = u; yout = ya; mt = m.mb; mo = m.ma; cw = 0.0; cy = dt; break;
+                default: yin = ya; uu = ya; yout = u; mt = m.ma; mo = m.mu; cw = c6; cy = 0.0; break;
+            }
+            args[r] = make_stage_args<T>(m.g, m.ph, m.pl, yin, uu, w, yout, mt, m.mpart, cw, cy);
+            tots[r] = TotArgs{m.mpart, mo, m.g.nch, (long long)m.g.nx * m.g.nz};
+            xgs[r] = xg_args(m.g, yin, sizeof(T));
+        }
+        off[st - 1][0] = im.put(args.data(), n * sizeof(StageArgs<T>));
+        off[st - 1][1] = im.put(tots.data(), n * sizeof(TotArgs));
+        off[st - 1][2] = im.put(xgs.data(), n * sizeof(XgArgs));
+    }
+    int blocks[3];
+    for (int k = 0; k < 3; ++k) off_map[k] = im.put_map(count[k], blocks[k]);
+    const std::vector<int> zeros(32, 0);
+    const size_t off_ctr = im.put(zeros.data(), zeros.size() * sizeof(int));
+    hipError_t e = im.upload(t.buf, t.bytes, s);
+    if (e != hipSuccess) return e;
+    // (stage 2, the largest, sets the count)
+    constexpr int R = StageShape<T>::R;
+    e = resident_blocks((const void*)k_stage_batch_q<T, R, 2, sizeof(T) == 4>, 64 * StageShape<T>::W, t.pgrid);
+    if (e != hipSuccess) return e;
+    char* d = static_cast<char*>(t.buf);
+    for (int st = 0; st < 4; ++st) {
+        t.args[st] = d + off[st][0];
+        t.tot[st] = d + off[st][1];
+        t.xg[st] = d + off[st][2];
+    }
+    t.bmap = (int*)(d + off_map[0]);
+    t.tmap = (int*)(d + off_map[1]);
+    t.xmap = (int*)(d + off_map[2]);
+    t.ctr = (int*)(d + off_ctr);
+    t.nblocks = blocks[0];
+    t.tblocks = blocks[1];
+    t.xblocks = blocks[2];
+    return hipSuccess;
+}
+
+hipError_t stage_batch_build(StageBatch& t, const std::vector<StageMember>& ms, int esize, int launch, hipStream_t s) {
+    t.esize = esize;
+    t.launch = launch;
+    t.nblocks = 0;
+    if (ms.empty()) return hipSuccess;
+    for (const auto& m : ms) {
+        if (!buffer_addressable(m.g, esize)) return hipErrorInvalidValue;
+        if (m.g.lpr != dirs_per_chunk(esize) || m.g.wpb != waves_per_block(esize) || m.g.nox)
+            return hipErrorInvalidValue;
+    }
+    return esize == 8 ? stage_batch_build_t<double>(t, ms, s) : stage_batch_build_t<float>(t, ms, s);
+}
+
+void stage_batch_free(StageBatch& t) {
+    if (t.buf) (void)hipFree(t.buf);
+    t = StageBatch{};
+}
+
+template <typename T, int STAGE>
+static hipError_t stage_batch_launch(const StageBatch& t, hipStream_t s) {
+    constexpr int R = StageShape<T>::R;
+    constexpr bool COMP = sizeof(T) == 4;
+    const dim3 block(64 * StageShape<T>::W);
+    const StageArgs<T>* a = (const StageArgs<T>*)t.args[STAGE - 1];
+    hipLaunchKernelGGL(k_xghosts_batch, dim3(t.xblocks), dim3(256), 0, s, (const XgArgs*)t.xg[STAGE - 1], t.xmap);
+    if (t.launch == kBatchPersistent) {
+        int* c = t.ctr + 8 * (STAGE - 1);
+        const hipError_t e = launch_zero_ints(c, 8, s);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL((k_stage_batch_q<T, R, STAGE, COMP>), dim3(t.pgrid), block, 0, s, a, t.bmap, c, t.nblocks);
+    } else {
+        hipLaunchKernelGGL((k_stage_batch<T, R, STAGE, COMP>), dim3(t.nblocks), block, 0, s, a, t.bmap);
+    }
+    hipLaunchKernelGGL((k_moment_totals_batch<COMP>), dim3(t.tblocks), dim3(256), 0, s,
+                       (const TotArgs*)t.tot[STAGE - 1], t.tmap);
+    return hipGetLastError();
+}
+template <typename T>
+static hipError_t stage_batch_step_t(const StageBatch& t, int nstages, hipStream_t s) {
+    hipError_t e = stage_batch_launch<T, 1>(t, s);
+    if (e == hipSuccess && nstages > 1) e = stage_batch_launch<T, 2>(t, s);
+    if (e == hipSuccess && nstages > 2) e = stage_batch_launch<T, 3>(t, s);
+    if (e == hipSuccess && nstages > 3) e = stage_batch_launch<T, 4>(t, s);
+    return e;
+}
+hipError_t stage_batch_step(const StageBatch& t, int nstages, hipStream_t s) {
+    if (t.nblocks == 0) return hipSuccess;
+    return t.esize == 8 ? stage_batch_step_t<double>(t, nstages, s) : stage_batch_step_t<float>(t, nstages, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -50,7 +50,6 @@
 #include "nuosc_lanes.h"
 
 #include <algorithm>
-#include <cstring>
 #include <type_traits>
 #include <vector>
 
@@ -852,11 +851,6 @@ void k_pair_batch_q(const PairArgs<T>* __restrict__ runs, const int* __restrict_
     }
 }
 
-__global__ void k_zero_ints(int* __restrict__ p, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
-}
-
 constexpr int kRowWaves = 4;   // waves per block of the one-row form, a unit each
 
 template <typename T, int R>
@@ -1396,13 +1390,7 @@ namespace {
 template <typename T>
 hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hipStream_t s) {
     const int n = (int)ms.size();
-    std::vector<char> host;
-    auto put = [&](const void* p, size_t bytes) {
-        const size_t at = (host.size() + 255) / 256 * 256;
-        host.resize(at + bytes);
-        std::memcpy(host.data() + at, p, bytes);
-        return at;
-    };
+    TableImage im;
     // blocks of the two pairs, the totals and the prediction -> (member, block of member)
     std::vector<long long> count[4];
     for (const BatchMember& m : ms) {
@@ -1413,20 +1401,6 @@ hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hip
         count[2].push_back((sites + kTotSites - 1) / kTotSites);
         count[3].push_back(predict_blocks(g.nx, g.nz));
     }
-    auto put_map = [&](const std::vector<long long>& c, int& blocks) {
-        long long total = 0;
-        for (long long k : c) total += k;
-        blocks = (int)total;
-        const size_t at = (host.size() + 255) / 256 * 256;
-        host.resize(at + total * 2 * sizeof(int));
-        int* p = (int*)(host.data() + at);
-        for (int r = 0; r < n; ++r)
-            for (int b = 0; b < (int)c[r]; ++b) {
-                *p++ = r;
-                *p++ = b;
-            }
-        return at;
-    };
     size_t off_args[2][2], off_pre[2][2], off_map[4];
     for (int flip = 0; flip < 2; ++flip)
         for (int pair = 1; pair <= 2; ++pair) {
@@ -1442,23 +1416,24 @@ hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hip
                 pa[r] = pair_args<T>(ms[r].g, ms[r].ph, ms[r].zlen, pair, b, ms[r].dt);
                 pp[r] = predict_args(ms[r].g, ms[r].ph, pair, b, ms[r].dt);
             }
-            off_args[pair - 1][flip] = put(pa.data(), n * sizeof(PairArgs<T>));
-            off_pre[pair - 1][flip] = put(pp.data(), n * sizeof(PredictArgs));
+            off_args[pair - 1][flip] = im.put(pa.data(), n * sizeof(PairArgs<T>));
+            off_pre[pair - 1][flip] = im.put(pp.data(), n * sizeof(PredictArgs));
         }
     std::vector<SumArgs> sa(n);
     for (int r = 0; r < n; ++r)
         sa[r] = SumArgs{ms[r].b.part, ms[r].b.tot, ms[r].g.nch, (long long)ms[r].g.nx * ms[r].g.nz};
-    const size_t off_sum = put(sa.data(), n * sizeof(SumArgs));
+    const size_t off_sum = im.put(sa.data(), n * sizeof(SumArgs));
     int blocks[4];
-    for (int k = 0; k < 4; ++k) off_map[k] = put_map(count[k], blocks[k]);
+    for (int k = 0; k < 4; ++k) off_map[k] = im.put_map(count[k], blocks[k]);
     const std::vector<int> zeros(kBatchCounters, 0);
-    const size_t off_ctr = put(zeros.data(), kBatchCounters * sizeof(int));
-    hipError_t e;
-    if (t.bytes < host.size()) {
-        batch_free(t);
-        if ((e = hipMalloc(&t.buf, host.size())) != hipSuccess) return e;
-        t.bytes = host.size();
-    }
+    const size_t off_ctr = im.put(zeros.data(), kBatchCounters * sizeof(int));
+    hipError_t e = im.upload(t.buf, t.bytes, s);
+    if (e != hipSuccess) return e;
+    // persistent launch: a grid of as many blocks as the GPU holds at once
+    e = resident_blocks((const void*)k_pair_batch_q<T, 1>, 64 * (PairShape<T, 1>::R + 4), t.pgrid[0]);
+    if (e != hipSuccess) return e;
+    e = resident_blocks((const void*)k_pair_batch_q<T, 2>, 64 * (PairShape<T, 2>::R + 4), t.pgrid[1]);
+    if (e != hipSuccess) return e;
     char* d = static_cast<char*>(t.buf);
     for (int p = 0; p < 2; ++p)
         for (int flip = 0; flip < 2; ++flip) {
@@ -1475,21 +1450,7 @@ hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hip
     t.ctr = (int*)(d + off_ctr);
     t.tblocks = blocks[2];
     t.pblocks = blocks[3];
-    // persistent launch: a grid of as many blocks as the GPU holds at once
-    {
-        int dev = 0, cus = 0, bpc[2] = {0, 0};
-        if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
-        if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
-        if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc[0], k_pair_batch_q<T, 1>,
-                                                              64 * (PairShape<T, 1>::R + 4), 0)) != hipSuccess)
-            return e;
-        if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpc[1], k_pair_batch_q<T, 2>,
-                                                              64 * (PairShape<T, 2>::R + 4), 0)) != hipSuccess)
-            return e;
-        for (int p = 0; p < 2; ++p) t.pgrid[p] = std::max(8, (cus * std::max(bpc[p], 1) + 7) / 8 * 8);
-    }
-    if ((e = hipMemcpyAsync(t.buf, host.data(), host.size(), hipMemcpyHostToDevice, s)) != hipSuccess) return e;
-    return hipStreamSynchronize(s);
+    return hipSuccess;
 }
 
 template <typename T, int PAIR>
@@ -1499,7 +1460,8 @@ hipError_t batch_pair_t(const BatchTables& t, int flip, hipStream_t s) {
     const int n = t.nblocks[PAIR - 1];
     if (t.launch == kBatchPersistent) {
         int* c = t.ctr + 8 * (PAIR - 1);
-        hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, c, 8);   // a kernel node, not a memset, in graphs
+        const hipError_t e = launch_zero_ints(c, 8, s);
+        if (e != hipSuccess) return e;
         hipLaunchKernelGGL((k_pair_batch_q<T, PAIR>), dim3(t.pgrid[PAIR - 1]), block, 0, s, a, t.bmap[PAIR - 1], c, n);
     } else {
         hipLaunchKernelGGL((k_pair_batch<T, PAIR>), dim3(n), block, 0, s, a, t.bmap[PAIR - 1]);
