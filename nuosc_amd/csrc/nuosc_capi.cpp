@@ -479,11 +479,19 @@ int refresh_step(nuosc_sim* s, StepKind kind = kRk4) {
 }
 bool step_ready(const nuosc_sim* s, StepKind kind = kRk4) { return s->pairs[kind] ? s->have_sums : s->have_moments; }
 
-// the stage pairs leave the new state in st_ya
-void state_stepped(nuosc_sim* s) {
-    std::swap(s->st_u, s->st_ya);
-    s->flip ^= 1;
-    s->have_moments = false;
+// no record of the state is current: it changes, or a step is being queued, which
+// has other records in their place until it is queued whole
+void forget_records(nuosc_sim* s) { s->have_moments = s->have_sums = false; }
+
+// a step is queued: the stage pairs leave the new state in st_ya; its records
+// are those the next step of this kind needs
+void state_stepped(nuosc_sim* s, StepKind kind = kRk4) {
+    if (s->pairs[kind]) {
+        std::swap(s->st_u, s->st_ya);
+        s->flip ^= 1;
+    }
+    (s->pairs[kind] ? s->have_sums : s->have_moments) = true;
+    s->phy_time += s->dt;   // accumulated, as nuosc_class.cpp:423, 448
 }
 
 // nsteps steps on the handle's stream, replayed from a captured graph if the
@@ -502,6 +510,7 @@ int run_steps(nuosc_sim* s, StepKind kind, int nsteps) {
     }
     HIPCK(s, hipEventRecord(s->ev0, s->stream));
     for (int n = 0; n < nsteps; ++n) {
+        forget_records(s);
         if (s->cfg.use_graph) {
             hipGraphExec_t& exec = s->graph_exec[kind][s->flip];
             if (!exec) {
@@ -522,9 +531,7 @@ int run_steps(nuosc_sim* s, StepKind kind, int nsteps) {
             const int rc = enqueue();
             if (rc) return rc;
         }
-        if (pairs) state_stepped(s);
-        else s->have_sums = false;
-        s->phy_time += s->dt;   // accumulated, as nuosc_class.cpp:423, 448
+        state_stepped(s, kind);
     }
     HIPCK(s, hipEventRecord(s->ev1, s->stream));
     s->steps_in_last_call = nsteps;
@@ -989,6 +996,7 @@ int nuosc_fill_init(nuosc_sim* s, int ipt, double alpha, double eps0, double sig
     int rc = ensure_tmp(s, sizeof(double) * 2 * (size_t)s->nz);
     if (rc) return rc;
     HIPCK(s, hipMemcpyAsync(s->d_tmp, tab.data(), sizeof(double) * 2 * s->nz, hipMemcpyHostToDevice, s->stream));
+    forget_records(s);
     if (is64(s))
         HIPCK(s, launch_init<double>(s->geo, ipt, s->d_g0, s->d_g0 + s->nv, s->d_tmp, s->d_tmp + s->nz, eps0, seed,
                                      (double*)s->st_u, s->stream));
@@ -1009,7 +1017,6 @@ int nuosc_fill_init(nuosc_sim* s, int ipt, double alpha, double eps0, double sig
     drop_graph(s);
     rc = set_device_time(s);
     if (rc) return rc;
-    s->have_moments = s->have_sums = false;
     rc = refresh_step(s);
     if (rc) return rc;
     HIPCK(s, hipStreamSynchronize(s->stream));
@@ -1048,12 +1055,11 @@ int nuosc_profile_stages(nuosc_sim* s, int nsteps, double* stage_ms) {
     double acc[4] = {0, 0, 0, 0};
     int rc = NUOSC_OK;
     for (int n = 0; n < nsteps && rc == NUOSC_OK; ++n) {
+        forget_records(s);
         if (pairs) rc = is64(s) ? enqueue_step_pairs<double>(s, kRk4, ev) : enqueue_step_pairs<float>(s, kRk4, ev);
         else rc = is64(s) ? enqueue_step<double>(s, ev) : enqueue_step<float>(s, ev);
         if (rc) break;
-        if (pairs) state_stepped(s);
-        else s->have_sums = false;
-        s->phy_time += s->dt;
+        state_stepped(s);
         if (hipEventSynchronize(ev[pairs ? 5 : 7]) != hipSuccess) {
             rc = fail(s, NUOSC_EHIP, "event sync failed");
             break;
@@ -1230,9 +1236,9 @@ int nuosc_analysis(nuosc_sim* s, nuosc_analysis_t* o) {
 
 int nuosc_renormalize(nuosc_sim* s) {
     if (!s) return NUOSC_EINVAL;
+    forget_records(s);
     if (is64(s)) HIPCK(s, launch_renorm<double>(s->geo, (double*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->stream));
     else HIPCK(s, launch_renorm<float>(s->geo, (float*)s->st_u, s->d_g0, s->d_g0 + s->nv, s->stream));
-    s->have_moments = s->have_sums = false;
     return refresh_step(s);
 }
 
@@ -1270,13 +1276,13 @@ int nuosc_upload_field(nuosc_sim* s, int f, const double* host) { return nuosc_u
 int nuosc_upload_fields(nuosc_sim* s, int f0, int nf, const double* host) {
     if (!s || !host) return NUOSC_EINVAL;
     if (f0 < 0 || nf < 1 || f0 > s->nf - nf) return fail(s, NUOSC_EINVAL, "field index out of range");
-    s->have_moments = s->have_sums = false;
+    forget_records(s);
     return fields_up(s, s->st_u, f0, nf, host);
 }
 
 int nuosc_state_updated(nuosc_sim* s) {
     if (!s) return NUOSC_EINVAL;
-    s->have_moments = s->have_sums = false;
+    forget_records(s);
     int rc = refresh_step(s);
     if (rc) return rc;
     HIPCK(s, hipStreamSynchronize(s->stream));
@@ -1502,13 +1508,10 @@ int nuosc_batch_step(nuosc_batch* b, int nsteps) {
             if (hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0) != hipSuccess)
                 return bfail(b, NUOSC_EHIP, "graph instantiation failed");
         }
+        for (nuosc_sim* m : b->members) forget_records(m);
         if (hipGraphLaunch(exec, b->stream) != hipSuccess) return bfail(b, NUOSC_EHIP, "graph launch failed");
         b->flip ^= 1;
-        for (nuosc_sim* m : b->members) {
-            if (m->pairs[kRk4]) state_stepped(m);
-            else m->have_sums = false;
-            m->phy_time += m->dt;
-        }
+        for (nuosc_sim* m : b->members) state_stepped(m);
     }
     if (hipStreamSynchronize(b->stream) != hipSuccess) return bfail(b, NUOSC_EHIP, "batch stream sync failed");
     return NUOSC_OK;

@@ -1,0 +1,113 @@
+"""The host code of the handles and batches on a stand-in HIP runtime
+(fake_hip.cpp): no GPU, every launch and allocation can be made to fail, and a
+kernel that is given another state's records is counted."""
+import numpy as np
+import pytest
+
+import fake_hip
+import nuosc_amd as N
+
+H = 0.125
+
+
+@pytest.fixture(scope="session")
+def fake_lib(tmp_path_factory):
+    return fake_hip.load(fake_hip.build(tmp_path_factory.mktemp("fake")))
+
+
+@pytest.fixture
+def fake(fake_lib, monkeypatch):
+    monkeypatch.setattr(N, "_lib", fake_lib)
+    fake_lib.fake_reset()
+    yield fake_lib
+    assert fake_lib.fake_mistakes() == 0
+    assert fake_lib.fake_device_bytes() == 0 and fake_lib.fake_graphs() == 0
+
+
+def make(nx=9, nz=40, nn=2, seed=7, **kw):
+    g = N.NuOsc(nv=nn, x0=-nx * H / 2, x1=nx * H / 2, z0=-nz * H / 2, z1=nz * H / 2, dx=H, dz=H, **kw)
+    g.fillInitValue(ipt=5, seed=seed)
+    return g
+
+
+def value(g):
+    return g.get_field(0).flat[0]
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(precision=32), dict(nx=701, nz=2), dict(bc=N.BC_OPEN_Z), dict(nflavor=3),
+                                dict(adv=N.ADV_CFD2), dict(renorm=True), dict(use_graph=False)])
+def test_steps(fake, kw):
+    """The stand-in itself: every route steps, in any order of the schemes."""
+    with make(**kw) as g:
+        g.step_rk4(3)
+        g.step_srk3(2)
+        g.step_rk4(2)
+        g.set_state(g.get_state())
+        g.step_srk3(1)
+        assert value(g) % 1000 == 7 + 8
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(precision=32), dict(nx=701, nz=2), dict(bc=N.BC_OPEN_Z), dict(nflavor=3),
+                                dict(renorm=True)])
+@pytest.mark.parametrize("use_graph", [True, False])
+@pytest.mark.parametrize("scheme", ["step_rk4", "step_srk3", "profile_stages"])
+def test_failed_launch_in_a_step(fake, kw, use_graph, scheme):
+    """Whichever launch of a step fails, the call says so and the next step does
+    not take the records the failed one left."""
+    with make(use_graph=use_graph, **kw) as g:
+        g.step_rk4(1)
+        pairs = g.plan()[0] == 15 and "nflavor" not in kw
+        for n in range(1, 15):
+            before, t = value(g), g.phy_time
+            fake.fake_fail(b"launch", n)
+            try:
+                getattr(g, scheme)(1)
+            except N.NuOscError:
+                assert g.phy_time == t
+                if pairs:   # (the other routes write the state in place)
+                    assert value(g) == before
+            fake.fake_fail(b"launch", 1 << 30)
+            g.step_srk3(1)
+            g.step_rk4(1)
+            assert fake.fake_mistakes() == 0, n
+
+
+@pytest.mark.parametrize("what", ["analysis", "pair_sums", "renorm"])
+def test_failed_refresh(fake, what):
+    """fillInitValue and renormalize that fail half-way leave no records of the
+    state before."""
+    with make() as g:
+        g.step_rk4(1)
+        fake.fake_fail(what.encode(), 1)
+        with pytest.raises(N.NuOscError):
+            if what == "renorm":
+                g.renormalize()
+            else:
+                g.fillInitValue(ipt=5, seed=50)
+        g.step_rk4(1)
+        assert value(g) == (9 if what == "renorm" else 51)
+
+
+@pytest.mark.parametrize("what", ["launch", "hipGraphLaunch"])
+def test_failed_batch_step(fake, what):
+    sims = [make(seed=10), make(nx=701, nz=2, seed=20)]
+    b = N.Batch()
+    for g in sims:
+        b.add(g)
+    b.step(1)
+    for n in range(1, 10):
+        before = [value(g) for g in sims]
+        fake.fake_fail(what.encode(), n)
+        sims[0].set_mu(1.0 + n)   # (a new capture)
+        try:
+            b.step(1)
+        except N.NuOscError:
+            assert [value(g) for g in sims] == before
+        fake.fake_fail(what.encode(), 1 << 30)
+        for g in sims:
+            g.step_rk4(1)
+        b.step(2)
+        assert fake.fake_mistakes() == 0, n
+    b.close()
+    for g in sims:
+        g.close()
