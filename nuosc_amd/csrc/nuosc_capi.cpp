@@ -523,8 +523,13 @@ int run_steps(nuosc_sim* s, StepKind kind, int nsteps) {
                     return rc;
                 }
                 if (e != hipSuccess) return fail(s, NUOSC_EHIP, std::string("graph capture: ") + hipGetErrorString(e));
+                const hipError_t ie = hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0);
+                if (ie != hipSuccess) {
+                    exec = nullptr;
+                    (void)hipGraphDestroy(gr);
+                    return fail(s, NUOSC_EHIP, std::string("graph instantiation: ") + hipGetErrorString(ie));
+                }
                 s->graph[kind][s->flip] = gr;
-                HIPCK(s, hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0));
             }
             HIPCK(s, hipGraphLaunch(exec, s->stream));
         } else {
@@ -1504,9 +1509,12 @@ int nuosc_batch_step(nuosc_batch* b, int nsteps) {
                 if (gr) (void)hipGraphDestroy(gr);
                 return bfail(b, NUOSC_EHIP, "batched step capture failed");
             }
-            b->graph[b->flip] = gr;
-            if (hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0) != hipSuccess)
+            if (hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0) != hipSuccess) {
+                exec = nullptr;
+                (void)hipGraphDestroy(gr);
                 return bfail(b, NUOSC_EHIP, "graph instantiation failed");
+            }
+            b->graph[b->flip] = gr;
         }
         for (nuosc_sim* m : b->members) forget_records(m);
         if (hipGraphLaunch(exec, b->stream) != hipSuccess) return bfail(b, NUOSC_EHIP, "graph launch failed");

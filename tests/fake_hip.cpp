@@ -212,7 +212,7 @@ hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) {
 }
 hipError_t hipGraphInstantiate(hipGraphExec_t* x, hipGraph_t g, hipGraphNode_t*, char*, size_t) {
     *x = nullptr;
-    if (fails("hipGraphInstantiate")) return err(hipErrorOutOfMemory);
+    if (fails("hipGraphInstantiate")) return hipErrorOutOfMemory;
     *x = new hipGraphExec{g->ops};
     return hipSuccess;
 }

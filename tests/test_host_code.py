@@ -111,3 +111,23 @@ def test_failed_batch_step(fake, what):
     b.close()
     for g in sims:
         g.close()
+
+
+def test_failed_instantiation(fake):
+    """A captured step that cannot be instantiated is given back (the fixture
+    counts graphs), and the next call captures it again."""
+    with make() as g:
+        b = N.Batch()
+        for n in range(2):
+            fake.fake_fail(b"hipGraphInstantiate", 1)
+            with pytest.raises(N.NuOscError):
+                g.step_rk4(1)
+        g.step_rk4(3)
+        b.add(g)
+        for n in range(2):
+            fake.fake_fail(b"hipGraphInstantiate", 1)
+            with pytest.raises(N.NuOscError):
+                b.step(1)
+        b.step(2)
+        assert value(g) == 7 + 5
+        b.close()
