@@ -35,12 +35,17 @@ void free_slot(Slot& s) {
     if (s.p) (void)hipHostFree(s.p);
     s = Slot{};
 }
-bool make_slot(Slot& s) {
-    if (hipHostMalloc(&s.p, kSlotBytes, hipHostMallocPortable) == hipSuccess &&
-        hipEventCreateWithFlags(&s.done, hipEventDisableTiming) == hipSuccess)
-        return true;
-    free_slot(s);
-    return false;
+// (an event belongs to the device that is current when it is made, and can be
+// recorded on that device's streams only: the caller may have another one current)
+bool make_slot(int device, Slot& s) {
+    int current = device;
+    (void)hipGetDevice(&current);
+    if (current != device) (void)hipSetDevice(device);
+    const bool ok = hipHostMalloc(&s.p, kSlotBytes, hipHostMallocPortable) == hipSuccess &&
+                    hipEventCreateWithFlags(&s.done, hipEventDisableTiming) == hipSuccess;
+    if (!ok) free_slot(s);
+    if (current != device) (void)hipSetDevice(current);
+    return ok;
 }
 
 // Adds up to want slots to got, which has room for them (at least one: waits
@@ -56,7 +61,7 @@ void take_slots(int device, int want, std::vector<Slot>& got) {
         }
         while ((int)got.size() < want && d.made < kMaxSlots) {
             Slot s;
-            if (!make_slot(s)) break;
+            if (!make_slot(device, s)) break;
             ++d.made;
             got.push_back(s);
         }

@@ -1,6 +1,8 @@
 """The host code of the handles and batches on a stand-in HIP runtime
 (fake_hip.cpp): no GPU, every launch and allocation can be made to fail, and a
 kernel that is given another state's records is counted."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -131,3 +133,22 @@ def test_failed_instantiation(fake):
         b.step(2)
         assert value(g) == 7 + 5
         b.close()
+
+
+def test_transfer_with_another_device_current(fake):
+    """A handle on device 1 moves fields whichever device its caller has current."""
+    with make(device=1) as g:
+        for current in (0, 1):
+            fake.hipSetDevice(current)
+            a = np.full((8, *g.shape), 3.0 + current)
+            g.set_state(a)
+            assert np.array_equal(g.get_state(), a)
+            g.analysis()
+    fake.hipSetDevice(0)
+    with N.NuOsc(nv=2, device=1) as g:
+        fake.hipSetDevice(0)
+        g.fillInitValue(ipt=5, seed=4)   # the first slot
+        assert value(g) == 4
+        dev = C.c_int()
+        fake.hipGetDevice(C.byref(dev))
+        assert dev.value == 0
