@@ -43,7 +43,10 @@ bool make_slot(int device, Slot& s) {
     if (current != device) (void)hipSetDevice(device);
     const bool ok = hipHostMalloc(&s.p, kSlotBytes, hipHostMallocPortable) == hipSuccess &&
                     hipEventCreateWithFlags(&s.done, hipEventDisableTiming) == hipSuccess;
-    if (!ok) free_slot(s);
+    if (!ok) {
+        free_slot(s);
+        (void)hipGetLastError();   // (else the next launch check reports it: fewer slots will do)
+    }
     if (current != device) (void)hipSetDevice(current);
     return ok;
 }

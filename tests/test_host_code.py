@@ -152,3 +152,13 @@ def test_transfer_with_another_device_current(fake):
         dev = C.c_int()
         fake.hipGetDevice(C.byref(dev))
         assert dev.value == 0
+
+
+def test_fewer_slots_than_asked_for(fake):
+    """A transfer that gets some of its slots goes on with those."""
+    with make(nx=128, nz=128) as g:   # 44 MB: eight slots
+        a = np.full((8, *g.shape), 3.0)
+        for what in (b"hipHostMalloc", b"hipEventCreate"):
+            fake.fake_fail(what, 2)
+            g.set_state(a)
+            assert np.array_equal(g.get_state(), a)
