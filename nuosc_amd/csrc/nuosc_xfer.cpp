@@ -110,7 +110,10 @@ hipError_t xfer_run(int device, hipStream_t s, long long nchunks, int nthreads, 
         take_slots(device, want, slots);
     } catch (const std::bad_alloc&) {
     }
-    if (slots.empty()) return hipErrorOutOfMemory;
+    if (slots.empty()) {
+        (void)hipStreamSynchronize(s);   // what the caller queued may read its own memory
+        return hipErrorOutOfMemory;
+    }
     std::atomic<long long> next{0};
     std::atomic<int> error{hipSuccess};
     auto work = [&](const Slot& slot, bool own_thread) {

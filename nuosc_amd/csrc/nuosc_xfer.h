@@ -35,7 +35,7 @@ inline int xfer_threads(long long bytes) { return bytes < (32 << 20) ? 1 : kXfer
 // slot, then host(c, slot) runs once it is done; up: host(c, slot) fills the
 // slot, then enqueue(c, slot) queues the work that reads it.  Returns when
 // all of it is done; an error (also of a chunk not started because of it) is
-// returned, hipErrorOutOfMemory if no slot can be had.
+// returned, hipErrorOutOfMemory if no slot can be had, with nothing left queued on s.
 hipError_t xfer_run(int device, hipStream_t s, long long nchunks, int nthreads, bool down,
                     const std::function<hipError_t(long long, void*)>& enqueue,
                     const std::function<void(long long, void*)>& host);

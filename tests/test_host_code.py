@@ -162,3 +162,15 @@ def test_fewer_slots_than_asked_for(fake):
             fake.fake_fail(what, 2)
             g.set_state(a)
             assert np.array_equal(g.get_state(), a)
+
+
+def test_no_slot_leaves_nothing_queued(fake):
+    """Calls that fail for want of a slot return once the copies that they queued
+    from their own memory are done."""
+    with N.NuOsc(nv=2) as g:
+        for call in (lambda: g.p3_slice([0, 1], [0, 2]), lambda: g.fillInitValue(ipt=0)):
+            fake.fake_fail(b"hipHostMalloc", 1)
+            with pytest.raises(N.NuOscError) as e:
+                call()
+            assert e.value.code == N.NUOSC_ENOMEM
+            assert fake.fake_pending() == 0
