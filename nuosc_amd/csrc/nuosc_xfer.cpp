@@ -17,6 +17,8 @@ namespace {
 
 struct Slot {
     void* p = nullptr;
+    // releases to the system: what a kernel wrote to the slot is in host memory once
+    // the event is over, also where pinned memory is not coherent by default
     hipEvent_t done = nullptr;
 };
 constexpr int kMaxSlots = 2 * kXferThreads;   // per device: 64 MiB of pinned memory
@@ -42,7 +44,7 @@ bool make_slot(int device, Slot& s) {
     (void)hipGetDevice(&current);
     if (current != device) (void)hipSetDevice(device);
     const bool ok = hipHostMalloc(&s.p, kSlotBytes, hipHostMallocPortable) == hipSuccess &&
-                    hipEventCreateWithFlags(&s.done, hipEventDisableTiming) == hipSuccess;
+                    hipEventCreateWithFlags(&s.done, hipEventDisableTiming | hipEventReleaseToSystem) == hipSuccess;
     if (!ok) {
         free_slot(s);
         (void)hipGetLastError();   // (else the next launch check reports it: fewer slots will do)

@@ -174,3 +174,10 @@ def test_no_slot_leaves_nothing_queued(fake):
                 call()
             assert e.value.code == N.NUOSC_ENOMEM
             assert fake.fake_pending() == 0
+
+
+def test_slot_events_release_to_the_system(fake):
+    """hipEventReleaseToSystem (0x40000000): the fence that makes a kernel's writes
+    to a slot visible to the host."""
+    with make():
+        assert fake.fake_event_flags() & 0x40000000
