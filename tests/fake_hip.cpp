@@ -63,6 +63,7 @@ bool fails(const char* what) {
 }
 void run(ihipStream_t* s) {
     std::lock_guard<std::recursive_mutex> g(mu);
+    if (std::find(streams.begin(), streams.end(), s) == streams.end()) return;   // (an event's, gone)
     std::vector<Op> q;
     q.swap(s->queue);
     for (Op& op : q) op();

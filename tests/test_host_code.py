@@ -177,7 +177,7 @@ def test_no_slot_leaves_nothing_queued(fake):
 
 
 def test_slot_events_release_to_the_system(fake):
-    """hipEventReleaseToSystem (0x40000000): the fence that makes a kernel's writes
+    """hipEventReleaseToSystem (0x80000000): the fence that makes a kernel's writes
     to a slot visible to the host."""
     with make():
-        assert fake.fake_event_flags() & 0x40000000
+        assert fake.fake_event_flags() & 0x80000000
