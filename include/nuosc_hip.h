@@ -257,14 +257,17 @@ int nuosc_last_step_ms(nuosc_sim* sim, double* ms);
 int nuosc_profile_stages(nuosc_sim* sim, int nsteps, double* stage_ms);
 
 /* Stage-kernel decomposition (no reference counterpart).  Each wavefront
- * marches along z over a segment of zlen sites; nuosc_autotune times RK4
- * stages 1-3 (with their boundary fills and moment totals), or the two stage
- * pairs, on this handle's own grid for zlen in {8, ..., 256}, the candidates in turn for trials
- * rounds after a warm-up round, keeps each candidate's fastest time and
- * selects the best.  Call it at a step boundary: it overwrites only the RK4
- * scratch copies, never the state.  Results are cached per (nx, nz, nv,
- * precision, bc, ko_order, adv, one-row form) for the process.  3-flavour handles have no segment length:
- * autotune returns NUOSC_OK with *best_zlen = 0 and set_zlen has no effect. */
+ * marches along z over a segment of zlen sites.  nuosc_autotune times RK4
+ * stages 1-3 (with their boundary fills and moment totals), or each of the two
+ * stage pairs, on this handle's own grid for zlen in {8, ..., 256}, the length
+ * planned and the one in force, in turn for trials rounds after a warm-up
+ * round, keeps each one's fastest time and takes it instead of the plan if it
+ * is faster by more than 2%; stage pairs have a length each (best_zlen: pair
+ * 1's; best_ms: both pairs' times).  Call it at a step boundary: it overwrites
+ * only the RK4 scratch copies, never the state.  Results are cached per (nx,
+ * nz, nv, precision, bc, ko_order, adv, one-row form) for the process.
+ * 3-flavour handles have no segment length: autotune returns NUOSC_OK with
+ * *best_zlen = 0 and set_zlen has no effect. */
 int nuosc_get_plan(const nuosc_sim* sim, int* zlen, int* waves);
 int nuosc_set_zlen(nuosc_sim* sim, int zlen);
 int nuosc_autotune(nuosc_sim* sim, int trials, int* best_zlen, double* best_ms);

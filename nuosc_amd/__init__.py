@@ -335,8 +335,9 @@ class NuOsc:
         self._check(lib().nuosc_set_zlen(self._h, int(zlen)))
 
     def autotune(self, trials=2):
-        """Pick the z-segment length of the stage kernel by timing it on this
-        grid (at a step boundary; the state is not modified)."""
+        """Pick the z-segment lengths of the stage kernels by timing them on this
+        grid (at a step boundary; the state is not modified); returns that of
+        the first kernel and the time (ms; -1: from an earlier call)."""
         z, ms = C.c_int(), C.c_double()
         self._check(lib().nuosc_autotune(self._h, int(trials), C.byref(z), C.byref(ms)))
         return z.value, ms.value

@@ -45,6 +45,7 @@ std::map<std::string, long long> count;      // how often it ran
 std::map<void*, size_t> device_mem;
 std::vector<ihipStream_t*> streams;
 double best_zlen[kLone + 1] = {};
+int last_zlen[kLone + 1] = {};
 std::vector<BatchMember> batch_members;
 thread_local int current = 0;
 thread_local hipError_t last = hipSuccess;
@@ -109,6 +110,7 @@ int fake_pending() {
     return (int)n;
 }
 void fake_best_zlen(int pair, double z) { best_zlen[pair] = z; }
+int fake_last_zlen(int pair) { return last_zlen[pair]; }
 
 const char* hipGetErrorString(hipError_t e) { return e == hipSuccess ? "ok" : "error"; }
 hipError_t hipGetLastError() {
@@ -246,7 +248,10 @@ int pair_waves(const Geometry&, int, int zlen) { return zlen; }
 int plan_pair_zlen(const Geometry& g, int, int pair, int) { return std::min(g.nz, pair == 2 ? 25 : (pair == kLone ? 20 : 15)); }
 int plan_batch_zlen(const std::vector<Geometry>&, int, int) { return 24; }
 // a kernel takes 1 ms where its segments have the best length, longer elsewhere
-static double pair_ms(int pair, int zlen) { return 1.0 + std::abs(zlen - best_zlen[pair]) / 100.0; }
+static double pair_ms(int pair, int zlen) {
+    last_zlen[pair] = zlen;
+    return 1.0 + std::abs(zlen - best_zlen[pair]) / 10.0;
+}
 
 template <typename T>
 hipError_t launch_init(const Geometry&, int, const double*, const double*, const double*, const double*, double,

@@ -169,3 +169,20 @@ def test_open_ghost_waves(nuosc_mod, oracle_mod, nx, nn, precision):
     tol = 1e-12 if precision == 64 else 3 * 18 * 2.0 ** -24 * 2
     for f in range(8):
         assert np.max(np.abs(a[f] - b[f])) <= tol * np.max(np.abs(b[:4] if f < 4 else b[4:])), f
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+def test_autotuned_steps_bitwise(nuosc_mod, precision):
+    """Steps on tuned segment lengths, on a second handle through the cached
+    ones, and on the plan: the same state."""
+    runs = []
+    for tune in (0, 2, 2):
+        g = make(nuosc_mod, 31, 83, 3, precision=precision)
+        if tune:
+            zlen, ms = g.autotune(tune)
+            assert zlen == g.plan()[0] and (ms > 0) == (len(runs) == 1)
+        g.step_rk4(3)
+        g.step_srk3(1)
+        runs.append(g.get_state())
+    for r in runs[1:]:
+        assert np.array_equal(r, runs[0])

@@ -181,3 +181,30 @@ def test_slot_events_release_to_the_system(fake):
     to a slot visible to the host."""
     with make():
         assert fake.fake_event_flags() & 0x80000000
+
+
+# best lengths of the two pair kernels; planned: 15 and 25
+@pytest.mark.parametrize("nx,best", [(100, (15, 25)), (101, (64, 16)), (102, (15, 32)), (103, (8, 25)), (104, (40, 33))])
+def test_autotune_takes_each_kernels_best(fake, nx, best):
+    """The tuner never leaves a kernel slower than it was planned, gives each its
+    own length, and a second handle of the grid gets the same from the cache."""
+    zl = [8, 16, 32, 64, 128, 256]
+    want = [min([p, *zl], key=lambda z: abs(z - b)) for p, b in zip((15, 25), best)]
+    for pair in (1, 2):
+        fake.fake_best_zlen(pair, best[pair - 1])
+    for handle in range(2):
+        with make(nx=nx, nz=300) as g:
+            got, ms = g.autotune(1)
+            assert (ms > 0) == (handle == 0) and got == want[0] == g.plan()[0]
+            g.step_rk4(1)
+            assert [fake.fake_last_zlen(p) for p in (1, 2)] == want
+            g.step_srk3(1)
+            assert [fake.fake_last_zlen(p) for p in (3, 4)] == [15, 20]
+
+
+def test_autotune_tries_the_length_in_force(fake):
+    fake.fake_best_zlen(1, 47)
+    fake.fake_best_zlen(2, 47)
+    with make(nx=110, nz=300) as g:
+        g.set_zlen(47)
+        assert g.autotune(1)[0] == 47
