@@ -1419,8 +1419,9 @@ int batch_tables(nuosc_batch* b) {
     }
     for (nuosc_sim* m : b->members) {
         if (m->pairs[kRk4]) {
-            const int zlen = shared > 0 ? std::min(shared, m->nz) : m->pair_zlen[1];
-            ms.push_back(BatchMember{m->geo, m->ph, zlen, pair_buffers(m), m->dt});
+            const int z[2] = {shared > 0 ? std::min(shared, m->nz) : m->pair_zlen[1],
+                              shared > 0 ? std::min(shared, m->nz) : m->pair_zlen[2]};
+            ms.push_back(BatchMember{m->geo, m->ph, {z[0], z[1]}, pair_buffers(m), m->dt});
             b->copies.push_back({m->st_u, m->st_ya});
         } else {
             const int zlen = b->zlen < 0 ? 64 : (b->zlen ? b->zlen : m->plan.zlen);

@@ -278,7 +278,7 @@ hipError_t launch_zero_ints(int* p, int n, hipStream_t s);
 struct BatchMember {
     Geometry g;
     Physics ph;
-    int zlen;
+    int zlen[2];     // of pairs 1 and 2
     PairBuffers b;   // of flip 0; with flip 1 u and unew change places
     double dt;
 };

@@ -1397,7 +1397,7 @@ hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hip
         const Geometry& g = m.g;
         const long long sites = (long long)g.nx * g.nz;
         // (the box form for every member, one-row grids included)
-        for (int pair : {1, 2}) count[pair - 1].push_back(pair_box_blocks(g, sizeof(T), pair, m.zlen));
+        for (int pair : {1, 2}) count[pair - 1].push_back(pair_box_blocks(g, sizeof(T), pair, m.zlen[pair - 1]));
         count[2].push_back((sites + kTotSites - 1) / kTotSites);
         count[3].push_back(predict_blocks(g.nx, g.nz));
     }
@@ -1413,7 +1413,7 @@ hipError_t batch_build_t(BatchTables& t, const std::vector<BatchMember>& ms, hip
                     b.u = b.unew;
                     b.unew = const_cast<void*>(u);
                 }
-                pa[r] = pair_args<T>(ms[r].g, ms[r].ph, ms[r].zlen, pair, b, ms[r].dt);
+                pa[r] = pair_args<T>(ms[r].g, ms[r].ph, ms[r].zlen[pair - 1], pair, b, ms[r].dt);
                 pp[r] = predict_args(ms[r].g, ms[r].ph, pair, b, ms[r].dt);
             }
             off_args[pair - 1][flip] = im.put(pa.data(), n * sizeof(PairArgs<T>));
@@ -1477,7 +1477,7 @@ hipError_t batch_build(BatchTables& t, const std::vector<BatchMember>& ms, int e
     t.nblocks[0] = t.nblocks[1] = 0;
     if (ms.empty()) return hipSuccess;
     for (const auto& m : ms)
-        if (!pair_capable(m.g) || m.zlen < 1 || m.g.lpr != 64) return hipErrorInvalidValue;
+        if (!pair_capable(m.g) || m.zlen[0] < 1 || m.zlen[1] < 1 || m.g.lpr != 64) return hipErrorInvalidValue;
     return esize == 8 ? batch_build_t<double>(t, ms, s) : batch_build_t<float>(t, ms, s);
 }
 

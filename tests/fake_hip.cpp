@@ -250,8 +250,10 @@ int plan_batch_zlen(const std::vector<Geometry>&, int, int) { return 24; }
 // a kernel takes 1 ms where its segments have the best length, longer elsewhere
 static double pair_ms(int pair, int zlen) {
     last_zlen[pair] = zlen;
-    return 1.0 + std::abs(zlen - best_zlen[pair]) / 10.0;
+    return 1.0 + std::abs(zlen - best_zlen[pair]) / (pair == 2 ? 5.0 : 10.0);   // (pair 2 the longer)
 }
+static int zlen_of(const int* z, int pair) { return z[pair - 1]; }
+[[maybe_unused]] static int zlen_of(int z, int) { return z; }
 
 template <typename T>
 hipError_t launch_init(const Geometry&, int, const double*, const double*, const double*, const double*, double,
@@ -383,7 +385,7 @@ hipError_t batch_pair(const BatchTables& t, int pair, int flip, hipStream_t s) {
     const std::vector<BatchMember> ms = batch_members;
     const int esize = t.esize;
     double ms_all = 0;
-    for (const BatchMember& m : ms) ms_all += pair_ms(pair, m.zlen);
+    for (const BatchMember& m : ms) ms_all += pair_ms(pair, zlen_of(m.zlen, pair));
     return launch("batch_pair", s, ms_all, [=] {
         for (const BatchMember& m : ms) pair_kernel(pair, esize, flipped(m.b, flip));
     });

@@ -208,3 +208,14 @@ def test_autotune_tries_the_length_in_force(fake):
     with make(nx=110, nz=300) as g:
         g.set_zlen(47)
         assert g.autotune(1)[0] == 47
+
+
+def test_batch_members_own_plans(fake):
+    """set_zlen(0): each member's own lengths, one for each kernel."""
+    with make(nz=300) as g:
+        b = N.Batch()
+        b.add(g)
+        b.set_zlen(0)
+        b.step(1)
+        assert [fake.fake_last_zlen(p) for p in (1, 2)] == [15, 25]
+        b.close()
