@@ -298,11 +298,13 @@ const char* nuosc_batch_last_error(const nuosc_batch* batch);
  * and capped at each member's nz (0 = each member's own plan; the default is
  * planned for the members).  A common length gives every block of a batched
  * launch the same work.
- * batch_autotune times the batched stages-1+2 kernel for zlen in {16, ..., 256}
- * and both launch forms (trials launches each, the fastest kept; only the
- * RK4 scratch copies are written) and keeps the best pair (the launch form
- * it chose: nuosc_batch_get_launch).  Results do not depend on zlen or the
- * launch form. */
+ * batch_autotune times both batched stage-pair kernels for zlen in {16, ...,
+ * 256}, for the planned length and for what is in force, in both launch forms
+ * (trials launches each, the fastest kept; only the RK4 scratch copies are
+ * written), and takes the best length and form if they are more than 2% faster
+ * than what is in force (the launch form it chose: nuosc_batch_get_launch).
+ * best_zlen, best_ms: the fastest of the listed lengths.  Results do not depend
+ * on zlen or the launch form. */
 int nuosc_batch_set_zlen(nuosc_batch* batch, int zlen);
 int nuosc_batch_autotune(nuosc_batch* batch, int trials, int* best_zlen, double* best_ms);
 /* Launch form of the batched stage-pair kernels: NUOSC_BATCH_GRID (default: one

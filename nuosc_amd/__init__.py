@@ -434,8 +434,9 @@ class Batch:
         self._check(lib().nuosc_batch_set_zlen(self._h, int(zlen)))
 
     def autotune(self, trials=2):
-        """Pick the fastest shared z-segment length and launch form; returns
-        (zlen, stages-1+2 ms); the form chosen is `launch`."""
+        """Pick the fastest shared z-segment length and launch form, unless those
+        in force are as fast; returns the fastest of the listed lengths and its
+        time (both pairs, ms); the form chosen is `launch`."""
         z, ms = C.c_int(), C.c_double()
         self._check(lib().nuosc_batch_autotune(self._h, int(trials), C.byref(z), C.byref(ms)))
         return z.value, ms.value

@@ -1584,10 +1584,12 @@ int nuosc_batch_autotune(nuosc_batch* b, int trials, int* best_zlen, double* bes
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
         return bfail(b, NUOSC_EHIP, "event creation failed");
     const int keep = b->zlen, keep_launch = b->launch;
-    // (z-segment length, launch form) pairs
-    std::vector<std::pair<int, int>> cand;
-    for (int zl : {16, 32, 64, 128, 256})
+    // (z-segment length, launch form): what is in force, the plan for the members,
+    // then the listed lengths
+    std::vector<std::pair<int, int>> cand{{keep, keep_launch}};
+    for (int zl : {-1, 16, 32, 64, 128, 256})
         for (int lf : {NUOSC_BATCH_GRID, NUOSC_BATCH_PERSISTENT}) cand.push_back({zl, lf});
+    const size_t listed = 3;
     std::vector<float> tmin(cand.size(), 1e30f);
     // candidates in turn (tables rebuilt per candidate), trials + 1 rounds,
     // the first a warm-up, so clock drift during the search favours none
@@ -1598,8 +1600,9 @@ int nuosc_batch_autotune(nuosc_batch* b, int trials, int* best_zlen, double* bes
             rc = batch_tables(b);
             if (rc) break;
             (void)hipEventRecord(e0, b->stream);
-            // pair 1 and stages 1-3 write only the RK4 scratch copies and records, never the state
+            // the pairs and stages 1-3 write only the RK4 scratch copies and records, never the state
             hipError_t le = batch_pair(b->tables, 1, 0, b->stream);
+            if (le == hipSuccess) le = batch_pair(b->tables, 2, 0, b->stream);
             if (le == hipSuccess) le = stage_batch_step(b->stages, 3, b->stream);
             (void)hipEventRecord(e1, b->stream);
             if (le != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
@@ -1615,16 +1618,19 @@ int nuosc_batch_autotune(nuosc_batch* b, int trials, int* best_zlen, double* bes
         }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    size_t kb = 0;
-    for (size_t k = 1; k < cand.size(); ++k)
+    size_t kb = 0, kl = listed;   // the fastest, and the fastest of the listed lengths
+    for (size_t k = 1; k < cand.size(); ++k) {
         if (tmin[k] < tmin[kb]) kb = k;
-    b->zlen = rc == NUOSC_OK ? cand[kb].first : keep;
-    b->launch = rc == NUOSC_OK ? cand[kb].second : keep_launch;
+        if (k > listed && tmin[k] < tmin[kl]) kl = k;
+    }
+    if (rc != NUOSC_OK || tmin[kb] > kTuneGain * tmin[0]) kb = 0;
+    b->zlen = cand[kb].first;
+    b->launch = cand[kb].second;
     b->dirty = true;
     batch_drop_graph(b);
     if (rc) return rc;
-    if (best_zlen) *best_zlen = cand[kb].first;
-    if (best_ms) *best_ms = tmin[kb];
+    if (best_zlen) *best_zlen = cand[kl].first;
+    if (best_ms) *best_ms = tmin[kl];
     return NUOSC_OK;
 }
 

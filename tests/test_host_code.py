@@ -210,6 +210,27 @@ def test_autotune_tries_the_length_in_force(fake):
         assert g.autotune(1)[0] == 47
 
 
+# best lengths of the two pair kernels (pair 2 the steeper), length after tuning; planned: 24
+@pytest.mark.parametrize("best,want", [((24, 24), 24), ((16, 64), 64), ((128, 128), 128), ((30, 20), 24)])
+def test_batch_autotune_times_both_pairs(fake, best, want):
+    """The batch is left on the length that is fastest for both kernels together,
+    the planned one included."""
+    for pair in (1, 2):
+        fake.fake_best_zlen(pair, best[pair - 1])
+    sims = [make(nx=20 + k, nz=300, seed=k) for k in range(2)]
+    b = N.Batch()
+    for g in sims:
+        b.add(g)
+    zlen, ms = b.autotune(1)
+    assert zlen in (16, 32, 64, 128, 256) and ms > 0
+    b.step(3)
+    assert [fake.fake_last_zlen(p) for p in (1, 2)] == [want, want]
+    assert [value(g) for g in sims] == [3, 4]
+    b.close()
+    for g in sims:
+        g.close()
+
+
 def test_batch_members_own_plans(fake):
     """set_zlen(0): each member's own lengths, one for each kernel."""
     with make(nz=300) as g:
