@@ -463,8 +463,9 @@ class Batch:
 
 
 def estimate_device_bytes(nv=4, x0=-1.0, x1=1.0, z0=-10.0, z1=10.0, dx=0.1, dz=0.1, precision=PREC_FP64, nflavor=2,
-                          **_):
-    cfg = Config(nn=nv, gx=2, gz=2, x0=x0, x1=x1, z0=z0, z1=z1, dx=dx, dz=dz, precision=precision, nflavor=nflavor)
+                          gx=2, gz=2, bc=BC_PERIODIC, ko_order=3, adv=ADV_CFD4, **_):
+    cfg = Config(nn=nv, gx=gx, gz=gz, x0=x0, x1=x1, z0=z0, z1=z1, dx=dx, dz=dz, precision=precision, bc=bc,
+                 ko_order=ko_order, adv=adv, nflavor=nflavor)
     b = C.c_longlong()
     rc = lib().nuosc_estimate_device_bytes(C.byref(cfg), C.byref(b))
     if rc != 0:

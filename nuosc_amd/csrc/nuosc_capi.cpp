@@ -37,7 +37,7 @@ struct nuosc_sim {
     int nx = 0, nz = 0, nv = 0, nvp = 0, nch = 0;
     int nf = kNVar;                 // fields per site record: 8 (2 flavours) or 18 (3 flavours)
     long long srec = 0, xrow = 0;   // site-record and x-row strides of the state copies (elements)
-    long long state_elems = 0;      // elements allocated for the four copies
+    long long copy_elems = 0;       // elements of a state copy
     double dt = 0, ds_L = 0, ct = 0, st = 0;
     double phy_time = 0;
     double n_nue0[2] = {0, 0};
@@ -108,12 +108,12 @@ void batch_detach(nuosc_batch* b, nuosc_sim* s);
 
 bool is64(const nuosc_sim* s) { return s->cfg.precision == NUOSC_PREC_FP64; }
 
-// Strides of the four state copies (separate allocations, site records of
+// Strides of the state copies (separate allocations, site records of
 // nf nvp elements); ok = false: the x rows one stage block addresses (2
 // flavours: also the moment records; 3 flavours with nx > 1: the z march's
 // block of rows) do not fit 32-bit buffer offsets.
 struct CopyLayout {
-    long long srec, xrow, elems;   // strides and elements allocated for all four copies
+    long long srec, xrow, elems;   // strides and elements of one copy
     bool ok;
 };
 CopyLayout copy_layout(int nx, int nz, int nzs, int nvp, int nch, int esize, int nf) {
@@ -127,7 +127,7 @@ CopyLayout copy_layout(int nx, int nz, int nzs, int nvp, int nch, int esize, int
     gq.xrow = (long long)nzs * gq.srec;
     if (nf == kNVar && !buffer_addressable(gq, esize)) return CopyLayout{0, 0, 0, false};
     if (nf == kNVar3 && !flavor3_addressable(gq, esize)) return CopyLayout{0, 0, 0, false};
-    return CopyLayout{gq.srec, gq.xrow, 4 * copy_elems(gq), true};
+    return CopyLayout{gq.srec, gq.xrow, copy_elems(gq), true};
 }
 
 // Steps in stage pairs: 2 flavours, the default discretisation, unless stage by
@@ -167,6 +167,8 @@ bool steps_in_pairs(const nuosc_config& c, StepKind kind, long long nx, long lon
     if (!f32) return nz >= 8;
     return nz >= (open && nv < 256 ? 32 : 12);
 }
+// State copies: u, yA, yB, and A (w), which FP64 stage pairs do without.
+bool keeps_a(const nuosc_config& c, bool rk4_pairs) { return !(rk4_pairs && c.precision == NUOSC_PREC_FP64); }
 // doubles of the partial moment records (with the spare x row's) and of the
 // partial direction sums, which share one buffer
 long long part_doubles(long long nx, long long nz, long long nv, long long nch, int nf, bool pairs) {
@@ -767,7 +769,7 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
         }
         s->srec = L.srec;
         s->xrow = L.xrow;
-        s->state_elems = L.elems;
+        s->copy_elems = L.elems;
     }
     // nuosc_class.cpp:461-464, nuosc_class.h:120-122
     s->ds_L = c.dx * c.dz / (c.z1 - c.z0) / (c.x1 - c.x0);
@@ -789,7 +791,6 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
     if (hipEventCreate(&s->ev0) != hipSuccess || hipEventCreate(&s->ev1) != hipSuccess)
         return bail(NUOSC_EHIP, "event creation failed");
 
-    const size_t state_bytes = (size_t)s->state_elems * s->esize;
     const bool three = s->nf == kNVar3;
     for (StepKind k : {kRk4, kSrk3}) s->pairs[k] = steps_in_pairs(c, k, s->nx, s->nz);
     const bool pairs = s->pairs[kRk4] || s->pairs[kSrk3];
@@ -797,8 +798,9 @@ int nuosc_create(const nuosc_config* cfg, nuosc_sim** out) {
     const size_t mom_bytes = (size_t)s->nx * s->nz * (three ? kNMom3 : kMomStride) * sizeof(double);
     void** states[4] = {&s->st_u, &s->st_w, &s->st_ya, &s->st_yb};
     {
-        const size_t copy_bytes = state_bytes / 4;
+        const size_t copy_bytes = (size_t)s->copy_elems * s->esize;
         for (void** p : states) {
+            if (p == &s->st_w && !keeps_a(c, s->pairs[kRk4])) continue;
             if (hipMalloc(p, copy_bytes) != hipSuccess) return bail(NUOSC_ENOMEM, "state allocation failed");
             s->device_bytes += (long long)copy_bytes;
             if (hipMemsetAsync(*p, 0, copy_bytes, s->stream) != hipSuccess) return bail(NUOSC_EHIP, "memset failed");
@@ -1646,8 +1648,8 @@ int nuosc_estimate_device_bytes(const nuosc_config* c, long long* bytes) {
     const int nf = c->nflavor == 3 ? kNVar3 : kNVar;
     const CopyLayout L = copy_layout((int)nx, (int)nz, (int)nzs, (int)nvp, (int)nch, esize, nf);
     if (!L.ok) return NUOSC_EINVAL;
-    long long b = L.elems * esize;                                     // u, w, yA, yB
-    const bool pairs = steps_in_pairs(*c, kRk4, nx, nz) || steps_in_pairs(*c, kSrk3, nx, nz);
+    const bool rk4_pairs = steps_in_pairs(*c, kRk4, nx, nz), pairs = rk4_pairs || steps_in_pairs(*c, kSrk3, nx, nz);
+    long long b = L.elems * esize * (keeps_a(*c, rk4_pairs) ? 4 : 3);  // u, w, yA, yB
     b += part_doubles(nx, nz, nv, nch, nf, pairs) * 8;                 // moments: partials, totals
     b += (nf == kNVar3 ? 2ll * kNMom3 : 3ll * kMomStride + (pairs ? kPairRec : 0)) * nx * nz * 8;
     if (pairs && c->bc == NUOSC_BC_OPEN_Z) b += pair_open_doubles(nx, nch, nvp) * 8;   // ghost sites

@@ -240,3 +240,18 @@ def test_batch_members_own_plans(fake):
         b.step(1)
         assert [fake.fake_last_zlen(p) for p in (1, 2)] == [15, 25]
         b.close()
+
+
+@pytest.mark.parametrize("kw,copies", [(dict(), 3), (dict(precision=32), 4), (dict(nx=701, nz=2), 4), (dict(nflavor=3), 4),
+                                       (dict(adv=N.ADV_CFD2), 4), (dict(bc=N.BC_OPEN_Z), 3), (dict(nx=701, nz=6), 3)])
+def test_state_copies(fake, kw, copies):
+    """FP64 stage pairs hold three copies of the state, the others four; the
+    estimate says so too."""
+    with make(**kw) as g:
+        es, fields = g.precision // 8, g.nvar
+        nvp = -(-g.nv * es // 128) * 128 // es
+        copy = (g.nx + 7) * (g.nz + (4 if "bc" in kw else 0)) * fields * nvp * es
+        assert copies * copy < g.device_bytes() < (copies + 0.5) * copy
+        est = N.estimate_device_bytes(nv=2, x0=-g.nx * H / 2, x1=g.nx * H / 2, z0=-g.nz * H / 2, z1=g.nz * H / 2, dx=H,
+                                      dz=H, **kw)
+        assert g.device_bytes() <= est < g.device_bytes() + (1 << 20)
