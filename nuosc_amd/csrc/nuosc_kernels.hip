@@ -700,7 +700,7 @@ __device__ __forceinline__ void stage_body(const StageArgs<T>& a, int lblock, in
                 yout.stv(bo, f, yo[f], vos, so);
             }
         }
-        if constexpr (STAGE != 0) {
+        if constexpr (STAGE != 0) {   // (never with NOX)
             // moment terms of the lane's V directions, summed per lane first
             // (exactly, with the rounding error carried, in the FP32 form)
             double t[16], te[16];
@@ -750,11 +750,9 @@ __device__ __forceinline__ void stage_body(const StageArgs<T>& a, int lblock, in
                 __builtin_amdgcn_make_buffer_rsrc((void*)bp, 0, (int)a.mpart_bytes, kRsrcWord3);
             const int sv = dl >> sh;                       // value index 0..15
             const bool used = sv < kNMom;
-            // (NOX: row groups past the last chunk write the spare row's records)
-            const bool rec_ok = row_ok && used && (!NOX || ch < nch);
+            const bool rec_ok = row_ok && used;
             const unsigned rec =
-                ((unsigned)((rec_ok ? r : nx) - ib) * (unsigned)nz * nch + (unsigned)(NOX ? min(ch, nch - 1) : ch)) *
-                (kMomRec * 8);
+                ((unsigned)((rec_ok ? r : nx) - ib) * (unsigned)nz * nch + (unsigned)ch) * (kMomRec * 8);
             const unsigned srec = (mbase + j) * (unsigned)(nch * kMomRec * 8);
             Lane<double>::st(tot, rp, rec + (unsigned)(used ? sv : sv - kNMom) * 8, srec);
         }
