@@ -233,3 +233,29 @@ def test_member_of_one_batch_only(nuosc_mod):
     b3 = N.Batch(precision=64)
     b3.add(g)
     g.close()
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+def test_members_stepped_alone_between(nuosc_mod, precision):
+    """A member that steps alone between batch steps has exchanged its state
+    copies an odd or even number of times since the tables were built: the batch
+    goes on from its state, not from the other copy."""
+    N = nuosc_mod
+    alone = [make(N, c, 500 + k, precision) for k, c in enumerate(RUNS)]
+    mixed = [make(N, c, 500 + k, precision) for k, c in enumerate(RUNS)]
+    b = N.Batch(precision=precision)
+    for g in mixed:
+        b.add(g)
+    for nbatch, who, n in ((1, 0, 1), (3, 1, 2), (2, 2, 3), (1, 3, 1), (2, 0, 1)):
+        b.step(nbatch)
+        mixed[who].step_rk4(n)
+        mixed[who].analysis()
+        for g in alone:
+            g.step_rk4(nbatch)
+        alone[who].step_rk4(n)
+    b.step(2)
+    for k, (a, m) in enumerate(zip(alone, mixed)):
+        a.step_rk4(2)
+        assert np.array_equal(a.get_state(), m.get_state()), k
+        assert a.phy_time == m.phy_time
+    b.close()

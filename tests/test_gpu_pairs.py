@@ -186,3 +186,28 @@ def test_autotuned_steps_bitwise(nuosc_mod, precision):
         runs.append(g.get_state())
     for r in runs[1:]:
         assert np.array_equal(r, runs[0])
+
+
+@pytest.mark.parametrize("shape", [(1, 40, 2, 7), (5, 33, 3, 0), (9, 20, 2, 5)])
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("scheme", ["rk4", "srk3"])
+def test_open_renormalised_pairs_match_oracle(nuosc_mod, oracle_mod, shape, precision, scheme):
+    """Open z with renormalisation in every step: the new state is renormalised
+    after its sums were formed, and its ghost sites follow.  Tolerances of
+    test_open_pairs_match_oracle, one more rounding a step."""
+    nx, nz, nn, zlen = shape
+    zc = -nz * H / 2 - 0.3
+    init = dict(ipt=0, alpha=0.85, eps0=0.3, sigma=0.5, lnue=0.6, lnueb=0.5)
+    g = nuosc_mod.NuOsc(nv=nn, CFL=0.4, bc=nuosc_mod.BC_OPEN_Z, zc=zc, precision=precision, renorm=True, **geo(nx, nz), **PHYS)
+    o = oracle_mod.OracleSim(nn=nn, cfl=0.4, bc=1, zc=zc, renorm=1, **geo(nx, nz), **PHYS)
+    g.fillInitValue(**init)
+    o.fill_init(**init)
+    if zlen:
+        g.set_zlen(zlen)
+    for n in (1, 2, 6):
+        (g.step_rk4 if scheme == "rk4" else g.step_srk3)(n)
+        (o.step if scheme == "rk4" else o.step_srk3)(n)
+    a, b = g.get_state(), o.get_state()
+    tol = 1e-12 if precision == 64 else 9 * 19 * 2.0 ** -24 * 2
+    for f in range(8):
+        assert np.max(np.abs(a[f] - b[f])) <= tol * np.max(np.abs(b[:4] if f < 4 else b[4:])), f

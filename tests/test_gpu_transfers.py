@@ -53,3 +53,26 @@ def test_threads(nuosc_mod):
     for t in ts:
         t.join()
     assert not bad
+
+
+def test_more_transfers_than_slots(nuosc_mod):
+    """Four handles with states of 57 MB, eight slots each of the sixteen there
+    are: the later ones wait for a slot."""
+    sims = [make(nuosc_mod, 60, 60 + k, 5) for k in range(4)]
+    bad = []
+
+    def work(k):
+        rng = np.random.default_rng(k)
+        for _ in range(3):
+            a = rng.normal(size=(8, *sims[k].shape))
+            assert a.nbytes >= 32 << 20
+            sims[k].set_state(a)
+            if not np.array_equal(sims[k].get_state(), a):
+                bad.append(k)
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
