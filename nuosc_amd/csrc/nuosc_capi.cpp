@@ -1589,34 +1589,51 @@ int nuosc_batch_autotune(nuosc_batch* b, int trials, int* best_zlen, double* bes
     // (z-segment length, launch form): what is in force, the plan for the members,
     // then the listed lengths
     std::vector<std::pair<int, int>> cand{{keep, keep_launch}};
-    for (int zl : {-1, 16, 32, 64, 128, 256})
+    for (int lf : {NUOSC_BATCH_GRID, NUOSC_BATCH_PERSISTENT})
+        if (cand[0] != std::make_pair(-1, lf)) cand.push_back({-1, lf});
+    const size_t listed = cand.size();
+    for (int zl : {16, 32, 64, 128, 256})
         for (int lf : {NUOSC_BATCH_GRID, NUOSC_BATCH_PERSISTENT}) cand.push_back({zl, lf});
-    const size_t listed = 3;
     std::vector<float> tmin(cand.size(), 1e30f);
-    // candidates in turn (tables rebuilt per candidate), trials + 1 rounds,
-    // the first a warm-up, so clock drift during the search favours none
-    for (int t = 0; t < trials + 1 && rc == NUOSC_OK; ++t)
-        for (size_t k = 0; k < cand.size() && rc == NUOSC_OK; ++k) {
+    // time of a pair kernel of the tables as they are (pair 2: with stages 1-3 of
+    // the members that step stage by stage); all of these write only the RK4
+    // scratch copies and records, never the state
+    auto kernel_ms = [&](int pair) {
+        (void)hipEventRecord(e0, b->stream);
+        hipError_t le = batch_pair(b->tables, pair, 0, b->stream);
+        if (le == hipSuccess && pair == 2) le = stage_batch_step(b->stages, 3, b->stream);
+        (void)hipEventRecord(e1, b->stream);
+        float ms = 0;
+        if (le != hipSuccess || hipEventSynchronize(e1) != hipSuccess) rc = bfail(b, NUOSC_EHIP, "autotune launch failed");
+        else if (hipEventElapsedTime(&ms, e0, e1) != hipSuccess) rc = bfail(b, NUOSC_EHIP, "autotune timing failed");
+        return ms;
+    };
+    // Candidates in turn (tables rebuilt per candidate) for trials rounds, what is
+    // in force first (once before that to warm up) and last, so clock drift
+    // favours none.  The longer kernel alone leaves out what is 5% behind, and the
+    // persistent form of a length whose ordinary grid is.
+    std::vector<char> out(cand.size(), 0);
+    float least = 1e30f, least_listed = 1e30f;   // of pair 2
+    for (int t = 0; t <= trials && rc == NUOSC_OK; ++t)
+        for (size_t k = 0; k < (t < trials ? cand.size() : 1) && rc == NUOSC_OK; ++k) {
+            if (out[k] || (k > listed && cand[k].first == cand[k - 1].first && out[k - 1])) continue;
             b->zlen = cand[k].first;
             b->launch = cand[k].second;
             rc = batch_tables(b);
+            if (rc == NUOSC_OK && t == 0 && k == 0) {
+                kernel_ms(1);
+                if (rc == NUOSC_OK) kernel_ms(2);
+            }
             if (rc) break;
-            (void)hipEventRecord(e0, b->stream);
-            // the pairs and stages 1-3 write only the RK4 scratch copies and records, never the state
-            hipError_t le = batch_pair(b->tables, 1, 0, b->stream);
-            if (le == hipSuccess) le = batch_pair(b->tables, 2, 0, b->stream);
-            if (le == hipSuccess) le = stage_batch_step(b->stages, 3, b->stream);
-            (void)hipEventRecord(e1, b->stream);
-            if (le != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
-                rc = bfail(b, NUOSC_EHIP, "autotune launch failed");
-                break;
+            const float ms2 = kernel_ms(2);
+            if (rc) break;
+            if (t == 0 && k > 0 && ms2 > 1.05f * least && (k < listed || ms2 > least_listed)) {
+                out[k] = 1;
+                continue;
             }
-            float ms = 0;
-            if (hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-                rc = bfail(b, NUOSC_EHIP, "autotune timing failed");
-                break;
-            }
-            if (t > 0) tmin[k] = std::min(tmin[k], ms);
+            least = std::min(least, ms2);
+            if (k >= listed) least_listed = std::min(least_listed, ms2);
+            tmin[k] = std::min(tmin[k], ms2 + kernel_ms(1));
         }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
