@@ -548,7 +548,7 @@ def batched_leg(N, a, runs=64, steps=20):
     aggregate updates/s stepped all together (at the autotuned z-segment
     length and launch form; the other launch form is timed too) and one
     after another, and each mode's HBM fraction at 224 B per FP32 update
-    (12 passes x 8 fields)."""
+    (7 passes x 8 fields)."""
     import numpy as np
     rng = np.random.default_rng(7)
     specs = [scan_run(rng, k) for k in range(runs)]

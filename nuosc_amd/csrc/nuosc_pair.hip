@@ -17,11 +17,11 @@
 //   pair 1: read u     -> Y2 (on chip) -> Y3
 //   pair 2: read Y3, u -> Y4 (on chip) -> u' = (2 Y3 + Y4)/3 + dt/6 (k1 + k4)
 // 2 + 3 = 5 passes (320 B per update instead of 768; 512 x 512 x 642: 28.9 ms
-// a step stage by stage, 19.3 in 7 passes, 18.1 in 5).  Pair 1 takes 6.8 ms (25
-// GB moved, 3.7 TB/s), pair 2 10.8 (38 GB); with every load from one z and
-// nothing stored they take 5.4 and 9.0, so pair 2 is bound by issuing its
-// instructions at 2 waves per SIMD and memory adds a part.  FP32 takes 4.9 and
-// 5.2 ms, 3.9 each without memory traffic: a third k in pair 2 would cost more
+// a step stage by stage, 19.3 in 7 passes, 17.8 in 5).  Pair 1 takes 6.7 ms (25
+// GB moved, 3.8 TB/s), pair 2 10.7 (38-40 GB); with every load from one z and
+// nothing stored they take 5.7 and 9.1, so pair 2 is bound by issuing its
+// instructions at 2 waves per SIMD and memory adds a part.  FP32 takes 4.8 and
+// 5.1 ms, 3.9 each without memory traffic: a third k in pair 2 would cost more
 // than the 2 passes, so there A is kept.  An SSP-RK3 step is a pair and a single stage, 2 + 3 = 5 passes instead of 8:
 //   pair 3: read u       -> u1 = u + dt k (on chip) -> u2 = 3/4 u + 1/4 (u1 + dt k)
 //   k_lone: read u2, u   -> u' = 1/3 u + 2/3 (u2 + dt k)
